@@ -258,7 +258,10 @@ int pdp3_density(pdp3_ctx *ctx, int index, double *out);
  * FP64 form has one shape.  pdp3_autotune runs steps_per_candidate real steps
  * of the simulation with each shape, times the plasma kernel and keeps the
  * fastest (the steps advance the simulation; results differ between shapes
- * only by the order of FP64 sums). */
+ * only by the order of FP64 sums).  Until one of the two is called, each
+ * species runs on the shape that suits its size (down to 256 particles per
+ * block, smaller than the shapes that can be set) and pdp3_get_tile returns
+ * 16 x 4. */
 int pdp3_set_tile(pdp3_ctx *ctx, int ppt, int waves);
 int pdp3_get_tile(const pdp3_ctx *ctx, int *ppt, int *waves);
 int pdp3_autotune(pdp3_ctx *ctx, int steps_per_candidate, int *ppt, int *waves);

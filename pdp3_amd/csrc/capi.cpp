@@ -1053,6 +1053,7 @@ int pdp3_set_tile(pdp3_ctx *ctx, int ppt, int waves) {
   for (int t = 0; t < kNumTiles; t++)
     if (kTileShapes[t][0] == ppt && kTileShapes[t][1] == waves) {
       ctx->c.tile = t;
+      ctx->c.tile_auto = false;
       return PDP3_OK;
     }
   return fail(ctx, PDP3_ERR_BAD_ARG, "unsupported tile shape");
@@ -1074,6 +1075,7 @@ int pdp3_autotune(pdp3_ctx *ctx, int steps_per_candidate, int *ppt, int *waves) 
   KernelTimer saved = c.timers[PDP3_KERNEL_PARTICLES];
   int st, best = 0;
   double best_ms = 1e300;
+  c.tile_auto = false;
   for (int t = 0; t < kNumTiles; t++) {
     c.tile = t;
     c.profiling = true;

@@ -76,6 +76,34 @@ __host__ __device__ __forceinline__ long long logical_of(long long p) {
 constexpr int kNumTiles = 6;
 constexpr int kTileShapes[kNumTiles][2] = {{16, 4}, {16, 2}, {16, 1}, {8, 4}, {8, 2}, {4, 4}};
 
+// Which slots of a chunked species a block of WAVES wavefronts walks with PPT
+// particles per lane.  A tile is kParticles consecutive logical particles: a
+// whole number of chunks, or, where that is less than a chunk, the kGroup
+// neighbouring lanes of one chunk in all kPPT iterations (thread t takes lane
+// t % kGroup and iterations t / kGroup * PPT ..), so that a small tile still
+// covers one run of cells and reads kGroup contiguous slots at a time.
+template <int PPT, int WAVES>
+struct TileMap {
+  static constexpr int kParticles = WAVES * 64 * PPT;
+  static constexpr bool kWhole = kParticles >= kChunk;
+  static constexpr int kGroup = kWhole ? 64 : kParticles / kPPT;
+  // slots from the tile's first one that its threads may reach
+  static constexpr int kSpan = kWhole ? kParticles : kChunk;
+  // slot of the tile's last logical particle, from its first slot
+  static constexpr int kLast = kWhole ? kParticles - 1 : (kPPT - 1) * 64 + kGroup - 1;
+  static_assert(kPPT % PPT == 0 && (kWhole ? kParticles % kChunk == 0 : kChunk % kParticles == 0), "tile shape");
+  __device__ __forceinline__ static long long base(long long tile) {
+    if (kWhole) return tile * kParticles;
+    constexpr int kPer = kWhole ? 1 : kChunk / kParticles;
+    return tile / kPer * kChunk + tile % kPer * kGroup;
+  }
+  // the thread's first slot, from the tile's
+  __device__ __forceinline__ static unsigned first(unsigned t) {
+    constexpr unsigned kTeam = kGroup * (kPPT / PPT);  // threads that share a chunk's lanes
+    return t / kTeam * kChunk + t % kTeam / kGroup * (PPT * 64) + t % kGroup;
+  }
+};
+
 // alive byte of the FP64 state: 0 dead, 1 alive, 2 padding slot
 constexpr uint8_t kPadSlot = 2;
 // FP32 cell word of a padding slot (a dead particle's word never equals it)
@@ -149,8 +177,10 @@ struct Ctx {
   bool profiling = false;
   KernelTimer timers[5];
   int sort_interval = 0;
-  // tile shape of the FP32 particle kernel (index into kTileShapes)
+  // tile shape of the FP32 particle kernel (index into kTileShapes); until it
+  // is set or autotuned each species runs on the shape that suits its size
   int tile = 0;
+  bool tile_auto = true;
   long long steps_done = 0;
   // sort workspace
   int32_t *sort_keys = nullptr;
@@ -251,6 +281,7 @@ void launch_bunch_inject_f64(Ctx &c, Species &sp, unsigned start, unsigned count
 
 // FP32 form
 void launch_fused_f32(Ctx &c, Species &sp);
+int auto_tile(const Ctx &c, const Species &sp);  // kTileShapes index, or 6 / 7: 2 / 1 particles per lane x 4
 void launch_charge_weighting_f32(Ctx &c, Species &sp, double *rho = nullptr);
 void launch_bunch_inject_f32(Ctx &c, Species &sp, unsigned start, unsigned count, double dl);
 bool launch_f32_from_f64(Ctx &c, Species &sp);  // pack absolute FP64 state into cell form

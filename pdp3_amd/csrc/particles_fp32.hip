@@ -68,6 +68,18 @@ __device__ __forceinline__ const double *field(const F32Args &p, int c) {
   return p.grid + (size_t)c * ((size_t)p.nr * (size_t)p.nz);
 }
 
+// the element at byte offset `off` from p: a 32-bit offset from a
+// uniform base is one VGPR and scalar-base addressing, where an element index
+// would be widened to a 64-bit address per array
+template <class T>
+__device__ __forceinline__ T &at(T *p, unsigned off) {
+  return *reinterpret_cast<T *>(reinterpret_cast<char *>(p) + off);
+}
+template <class T>
+__device__ __forceinline__ const T &at(const T *p, unsigned off) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + off);
+}
+
 // radial weights of the four-node gathers (src/eField.cpp:204-316,
 // src/hField.cpp:159-267) in cell units.  "lo" family (E_r, H_z, H_phi):
 // staggered index from r - dr/2; otherwise (E_phi, E_z, H_r) the particle's
@@ -114,8 +126,20 @@ __device__ __forceinline__ AxW ax_half(int k, float b) {
   return AxW{down ? k - 1 : k, down ? b + 0.5f : b - 0.5f};
 }
 
+// the four-node interpolation, its multiply-adds written out so that every
+// field source rounds alike however its code is compiled; HZ: the order H_z
+// is interpolated in
+template <bool HZ = false>
+__device__ __forceinline__ float stencil(float f00, float f01, float f10, float f11, RadW rw, AxW aw) {
+  const float b = aw.b, ob = 1.f - aw.b;
+  const float t0 = fmaf(f00, ob, f01 * b);
+  if (HZ) return fmaf(rw.B, fmaf(f11, b, f10 * ob), t0 * rw.A);
+  return fmaf(rw.A, t0, fmaf(f10, ob, f11 * b) * rw.B);
+}
+
 // node values are rounded to FP32 and multiplied by the push's scale s
 // (escale for E, bscale for H) before the interpolation
+template <bool HZ = false>
 __device__ __forceinline__ float gather(const F32Args &p, const double *__restrict__ F, float s, RadW rw, AxW aw) {
   int ir = rw.ir, kz = aw.kz;
   if (ir > p.nr - 2 || kz > p.nz - 2) {
@@ -126,8 +150,7 @@ __device__ __forceinline__ float gather(const F32Args &p, const double *__restri
   const double *row0 = F + (size_t)ir * (size_t)p.nz + kz;
   const double *row1 = row0 + p.nz;
   float f00 = (float)row0[0] * s, f01 = (float)row0[1] * s, f10 = (float)row1[0] * s, f11 = (float)row1[1] * s;
-  float b = aw.b, ob = 1.f - aw.b;
-  return (f00 * ob + f01 * b) * rw.A + (f10 * ob + f11 * b) * rw.B;
+  return stencil<HZ>(f00, f01, f10, f11, rw, aw);
 }
 
 // field sources of the push.  GlobalFields reads the six FP64 components
@@ -164,30 +187,34 @@ struct GlobalFields {
   }
 };
 
-// rows bi..bi+kFR-1, columns bk..bk+kFK-1 of the six components, anchored two
-// rows and two columns below the tile's anchor cell (ai, ak): a particle in
-// cell (i, k) reads rows i-1..i+1 and columns k-1..k+1, so every cell with
-// i in [ai-1, ai+1] and k in [ak-1, ak+kFK-4] is served from the box (a
+// rows bi..bi+kFR-1, columns bk..bk+width-1 of the six components, anchored
+// two rows and two columns below the tile's anchor cell (ai, ak): a particle
+// in cell (i, k) reads rows i-1..i+1 and columns k-1..k+1, so every cell with
+// i in [ai-1, ai+1] and k in [ak-1, ak+width-4] is served from the box (a
 // sorted tile lies along row ai; between sorts some of its particles have
-// moved to the rows next to it, or to the column before its first).  Each
-// entry is a pair (node k, node k+1) of its row, so that the four nodes of
-// one component's stencil are two 8-byte entries kFK apart (one LDS
-// instruction) and the six components differ only by a constant offset.
-constexpr int kFR = 5, kFK = 64, kFComp = 6, kFSize = kFComp * kFR * kFK;
+// moved to the rows next to it, or to the column before its first).  width is
+// kFK, or half of it for a tile that ends within the first half.  (With 64
+// columns a 4096-particle tile overran the box below 66 particles per cell and
+// its other particles gathered from HBM: the kernel on 4096-particle tiles at
+// 40 per cell took 338 us for 2.1e7 particles, with 128 columns 238 us.)
+// Components with the same stencil are stored together: {E_r, H_z} and
+// {E_z, H_r} as pairs, E_phi and H_phi alone, so that a stencil is four
+// addresses and eight LDS reads.
+constexpr int kFR = 5, kFK = 128, kFComp = 6, kFPlane = kFR * kFK;
 constexpr int kFBelow = 2;  // box rows and columns below the anchor cell
-// the LDS array (floats): the field box (two floats per entry), then two
+// the LDS array (floats): {E_r, H_z}, {E_z, H_r}, E_phi, H_phi, then two
 // float4 row entries for each box row
-constexpr int kFBoxFloats = 2 * kFSize + 8 * kFR;
+constexpr int kFErHz = 0, kFEzHr = 2 * kFPlane, kFEphi = 4 * kFPlane, kFHphi = 5 * kFPlane, kFRows = 6 * kFPlane;
+constexpr int kFBoxFloats = kFRows + 8 * kFR;
 
-__device__ __forceinline__ float gather_box(const float2 *e, RadW rw, AxW aw) {
-  const float2 lo = e[0], hi = e[kFK];
-  float b = aw.b, ob = 1.f - aw.b;
-  return (lo.x * ob + lo.y * b) * rw.A + (hi.x * ob + hi.y * b) * rw.B;
+__device__ __forceinline__ float gather_box(const float *e, RadW rw, AxW aw) {
+  return stencil(e[0], e[1], e[kFK], e[kFK + 1], rw, aw);
 }
 
 struct BoxFields {
-  const float *box;  // LDS, kFComp x kFR x kFK pairs, then the row entries of rows ai-2 .. ai+2
+  const float *box;  // LDS
   int ai, ak;        // anchor cell of the tile
+  int width;         // columns filled
   // the box's row entries (an LDS read for every particle), replaced by the
   // entries evaluated in place for a row outside the box.  A global load here
   // would make the read a flat load, whose wait also waits for the next
@@ -195,7 +222,7 @@ struct BoxFields {
   __device__ __forceinline__ void row(const F32Args &p, int i, float4 &t0, float4 &t1) const {
     const int li = i - ai + kFBelow;
     const int lc = min(max(li, 0), kFR - 1);
-    const float4 *t = reinterpret_cast<const float4 *>(box + 2 * kFSize);
+    const float4 *t = reinterpret_cast<const float4 *>(box + kFRows);
     t0 = t[2 * lc];
     t1 = t[2 * lc + 1];
     if ((unsigned)li >= (unsigned)kFR) row_entries(min(max(i, 0), p.nr - 1), t0, t1);
@@ -203,20 +230,21 @@ struct BoxFields {
   __device__ __forceinline__ void get(const F32Args &p, int i, int k, RadW rl, RadW ro, AxW zo, AxW zh, float e[3],
                                       float h[3]) const {
     const bool inbox = (unsigned)(i - ai + kFBelow - 1) < (unsigned)(kFR - 2) &&
-                       (unsigned)(k - ak + kFBelow - 1) < (unsigned)(kFK - 2) && i <= p.nr - 2 && k <= p.nz - 2;
+                       (unsigned)(k - ak + kFBelow - 1) < (unsigned)(width - 2) && i <= p.nr - 2 && k <= p.nz - 2;
     if (inbox) {
       const int bi = ai - kFBelow, bk = ak - kFBelow;
-      constexpr int C = kFR * kFK;
-      const float2 *f = reinterpret_cast<const float2 *>(box);
       // the stencil's first entry for each (radial, axial) weight pair
       const int rlo = (rl.ir - bi) * kFK, roo = (ro.ir - bi) * kFK, zoo = zo.kz - bk, zho = zh.kz - bk;
-      const float2 *lo_o = f + (rlo + zoo), *oo_o = f + (roo + zoo), *oo_h = f + (roo + zho), *lo_h = f + (rlo + zho);
-      const float e0 = gather_box(lo_o + 0 * C, rl, zo);
-      const float e1 = gather_box(oo_o + 1 * C, ro, zo);
-      const float e2 = gather_box(oo_h + 2 * C, ro, zh);
-      const float h0 = gather_box(oo_h + 3 * C, ro, zh);
-      const float h1 = gather_box(lo_h + 4 * C, rl, zh);
-      const float h2 = gather_box(lo_o + 5 * C, rl, zo);
+      const float2 *erhz = reinterpret_cast<const float2 *>(box + kFErHz) + (rlo + zoo);
+      const float2 *ezhr = reinterpret_cast<const float2 *>(box + kFEzHr) + (roo + zho);
+      const float2 p00 = erhz[0], p01 = erhz[1], p10 = erhz[kFK], p11 = erhz[kFK + 1];
+      const float e0 = stencil(p00.x, p01.x, p10.x, p11.x, rl, zo);
+      const float h2 = stencil<true>(p00.y, p01.y, p10.y, p11.y, rl, zo);
+      const float e1 = gather_box(box + kFEphi + (roo + zoo), ro, zo);
+      const float2 q00 = ezhr[0], q01 = ezhr[1], q10 = ezhr[kFK], q11 = ezhr[kFK + 1];
+      const float e2 = stencil(q00.x, q01.x, q10.x, q11.x, ro, zh);
+      const float h0 = stencil(q00.y, q01.y, q10.y, q11.y, ro, zh);
+      const float h1 = gather_box(box + kFHphi + (rlo + zho), rl, zh);
       e[0] = e0; e[1] = e1; e[2] = e2;
       h[0] = h0; h[1] = h1; h[2] = h2;
     } else {
@@ -225,38 +253,48 @@ struct BoxFields {
       const float e2 = gather(p, field(p, kEZ), p.escale, ro, zh);
       const float h0 = gather(p, field(p, kHHR), p.bscale, ro, zh);
       const float h1 = gather(p, field(p, kHHPhi), p.bscale, rl, zh);
-      const float h2 = gather(p, field(p, kHHZ), p.bscale, rl, zo);
+      const float h2 = gather<true>(p, field(p, kHHZ), p.bscale, rl, zo);
       e[0] = e0; e[1] = e1; e[2] = e2;
       h[0] = h0; h[1] = h1; h[2] = h2;
     }
   }
 };
 
-// block prologue: fill the field box (nodes outside the grid read as 0; no
-// particle that the box serves reads them, nor the second half of a row's
-// last entry)
-__device__ __forceinline__ void field_box_fill(const F32Args &p, float *box, int ai, int ak) {
+// block prologue: fill the field box's first `width` columns (nodes outside
+// the grid hold the nearest node's value; no particle that the box serves
+// reads them).  One wavefront per 64 columns of a box row of one component,
+// the kFComp * kFR rows dealt out evenly; a wave's loads are all in flight
+// before the first is used (a branch or a use between them had made the
+// prologue a chain of load latencies).
+template <int WAVES>
+__device__ __forceinline__ void field_box_fill(const F32Args &p, float *box, int ai, int ak, int width) {
   const int bi = ai - kFBelow, bk = ak - kFBelow;
   if (threadIdx.x < 2 * kFR) {
     const int r = min(max(bi + (int)(threadIdx.x >> 1), 0), p.nr - 1);
-    reinterpret_cast<float4 *>(box + 2 * kFSize)[threadIdx.x] = p.rows[2 * r + (threadIdx.x & 1)];
+    reinterpret_cast<float4 *>(box + kFRows)[threadIdx.x] = p.rows[2 * r + (threadIdx.x & 1)];
   }
-  const double *src[kFComp] = {field(p, kER), field(p, kEPhi), field(p, kEZ), field(p, kHHR), field(p, kHHPhi),
-                               field(p, kHHZ)};
-  float2 *f = reinterpret_cast<float2 *>(box);
+  constexpr int kLines = kFComp * kFR, kBatch = 8;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  for (int col = threadIdx.x & 63; col < width; col += 64) {
+    const unsigned gk = min(max(bk + col, 0), p.nz - 1);
+    for (int t0 = wave; t0 < kLines; t0 += WAVES * kBatch) {
+      double v[kBatch];
 #pragma unroll
-  for (int comp = 0; comp < kFComp; comp++) {
-    const double *F = src[comp];
-    const float sc = comp < 3 ? p.escale : p.bscale;
-    // one wavefront per box row (kFK = 64 columns): each node is loaded once
-    // and the next column's value comes from the next lane
-    for (int t = threadIdx.x; t < kFR * kFK; t += blockDim.x) {
-      const int r = t / kFK, col = t - r * kFK;
-      const int gi = bi + r, gk = bk + col;
-      float v0 = 0.f;
-      if ((unsigned)gi < (unsigned)p.nr && (unsigned)gk < (unsigned)p.nz) v0 = (float)F[(size_t)gi * p.nz + gk] * sc;
-      const float v1 = __shfl_down(v0, 1);  // lane 63 (the row's last entry) gets its own value: never read
-      f[comp * kFR * kFK + t] = make_float2(v0, v1);
+      for (int u = 0; u < kBatch; u++) {
+        const int line = min(t0 + u * WAVES, kLines - 1), comp = line / kFR;
+        const int gi = min(max(bi + line - comp * kFR, 0), p.nr - 1);
+        // kHHR .. kHHZ are components 6 .. 8 of the grid
+        v[u] = at(field(p, comp < 3 ? comp : comp + 3) + (size_t)gi * p.nz, gk * 8u);
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; u++) {
+        const int line = t0 + u * WAVES, comp = line / kFR, row = line - comp * kFR;
+        if (line >= kLines) break;
+        // E_r, E_phi, E_z, H_r, H_phi, H_z
+        const int plane = comp == 0 ? kFErHz : comp == 1 ? kFEphi : comp == 2 ? kFEzHr : comp == 3 ? kFEzHr + 1 : comp == 4 ? kFHphi : kFErHz + 1;
+        const int step = comp == 1 || comp == 4 ? 1 : 2;
+        box[plane + (row * kFK + col) * step] = (float)v[u] * (comp < 3 ? p.escale : p.bscale);
+      }
     }
   }
 }
@@ -293,7 +331,7 @@ __device__ __forceinline__ void vay_u(const F32Args &p, const float e[3], const 
   float alpha = 1.f + dot3f(up, up) * p.inv_c2;  // gamma'^2
   float B2 = dot3f(b, b);
   float s = alpha - B2;
-  float ub = dot3f(up, b);
+  const float ub = fmaf(up[2], b[2], fmaf(up[1], b[1], up[0] * b[0]));
   float us2 = ub * ub;
   float ig = frsq(0.5f * (s + fsqrt(s * s + 4.f * (B2 + us2))));  // 1/gamma^{n+1}
   for (int j = 0; j < 3; j++) b[j] *= ig;
@@ -544,18 +582,6 @@ struct PState {
   float a, b, u0, u1, u2, w;
 };
 
-// the 4-byte element at byte offset `off` from p: a 32-bit offset from a
-// uniform base is one VGPR and scalar-base addressing, where an element index
-// would be widened to a 64-bit address per array
-template <class T>
-__device__ __forceinline__ T &at(T *p, unsigned off) {
-  return *reinterpret_cast<T *>(reinterpret_cast<char *>(p) + off);
-}
-template <class T>
-__device__ __forceinline__ const T &at(const T *p, unsigned off) {
-  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + off);
-}
-
 __device__ __forceinline__ PState load_state(const F32Args &p, unsigned off) {
   PState s;
   // streaming (non-temporal) loads and stores: each slot is touched once per
@@ -689,16 +715,20 @@ __device__ __forceinline__ F32Args from_slot(const F32Args &p, long long base) {
   return q;
 }
 
-// one tile of a cell-sorted (chunked) species: CB = WAVES * PPT / kPPT chunks
-// starting at slot `base`.  Wave w takes chunk w / (kPPT / PPT) and, in it,
-// the slots of iterations j0 .. j0+PPT-1, j0 = (w % (kPPT / PPT)) * PPT: its
-// lanes read contiguous slots (coalesced) and lane L walks the consecutive
-// logical particles L*kPPT+j0 .. L*kPPT+j0+PPT-1, mostly of one cell.
-template <int PPT, int WAVES>
+// one tile of a cell-sorted (chunked) species from slot `base` (TileMap): its
+// lanes read contiguous slots (coalesced) and each walks PPT consecutive
+// logical particles, mostly of one cell.
+template <int PPT, int WAVES, class Sink>
 __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink &gs, long long base, long long n_cap,
                                              double *box, float *fbox) {
-  static_assert(kFK == 64, "one wavefront per field box row");
-  static_assert(kPPT % PPT == 0 && (WAVES * PPT) % kPPT == 0, "tile shape");
+  static_assert(kFK == Sink::kK, "the two boxes share their width");
+  using Map = TileMap<PPT, WAVES>;
+  const F32Args q = from_slot(p, base);
+  const unsigned lim = (unsigned)min(n_cap - base, (long long)Map::kSpan);
+  const unsigned off0 = Map::first(threadIdx.x);
+  // the lane's first particle is on its way while the boxes are set up
+  PState nx{kDead, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (off0 < lim) nx = load_state_next(q, off0 * 4u);
   // anchor samples: slot base + j is the logical particle 16 j of a plasma
   // tile (the chunk-transposed layout), particle j of an ensemble's bunch block
   int ai, ak;
@@ -714,23 +744,20 @@ __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink 
     }
     tile_anchor(live, ri, kk, ai, ak);
   }
-  TileSink sk;
-  box_init(box, ai, ak, sk, gs);
-  field_box_fill(p, fbox, ai, ak);
+  // the boxes' width: half of it when the tile's last particle (the last
+  // slot its threads reach) lies within the first half of the anchor's row,
+  // with one column to spare
+  const uint32_t cl = base + Map::kLast < n_cap ? p.cell[base + Map::kLast] : kDead;
+  const bool narrow = !(cl & kDead) && cell_i(cl) == ai && cell_k(cl) - ak <= kFK / 2 - 5;
+  const int width = narrow ? kFK / 2 : kFK;
+  Sink sk;
+  box_init(box, ai, ak, width, sk, gs);
+  field_box_fill<WAVES>(p, fbox, ai, ak, width);
   __syncthreads();
-  const BoxFields fs{fbox, ai, ak};
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  constexpr int kSplit = kPPT / PPT;
-  const int chunk = wave / kSplit, j0 = (wave % kSplit) * PPT;
-  constexpr long long kTile = (long long)WAVES * PPT / kPPT * kChunk;
-  const F32Args q = from_slot(p, base);
-  const unsigned lim = (unsigned)min(n_cap - base, kTile);
-  const unsigned off0 = (unsigned)(chunk * kChunk + j0 * 64 + lane);
+  const BoxFields fs{fbox, ai, ak, width};
   // software pipeline: the state of the lane's next particle is loaded before
   // the current one is pushed; all its loads are waited for before the
   // current particle's stores, so the wait never includes stores in flight
-  PState nx{kDead, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (off0 < lim) nx = load_state_next(q, off0 * 4u);
   for (int j = 0; j < PPT; j++) {
     const PState cur = nx;
     unsigned n = off0 + (unsigned)j * 64u, n1 = n + 64u;
@@ -750,7 +777,6 @@ template <int PPT, int WAVES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_fused32_tiled(F32Args p, GlobalSink gs, long long n_cap) {
   __shared__ double box[TileSink::kSize];
   __shared__ __align__(16) float fbox[kFBoxFloats];
-  constexpr long long kTile = (long long)WAVES * PPT / kPPT * kChunk;
   // launched for the chunked layout only, i.e. plasma species: no bunch walls
   // and no charge density (constants here drop their code and registers)
   F32Args q = p;
@@ -762,7 +788,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
   g.nr = q.nr;
   g.nz = q.nz;
   g.err = q.err;
-  fused32_tile<PPT, WAVES>(q, g, (long long)blockIdx.x * kTile, n_cap, box, fbox);
+  fused32_tile<PPT, WAVES, TileSink>(q, g, TileMap<PPT, WAVES>::base(blockIdx.x), n_cap, box, fbox);
 }
 
 // bunches (plain layout): the same walk, the box anchored at the smallest
@@ -789,7 +815,7 @@ __device__ __forceinline__ void fused32_bunch_tile(const F32Args &p, const Globa
   block_min2(ai, ak);
   if (ai == 0x7fffffff) return;  // no living particle in the block (uniform over the block)
   BunchSink sk;
-  box_init(box, ai, ak, sk, gs);
+  box_init(box, ai, ak, BunchSink::kK, sk, gs);
   __syncthreads();
   const F32Args q = from_slot(p, base);
   const unsigned lim = (unsigned)min(n_cap - base, (long long)WAVES * 64 * PPT);
@@ -901,7 +927,7 @@ template <int PPT, int WAVES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
 k_ens_fused32(const F32Args *__restrict__ args, const GlobalSink *__restrict__ sinks,
               const EnsItem *__restrict__ items, int n_items) {
-  __shared__ double box[TileSink::kSize];
+  __shared__ double box[TileRhoSink::kSize];
   __shared__ __align__(16) float fbox[kFBoxFloats];
   const int it = blockIdx.x;
   if (it >= n_items) return;
@@ -913,7 +939,7 @@ k_ens_fused32(const F32Args *__restrict__ args, const GlobalSink *__restrict__ s
   g.nr = a.nr;  // one copy of the grid size and error word (scalar registers)
   g.nz = a.nz;
   g.err = a.err;
-  fused32_tile<PPT, WAVES>(a, g, item.base, item.n_cap, box, fbox);
+  fused32_tile<PPT, WAVES, TileRhoSink>(a, g, item.base, item.n_cap, box, fbox);
 }
 
 // plain layout (bunches): one particle per thread, deposits straight to HBM
@@ -1096,7 +1122,7 @@ unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
 
 template <int PPT, int WAVES>
 void launch_tile_t(hipStream_t st, const F32Args &p, const GlobalSink &gs, long long n_cap) {
-  constexpr long long kTile = (long long)WAVES * PPT / kPPT * kChunk;
+  constexpr long long kTile = TileMap<PPT, WAVES>::kParticles;
   unsigned blocks = (unsigned)((n_cap + kTile - 1) / kTile);
   hipLaunchKernelGGL((k_fused32_tiled<PPT, WAVES>), dim3(blocks), dim3(WAVES * 64), 0, st, p, gs, n_cap);
 }
@@ -1108,14 +1134,39 @@ void launch_tile(int tile, hipStream_t st, const F32Args &p, const GlobalSink &g
     case 2: launch_tile_t<16, 1>(st, p, gs, n_cap); break;
     case 3: launch_tile_t<8, 4>(st, p, gs, n_cap); break;
     case 4: launch_tile_t<8, 2>(st, p, gs, n_cap); break;
-    default: launch_tile_t<4, 4>(st, p, gs, n_cap); break;
+    case 5: launch_tile_t<4, 4>(st, p, gs, n_cap); break;
+    case 6: launch_tile_t<2, 4>(st, p, gs, n_cap); break;
+    default: launch_tile_t<1, 4>(st, p, gs, n_cap); break;
   }
+}
+
+// the shape for a species of a context whose shape was neither set nor
+// autotuned: the largest that covers at most kFK - 8 cells of a sorted species
+// (its boxes then serve all of its particles) and still fills the GPU; a
+// species without either runs on 256-particle tiles.  A shape of 4 or 8
+// particles per lane and more needs two full rounds or more of blocks (five
+// blocks on each of 256 CUs) to be worth its longer walk.  Kernel times in us,
+// shapes 16x4, 8x4, 4x4, 2x4, 1x4:
+//   1.6e5 particles, 10 per cell:  56.4   34.9   22.7   17.3   15.0
+//   9.8e5 particles, 30 per cell:  55.6   37.8   30.2   30.0   41.6
+//   1.3e6 particles, 10 per cell:  73.6   51.6   34.7   37.4   48.5
+//   2.6e6 particles, 20 per cell:  79.3   57.5   53.0   60.2   91.8
+//   2.1e7 particles, 40 per cell: 238    273    303    428    671
+//   2.1e8 particles, 100 per cell: 2126  2432   2866   4048   6755
+int auto_tile(const Ctx &c, const Species &sp) {
+  const double cells = (double)(c.g.nr - 1) * (c.g.nz - 1);
+  const struct {
+    int tile, particles, blocks;
+  } shapes[] = {{0, 4096, 4096}, {3, 2048, 4096}, {5, 1024, 800}, {6, 512, 400}};
+  for (const auto &s : shapes)
+    if (sp.n >= (long long)s.particles * s.blocks && s.particles * cells <= (kFK - 8) * (double)sp.n) return s.tile;
+  return 7;
 }
 
 void launch_fused_f32(Ctx &c, Species &sp) {
   if (sp.n_cap <= 0 || !sp.f32.cell) return;
   if (sp.chunked) {
-    launch_tile(c.tile, c.stream, args32(c, sp), sink32(c), sp.n_cap);
+    launch_tile(c.tile_auto ? auto_tile(c, sp) : c.tile, c.stream, args32(c, sp), sink32(c), sp.n_cap);
   } else {
     // the most particles per lane that still give 1024 blocks
     const long long n = sp.n_cap, per = (long long)kWavesPerBlock * 64;

@@ -700,7 +700,7 @@ k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_ca
     tile_anchor(live, ri, kk, ai, ak);
   }
   TileSink sk;
-  box_init(box, ai, ak, sk, gs);
+  box_init(box, ai, ak, TileSink::kK, sk, gs);
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long long cbase = base + (long long)wave * kChunk + lane;
@@ -735,7 +735,7 @@ __global__ void __launch_bounds__(256) k_fused_bunch(GridDesc g, Fields f, Globa
   block_min2(ai, ak);
   if (ai == 0x7fffffff) return;
   BunchSink sk;
-  box_init(box, ai, ak, sk, gs);
+  box_init(box, ai, ak, BunchSink::kK, sk, gs);
   __syncthreads();
   for (int j = 0; j < PPT; j++) {
     long long p = cbase + (long long)j * 64;

@@ -63,18 +63,21 @@ struct GlobalSink {
   __device__ __forceinline__ void flush() {}
 };
 
-constexpr int kBoxComps = 4;
-
 // BR x BK nodes per component; the plasma box spans 4 rows (i0-1 .. i0+2) by
 // 128 columns (a sorted block covers a run of cells along one row), the bunch
 // box 16 rows by 32 columns (a bunch block is a thin disc of particles
 // injected in the same step)
-template <bool RHO, int BR = 4, int BK = 128>
+// COMPS: 3, or 4 where rho is deposited too (RHO: also summed in registers)
+template <bool RHO, int COMPS, int BR = 4, int BK = 128>
 struct TileSinkT {
-  static constexpr int kR = BR, kK = BK, kSize = kBoxComps * BR * BK;
+  static constexpr int kComps = COMPS;
+  static_assert(COMPS == 3 || COMPS == 4, "J_r, J_phi, J_z and rho");
+  static_assert(COMPS == 4 || !RHO, "rho sums need the box's fourth component");
+  static constexpr int kR = BR, kK = BK, kSize = kComps * BR * BK;
   GlobalSink g;
-  double *box;  // LDS, kBoxComps x kBoxR x kBoxK
+  double *box;  // LDS, kComps x kR x kK
   int bi, bk;   // node coordinates of box[.][0][0]
+  int bw;       // columns of the box in use (a multiple of the wavefront or kK)
   int ic, kc;   // cell of the register accumulator
   // scalar accumulators (no arrays: a runtime index would push them to scratch)
   double p00, p10, p01, p11;  // J_phi corners (ic+di, kc+dk)
@@ -84,7 +87,7 @@ struct TileSinkT {
 
   __device__ __forceinline__ void box_put(int comp, int i, int k, double v) {
     int li = i - bi, lk = k - bk;
-    if ((unsigned)li < (unsigned)BR && (unsigned)lk < (unsigned)BK)
+    if (comp < COMPS && (unsigned)li < (unsigned)BR && (unsigned)lk < (unsigned)bw)
       atomicAdd(box + (comp * BR + li) * BK + lk, v);
     else
       g.put(comp, i, k, v);
@@ -163,7 +166,7 @@ struct TileSinkT {
   __device__ __forceinline__ void flush() {
     if (ic < 0) return;
     const int li = ic - bi, lk = kc - bk;
-    if ((unsigned)li < (unsigned)(BR - 1) && (unsigned)lk < (unsigned)(BK - 1)) {
+    if ((unsigned)li < (unsigned)(BR - 1) && (unsigned)lk < (unsigned)(bw - 1)) {
       double *q = box + li * BK + lk;
       constexpr int C = BR * BK;
       atomicAdd(q + kCPhi * C, p00);
@@ -209,8 +212,9 @@ struct TileSinkT {
     }
   }
 };
-using TileSink = TileSinkT<false>;
-using BunchSink = TileSinkT<true, 16, 32>;
+using TileSink = TileSinkT<false, 3>;       // plasma species
+using TileRhoSink = TileSinkT<false, 4>;    // an ensemble's tiles, bunch blocks among them
+using BunchSink = TileSinkT<true, 4, 16, 32>;
 
 // The anchor cell of a tile of cell-sorted particles, from the cells (i, k)
 // of its logical particles 0, 16 and 32 (live: a living particle; uniform
@@ -243,14 +247,19 @@ __device__ __forceinline__ void tile_anchor(const bool (&live)[3], const int (&i
 }
 
 // block prologue: anchor the box one row and two columns below the given
-// cell (the tile's anchor, or a bunch block's smallest cell) and clear it
+// cell (the tile's anchor, or a bunch block's smallest cell) and clear its
+// first `width` columns
 template <class T>
-__device__ __forceinline__ void box_init(double *box, int anchor_i, int anchor_k, T &s, const GlobalSink &g) {
-  for (int t = threadIdx.x; t < T::kSize; t += blockDim.x) box[t] = 0.0;
+__device__ __forceinline__ void box_init(double *box, int anchor_i, int anchor_k, int width, T &s,
+                                         const GlobalSink &g) {
+  constexpr int kRow = T::kK < 64 ? T::kK : 64;  // columns cleared or added at a time
+  for (int t = threadIdx.x / kRow; t < T::kComps * T::kR; t += blockDim.x / kRow)
+    for (int c = threadIdx.x % kRow; c < width; c += kRow) box[t * T::kK + c] = 0.0;
   s.g = g;
   s.box = box;
   s.bi = anchor_i - 1;
   s.bk = anchor_k - 2;
+  s.bw = width;
   s.ic = -1;
   s.kc = -1;
   s.p00 = s.p10 = s.p01 = s.p11 = 0.0;
@@ -261,14 +270,14 @@ __device__ __forceinline__ void box_init(double *box, int anchor_i, int anchor_k
 // block epilogue: add the box to the grid (after __syncthreads)
 template <class T>
 __device__ __forceinline__ void box_flush(const double *box, const T &s) {
-  for (int t = threadIdx.x; t < T::kSize; t += blockDim.x) {
-    double v = box[t];
-    if (v == 0.0) continue;
-    int comp = t / (T::kR * T::kK);
-    int rem = t - comp * T::kR * T::kK;
-    int li = rem / T::kK, lk = rem - li * T::kK;
-    s.g.put(comp, s.bi + li, s.bk + lk, v);
-  }
+  constexpr int kRow = T::kK < 64 ? T::kK : 64;
+  for (int t = threadIdx.x / kRow; t < T::kComps * T::kR; t += blockDim.x / kRow)
+    for (int c = threadIdx.x % kRow; c < s.bw; c += kRow) {
+      const double v = box[t * T::kK + c];
+      if (v == 0.0) continue;
+      const int comp = t / T::kR;
+      s.g.put(comp, s.bi + t - comp * T::kR, s.bk + c, v);
+    }
 }
 
 }  // namespace pdp3

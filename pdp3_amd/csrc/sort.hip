@@ -712,10 +712,10 @@ int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream) 
     d.slot_base = n;
     d.key_base = (uint32_t)keys;
     d.nzm1 = (uint32_t)(c.g.nz - 1);
-    // A particle tile (a few chunks of consecutive particles) spans
-    // tile / ppc cells; in row order that overruns the tile's 64-column field
-    // box below about 32 particles per cell, in bands of two rows only below
-    // about 16.  Instances with fewer particles per cell sort in bands.
+    // A particle tile of 4096 consecutive particles spans 4096 / ppc cells; in
+    // row order that overruns the tile's 128-column field box below about 32
+    // particles per cell, in bands of two rows only below about 16.  Instances
+    // with fewer particles per cell sort in bands.
     const long long rows = c.g.nr - 1;
     d.band = sp.n < 32LL * rows * (long long)d.nzm1 ? 1u : 0u;
     d.ncell = d.band ? (uint32_t)(2 * ((rows + 1) / 2)) * d.nzm1 : (uint32_t)rows * d.nzm1;

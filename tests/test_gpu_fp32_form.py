@@ -249,3 +249,38 @@ def test_tile_shapes_agree_and_autotune():
             sim2.set_tile(3, 3)
         finally:
             sim2.close()
+
+
+@pytest.mark.parametrize("cells_r,cells_z,ppc", [
+    (21, 43, 3),      # 256-particle tiles, the last chunk mostly padding
+    (9, 1000, 1),     # the same, tiles that overrun the field box
+    (64, 256, 16),    # 512-particle tiles
+    (128, 512, 15),   # one chunk per tile
+    (256, 1024, 33),  # 2048-particle tiles, half the field box's width
+    (512, 2048, 17),  # the same, its whole width
+])
+def test_tile_chosen_by_size(cells_r, cells_z, ppc):
+    """Without a set or autotuned shape a species runs on the tile that suits
+    its size; the step is that of the 16 x 4 shape up to the order of the FP64
+    sums (per-particle arithmetic is identical: a deposit of n FP64 terms
+    reordered moves by at most n ulps, far below 1e-11 of the maximum)."""
+    from pdp3_amd import capi
+
+    d = 5e-4
+    out = []
+    for shape in (None, (16, 4)):
+        sim = capi.Simulation(cells_r + 1, cells_z + 1, cells_r * d, cells_z * d, 0.5 * d / 3e8,
+                              precision=capi.PREC_FP32)
+        sim.boundary_conditions()
+        idx = sim.add_species(-1, 1.0, ppc * cells_r * cells_z)
+        sim.init_uniform(idx, 11, ppc, 1e17, 0, 50.0)
+        if shape:
+            sim.set_tile(*shape)
+        assert sim.tile() == (16, 4)
+        sim.step(4)
+        out.append({n: sim.field(n) for n in ("E_r", "E_phi", "E_z", "H_phi", "J_r", "J_phi", "J_z")})
+        out[-1].update({k: v for k, v in sim.download(idx).items() if k in ("r", "z", "vr", "vphi", "vz")}
+                       if cells_r < 200 else {})
+        sim.close()
+    for n in out[0]:
+        assert normwise(out[0][n], out[1][n]) <= 1e-11, (n, normwise(out[0][n], out[1][n]))
