@@ -60,7 +60,6 @@ struct GridDesc {
 constexpr int kPPT = 16;
 constexpr int kChunk = 64 * kPPT;
 constexpr int kWavesPerBlock = 4;
-constexpr int kBlockParticles = kWavesPerBlock * kChunk;
 
 __host__ __device__ __forceinline__ long long phys_of(long long s) {
   long long c = s / kChunk, w = s - c * kChunk;

@@ -676,17 +676,18 @@ __device__ __forceinline__ void step_particle(const GridDesc &g, const Fields &f
   if (!alive) s.alive[i] = 0;
 }
 
-// chunked plasma species: 4 wavefronts per block, each walking one chunk of
-// kChunk slots kPPT particles per lane, deposits through the tile sink
-// with the divisions taken from shared reciprocals (div_cr) the compiler's own
-// choice, 227 VGPRs at 2 waves per SIMD without spills, is the fastest: 25.9 ms
+// chunked plasma species: 4 wavefronts per block on one tile (TileMap), PPT
+// particles per lane, deposits through the tile sink; with the divisions taken from shared reciprocals (div_cr) the compiler's own
+// choice, 227 VGPRs (PPT > 1) at 2 waves per SIMD without spills, is the fastest: 25.9 ms
 // at cfg3 against 26.7 ms for the IEEE divisions at 3 waves (168 VGPRs, 12
 // spilled); forcing 3 waves with div_cr spills 146 VGPRs (43 ms)
+template <int PPT>
 __global__ void __launch_bounds__(256)
 k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_cap, int pusher) {
   __shared__ double box[TileSink::kSize];
-  const long long base = (long long)blockIdx.x * kBlockParticles;
-  // anchor samples: slot base + j is the logical particle 16 j of the block
+  using Map = TileMap<PPT, kWavesPerBlock>;
+  const long long base = Map::base(blockIdx.x);
+  // anchor samples: slot base + j is the logical particle 16 j of the tile
   int ai, ak;
   {
     bool live[3];
@@ -702,10 +703,9 @@ k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_ca
   TileSink sk;
   box_init(box, ai, ak, TileSink::kK, sk, gs);
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long long cbase = base + (long long)wave * kChunk + lane;
-  for (int j = 0; j < kPPT; j++) {
-    long long p = cbase + (long long)j * 64;
+  const long long first = base + Map::first(threadIdx.x);
+  for (int j = 0; j < PPT; j++) {
+    long long p = first + (long long)j * 64;
     if (p < n_cap) step_particle(g, f, sk, gs.err, s, pusher, false, p);
   }
   sk.flush();
@@ -869,12 +869,33 @@ unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
+template <int PPT>
+void launch_tile64(Ctx &c, Species &sp) {
+  constexpr long long kTile = TileMap<PPT, kWavesPerBlock>::kParticles;
+  hipLaunchKernelGGL(k_fused_tiled<PPT>, dim3((unsigned)((sp.n_cap + kTile - 1) / kTile)), dim3(256), 0, c.stream, c.g,
+                     fields_of(c), sink_of(c), args_of(sp), sp.n_cap, c.pusher);
+}
+
+// Particles per lane by the size of the species.  Without a walk the kernel
+// needs 156 VGPRs (three waves per SIMD) and fills the GPU from the fewest
+// particles; a walk's hoisted constants and register sums bring it to 227 (two
+// waves), but it adds to LDS only when a lane changes cell, which wins once
+// every lane has many particles.  Kernel times in us, 16, 8, 4, 2, 1 per lane:
+//   1.6e5 particles, 10 per cell: 106   60   35   27   22
+//   2.6e6 particles, 20 per cell: 236  189  184  195  181
+//   1.0e7 particles, 20 per cell: 796  719  749  809  752
+//   1.0e8 particles, 100 per cell: 6448 6681 7118 7866 7288
+constexpr long long kOneEach = 8000000, kEightEach = 16000000;
+
 void launch_fused_f64(Ctx &c, Species &sp) {
   if (sp.n_cap <= 0) return;
   if (sp.chunked) {
-    unsigned blocks = (unsigned)((sp.n_cap + kBlockParticles - 1) / kBlockParticles);
-    hipLaunchKernelGGL(k_fused_tiled, dim3(blocks), dim3(256), 0, c.stream, c.g, fields_of(c), sink_of(c),
-                       args_of(sp), sp.n_cap, c.pusher);
+    if (sp.n_cap < kOneEach)
+      launch_tile64<1>(c, sp);
+    else if (sp.n_cap < kEightEach)
+      launch_tile64<8>(c, sp);
+    else
+      launch_tile64<16>(c, sp);
   } else {
     // the most particles per lane that still give 1024 blocks
     const long long n = sp.n_cap, per = (long long)kWavesPerBlock * 64;

@@ -282,3 +282,38 @@ def test_superluminal_velocity_is_reported(capi):
     with pytest.raises(capi.Pdp3Error) as ei:
         sim.step(1)
     assert ei.value.code == capi.ERR_SUPERLUMINAL
+
+
+@pytest.mark.parametrize("cells_r,cells_z,ppc", [
+    (21, 43, 3),      # one particle per lane, the last chunk mostly padding
+    (64, 256, 10),
+    (256, 1024, 31),  # eight per lane
+    (256, 1024, 62),  # sixteen per lane
+])
+def test_fused_step_by_size(capi, cells_r, cells_z, ppc):
+    """The fused kernel's walk follows the species' size; at every size its step
+    is that of the split entry points: the same arithmetic per particle, so the
+    grids agree up to the order of their FP64 sums (at most some hundred terms
+    a node, each reordering an ulp: 1e-12 of the maximum holds with room)."""
+    d = 5e-4
+    f = []
+    for fused in (True, False):
+        sim = capi.Simulation(cells_r + 1, cells_z + 1, cells_r * d, cells_z * d, 0.5 * d / 3e8)
+        sim.boundary_conditions()
+        idx = sim.add_species(-1, 1.0, ppc * cells_r * cells_z)
+        sim.init_uniform(idx, 12, ppc, 1e17, 0, 50.0)
+        for _ in range(2):
+            if fused:
+                sim.step(1)
+                continue
+            sim.h_calc()
+            sim.reset_j()
+            sim.step_v(idx)
+            sim.full_current_distribution(idx)
+            sim.e_calc()
+        f.append({n: sim.field(n) for n in ("E_r", "E_phi", "E_z", "H_phi", "J_r", "J_phi", "J_z")})
+        if cells_r < 100:
+            f[-1].update({k: v for k, v in sim.download(idx).items() if k != "alive"})
+        sim.close()
+    for n in f[0]:
+        assert normwise(f[0][n], f[1][n]) <= 1e-12, (n, normwise(f[0][n], f[1][n]))
