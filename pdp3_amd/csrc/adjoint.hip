@@ -28,10 +28,8 @@ namespace pdp3 {
 
 namespace {
 
-constexpr int kDN = 4;       // directions per pass
+constexpr int kDN = 4;  // directions
 static_assert(kDN == kTangentDirs, "the tangent-linear model runs one direction per dual slot");
-constexpr int kInputs = 12;  // r, z, v0, v1, v2, e0, e1, e2, h0, h1, h2, w
-constexpr int kPasses = kInputs / kDN;
 
 struct D {
   double v;
@@ -44,14 +42,13 @@ __device__ __forceinline__ D cst(double x) {
   for (int j = 0; j < kDN; j++) r.d[j] = 0.0;
   return r;
 }
-// x as input `input` of pass `pass` (derivative 1 in its direction); selects
-// on constant indices, so that no dual number is addressed through memory
-__device__ __forceinline__ D seed(double x, int input, int pass) {
+// x as direction `dir` (derivative 1 there); selects on constant indices, so
+// that no dual number is addressed through memory
+__device__ __forceinline__ D seed(double x, int dir) {
   D r;
   r.v = x;
-  const int jin = input - pass * kDN;
 #pragma unroll
-  for (int j = 0; j < kDN; j++) r.d[j] = j == jin ? 1.0 : 0.0;
+  for (int j = 0; j < kDN; j++) r.d[j] = j == dir ? 1.0 : 0.0;
   return r;
 }
 __device__ __forceinline__ D operator+(D a, D b) {
@@ -209,51 +206,6 @@ __device__ __forceinline__ D gather_d(const GridDesc &g, const double *F, D r, D
   return gw.w[0] * row0[0] + gw.w[1] * row1[0] + gw.w[2] * row0[1] + gw.w[3] * row1[1];
 }
 
-// the adjoints of the gathered fields of one block's particles are summed in
-// an LDS box of kABR x kABK nodes per component (anchored one row and two
-// columns below the block's smallest cell) and added to the grid once per
-// block; stencils outside the box go to the grid directly
-constexpr int kABR = 4, kABK = 64, kABComp = 6;
-struct AdjBox {
-  double *box;  // LDS, kABComp x kABR x kABK
-  int bi, bk;   // node of box[.][0][0]
-};
-__device__ __forceinline__ void box_scatter(const GridDesc &g, const AdjBox &b, int comp, double *LF, double r,
-                                            double z, bool lo, bool zhalf, double lam) {
-  if (lam == 0.0) return;
-  GatherW gw = gather_w(g, cst(r), cst(z), lo, zhalf);
-  // weights 0..3 multiply the nodes (ir, kz), (ir+1, kz), (ir, kz+1), (ir+1, kz+1)
-  const double v00 = gw.w[0].v * lam, v10 = gw.w[1].v * lam, v01 = gw.w[2].v * lam, v11 = gw.w[3].v * lam;
-  const int li = gw.ir - b.bi, lk = gw.kz - b.bk;
-  if ((unsigned)li < (unsigned)(kABR - 1) && (unsigned)lk < (unsigned)(kABK - 1)) {
-    double *q = b.box + (comp * kABR + li) * kABK + lk;
-    atomicAdd(q, v00);
-    atomicAdd(q + kABK, v10);
-    atomicAdd(q + 1, v01);
-    atomicAdd(q + kABK + 1, v11);
-  } else {
-    double *row0 = LF + (size_t)gw.ir * (size_t)g.nz + gw.kz;
-    double *row1 = row0 + g.nz;
-    unsafeAtomicAdd(row0, v00);
-    unsafeAtomicAdd(row1, v10);
-    unsafeAtomicAdd(row0 + 1, v01);
-    unsafeAtomicAdd(row1 + 1, v11);
-  }
-}
-
-// the deposit "sink" of the adjoint: every contribution v at node (i, k) of
-// component C adds lambda_J[C](i, k) * dv to the accumulated input adjoints
-struct AdjSink {
-  const GridDesc *g;
-  const double *ljr, *ljphi, *ljz;
-  double acc[kDN];
-  __device__ __forceinline__ void add(int comp, int i, int k, D v) {
-    if ((unsigned)i >= (unsigned)g->nr || (unsigned)k >= (unsigned)g->nz) return;
-    const double *L = comp == 0 ? ljr : comp == 1 ? ljphi : ljz;
-    const double l = L[(size_t)i * (size_t)g->nz + (size_t)k];
-    for (int j = 0; j < kDN; j++) acc[j] += l * v.d[j];
-  }
-};
 constexpr int kAR = 0, kAPhi = 1, kAZ = 2;
 
 __device__ __forceinline__ D dot3(const D *a, const D *b) {
@@ -707,81 +659,567 @@ __device__ __forceinline__ void walls_d(const GridDesc &g, bool is_bunch, D &x, 
   }
 }
 
-// vector-Jacobian product of one particle's step
-// the vector-Jacobian product of one living particle's step
-__device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields &f, const AdjGrid &lg,
-                                             const AdjSpecies &s, int pusher, long long i, const AdjBox &b) {
-  const double r0v = s.r[i], z0v = s.z[i];
-  const double lam_r = s.lr[i], lam_z = s.lz[i], lam_v0 = s.lvr[i], lam_v1 = s.lvphi[i], lam_v2 = s.lvz[i];
-  double lin[kInputs] = {};
-  for (int pass = 0; pass < kPasses; pass++) {
-    AdjSink sk;
-    sk.g = &g;
-    sk.ljr = lg.ljr;
-    sk.ljphi = lg.ljphi;
-    sk.ljz = lg.ljz;
-    for (int j = 0; j < kDN; j++) sk.acc[j] = 0.0;
-    D r = seed(r0v, 0, pass), z = seed(z0v, 1, pass);
-    D v[3] = {seed(s.vr[i], 2, pass), seed(s.vphi[i], 3, pass), seed(s.vz[i], 4, pass)};
-    D w = seed(s.w[i], 11, pass);
-    D q = s.charge * w, m = s.mass * w;
-    const D r_old = r, z_old = z;
-    D e[3], h[3];
-    e[0] = gather_d(g, f.er, r, z, true, false) + seed(0.0, 5, pass);
-    e[1] = gather_d(g, f.ephi, r, z, false, false) + seed(0.0, 6, pass);
-    e[2] = gather_d(g, f.ez, r, z, false, true) + seed(0.0, 7, pass);
-    h[0] = gather_d(g, f.hhr, r, z, false, true) + seed(0.0, 8, pass);
-    h[1] = gather_d(g, f.hhphi, r, z, true, true) + seed(0.0, 9, pass);
-    h[2] = gather_d(g, f.hhz, r, z, true, false) + seed(0.0, 10, pass);
-    if (pusher == 1)
-      vay_d(q, m, g.dt, e, h, v);
-    else
-      boris_d(q, m, g.dt, e, h, v);
-    const double half_dt = g.dt / 2.;
-    // first half step and rotation (step_v)
-    D x = r + v[0] * half_dt;
-    D y = 0.0 + v[1] * half_dt;
-    z = z + v[2] * half_dt;
-    r = dsqrt(x * x + y * y);
-    // full_current_distribution
-    jphi_d(g, sk, q, r, z, v[1]);
-    x = r + v[0] * half_dt;
-    y = 0.0 + v[1] * half_dt;
-    z = z + v[2] * half_dt;
-    bool alive = true;
-    walls_d(g, s.is_bunch != 0, x, z, v[0], v[2], alive);
-    D rr = dsqrt(x * x + y * y);
-    D st = y / rr;
-    r = rr;
-    if (alive) {
-      deposit_j_d(g, sk, q, r, z, r_old, z_old);
-      D ct = dsqrt(1 - st * st);
-      D u2 = ct * v[0] - st * v[1];
-      D w2 = st * v[0] + ct * v[1];
-      v[0] = u2;
-      v[1] = w2;
-      for (int j = 0; j < kDN; j++)
-        sk.acc[j] += lam_r * r.d[j] + lam_z * z.d[j] + lam_v0 * v[0].d[j] + lam_v1 * v[1].d[j] + lam_v2 * v[2].d[j];
-    }
-#pragma unroll
-    for (int o = 0; o < kInputs; o++) lin[o] = o / kDN == pass ? sk.acc[o % kDN] : lin[o];
-  }
-  s.lr[i] = lin[0];
-  s.lz[i] = lin[1];
-  s.lvr[i] = lin[2];
-  s.lvphi[i] = lin[3];
-  s.lvz[i] = lin[4];
-  s.lw[i] += lin[11];
-  box_scatter(g, b, 0, lg.ler, r0v, z0v, true, false, lin[5]);
-  box_scatter(g, b, 1, lg.lephi, r0v, z0v, false, false, lin[6]);
-  box_scatter(g, b, 2, lg.lez, r0v, z0v, false, true, lin[7]);
-  box_scatter(g, b, 3, lg.lhr, r0v, z0v, false, true, lin[8]);
-  box_scatter(g, b, 4, lg.lhphi, r0v, z0v, true, true, lin[9]);
-  box_scatter(g, b, 5, lg.lhz, r0v, z0v, true, false, lin[10]);
+// ------------------------------------------------ reverse mode, one particle
+#pragma clang fp contract(fast)
+// The vector-Jacobian product of one particle's step, written out stage by
+// stage in reverse.  Every deposit is linear in the weight and the push does
+// not depend on it (q / m), so the weight's adjoint is the sum of lambda_J
+// times the deposits of a unit weight.  One forward evaluation and one reverse sweep
+// replace 12 directional derivatives of the step.
+
+struct V3 {
+  double x, y, z;
+};
+__device__ __forceinline__ V3 operator+(V3 a, V3 b) { return V3{a.x + b.x, a.y + b.y, a.z + b.z}; }
+__device__ __forceinline__ V3 operator*(double s, V3 a) { return V3{s * a.x, s * a.y, s * a.z}; }
+__device__ __forceinline__ double dot(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+__device__ __forceinline__ V3 cross(V3 a, V3 b) {
+  return V3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
+}
+__device__ __forceinline__ V3 fma3(double s, V3 a, V3 b) { return V3{s * a.x + b.x, s * a.y + b.y, s * a.z + b.z}; }
+
+// u = v gamma(v) and gamma = (1 + u^2/c^2)^(-1/2) with their reverse steps
+struct Boost {
+  V3 u;       // v with the components below MNZL dropped
+  double g0;  // 1 / sqrt(1 - v^2/c^2)
+};
+__device__ __forceinline__ Boost boost_of(V3 v) {
+  Boost b;
+  b.u = V3{fabs(v.x) < kMnzl ? 0.0 : v.x, fabs(v.y) < kMnzl ? 0.0 : v.y, fabs(v.z) < kMnzl ? 0.0 : v.z};
+  b.g0 = 1.0 / sqrt(1.0 - dot(b.u, b.u) / kC2);
+  return b;
+}
+// adjoint of v from the adjoint of U = g0 u
+__device__ __forceinline__ V3 boost_back(const Boost &b, V3 v, V3 lU) {
+  const double s = b.g0 * b.g0 * b.g0 / kC2 * dot(lU, b.u);
+  const V3 l = fma3(s, b.u, b.g0 * lU);
+  return V3{fabs(v.x) < kMnzl ? 0.0 : l.x, fabs(v.y) < kMnzl ? 0.0 : l.y, fabs(v.z) < kMnzl ? 0.0 : l.z};
+}
+__device__ __forceinline__ double inv_gamma(V3 u) { return 1.0 / sqrt(1.0 + dot(u, u) / kC2); }
+// adjoint of u added for an adjoint lg of g = inv_gamma(u)
+__device__ __forceinline__ V3 inv_gamma_back(double g, V3 u, double lg, V3 l) {
+  return fma3(-(g * g * g) / kC2 * lg, u, l);
 }
 
-__global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, AdjGrid lg, AdjSpecies s,
-                                                       int pusher) {
+// what the reverse sweep of a push keeps of its forward evaluation, recomputed
+// from the inputs: v, and the fields multiplied by the species' scales
+struct PushBack {
+  V3 v, e, b;  // adjoints of v and of the scaled fields
+};
+
+// relativistic Boris (src/particles.cpp:1025-1150)
+__device__ __forceinline__ V3 boris_fwd(V3 v, V3 e, V3 h) {
+  const Boost b0 = boost_of(v);
+  const V3 t = fma3(b0.g0, b0.u, e);
+  const V3 b = inv_gamma(t) * h;
+  const V3 w = cross(t + cross(t, b), b);
+  const V3 u = fma3(2.0 / (1.0 + dot(b, b)), w, t) + e;
+  return inv_gamma(u) * u;
+}
+__device__ __forceinline__ PushBack boris_back(V3 v, V3 e, V3 h, V3 lv) {
+  const Boost b0 = boost_of(v);
+  const V3 t = fma3(b0.g0, b0.u, e);
+  const double g1 = inv_gamma(t);
+  const V3 b = g1 * h;
+  const V3 tp = t + cross(t, b);
+  const double c2 = 2.0 / (1.0 + dot(b, b));
+  const V3 w = cross(tp, b);
+  const V3 u = fma3(c2, w, t) + e;
+  const double g2 = inv_gamma(u);
+  PushBack o;
+  const V3 lu = inv_gamma_back(g2, u, dot(lv, u), g2 * lv);
+  const double lc2 = dot(lu, w);
+  const V3 lw = c2 * lu;
+  const V3 ltp = cross(b, lw);
+  V3 lt = lu + ltp + cross(b, ltp);
+  V3 lb = cross(lw, tp) + cross(ltp, t);
+  lb = fma3(-c2 * c2 * lc2, b, lb);
+  o.b = g1 * lb;
+  lt = inv_gamma_back(g1, t, dot(lb, h), lt);
+  o.e = lu + lt;
+  o.v = boost_back(b0, v, lt);
+  return o;
+}
+
+// Vay with the reference's scaling (src/particles.cpp:1152-1254)
+__device__ __forceinline__ V3 vay_fwd(V3 v, V3 e, V3 h) {
+  const Boost b0 = boost_of(v);
+  const V3 t = b0.g0 * b0.u;
+  const V3 up = fma3(inv_gamma(t), cross(t, h), t + e);
+  const double B2 = dot(h, h), ub = dot(up, h), sg = 1.0 + dot(up, up) / kC2 - B2;
+  const double al = 1.0 / sqrt(0.5 * (sg + sqrt(sg * sg + 4. * (B2 + ub * ub))));
+  const V3 b = al * h;
+  const V3 u = (1.0 / (1.0 + dot(b, b))) * (fma3(dot(up, b), b, up) + cross(up, b));
+  return inv_gamma(u) * u;
+}
+__device__ __forceinline__ PushBack vay_back(V3 v, V3 e, V3 h, V3 lv) {
+  const Boost b0 = boost_of(v);
+  const V3 t = b0.g0 * b0.u;
+  const double g1 = inv_gamma(t);
+  const V3 th = cross(t, h);
+  const V3 up = fma3(g1, th, t + e);
+  const double B2 = dot(h, h), ub = dot(up, h), sg = 1.0 + dot(up, up) / kC2 - B2;
+  const double root = sqrt(sg * sg + 4. * (B2 + ub * ub));
+  const double al = 1.0 / sqrt(0.5 * (sg + root));
+  const V3 b = al * h;
+  const double s = 1.0 / (1.0 + dot(b, b)), al2 = dot(up, b);
+  const V3 q = fma3(al2, b, up) + cross(up, b);
+  const V3 u = s * q;
+  const double g3 = inv_gamma(u);
+  PushBack o;
+  const V3 lu = inv_gamma_back(g3, u, dot(lv, u), g3 * lv);
+  const double ls = dot(lu, q);
+  const V3 lq = s * lu;
+  const double lal2 = dot(lq, b);
+  V3 lup = fma3(lal2, b, lq + cross(b, lq));
+  V3 lb = fma3(lal2, up, fma3(al2, lq, cross(lq, up)));
+  lb = fma3(-2.0 * s * s * ls, b, lb);
+  const double lx = -0.5 * al * al * al * dot(lb, h);
+  const double lin = 0.5 * lx * 0.5 / root;
+  const double lsg = 0.5 * lx + 2.0 * sg * lin, lub = 2.0 * ub * 4.0 * lin, lB2 = 4.0 * lin - lsg;
+  lup = fma3(lub, h, fma3(lsg * (2.0 / kC2), up, lup));
+  V3 lh = fma3(al, lb, fma3(lub, up, (2.0 * lB2) * h));
+  const V3 mu = g1 * lup;
+  lh = lh + cross(mu, t);
+  const V3 lt = inv_gamma_back(g1, t, dot(lup, th), cross(h, mu));
+  o.e = lup;
+  o.b = lh;
+  o.v = boost_back(b0, v, lup + lt);
+  return o;
+}
+
+// the four-node gather of one component and its derivatives along r and z
+// (src/eField.cpp:204-316), from the shares of the rings (per unit of z) of
+// its radial family
+struct RingW {
+  int ir;
+  double in, out, din, dout;  // shares of nodes ir, ir+1 and their r derivatives
+};
+__device__ __forceinline__ RingW ring_lo(const GridDesc &g, double r) {
+  RingW w;
+  w.ir = min(max(cell_number(r - 0.5 * g.dr, g.dr), 0), g.nr - 2);
+  const double r1 = r - 0.5 * g.dr, r3 = r + 0.5 * g.dr, r2 = (w.ir + 1) * g.dr;
+  const double p1 = kPi / cell_volume(w.ir + 1, g.dr, g.dz), p2 = kPi / cell_volume(w.ir + 3, g.dr, g.dz);
+  w.in = p1 * (r2 * r2 - r1 * r1);
+  w.out = p2 * (r3 * r3 - r2 * r2);
+  w.din = -2.0 * p1 * r1;
+  w.dout = 2.0 * p2 * r3;
+  return w;
+}
+__device__ __forceinline__ RingW ring_own(const GridDesc &g, double r) {
+  RingW w;
+  w.ir = min(max(cell_number(r, g.dr), 0), g.nr - 2);
+  const double r1 = r - 0.5 * g.dr, r3 = r + 0.5 * g.dr, r2 = (w.ir + 0.5) * g.dr;
+  const double p1 = kPi / ((r > g.dr) ? cell_volume(w.ir, g.dr, g.dz) : cyl_vol(g.dz, g.dr));
+  const double p2 = kPi / cell_volume(w.ir + 2, g.dr, g.dz);
+  w.in = p1 * (r2 * r2 - r1 * r1);
+  w.out = p2 * (r3 * r3 - r2 * r2);
+  w.din = -2.0 * p1 * r1;
+  w.dout = 2.0 * p2 * r3;
+  return w;
+}
+struct ColW {
+  int kz;
+  double d1, d2;  // distances to column kz+1 and from column kz
+};
+__device__ __forceinline__ ColW col_w(const GridDesc &g, double z, bool half) {
+  ColW c;
+  c.kz = min(max(cell_number(half ? z - 0.5 * g.dz : z, g.dz), 0), g.nz - 2);
+  const double z0 = (half ? c.kz + 0.5 : c.kz) * g.dz;
+  c.d1 = z0 + g.dz - z;
+  c.d2 = z - z0;
+  return c;
+}
+struct Gathered {
+  double v, dr, dz;
+};
+__device__ __forceinline__ Gathered gather_grad(const GridDesc &g, const double *F, const RingW &w, const ColW &c) {
+  const double *row0 = F + (size_t)w.ir * (size_t)g.nz + c.kz;
+  const double *row1 = row0 + g.nz;
+  const double f00 = row0[0], f01 = row0[1], f10 = row1[0], f11 = row1[1];
+  const double lo = f00 * c.d1 + f01 * c.d2, hi = f10 * c.d1 + f11 * c.d2;
+  return Gathered{w.in * lo + w.out * hi, w.din * lo + w.dout * hi, w.in * (f01 - f00) + w.out * (f11 - f10)};
+}
+
+// the adjoints of the gathered fields of one block's particles are summed in
+// an LDS box of kABR x kABK nodes per component (anchored one row and two
+// columns below the block's smallest cell) and added to the grid once per
+// block; stencils outside the box go to the grid directly
+constexpr int kABR = 4, kABK = 64, kABComp = 6;
+struct AdjBox {
+  double *box;  // LDS, kABComp x kABR x kABK
+  int bi, bk;   // node of box[.][0][0]
+};
+__device__ __forceinline__ void box_scatter(const GridDesc &g, const AdjBox &b, int comp, double *LF, const RingW &w,
+                                            const ColW &c, double lam) {
+  if (lam == 0.0) return;
+  // the shares of the nodes (ir, kz), (ir+1, kz), (ir, kz+1), (ir+1, kz+1)
+  const double v00 = w.in * c.d1 * lam, v10 = w.out * c.d1 * lam, v01 = w.in * c.d2 * lam, v11 = w.out * c.d2 * lam;
+  const int li = w.ir - b.bi, lk = c.kz - b.bk;
+  if ((unsigned)li < (unsigned)(kABR - 1) && (unsigned)lk < (unsigned)(kABK - 1)) {
+    double *q = b.box + (comp * kABR + li) * kABK + lk;
+    atomicAdd(q, v00);
+    atomicAdd(q + kABK, v10);
+    atomicAdd(q + 1, v01);
+    atomicAdd(q + kABK + 1, v11);
+  } else {
+    double *row0 = LF + (size_t)w.ir * (size_t)g.nz + c.kz;
+    double *row1 = row0 + g.nz;
+    unsafeAtomicAdd(row0, v00);
+    unsafeAtomicAdd(row1, v10);
+    unsafeAtomicAdd(row0 + 1, v01);
+    unsafeAtomicAdd(row1 + 1, v11);
+  }
+}
+
+// lambda_J at node (i, k), 0 off the grid
+__device__ __forceinline__ double lam_at(const GridDesc &g, const double *L, int i, int k) {
+  if ((unsigned)i >= (unsigned)g.nr || (unsigned)k >= (unsigned)g.nz) return 0.0;
+  return L[(size_t)i * (size_t)g.nz + (size_t)k];
+}
+
+// reverse of the J_phi deposit (azimuthal_current_distribution,
+// src/particles.cpp:688-784) of w charges q: adds to the adjoints of r, z,
+// v_phi; returns the weight's, sum lambda_J J / w
+__device__ __forceinline__ double jphi_back(const GridDesc &g, const double *L, double q, double w, double r, double z,
+                                            double vphi, double &lr, double &lz, double &lvphi) {
+  const double dr = g.dr, dz = g.dz;
+  const int i = max(cell_number(r, dr), 0), k = max(cell_number(z, dz), 0);
+  const double r1 = r - 0.5 * dr, r2 = (i + 0.5) * dr, r3 = r + 0.5 * dr;
+  const double i1 = 1.0 / ((r > dr) ? cell_volume(i, dr, dz) : cyl_vol(dz, dr)), i2 = 1.0 / cell_volume(i + 1, dr, dz);
+  const double d1 = (k + 0.5) * dz - (z - 0.5 * dz), d2 = (z + 0.5 * dz) - (k + 0.5) * dz;
+  const double l00 = lam_at(g, L, i, k) * i1, l10 = lam_at(g, L, i + 1, k) * i2;
+  const double l01 = lam_at(g, L, i, k + 1) * i1, l11 = lam_at(g, L, i + 1, k + 1) * i2;
+  const double in = r2 * r2 - r1 * r1, out = r3 * r3 - r2 * r2;
+  const double lo = l00 * d1 + l01 * d2, hi = l10 * d1 + l11 * d2;
+  const double G = in * lo + out * hi;
+  const double ir = 1.0 / r, K = q * ir / (2. * dz * dr);
+  lvphi += w * K * G;
+  lr += w * K * vphi * (2.0 * (r3 * hi - r1 * lo) - G * ir);
+  lz += w * K * vphi * (in * (l01 - l00) + out * (l11 - l10));
+  return K * vphi * G;
+}
+
+// M(x) = (log(1+x) - x) / x and its derivative (series below |x| = 0.1)
+__device__ __forceinline__ void m_and_slope(double x, double &M, double &dM) {
+  if (fabs(x) < 0.1) {
+    const double c[] = {1.0 / 11.0, -0.1, 1.0 / 9.0, -0.125, 1.0 / 7.0, -1.0 / 6.0, 0.2, -0.25, 1.0 / 3.0, -0.5};
+    double s = -1.0 / 12.0, d = 0.0;
+    for (double ck : c) {
+      d = s + x * d;
+      s = ck + x * s;
+    }
+    M = x * s;
+    dM = s + x * d;
+  } else {
+    M = (log1p(x) - x) / x;
+    dM = (1.0 / (1.0 + x) - 1.0 - M) / x;
+  }
+}
+
+// reverse of one straight piece inside cell (i, k), from the closed forms
+// above segment_d: S = sum lambda_J J and its derivatives with respect to the
+// piece's ends
+struct PieceAdj {
+  double s, rn, zn, ro, zo;
+};
+__device__ __forceinline__ PieceAdj segment_back(const GridDesc &g, const AdjGrid &lg, double q, double rn, double zn,
+                                                 double ro, double zo, int i, int k) {
+  const double dr = g.dr, dz = g.dz;
+  PieceAdj o{0.0, 0.0, 0.0, 0.0, 0.0};
+  if ((fabs(rn - ro) < kMnzl) || (fabs(zn - zo) < kMnzl)) return o;
+  const double fi = (double)i, idr = 1.0 / dr, idz = 1.0 / dz;
+  const double a = ro / dr - fi, b = zo / dz - (double)k, drho = (rn - ro) / dr, dzeta = (zn - zo) / dz;
+  const double kz = q / (4.0 * kPi * dr * dr * g.dt), kr = q / (2.0 * kPi * dr * dz * g.dt);
+  // lambda_J times the scales of the pairs (without the dzeta of J_z)
+  double gz0 = kz * lam_at(g, lg.ljz, i, k), gz1 = kz * lam_at(g, lg.ljz, i + 1, k);
+  double gr0 = kr * lam_at(g, lg.ljr, i, k), gr1 = kr * lam_at(g, lg.ljr, i, k + 1);
+  const double hdr = 0.5 * drho, ub = 1.0 - b, qdz = 0.25 * dzeta;
+  double sa, sb, sdr, sdz;
+  if (i == 0) {
+    const double j0 = 8.0 * (1.0 - hdr - a), j1 = hdr + 1.0 + a;
+    gr0 *= 2.0;
+    gr1 *= 2.0;
+    const double p0 = 0.5 * ub - qdz, p1 = 0.5 * b + qdz;
+    sdz = gz0 * j0 + gz1 * j1;
+    o.s = dzeta * sdz + drho * (gr0 * p0 + gr1 * p1);
+    sa = dzeta * (gz1 - 8.0 * gz0);
+    sdr = dzeta * (0.5 * gz1 - 4.0 * gz0) + gr0 * p0 + gr1 * p1;
+    sb = 0.5 * drho * (gr1 - gr0);
+    sdz += 0.25 * drho * (gr1 - gr0);
+  } else {
+    gz0 /= fi;
+    gz1 /= fi + 1.0;
+    const double ih = 1.0 / (fi + 0.5);
+    gr0 *= ih;
+    gr1 *= ih;
+    const double rs = fi + a, re = rs + drho, irs = 1.0 / rs, ire = 1.0 / re;
+    const double ii = fi * (fi + 1.0), x = drho * irs, t = drho * ire;
+    double M, dM;
+    m_and_slope(x, M, dM);
+    const double N = -t - M, iiM = ii * M, cc = 0.5 * ii * irs;
+    const double A0 = (1.0 - a) * (2.0 * fi + a) + iiM, A1 = a * (2.0 * fi + 1.0 + a) - iiM;
+    const double R0 = t * ub + dzeta * N, R1 = t * b - dzeta * N;
+    const double p0 = 0.5 * ub - qdz, p1 = 0.5 * b + qdz;
+    const double gd = gr0 - gr1;
+    const double jz = gz0 * (A0 * irs - hdr) + gz1 * (A1 * irs + hdr);  // per unit of dzeta
+    const double grR = gr0 * R0 + gr1 * R1, grp = gr0 * p0 + gr1 * p1;
+    o.s = dzeta * jz + drho * grp + cc * grR;
+    sdz = jz + gd * (cc * N - 0.25 * drho);
+    sb = -gd * (hdr + cc * t);
+    const double sM = dzeta * (gz0 - gz1) * ii * irs - gd * cc * dzeta;
+    const double st = cc * (gr0 * ub + gr1 * b - dzeta * gd);
+    const double sirs = dzeta * (gz0 * A0 + gz1 * A1) + 0.5 * ii * grR;
+    const double sx = sM * dM;
+    sa = dzeta * irs * (gz0 * (1.0 - 2.0 * fi - 2.0 * a) + gz1 * (2.0 * fi + 1.0 + 2.0 * a)) - sirs * irs * irs -
+         sx * x * irs - st * t * ire;
+    sdr = 0.5 * dzeta * (gz1 - gz0) + grp + sx * irs + st * rs * ire * ire;
+  }
+  o.rn = sdr * idr;
+  o.ro = (sa - sdr) * idr;
+  o.zn = sdz * idz;
+  o.zo = (sb - sdz) * idz;
+  return o;
+}
+
+// strict_d's sink in the reverse sweep: its four inputs are the dual
+// directions, the deposits are linear in q
+struct StrictSink {
+  const GridDesc *g;
+  const AdjGrid *lg;
+  PieceAdj o;
+  __device__ __forceinline__ void add(int comp, int i, int k, D v) {
+    const double l = lam_at(*g, comp == kAR ? lg->ljr : lg->ljz, i, k);
+    o.s += l * v.v;
+    o.rn += l * v.d[0];
+    o.zn += l * v.d[1];
+    o.ro += l * v.d[2];
+    o.zo += l * v.d[3];
+  }
+};
+
+// reverse of the J_r / J_z deposit of the straight path (ro, zo) -> (rn, zn)
+// (current_distribution, src/particles.cpp:480-685): the path is split at the
+// radial face r = rb (met at z1) and the axial face z = zb (met at r2) that it
+// crosses; with s the path parameter of the crossing, the adjoint of z1 goes
+// to the ends as (1-s, s) along z and times -dz/dr along r, that of r2 likewise
+__device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjGrid &lg, double q, double rn, double zn,
+                                                   double ro, double zo) {
+  const double dr = g.dr, dz = g.dz;
+  int i_n = max(cell_number(rn, dr), 0), k_n = max(cell_number(zn, dz), 0);
+  int i_o = max(cell_number(ro, dr), 0), k_o = max(cell_number(zo, dz), 0);
+  if (ro == (i_o + 1) * dr) i_o = i_n;
+  if (zo == (k_o + 1) * dz) k_o = k_n;
+  if (rn == (i_n + 1) * dr) i_n = i_o;
+  if (zn == (k_n + 1) * dz) k_n = k_o;
+  const int di = i_n - i_o, dk = k_n - k_o, res = abs(di) + abs(dk);
+  if ((fabs(rn - ro) < kMnzl) || (fabs(zn - zo) < kMnzl)) {
+    StrictSink sk{&g, &lg, {0.0, 0.0, 0.0, 0.0, 0.0}};
+    strict_d(g, sk, cst(q), seed(rn, 0), seed(zn, 1), seed(ro, 2), seed(zo, 3));
+    return sk.o;
+  }
+  // pieces: ns, the crossings in order (first / second), the cells before the last
+  int ns = 1, i0 = i_n, k0 = k_n, i1 = i_n, k1 = k_n;
+  bool rad = false, axi = false, rfirst = false;
+  double rb = 0.0, zb = 0.0, z1 = 0.0, r2 = 0.0;
+  const double slope = (rn - ro) / (zn - zo);
+  if (res == 1) {
+    ns = 2;
+    if (di != 0) {
+      rad = rfirst = true;
+      const bool up = !(ro > (i_n + 1) * dr);
+      rb = (up ? i_n : i_n + 1) * dr;
+      z1 = up ? zo + (rb - ro) / slope : zn + (rb - rn) / slope;
+      i0 = up ? i_n - 1 : i_n + 1;
+    } else {
+      axi = true;
+      const bool up = zo < k_n * dz;
+      zb = (up ? k_n : k_n + 1) * dz;
+      r2 = up ? ro + slope * (zb - zo) : rn + slope * (zb - zn);
+      k0 = up ? k_n - 1 : k_n + 1;
+    }
+  } else if (res == 2) {
+    // a path across a radial and an axial face; the other two-cell jumps are
+    // too long for a step and are treated as the forward pass treats them
+    const bool up = di > 0, right = dk > 0;
+    if (di == 0 || (!up && dk == 0)) {
+      ns = 0;
+    } else {
+      rad = axi = true;
+      rb = (up ? i_n : i_n + 1) * dr;
+      zb = (right ? k_n : k_n + 1) * dz;
+      const bool from_new = !up && !right;
+      z1 = from_new ? zn + (rb - rn) / slope : zo + (rb - ro) / slope;
+      r2 = from_new ? rn + (zb - zn) * slope : ro + (zb - zo) * slope;
+      ns = z1 == zb ? 0 : 3;
+      rfirst = right ? z1 < zb : z1 > zb;
+      i0 = up ? i_n - 1 : i_n + 1;
+      k0 = right ? k_n - 1 : k_n + 1;
+      i1 = rfirst ? i_n : i0;
+      k1 = rfirst ? k0 : k_n;
+    }
+  } else if (res > 2) {
+    ns = 0;
+  }
+  // the crossings in path order
+  const double cr0 = rfirst ? rb : r2, cz0 = rfirst ? z1 : zb;
+  const double cr1 = rfirst ? r2 : rb, cz1 = rfirst ? zb : z1;
+  PieceAdj o{0.0, 0.0, 0.0, 0.0, 0.0};
+  double c0r = 0.0, c0z = 0.0, c1r = 0.0, c1z = 0.0;  // adjoints of the crossings
+#pragma nounroll
+  for (int t = 0; t < ns; t++) {
+    const bool first = t == 0, last = t == ns - 1;
+    const PieceAdj p = segment_back(g, lg, q, last ? rn : first ? cr0 : cr1, last ? zn : first ? cz0 : cz1,
+                                    first ? ro : t == 1 ? cr0 : cr1, first ? zo : t == 1 ? cz0 : cz1,
+                                    last ? i_n : first ? i0 : i1, last ? k_n : first ? k0 : k1);
+    o.s += p.s;
+    if (first) {
+      o.ro += p.ro;
+      o.zo += p.zo;
+    } else if (t == 1) {
+      c0r += p.ro;
+      c0z += p.zo;
+    } else {
+      c1r += p.ro;
+      c1z += p.zo;
+    }
+    if (last) {
+      o.rn += p.rn;
+      o.zn += p.zn;
+    } else if (first) {
+      c0r += p.rn;
+      c0z += p.zn;
+    } else {
+      c1r += p.rn;
+      c1z += p.zn;
+    }
+  }
+  if (rad) {
+    const double l = rfirst ? c0z : c1z, s = (rb - ro) / (rn - ro), is = 1.0 / slope;
+    o.zo += (1.0 - s) * l;
+    o.zn += s * l;
+    o.ro -= is * (1.0 - s) * l;
+    o.rn -= is * s * l;
+  }
+  if (axi) {
+    const double l = rfirst ? c1r : c0r, s = (zb - zo) / (zn - zo);
+    o.ro += (1.0 - s) * l;
+    o.rn += s * l;
+    o.zo -= slope * (1.0 - s) * l;
+    o.zn -= slope * s * l;
+  }
+  return o;
+}
+
+// reflection_single / Bunch::reflection_single on the half-step point; sx, sz:
+// the signs that the reflections leave on (x, v_0) and (z, v_2)
+__device__ __forceinline__ void walls_sign(const GridDesc &g, bool is_bunch, double &x, double &z, double &sx,
+                                           double &sz, bool &alive) {
+  const double dr = g.dr, dz = g.dz;
+  const double radius_wall = g.r_size - dr / 2., longitude_wall = g.z_size - dz / 2.;
+  sx = sz = 1.0;
+  if (is_bunch) {
+    if (x > radius_wall || z > longitude_wall) alive = false;
+  } else {
+    if (x > radius_wall) {
+      x = radius_wall * 2. - x;
+      sx = -sx;
+    }
+    if (z > longitude_wall) {
+      z = longitude_wall * 2. - z;
+      sz = -sz;
+    }
+  }
+  if (x < dr / 2.) {
+    x = dr - x;
+    sx = -sx;
+  }
+  if (z < dz / 2.) {
+    z = dz - z;
+    sz = -sz;
+  }
+}
+
+// the vector-Jacobian product of one living particle's step
+template <bool VAY>
+__device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields &f, const AdjGrid &lg,
+                                             const AdjSpecies &s, long long i, const AdjBox &box) {
+  const double r0 = s.r[i], z0 = s.z[i], w = s.w[i];
+  const V3 v0 = {s.vr[i], s.vphi[i], s.vz[i]};
+  const double half_dt = g.dt / 2.;
+  // the scales of the push's fields: q / m does not depend on w
+  const double c1 = s.charge * g.dt / (2 * s.mass);
+  const double es = VAY ? 2 * c1 : c1, bs = VAY ? kMagnConst * c1 * (2 * c1) * c1 : kMagnConst * c1;
+  V3 e, h;
+  {
+    const RingW wl = ring_lo(g, r0), wo = ring_own(g, r0);
+    const ColW co = col_w(g, z0, false), ch = col_w(g, z0, true);
+    e = es * V3{gather_grad(g, f.er, wl, co).v, gather_grad(g, f.ephi, wo, co).v, gather_grad(g, f.ez, wo, ch).v};
+    h = bs * V3{gather_grad(g, f.hhr, wo, ch).v, gather_grad(g, f.hhphi, wl, ch).v, gather_grad(g, f.hhz, wl, co).v};
+  }
+  const V3 v = VAY ? vay_fwd(v0, e, h) : boris_fwd(v0, e, h);
+  // first half step and rotation (step_v), then full_current_distribution
+  const double x1 = r0 + v.x * half_dt, y = v.y * half_dt, z1 = z0 + v.z * half_dt;
+  const double r1 = sqrt(x1 * x1 + y * y);
+  double x2 = r1 + v.x * half_dt, z2 = z1 + v.z * half_dt, sx, sz;
+  bool alive = true;
+  walls_sign(g, s.is_bunch != 0, x2, z2, sx, sz, alive);
+  // adjoints: of v after the push, of the half-step point and of the start
+  V3 lv = {0.0, 0.0, 0.0};
+  double lr1 = 0.0, lz1 = 0.0, lr0 = 0.0, lz0 = 0.0, lw = 0.0;
+  if (alive) {
+    const double r2 = sqrt(x2 * x2 + y * y), ir2 = 1.0 / r2, st = y * ir2, ct = sqrt(1 - st * st);
+    const double o0 = s.lvr[i], o1 = s.lvphi[i], o2 = s.lvz[i];
+    const double vx = sx * v.x;  // after the walls
+    // rotation of the velocity by the second half step's angle
+    const double lst = vx * o1 - v.y * o0 - st / ct * (vx * o0 + v.y * o1);
+    const PieceAdj p = deposit_j_back(g, lg, s.charge, r2, z2, r0, z0);
+    lw += p.s;
+    lr0 = w * p.ro;
+    lz0 = w * p.zo;
+    const double lr2 = s.lr[i] + w * p.rn - lst * st * ir2, lz2 = s.lz[i] + w * p.zn;
+    const double lx2 = lr2 * x2 * ir2, ly2 = lr2 * st + lst * ir2;
+    lr1 = sx * lx2;
+    lz1 = sz * lz2;
+    lv.x = sx * (ct * o0 + st * o1) + half_dt * lr1;
+    lv.y = ct * o1 - st * o0 + half_dt * ly2;
+    lv.z = sz * o2 + half_dt * lz1;
+  }
+  lw += jphi_back(g, lg.ljphi, s.charge, w, r1, z1, v.y, lr1, lz1, lv.y);
+  const double ir1 = 1.0 / r1, lx1 = lr1 * x1 * ir1;
+  lr0 += lx1;
+  lz0 += lz1;
+  lv.x += half_dt * lx1;
+  lv.y += half_dt * (lr1 * y * ir1);
+  lv.z += half_dt * lz1;
+  V3 vb = v0, eb = e, hb = h;
+  asm volatile("" : "+v"(vb.x), "+v"(vb.y), "+v"(vb.z), "+v"(eb.x), "+v"(eb.y), "+v"(eb.z), "+v"(hb.x), "+v"(hb.y), "+v"(hb.z));
+  const PushBack p = VAY ? vay_back(vb, eb, hb, lv) : boris_back(vb, eb, hb, lv);
+  const V3 le = es * p.e, lh = bs * p.b;
+  double rg = r0, zg = z0;
+  asm volatile("" : "+v"(rg), "+v"(zg));
+  const RingW wl = ring_lo(g, rg), wo = ring_own(g, rg);
+  const ColW co = col_w(g, zg, false), ch = col_w(g, zg, true);
+  const Gathered e0 = gather_grad(g, f.er, wl, co), e1 = gather_grad(g, f.ephi, wo, co);
+  const Gathered e2 = gather_grad(g, f.ez, wo, ch), h0 = gather_grad(g, f.hhr, wo, ch);
+  const Gathered h1 = gather_grad(g, f.hhphi, wl, ch), h2 = gather_grad(g, f.hhz, wl, co);
+  s.lr[i] = lr0 + (le.x * e0.dr + le.y * e1.dr + le.z * e2.dr + lh.x * h0.dr + lh.y * h1.dr + lh.z * h2.dr);
+  s.lz[i] = lz0 + (le.x * e0.dz + le.y * e1.dz + le.z * e2.dz + lh.x * h0.dz + lh.y * h1.dz + lh.z * h2.dz);
+  s.lvr[i] = p.v.x;
+  s.lvphi[i] = p.v.y;
+  s.lvz[i] = p.v.z;
+  s.lw[i] += lw;
+  box_scatter(g, box, 0, lg.ler, wl, co, le.x);
+  box_scatter(g, box, 1, lg.lephi, wo, co, le.y);
+  box_scatter(g, box, 2, lg.lez, wo, ch, le.z);
+  box_scatter(g, box, 3, lg.lhr, wo, ch, lh.x);
+  box_scatter(g, box, 4, lg.lhphi, wl, ch, lh.y);
+  box_scatter(g, box, 5, lg.lhz, wl, co, lh.z);
+}
+
+#pragma clang fp contract(off)
+template <bool VAY>
+__global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, AdjGrid lg, AdjSpecies s) {
   __shared__ double box[kABComp * kABR * kABK];
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const bool live = i < s.n && s.alive[i] == 1;
@@ -796,7 +1234,7 @@ __global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, 
   for (int t = threadIdx.x; t < kABComp * kABR * kABK; t += blockDim.x) box[t] = 0.0;
   __syncthreads();
   const AdjBox b{box, ci - 1, ck - 2};
-  if (live) adj_particle(g, f, lg, s, pusher, i, b);
+  if (live) adj_particle<VAY>(g, f, lg, s, i, b);
   else if (i < s.n) s.lr[i] = s.lz[i] = s.lvr[i] = s.lvphi[i] = s.lvz[i] = 0.0;
   __syncthreads();
   double *const lf[kABComp] = {lg.ler, lg.lephi, lg.lez, lg.lhr, lg.lhphi, lg.lhz};
@@ -1148,7 +1586,11 @@ void launch_adj_particles(const GridDesc &g, const double *const *fields6, doubl
   AdjGrid lg{lam[9], lam[10], lam[11], lam[0], lam[1], lam[2], lam[6], lam[7], lam[8]};
   AdjSpecies s{r, z, vr, vphi, vz, w, alive, lstate[0], lstate[1], lstate[2], lstate[3], lstate[4], lw,
                charge, mass, n, is_bunch};
-  hipLaunchKernelGGL(k_adj_particles, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, f, lg, s, pusher);
+  const dim3 grid((unsigned)((n + 255) / 256));
+  if (pusher == 1)
+    hipLaunchKernelGGL(k_adj_particles<true>, grid, dim3(256), 0, st, g, f, lg, s);
+  else
+    hipLaunchKernelGGL(k_adj_particles<false>, grid, dim3(256), 0, st, g, f, lg, s);
 }
 
 void launch_adj_seed(const GridDesc &g, const double *ez, double *lez, int k0, int k1, double scale, double *phi,
