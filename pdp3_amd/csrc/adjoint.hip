@@ -842,22 +842,29 @@ __device__ __forceinline__ Gathered gather_grad(const GridDesc &g, const double 
 }
 
 // the adjoints of the gathered fields of one block's particles are summed in
-// an LDS box of kABR x kABK nodes per component (anchored one row and two
+// an LDS box of kR x kABK nodes per component (anchored one row and two
 // columns below the block's smallest cell) and added to the grid once per
-// block; stencils outside the box go to the grid directly
-constexpr int kABR = 4, kABK = 64, kABComp = 6;
+// block; stencils outside the box go to the grid directly.  A plasma block
+// lies along one row.  A bunch block spans the bunch's radius: in four rows
+// most of its 24 atomics a particle went to the same few grid nodes, and 6.4e4
+// bunch particles took as long as 2.6e6 plasma particles (330 us).
+constexpr int kABK = 64, kABComp = 6;
+template <bool BUNCH>
 struct AdjBox {
-  double *box;  // LDS, kABComp x kABR x kABK
+  static constexpr bool kBunch = BUNCH;
+  static constexpr int kR = BUNCH ? 16 : 4;
+  double *box;  // LDS, kABComp x kR x kABK
   int bi, bk;   // node of box[.][0][0]
 };
-__device__ __forceinline__ void box_scatter(const GridDesc &g, const AdjBox &b, int comp, double *LF, const RingW &w,
+template <class Box>
+__device__ __forceinline__ void box_scatter(const GridDesc &g, const Box &b, int comp, double *LF, const RingW &w,
                                             const ColW &c, double lam) {
   if (lam == 0.0) return;
   // the shares of the nodes (ir, kz), (ir+1, kz), (ir, kz+1), (ir+1, kz+1)
   const double v00 = w.in * c.d1 * lam, v10 = w.out * c.d1 * lam, v01 = w.in * c.d2 * lam, v11 = w.out * c.d2 * lam;
   const int li = w.ir - b.bi, lk = c.kz - b.bk;
-  if ((unsigned)li < (unsigned)(kABR - 1) && (unsigned)lk < (unsigned)(kABK - 1)) {
-    double *q = b.box + (comp * kABR + li) * kABK + lk;
+  if ((unsigned)li < (unsigned)(Box::kR - 1) && (unsigned)lk < (unsigned)(kABK - 1)) {
+    double *q = b.box + (comp * Box::kR + li) * kABK + lk;
     atomicAdd(q, v00);
     atomicAdd(q + kABK, v10);
     atomicAdd(q + 1, v01);
@@ -1141,9 +1148,9 @@ __device__ __forceinline__ void walls_sign(const GridDesc &g, bool is_bunch, dou
 }
 
 // the vector-Jacobian product of one living particle's step
-template <bool VAY>
+template <bool VAY, class Box>
 __device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields &f, const AdjGrid &lg,
-                                             const AdjSpecies &s, long long i, const AdjBox &box) {
+                                             const AdjSpecies &s, long long i, const Box &box) {
   const double r0 = s.r[i], z0 = s.z[i], w = s.w[i];
   const V3 v0 = {s.vr[i], s.vphi[i], s.vz[i]};
   const double half_dt = g.dt / 2.;
@@ -1163,7 +1170,7 @@ __device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields 
   const double r1 = sqrt(x1 * x1 + y * y);
   double x2 = r1 + v.x * half_dt, z2 = z1 + v.z * half_dt, sx, sz;
   bool alive = true;
-  walls_sign(g, s.is_bunch != 0, x2, z2, sx, sz, alive);
+  walls_sign(g, Box::kBunch, x2, z2, sx, sz, alive);
   // adjoints: of v after the push, of the half-step point and of the start
   V3 lv = {0.0, 0.0, 0.0};
   double lr1 = 0.0, lz1 = 0.0, lr0 = 0.0, lz0 = 0.0, lw = 0.0;
@@ -1218,9 +1225,11 @@ __device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields 
 }
 
 #pragma clang fp contract(off)
-template <bool VAY>
+template <bool VAY, bool BUNCH>
 __global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, AdjGrid lg, AdjSpecies s) {
-  __shared__ double box[kABComp * kABR * kABK];
+  using Box = AdjBox<BUNCH>;
+  constexpr int kSize = kABComp * Box::kR * kABK;
+  __shared__ double box[kSize];
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   const bool live = i < s.n && s.alive[i] == 1;
   // the box anchor: the smallest cell of the block's living particles
@@ -1231,17 +1240,17 @@ __global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, 
   }
   block_min2(ci, ck);
   if (ci == INT_MAX) ci = ck = 0;
-  for (int t = threadIdx.x; t < kABComp * kABR * kABK; t += blockDim.x) box[t] = 0.0;
+  for (int t = threadIdx.x; t < kSize; t += blockDim.x) box[t] = 0.0;
   __syncthreads();
-  const AdjBox b{box, ci - 1, ck - 2};
+  const Box b{box, ci - 1, ck - 2};
   if (live) adj_particle<VAY>(g, f, lg, s, i, b);
   else if (i < s.n) s.lr[i] = s.lz[i] = s.lvr[i] = s.lvphi[i] = s.lvz[i] = 0.0;
   __syncthreads();
   double *const lf[kABComp] = {lg.ler, lg.lephi, lg.lez, lg.lhr, lg.lhphi, lg.lhz};
-  for (int t = threadIdx.x; t < kABComp * kABR * kABK; t += blockDim.x) {
+  for (int t = threadIdx.x; t < kSize; t += blockDim.x) {
     const double v = box[t];
     if (v == 0.0) continue;
-    const int comp = t / (kABR * kABK), rem = t - comp * kABR * kABK;
+    const int comp = t / (Box::kR * kABK), rem = t - comp * Box::kR * kABK;
     const int gi = b.bi + rem / kABK, gk = b.bk + rem % kABK;
     // nodes off the grid never receive a stencil (gather_w clamps its cell)
     if ((unsigned)gi < (unsigned)g.nr && (unsigned)gk < (unsigned)g.nz)
@@ -1587,10 +1596,9 @@ void launch_adj_particles(const GridDesc &g, const double *const *fields6, doubl
   AdjSpecies s{r, z, vr, vphi, vz, w, alive, lstate[0], lstate[1], lstate[2], lstate[3], lstate[4], lw,
                charge, mass, n, is_bunch};
   const dim3 grid((unsigned)((n + 255) / 256));
-  if (pusher == 1)
-    hipLaunchKernelGGL(k_adj_particles<true>, grid, dim3(256), 0, st, g, f, lg, s);
-  else
-    hipLaunchKernelGGL(k_adj_particles<false>, grid, dim3(256), 0, st, g, f, lg, s);
+  auto kernel = pusher == 1 ? (is_bunch ? k_adj_particles<true, true> : k_adj_particles<true, false>)
+                            : (is_bunch ? k_adj_particles<false, true> : k_adj_particles<false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, g, f, lg, s);
 }
 
 void launch_adj_seed(const GridDesc &g, const double *ez, double *lez, int k0, int k1, double scale, double *phi,
