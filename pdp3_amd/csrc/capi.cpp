@@ -256,9 +256,9 @@ int init_beam(pdp3_ctx *ctx, bool inject = true) {
   return PDP3_OK;
 }
 
-int zero_grid(pdp3_ctx *ctx, int comp, int count = 1) {
+int zero_grid(pdp3_ctx *ctx, int comp) {
   Ctx &c = ctx->c;
-  launch_fill(c.a[comp], c.cells() * (size_t)count, 0.0, c.stream);  // the components are contiguous
+  launch_fill(c.a[comp], c.cells(), 0.0, c.stream);
   CHECK_LAUNCH(ctx);
   return PDP3_OK;
 }
@@ -980,14 +980,22 @@ int step_one(pdp3_ctx *ctx, const std::function<int()> *after_h) {
     if ((st = sort_plasma(ctx, false))) return st;
   }
   if ((st = init_beam(ctx))) return st;
-  if ((st = pdp3_hfield_calc(ctx))) return st;
+  {
+    // Current::reset_j and the bunch rho's reset in the H update's launch (J_r,
+    // J_phi, J_z and rho_bunch are consecutive components of the grid)
+    static_assert(kJPhi == kJR + 1 && kJZ == kJR + 2 && kRhoBunch == kJR + 3, "grid component order");
+    TimedScope ts(c, PDP3_KERNEL_H);
+    launch_h_update(c, true);
+    CHECK_LAUNCH(ctx);
+  }
   if (after_h && (st = (*after_h)())) return st;
-  // Current::reset_j and the bunch rho's reset in one launch (J_r, J_phi,
-  // J_z and rho_bunch are consecutive components of the grid)
-  static_assert(kJPhi == kJR + 1 && kJZ == kJR + 2 && kRhoBunch == kJR + 3, "grid component order");
-  if ((st = zero_grid(ctx, kJR, 4))) return st;
-  for (int j : c.order)
-    if ((st = particles_fused(ctx, c.species[j]))) return st;
+  // (live timing keeps plasma and bunch launches apart)
+  if (!c.profiling && (is_f32(c) ? launch_group_f32(c) : launch_group_f64(c))) {
+    CHECK_LAUNCH(ctx);
+  } else {
+    for (int j : c.order)
+      if ((st = particles_fused(ctx, c.species[j]))) return st;
+  }
   if ((st = pdp3_efield_calc(ctx))) return st;
   c.current_time = c.current_time + c.g.dt;  // src/loadInitParam.cpp:586
   c.steps_done++;

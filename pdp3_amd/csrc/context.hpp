@@ -205,8 +205,12 @@ struct Ctx {
   size_t cells() const { return (size_t)g.nr * (size_t)g.nz; }
 };
 
+// species that one launch can take (more are launched one by one)
+constexpr int kMaxGroup = 4;
+
 // ---- launchers (each enqueues on ctx.stream) ----
-void launch_h_update(Ctx &c);
+// reset_j: the same launch clears J and the bunch density
+void launch_h_update(Ctx &c, bool reset_j = false);
 void launch_e_update(Ctx &c);
 void launch_fill(double *p, size_t n, double v, hipStream_t s);
 void launch_gauss_residual(Ctx &c, const double *rho, double *out);
@@ -271,6 +275,9 @@ void launch_tlm_objective(const GridDesc &g, const double *ez, double *const *co
 
 // FP64 plain form
 void launch_fused_f64(Ctx &c, Species &sp);
+// every species of the loop in one launch, where they are small enough to be
+// bound by latency; false: not launched
+bool launch_group_f64(Ctx &c);
 void launch_step_v_f64(Ctx &c, Species &sp);
 void launch_full_current_f64(Ctx &c, Species &sp);
 // rho: target grid (nullptr: the bunch density)
@@ -280,6 +287,7 @@ void launch_bunch_inject_f64(Ctx &c, Species &sp, unsigned start, unsigned count
 
 // FP32 form
 void launch_fused_f32(Ctx &c, Species &sp);
+bool launch_group_f32(Ctx &c);  // as launch_group_f64
 int auto_tile(const Ctx &c, const Species &sp);  // kTileShapes index, or 6 / 7: 2 / 1 particles per lane x 4
 void launch_charge_weighting_f32(Ctx &c, Species &sp, double *rho = nullptr);
 void launch_bunch_inject_f32(Ctx &c, Species &sp, unsigned start, unsigned count, double dl);

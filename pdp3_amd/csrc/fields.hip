@@ -92,8 +92,20 @@ __device__ __forceinline__ void h_tile(const GridDesc &g, const HPtrs &f, int i0
   }
 }
 
-__global__ void __launch_bounds__(HTile::kThreads) k_h_update(GridDesc g, HPtrs f) {
+// j (may be null): J_r, J_phi, J_z and rho_bunch, consecutive grids of the same
+// shape, cleared by the threads of their nodes (Current::reset_j and
+// ChargeDensity::reset_rho of the loop, which nothing between the two reads):
+// a launch of its own for that took 4.3 us of a small run's 39 us step
+__global__ void __launch_bounds__(HTile::kThreads) k_h_update(GridDesc g, HPtrs f, double *j) {
   __shared__ double s[3 * HTile::kLds];
+  if (j) {
+    const int r = threadIdx.x / HTile::kCols, c = threadIdx.x - r * HTile::kCols;
+    const int i = blockIdx.y * HTile::kRows + r, k = blockIdx.x * HTile::kCols + c;
+    const size_t n = (size_t)g.nr * (size_t)g.nz;
+    if (i < g.nr && k < g.nz)
+#pragma unroll
+      for (int a = 0; a < 4; a++) j[a * n + at(g, i, k)] = 0.0;
+  }
   h_tile<HTile>(g, f, blockIdx.y * HTile::kRows, blockIdx.x * HTile::kCols, s);
 }
 
@@ -282,9 +294,11 @@ EPtrs eptrs(Ctx &c) {
                c.a[kER], c.a[kEPhi], c.a[kEZ]};
 }
 
-void launch_h_update(Ctx &c) {
-  dim3 grid((c.g.nz - 1 + HTile::kCols - 1) / HTile::kCols, (c.g.nr + HTile::kRows - 1) / HTile::kRows);
-  hipLaunchKernelGGL(k_h_update, grid, dim3(HTile::kThreads), 0, c.stream, c.g, hptrs(c));
+void launch_h_update(Ctx &c, bool reset_j) {
+  // (all nz columns of tiles: the last column of J is cleared too)
+  dim3 grid((c.g.nz + HTile::kCols - 1) / HTile::kCols, (c.g.nr + HTile::kRows - 1) / HTile::kRows);
+  hipLaunchKernelGGL(k_h_update, grid, dim3(HTile::kThreads), 0, c.stream, c.g, hptrs(c),
+                     reset_j ? c.a[kJR] : nullptr);
 }
 
 void launch_e_update(Ctx &c) {

@@ -16,6 +16,7 @@
 // is evaluated in FP64; the grid accumulation is FP64 (hardware FP64
 // atomics); fields and the PML stay FP64.
 #include <algorithm>
+#include <cstring>
 #include <vector>
 
 #include "context.hpp"
@@ -838,18 +839,6 @@ __global__ void __launch_bounds__(256) k_fused32_bunch(F32Args p, GlobalSink gs,
   fused32_bunch_tile<kWavesPerBlock, PPT>(p, gs, (long long)blockIdx.x * (kWavesPerBlock * 64 * PPT), n_cap, box);
 }
 
-// ensembles: the plasma tiles and bunch blocks of every instance in one
-// launch, one block per item of the work list (a persistent grid striding
-// over the list kept the loop's state in scalar registers, which spilled).
-// Bunch blocks take the plasma tile path too (their particles are not cell
-// sorted, so most of their gathers and deposits take the boxes' HBM
-// fallbacks), which keeps the kernel at the plasma path's register count.
-struct EnsItem {
-  int arg;   // index into the per-(instance, species) argument tables
-  int kind;  // 0 plasma tile, 1 bunch block
-  long long base, n_cap;
-};
-
 // A pointer read from device memory is generic (flat) to the compiler: its
 // loads, stores and atomics become flat instructions on 64-bit per-lane
 // addresses, which also hold up the kernel's LDS waits.  The ensemble's
@@ -919,6 +908,53 @@ __device__ __forceinline__ GlobalSink from_global(const GlobalSinkG &g) {
   s.err = (int *)g.err;
   return s;
 }
+
+// The species of one simulation in one launch: where none of them fills the
+// GPU a launch is bound by the latency of its blocks (a 1e3-particle bunch
+// takes 9.6 us beside a 1.6e5-particle plasma's 15), and they overlap.
+// first[s]: the first block of species s; the bunches come first, their
+// blocks (one particle per lane, global gathers) take the longest.
+struct F32Group {
+  F32ArgsG a[kMaxGroup];
+  GlobalSinkG sink;
+  int first[kMaxGroup];
+  long long n_cap[kMaxGroup];
+};
+
+template <int PPT>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_fused32_group(F32Group g) {
+  constexpr int kBunch = BunchSink::kSize, kTile = TileSink::kSize + (kFBoxFloats + 1) / 2;
+  __shared__ __align__(16) double lds[kBunch > kTile ? kBunch : kTile];
+  static_assert(TileSink::kSize % 2 == 0, "the field box behind the current box is 16-byte aligned");
+  int s = 0;
+#pragma unroll
+  for (int t = 1; t < kMaxGroup; t++) s += (int)blockIdx.x >= g.first[t] ? 1 : 0;
+  F32Args p = from_global(g.a[s]);
+  GlobalSink gs = from_global(g.sink);
+  gs.nr = p.nr;
+  gs.nz = p.nz;
+  gs.err = p.err;
+  const long long block = (int)blockIdx.x - g.first[s];
+  if (p.is_bunch) {
+    fused32_bunch_tile<kWavesPerBlock, 1>(p, gs, block * (kWavesPerBlock * 64), g.n_cap[s], lds);
+  } else {
+    p.want_rho = 0;
+    fused32_tile<PPT, kWavesPerBlock, TileSink>(p, gs, TileMap<PPT, kWavesPerBlock>::base(block), g.n_cap[s], lds,
+                                                reinterpret_cast<float *>(lds + TileSink::kSize));
+  }
+}
+
+// ensembles: the plasma tiles and bunch blocks of every instance in one
+// launch, one block per item of the work list (a persistent grid striding
+// over the list kept the loop's state in scalar registers, which spilled).
+// Bunch blocks take the plasma tile path too (their particles are not cell
+// sorted, so most of their gathers and deposits take the boxes' HBM
+// fallbacks), which keeps the kernel at the plasma path's register count.
+struct EnsItem {
+  int arg;   // index into the per-(instance, species) argument tables
+  int kind;  // 0 plasma tile, 1 bunch block
+  long long base, n_cap;
+};
 
 template <int PPT, int WAVES>
 // 5 waves per SIMD (96 VGPRs, 6 scalar registers spilled into vector lanes)
@@ -1118,6 +1154,9 @@ bool ensure_f32(Species &sp) {
 
 unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
 
+constexpr int kChunkTile = kNumTiles - 1;  // 4 x 4: one chunk per tile (the next shapes: 2 x 4 and 1 x 4)
+static_assert(kTileShapes[kChunkTile][0] * kTileShapes[kChunkTile][1] == kPPT, "one-chunk tile shape");
+
 }  // namespace
 
 template <int PPT, int WAVES>
@@ -1183,6 +1222,51 @@ void launch_fused_f32(Ctx &c, Species &sp) {
   }
 }
 
+template <int PPT>
+void launch_group_t(hipStream_t st, const F32Group &g, int blocks) {
+  hipLaunchKernelGGL(k_fused32_group<PPT>, dim3(blocks), dim3(256), 0, st, g);
+}
+
+bool launch_group_f32(Ctx &c) {
+  F32Group g;
+  int n = 0, tile = -1;
+  long long blocks = 0;
+  // bunches, then plasma species
+  for (int kind = 1; kind >= 0; kind--)
+    for (int j : c.order) {
+      Species &sp = c.species[j];
+      if (sp.n_cap <= 0 || !sp.f32.cell || (sp.kind == 1) != (kind == 1)) continue;
+      if (n == kMaxGroup) return false;
+      long long per = kWavesPerBlock * 64;
+      if (sp.chunked) {
+        // one shape, of at most a chunk, for all plasma species
+        const int t = c.tile_auto ? auto_tile(c, sp) : c.tile;
+        if (t < kChunkTile || (tile >= 0 && t != tile)) return false;
+        tile = t;
+        per *= t == kChunkTile ? 4 : t == kChunkTile + 1 ? 2 : 1;
+      } else if (sp.n_cap >= 1024 * per * 4) {
+        return false;  // a bunch that walks several particles per lane
+      }
+      const F32Args a = args32(c, sp);
+      memcpy(&g.a[n], &a, sizeof(a));
+      g.first[n] = (int)blocks;
+      g.n_cap[n] = sp.n_cap;
+      blocks += (sp.n_cap + per - 1) / per;
+      n++;
+    }
+  if (n < 2 || tile < 0 || blocks > 0x7fffffff) return false;
+  for (int t = n; t < kMaxGroup; t++) g.first[t] = 0x7fffffff;
+  const GlobalSink gs = sink32(c);
+  memcpy(&g.sink, &gs, sizeof(gs));
+  if (tile == kChunkTile)
+    launch_group_t<4>(c.stream, g, (int)blocks);
+  else if (tile == kChunkTile + 1)
+    launch_group_t<2>(c.stream, g, (int)blocks);
+  else
+    launch_group_t<1>(c.stream, g, (int)blocks);
+  return true;
+}
+
 void launch_charge_weighting_f32(Ctx &c, Species &sp, double *rho) {
   if (sp.n_cap <= 0 || !sp.f32.cell) return;
   GlobalSink gs = sink32(c);
@@ -1228,8 +1312,6 @@ struct EnsParticles {
 
 namespace {
 constexpr int kSparsePpc = 16;
-constexpr int kChunkTile = kNumTiles - 1;  // 4 x 4: one chunk per tile
-static_assert(kTileShapes[kChunkTile][0] * kTileShapes[kChunkTile][1] == kPPT, "one-chunk tile shape");
 // the argument table and the work lists of the ensemble's species
 void ens_lists(const std::vector<Ctx *> &ctxs, std::vector<F32Args> *args,
                std::vector<EnsItem> items[kNumTiles + 1]) {

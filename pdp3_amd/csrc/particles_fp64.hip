@@ -682,11 +682,11 @@ __device__ __forceinline__ void step_particle(const GridDesc &g, const Fields &f
 // at cfg3 against 26.7 ms for the IEEE divisions at 3 waves (168 VGPRs, 12
 // spilled); forcing 3 waves with div_cr spills 146 VGPRs (43 ms)
 template <int PPT>
-__global__ void __launch_bounds__(256)
-k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_cap, int pusher) {
-  __shared__ double box[TileSink::kSize];
+__device__ __forceinline__ void fused_tile(const GridDesc &g, const Fields &f, const GlobalSink &gs,
+                                           const SpeciesArgs &s, long long n_cap, int pusher, long long tile,
+                                           double *box) {
   using Map = TileMap<PPT, kWavesPerBlock>;
-  const long long base = Map::base(blockIdx.x);
+  const long long base = Map::base(tile);
   // anchor samples: slot base + j is the logical particle 16 j of the tile
   int ai, ak;
   {
@@ -713,15 +713,22 @@ k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_ca
   box_flush(box, sk);
 }
 
+template <int PPT>
+__global__ void __launch_bounds__(256)
+k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_cap, int pusher) {
+  __shared__ double box[TileSink::kSize];
+  fused_tile<PPT>(g, f, gs, s, n_cap, pusher, blockIdx.x, box);
+}
+
 // bunches (plain layout): the tiled walk with the box anchored at the
 // smallest living cell of the block; PPT particles per lane (wave w of a
 // block takes the 64 * PPT slots from w * 64 * PPT), few for a small bunch so
 // that its blocks still spread over the GPU
 template <int PPT>
-__global__ void __launch_bounds__(256) k_fused_bunch(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s,
-                                                     long long n_cap, int pusher) {
-  __shared__ double box[BunchSink::kSize];
-  const long long base = (long long)blockIdx.x * (kWavesPerBlock * 64 * PPT);
+__device__ __forceinline__ void fused_bunch(const GridDesc &g, const Fields &f, const GlobalSink &gs,
+                                            const SpeciesArgs &s, long long n_cap, int pusher, long long block,
+                                            double *box) {
+  const long long base = block * (kWavesPerBlock * 64 * PPT);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long long cbase = base + (long long)wave * (64 * PPT) + lane;
   int ai = 0x7fffffff, ak = 0x7fffffff;
@@ -744,6 +751,55 @@ __global__ void __launch_bounds__(256) k_fused_bunch(GridDesc g, Fields f, Globa
   sk.flush();
   __syncthreads();
   box_flush(box, sk);
+}
+
+template <int PPT>
+__global__ void __launch_bounds__(256) k_fused_bunch(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s,
+                                                     long long n_cap, int pusher) {
+  __shared__ double box[BunchSink::kSize];
+  fused_bunch<PPT>(g, f, gs, s, n_cap, pusher, blockIdx.x, box);
+}
+
+// The species of one simulation in one launch, one particle per lane: where
+// none of them fills the GPU a launch is bound by the latency of its blocks (a
+// 1e3-particle bunch takes 14 us beside a 1.6e5-particle plasma's 22), and they
+// overlap.  first[s]: the first block of species s.  The pointers are in the
+// global address space (SpeciesArgs read from an array would have generic ones).
+template <class T>
+using gptr = __attribute__((address_space(1))) T *;
+struct SpeciesArgsG {
+  gptr<double> r, z, vr, vphi, vz;
+  gptr<const double> w;
+  gptr<uint8_t> alive;
+  double charge, mass;
+  long long n_cap;
+  int first, is_bunch;
+};
+struct F64Group {
+  SpeciesArgsG a[kMaxGroup];
+};
+__global__ void __launch_bounds__(256) k_fused_group(GridDesc g, Fields f, GlobalSink gs, F64Group grp, int pusher) {
+  __shared__ double box[BunchSink::kSize > TileSink::kSize ? BunchSink::kSize : TileSink::kSize];
+  int t = 0;
+#pragma unroll
+  for (int j = 1; j < kMaxGroup; j++) t += (int)blockIdx.x >= grp.a[j].first ? 1 : 0;
+  const SpeciesArgsG &a = grp.a[t];
+  SpeciesArgs s{};
+  s.r = (double *)a.r;
+  s.z = (double *)a.z;
+  s.vr = (double *)a.vr;
+  s.vphi = (double *)a.vphi;
+  s.vz = (double *)a.vz;
+  s.w = (const double *)a.w;
+  s.alive = (uint8_t *)a.alive;
+  s.charge = a.charge;
+  s.mass = a.mass;
+  s.is_bunch = a.is_bunch;
+  const long long block = (int)blockIdx.x - a.first;
+  if (a.is_bunch)
+    fused_bunch<1>(g, f, gs, s, a.n_cap, pusher, block, box);
+  else
+    fused_tile<1>(g, f, gs, s, a.n_cap, pusher, block, box);
 }
 
 // plain layout, one particle per thread, deposits straight to HBM
@@ -909,6 +965,40 @@ void launch_fused_f64(Ctx &c, Species &sp) {
       hipLaunchKernelGGL(k_fused_bunch<1>, dim3((unsigned)((n + per - 1) / per)), dim3(256), 0, c.stream, c.g,
                          fields_of(c), sink_of(c), args_of(sp), n, c.pusher);
   }
+}
+
+bool launch_group_f64(Ctx &c) {
+  F64Group g;
+  int n = 0;
+  long long blocks = 0;
+  // bunches first: their blocks take the longest
+  for (int kind = 1; kind >= 0; kind--)
+    for (int j : c.order) {
+      Species &sp = c.species[j];
+      if (sp.n_cap <= 0 || (sp.kind == 1) != (kind == 1)) continue;
+      constexpr long long kPer = kWavesPerBlock * 64;
+      if (n == kMaxGroup || sp.n_cap >= (sp.chunked ? kOneEach : 1024 * kPer * 4)) return false;
+      const SpeciesArgs s = args_of(sp);
+      SpeciesArgsG &a = g.a[n++];
+      a.r = (gptr<double>)s.r;
+      a.z = (gptr<double>)s.z;
+      a.vr = (gptr<double>)s.vr;
+      a.vphi = (gptr<double>)s.vphi;
+      a.vz = (gptr<double>)s.vz;
+      a.w = (gptr<const double>)s.w;
+      a.alive = (gptr<uint8_t>)s.alive;
+      a.charge = s.charge;
+      a.mass = s.mass;
+      a.is_bunch = s.is_bunch;
+      a.n_cap = sp.n_cap;
+      a.first = (int)blocks;
+      blocks += (sp.n_cap + kPer - 1) / kPer;
+    }
+  if (n < 2) return false;
+  for (int t = n; t < kMaxGroup; t++) g.a[t].first = 0x7fffffff;
+  hipLaunchKernelGGL(k_fused_group, dim3((unsigned)blocks), dim3(256), 0, c.stream, c.g, fields_of(c), sink_of(c), g,
+                     c.pusher);
+  return true;
 }
 
 void launch_step_v_f64(Ctx &c, Species &sp) {
