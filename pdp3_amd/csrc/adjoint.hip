@@ -20,6 +20,9 @@
 // (EField::calc_field, src/eField.cpp:85-170, PML in Ke / Kh) are transposed
 // node by node in pull form (no atomics).  The particle step follows
 // particles_fp64.hip expression for expression.
+#include <algorithm>
+#include <climits>
+
 #include "context.hpp"
 #include "crmath.hpp"
 #include "sink.hpp"
@@ -139,14 +142,49 @@ struct AdjGrid {
   double *ler, *lephi, *lez, *lhr, *lhphi, *lhz;  // adjoint of E^n, Hh^n (scatter, atomics)
 };
 struct AdjSpecies {
-  const double *r, *z, *vr, *vphi, *vz, *w;  // state at step n
-  const uint8_t *alive;
+  StateRef st;                          // state at step n
   double *lr, *lz, *lvr, *lvphi, *lvz;  // in: adjoint of the state after step n; out: before
   double *lw;                           // accumulated adjoint of the weight
   double charge, mass;
-  long long n;
-  int is_bunch;
+  long long n;                          // slots
 };
+
+// the particle in slot i of either form, in FP64 as a download gives it (r and
+// z from the cell and its offsets, v = u / gamma in the FP32 form); false: dead
+struct AdjParticle {
+  double r, z, vr, vphi, vz, w;
+};
+template <bool F32>
+__device__ __forceinline__ bool adj_load(const GridDesc &g, const StateRef &s, long long i, AdjParticle &p) {
+  if (F32) {
+    const uint32_t c = s.cell[i];
+    if (c & 0x80000000u) return false;
+    p.r = ((double)(int)((c >> 16) & 0x7FFF) + (double)s.fa[i]) * g.dr;
+    p.z = ((double)(int)(c & 0xFFFF) + (double)s.fb[i]) * g.dz;
+    const double u0 = s.ur[i], u1 = s.uphi[i], u2 = s.uz[i];
+    const double ig = 1.0 / sqrt(1.0 + (u0 * u0 + u1 * u1 + u2 * u2) / (kLightSpeed * kLightSpeed));
+    p.vr = u0 * ig;
+    p.vphi = u1 * ig;
+    p.vz = u2 * ig;
+    p.w = s.fw[i];
+  } else {
+    if (s.alive[i] != 1) return false;
+    p.r = s.r[i];
+    p.z = s.z[i];
+    p.vr = s.vr[i];
+    p.vphi = s.vphi[i];
+    p.vz = s.vz[i];
+    p.w = s.w[i];
+  }
+  return true;
+}
+// the slot of this thread: plasma blocks take 256 consecutive logical
+// particles of the chunked layout, which lie along one run of cells
+template <bool BUNCH>
+__device__ __forceinline__ long long adj_slot() {
+  if (BUNCH) return (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  return TileMap<1, 4>::base(blockIdx.x) + TileMap<1, 4>::first(threadIdx.x);
+}
 
 __device__ __forceinline__ int cell_number(double x, double dx) { return (int)ceil(x / dx) - 1; }
 __device__ __forceinline__ double cell_volume(int i, double dr, double dz) { return kPi * dz * dr * dr * 2.0 * i; }
@@ -1150,9 +1188,9 @@ __device__ __forceinline__ void walls_sign(const GridDesc &g, bool is_bunch, dou
 // the vector-Jacobian product of one living particle's step
 template <bool VAY, class Box>
 __device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields &f, const AdjGrid &lg,
-                                             const AdjSpecies &s, long long i, const Box &box) {
-  const double r0 = s.r[i], z0 = s.z[i], w = s.w[i];
-  const V3 v0 = {s.vr[i], s.vphi[i], s.vz[i]};
+                                             const AdjSpecies &s, long long i, const AdjParticle &pt, const Box &box) {
+  const double r0 = pt.r, z0 = pt.z, w = pt.w;
+  const V3 v0 = {pt.vr, pt.vphi, pt.vz};
   const double half_dt = g.dt / 2.;
   // the scales of the push's fields: q / m does not depend on w
   const double c1 = s.charge * g.dt / (2 * s.mass);
@@ -1225,25 +1263,26 @@ __device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields 
 }
 
 #pragma clang fp contract(off)
-template <bool VAY, bool BUNCH>
+template <bool VAY, bool BUNCH, bool F32>
 __global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, AdjGrid lg, AdjSpecies s) {
   using Box = AdjBox<BUNCH>;
   constexpr int kSize = kABComp * Box::kR * kABK;
   __shared__ double box[kSize];
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool live = i < s.n && s.alive[i] == 1;
+  const long long i = adj_slot<BUNCH>();
+  AdjParticle pt;
+  const bool live = i < s.n && adj_load<F32>(g, s.st, i, pt);
   // the box anchor: the smallest cell of the block's living particles
   int ci = INT_MAX, ck = INT_MAX;
   if (live) {
-    ci = max(cell_number(s.r[i], g.dr), 0);
-    ck = max(cell_number(s.z[i], g.dz), 0);
+    ci = max(cell_number(pt.r, g.dr), 0);
+    ck = max(cell_number(pt.z, g.dz), 0);
   }
   block_min2(ci, ck);
   if (ci == INT_MAX) ci = ck = 0;
   for (int t = threadIdx.x; t < kSize; t += blockDim.x) box[t] = 0.0;
   __syncthreads();
   const Box b{box, ci - 1, ck - 2};
-  if (live) adj_particle<VAY>(g, f, lg, s, i, b);
+  if (live) adj_particle<VAY>(g, f, lg, s, i, pt, b);
   else if (i < s.n) s.lr[i] = s.lz[i] = s.lvr[i] = s.lvphi[i] = s.lvz[i] = 0.0;
   __syncthreads();
   double *const lf[kABComp] = {lg.ler, lg.lephi, lg.lez, lg.lhr, lg.lhphi, lg.lhz};
@@ -1275,27 +1314,50 @@ struct TlmJ {  // tangents of J^n, one set per direction
   double *jr[kDN], *jphi[kDN], *jz[kDN];
 };
 struct TlmSpecies {
-  const double *r, *z, *vr, *vphi, *vz, *w;  // state at step n (values)
-  const uint8_t *alive;
+  StateRef st;                          // state at step n (values)
   double *tr, *tz, *tvr, *tvphi, *tvz;  // kDN x n tangents: in at step n, out at n+1
   const double *tw;                     // kDN x n tangents of the weight
   double charge, mass;
-  long long n;
-  int is_bunch;
+  long long n;                          // slots
 };
 
 // deposit tangents: every contribution v at node (i, k) adds its derivative
-// part (one per direction) to the tangent J grids
+// part (one per direction) to the tangent J grids, through an LDS box of kR x
+// kK nodes per component and direction for the nodes around the block's
+// smallest cell (a particle's 48 global atomics, those of a bunch all on the
+// same few nodes, were most of the kernel)
+template <bool BUNCH>
 struct TlmSink {
+  static constexpr int kR = BUNCH ? 16 : 4, kK = BUNCH ? 32 : 64, kSize = 3 * kDN * kR * kK;
   const GridDesc *g;
   TlmJ j;
+  double *box;  // LDS
+  int bi, bk;   // node of box[.][0][0]
   __device__ __forceinline__ void add(int comp, int i, int k, D v) {
     if ((unsigned)i >= (unsigned)g->nr || (unsigned)k >= (unsigned)g->nz) return;
+    const int li = i - bi, lk = k - bk;
+    if ((unsigned)li < (unsigned)kR && (unsigned)lk < (unsigned)kK) {
+      double *q = box + (comp * kDN * kR + li) * kK + lk;
+#pragma unroll
+      for (int d = 0; d < kDN; d++)
+        if (v.d[d] != 0.0) atomicAdd(q + d * kR * kK, v.d[d]);
+      return;
+    }
     const size_t p = (size_t)i * (size_t)g->nz + (size_t)k;
 #pragma unroll
     for (int d = 0; d < kDN; d++) {
       double *J = comp == kAR ? j.jr[d] : comp == kAPhi ? j.jphi[d] : j.jz[d];
       if (v.d[d] != 0.0) unsafeAtomicAdd(J + p, v.d[d]);
+    }
+  }
+  __device__ __forceinline__ void flush() const {
+    for (int t = threadIdx.x; t < kSize; t += blockDim.x) {
+      const double v = box[t];
+      if (v == 0.0) continue;
+      const int plane = t / (kR * kK), rem = t - plane * kR * kK;
+      const int i = bi + rem / kK, k = bk + rem % kK, comp = plane / kDN, d = plane - comp * kDN;
+      double *const *J = comp == kAR ? j.jr : comp == kAPhi ? j.jphi : j.jz;
+      unsafeAtomicAdd(J[d] + (size_t)i * (size_t)g->nz + k, v);  // add() keeps off-grid nodes out
     }
   }
 };
@@ -1311,12 +1373,12 @@ __device__ __forceinline__ double gather_value(const GridDesc &g, const double *
   return gw.w[0].v * row0[0] + gw.w[1].v * row1[0] + gw.w[2].v * row0[1] + gw.w[3].v * row1[1];
 }
 
-__global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, TlmFields tf, TlmJ tj,
-                                                       TlmSpecies s, int pusher) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= s.n) return;
+template <bool BUNCH, class Sink>
+__device__ __forceinline__ void tlm_particle(const GridDesc &g, const AdjFields &f, const TlmFields &tf, Sink &sk,
+                                             const TlmSpecies &s, int pusher, long long i, bool live,
+                                             const AdjParticle &pt) {
   const long long n = s.n;
-  if (s.alive[i] != 1) {
+  if (!live) {
     // dead (or padding) slots keep zero tangents; a particle injected later
     // starts with zero tangents, as its injected state does not depend on w
 #pragma unroll
@@ -1331,10 +1393,9 @@ __global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, 
     for (int d = 0; d < kDN; d++) x.d[d] = t[d * n + i];
     return x;
   };
-  TlmSink sk{&g, tj};
-  D r = dual(s.r[i], s.tr), z = dual(s.z[i], s.tz);
-  D v[3] = {dual(s.vr[i], s.tvr), dual(s.vphi[i], s.tvphi), dual(s.vz[i], s.tvz)};
-  D w = dual(s.w[i], s.tw);
+  D r = dual(pt.r, s.tr), z = dual(pt.z, s.tz);
+  D v[3] = {dual(pt.vr, s.tvr), dual(pt.vphi, s.tvphi), dual(pt.vz, s.tvz)};
+  D w = dual(pt.w, s.tw);
   D q = s.charge * w, m = s.mass * w;
   const D r_old = r, z_old = z;
   const double r0v = r.v, z0v = z.v;
@@ -1368,7 +1429,7 @@ __global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, 
   y = 0.0 + v[1] * half_dt;
   z = z + v[2] * half_dt;
   bool alive = true;
-  walls_d(g, s.is_bunch != 0, x, z, v[0], v[2], alive);
+  walls_d(g, BUNCH, x, z, v[0], v[2], alive);
   D rr = dsqrt(x * x + y * y);
   D st = y / rr;
   r = rr;
@@ -1389,6 +1450,29 @@ __global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, 
     s.tvphi[d * n + i] = keep ? v[1].d[d] : 0.0;
     s.tvz[d * n + i] = keep ? v[2].d[d] : 0.0;
   }
+}
+
+template <bool BUNCH, bool F32>
+__global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, TlmFields tf, TlmJ tj, TlmSpecies s,
+                                                       int pusher) {
+  using Sink = TlmSink<BUNCH>;
+  __shared__ double box[Sink::kSize];
+  const long long i = adj_slot<BUNCH>();
+  AdjParticle pt;
+  const bool live = i < s.n && adj_load<F32>(g, s.st, i, pt);
+  int ci = INT_MAX, ck = INT_MAX;
+  if (live) {
+    ci = max(cell_number(pt.r, g.dr), 0);
+    ck = max(cell_number(pt.z, g.dz), 0);
+  }
+  block_min2(ci, ck);
+  if (ci == INT_MAX) ci = ck = 0;
+  for (int t = threadIdx.x; t < Sink::kSize; t += blockDim.x) box[t] = 0.0;
+  __syncthreads();
+  Sink sk{&g, tj, box, ci - 1, ck - 2};
+  if (i < s.n) tlm_particle<BUNCH>(g, f, tf, sk, s, pusher, i, live, pt);
+  __syncthreads();
+  sk.flush();
 }
 
 // tangent of the objective: phi_dot[d] += scale * sum 2 E_z(0, k) E_z-dot_d(0, k)
@@ -1419,8 +1503,9 @@ __global__ void __launch_bounds__(256) k_tlm_objective(GridDesc g, const double 
 
 // ------------------------------------------------------------- the fields
 
-struct AdjE {  // adjoints of E, H (after step), Hh, J and the coefficients
+struct AdjE {  // adjoints of E, H (after step), Hh, J and the coefficients; E of the pass before: ler.., scaled: ser..
   double *ler, *lephi, *lez, *lhr, *lhphi, *lhz, *lhhr, *lhhphi, *lhhz, *ljr, *ljphi, *ljz;
+  double *ser, *sephi, *sez;
   const double *ke, *kh;
 };
 
@@ -1433,8 +1518,11 @@ __device__ __forceinline__ bool upd_ephi(const GridDesc &g, int i, int k) {
 }
 __device__ __forceinline__ bool upd_ez(const GridDesc &g, int i, int k) { return i <= g.nr - 2 && k <= g.nz - 2; }
 
-// step 1a: lambda_H += C^T (Kh lambda_E), lambda_J = -Kh lambda_E (pull form:
-// each H node sums the E nodes whose update reads it)
+// step 1, with step 3b of the iteration after it (lambda_H <- lambda_H +
+// lambda_Hh, lambda_Hh <- 0, each node its own): lambda_H += C^T (Kh lambda_E),
+// lambda_J = -Kh lambda_E (pull form: each H node sums the E nodes whose update
+// reads it), and lambda_E scaled by Ke on the updated entries into the other
+// set of E grids, as the neighbours still read this one
 __global__ void __launch_bounds__(256) k_adj_e_curl(GridDesc g, AdjE a) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   const int i = blockIdx.y;
@@ -1462,28 +1550,23 @@ __global__ void __launch_bounds__(256) k_adj_e_curl(GridDesc g, AdjE a) {
     const size_t pu = p + g.nz;
     lhphi += a.kh[pu] * (-1.0 / dr + 1.0 / (2.0 * dr * (i + 1))) * a.lez[pu];
   }
-  a.lhphi[p] += lhphi;
+  a.lhphi[p] = (a.lhphi[p] + a.lhhphi[p]) + lhphi;
   // H_r(i, k): E_phi(i, k) has +Kh (H_r(i,k) - H_r(i,k-1)) / dz, E_phi(i, k+1) -
   double lhr = 0.0;
   if (upd_ephi(g, i, k)) lhr += a.kh[p] / dz * a.lephi[p];
   if (k + 1 < g.nz && upd_ephi(g, i, k + 1)) lhr += -a.kh[p + 1] / dz * a.lephi[p + 1];
-  a.lhr[p] += lhr;
+  a.lhr[p] = (a.lhr[p] + a.lhhr[p]) + lhr;
   // H_z(i, k): E_phi(i, k) has -Kh (H_z(i,k) - H_z(i-1,k)) / dr, E_phi(i+1, k) +
   double lhz = 0.0;
   if (upd_ephi(g, i, k)) lhz += -a.kh[p] / dr * a.lephi[p];
   if (i + 1 < g.nr && upd_ephi(g, i + 1, k)) lhz += a.kh[p + g.nz] / dr * a.lephi[p + g.nz];
-  a.lhz[p] += lhz;
-}
-
-// step 1b: lambda_E <- Ke lambda_E on the updated entries
-__global__ void __launch_bounds__(256) k_adj_e_scale(GridDesc g, AdjE a) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = blockIdx.y;
-  if (k >= g.nz) return;
-  const size_t p = at(g, i, k);
-  if (upd_er(g, i, k)) a.ler[p] *= a.ke[p];
-  if (upd_ephi(g, i, k)) a.lephi[p] *= a.ke[p];
-  if (upd_ez(g, i, k)) a.lez[p] *= a.ke[p];
+  a.lhz[p] = (a.lhz[p] + a.lhhz[p]) + lhz;
+  a.lhhr[p] = 0.0;
+  a.lhhphi[p] = 0.0;
+  a.lhhz[p] = 0.0;
+  a.ser[p] = upd_er(g, i, k) ? a.ler[p] * a.ke[p] : a.ler[p];
+  a.sephi[p] = upd_ephi(g, i, k) ? a.lephi[p] * a.ke[p] : a.lephi[p];
+  a.sez[p] = upd_ez(g, i, k) ? a.lez[p] * a.ke[p] : a.lez[p];
 }
 
 // step 3a: lambda_alpha = lambda_H + lambda_Hh / 2 (H_z: -(...)), pulled into
@@ -1522,23 +1605,9 @@ __global__ void __launch_bounds__(256) k_adj_h(GridDesc g, AdjE a) {
   double le_z = dt / (dr * mu) * (la_phi(i - 1, k) - la_phi(i, k));
   // E_r(i,k): H_phi(i,k-1) -dt/(dz mu), H_phi(i,k) +dt/(dz mu)
   double le_r = dt / (dz * mu) * (la_phi(i, k) - la_phi(i, k - 1));
-  a.ler[p] += le_r;
-  a.lephi[p] += le_phi;
-  a.lez[p] += le_z;
-}
-
-// step 3b: lambda_H <- lambda_H + lambda_Hh, lambda_Hh <- 0
-__global__ void __launch_bounds__(256) k_adj_h_fin(GridDesc g, AdjE a) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  const int i = blockIdx.y;
-  if (k >= g.nz) return;
-  const size_t p = at(g, i, k);
-  a.lhr[p] += a.lhhr[p];
-  a.lhphi[p] += a.lhhphi[p];
-  a.lhz[p] += a.lhhz[p];
-  a.lhhr[p] = 0.0;
-  a.lhhphi[p] = 0.0;
-  a.lhhz[p] = 0.0;
+  a.ser[p] += le_r;
+  a.sephi[p] += le_phi;
+  a.sez[p] += le_z;
 }
 
 // objective seed: lambda_Ez(0, k) += scale * 2 E_z(0, k) on k0..k1, and the
@@ -1561,44 +1630,70 @@ __global__ void __launch_bounds__(256) k_adj_seed(GridDesc g, const double *ez, 
   if (threadIdx.x == 0) *phi += part[0];
 }
 
+// several device-to-device copies in one launch (grid.y: the copy), 16 bytes a
+// thread and pass
+constexpr int kCopies = 24;
+struct CopyArgs {
+  CopySeg seg[kCopies];
+};
+__global__ void __launch_bounds__(256) k_copy(CopyArgs a) {
+  const CopySeg s = a.seg[blockIdx.y];
+  const size_t n = s.bytes / sizeof(uint4), stride = (size_t)gridDim.x * blockDim.x;
+  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (size_t i = t; i < n; i += stride) ((uint4 *)s.dst)[i] = ((const uint4 *)s.src)[i];
+  if (t < s.bytes - n * sizeof(uint4)) ((uint8_t *)s.dst)[n * sizeof(uint4) + t] = ((const uint8_t *)s.src)[n * sizeof(uint4) + t];
+}
+
 }  // namespace
 
 // ------------------------------------------------------------- launchers
 
-struct AdjLaunch {
-  GridDesc g;
-  AdjE e;
-};
-
-void launch_adj_fields_pre(const GridDesc &g, double *const *lam, const double *ke, const double *kh,
-                           hipStream_t st) {
-  AdjE a{lam[0], lam[1], lam[2], lam[3], lam[4], lam[5], lam[6], lam[7], lam[8], lam[9], lam[10], lam[11], ke, kh};
-  dim3 grid((g.nz + 255) / 256, g.nr);
-  hipLaunchKernelGGL(k_adj_e_curl, grid, dim3(256), 0, st, g, a);
-  hipLaunchKernelGGL(k_adj_e_scale, grid, dim3(256), 0, st, g, a);
+void launch_copies(const std::vector<CopySeg> &segs, hipStream_t st) {
+  for (size_t at = 0; at < segs.size(); at += kCopies) {
+    CopyArgs a;
+    const int n = (int)std::min<size_t>(kCopies, segs.size() - at);
+    size_t most = 0;
+    for (int j = 0; j < n; j++) {
+      a.seg[j] = segs[at + j];
+      most = std::max(most, a.seg[j].bytes);
+    }
+    const unsigned blocks = (unsigned)std::min<size_t>(1024, most / (sizeof(uint4) * 256) + 1);
+    hipLaunchKernelGGL(k_copy, dim3(blocks, n), dim3(256), 0, st, a);
+  }
 }
 
-void launch_adj_fields_post(const GridDesc &g, double *const *lam, const double *ke, const double *kh,
-                            hipStream_t st) {
-  AdjE a{lam[0], lam[1], lam[2], lam[3], lam[4], lam[5], lam[6], lam[7], lam[8], lam[9], lam[10], lam[11], ke, kh};
-  dim3 grid((g.nz + 255) / 256, g.nr);
-  hipLaunchKernelGGL(k_adj_h, grid, dim3(256), 0, st, g, a);
-  hipLaunchKernelGGL(k_adj_h_fin, grid, dim3(256), 0, st, g, a);
+AdjE adj_e(double *const *lam, double *const *scaled, const double *ke, const double *kh) {
+  return AdjE{lam[0], lam[1], lam[2], lam[3], lam[4], lam[5], lam[6], lam[7], lam[8], lam[9], lam[10], lam[11],
+              scaled[0], scaled[1], scaled[2], ke, kh};
 }
 
-void launch_adj_particles(const GridDesc &g, const double *const *fields6, double *const *lam, const double *r,
-                          const double *z, const double *vr, const double *vphi, const double *vz, const double *w,
-                          const uint8_t *alive, double *const *lstate, double *lw, double charge, double mass,
+void launch_adj_fields_pre(const GridDesc &g, double *const *lam, double *const *scaled, const double *ke,
+                           const double *kh, hipStream_t st) {
+  dim3 grid((g.nz + 255) / 256, g.nr);
+  hipLaunchKernelGGL(k_adj_e_curl, grid, dim3(256), 0, st, g, adj_e(lam, scaled, ke, kh));
+}
+
+void launch_adj_fields_post(const GridDesc &g, double *const *lam, double *const *scaled, const double *ke,
+                            const double *kh, hipStream_t st) {
+  dim3 grid((g.nz + 255) / 256, g.nr);
+  hipLaunchKernelGGL(k_adj_h, grid, dim3(256), 0, st, g, adj_e(lam, scaled, ke, kh));
+}
+
+void launch_adj_particles(const GridDesc &g, const double *const *fields6, double *const *lam, double *const *scaled,
+                          const StateRef &state, double *const *lstate, double *lw, double charge, double mass,
                           long long n, int is_bunch, int pusher, hipStream_t st) {
   if (n <= 0) return;
   AdjFields f{fields6[0], fields6[1], fields6[2], fields6[3], fields6[4], fields6[5]};
-  AdjGrid lg{lam[9], lam[10], lam[11], lam[0], lam[1], lam[2], lam[6], lam[7], lam[8]};
-  AdjSpecies s{r, z, vr, vphi, vz, w, alive, lstate[0], lstate[1], lstate[2], lstate[3], lstate[4], lw,
-               charge, mass, n, is_bunch};
+  AdjGrid lg{lam[9], lam[10], lam[11], scaled[0], scaled[1], scaled[2], lam[6], lam[7], lam[8]};
+  AdjSpecies s{state, lstate[0], lstate[1], lstate[2], lstate[3], lstate[4], lw, charge, mass, n};
   const dim3 grid((unsigned)((n + 255) / 256));
-  auto kernel = pusher == 1 ? (is_bunch ? k_adj_particles<true, true> : k_adj_particles<true, false>)
-                            : (is_bunch ? k_adj_particles<false, true> : k_adj_particles<false, false>);
-  hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, g, f, lg, s);
+  using K = void (*)(GridDesc, AdjFields, AdjGrid, AdjSpecies);
+  static const K kernels[8] = {k_adj_particles<false, false, false>, k_adj_particles<true, false, false>,
+                               k_adj_particles<false, true, false>,  k_adj_particles<true, true, false>,
+                               k_adj_particles<false, false, true>,  k_adj_particles<true, false, true>,
+                               k_adj_particles<false, true, true>,   k_adj_particles<true, true, true>};
+  hipLaunchKernelGGL(kernels[(pusher == 1) + 2 * (is_bunch != 0) + 4 * (state.cell != nullptr)], grid, dim3(256), 0, st,
+                     g, f, lg, s);
 }
 
 void launch_adj_seed(const GridDesc &g, const double *ez, double *lez, int k0, int k1, double scale, double *phi,
@@ -1607,9 +1702,8 @@ void launch_adj_seed(const GridDesc &g, const double *ez, double *lez, int k0, i
 }
 
 void launch_tlm_particles(const GridDesc &g, const double *const *fields6, double *const *const *tgrid,
-                          const double *r, const double *z, const double *vr, const double *vphi, const double *vz,
-                          const double *w, const uint8_t *alive, double *const *tstate, const double *tw,
-                          double charge, double mass, long long n, int is_bunch, int pusher, hipStream_t st) {
+                          const StateRef &state, double *const *tstate, const double *tw, double charge, double mass,
+                          long long n, int is_bunch, int pusher, hipStream_t st) {
   if (n <= 0) return;
   AdjFields f{fields6[0], fields6[1], fields6[2], fields6[3], fields6[4], fields6[5]};
   TlmFields tf;
@@ -1626,9 +1720,13 @@ void launch_tlm_particles(const GridDesc &g, const double *const *fields6, doubl
     tj.jphi[d] = a[kJPhi];
     tj.jz[d] = a[kJZ];
   }
-  TlmSpecies s{r, z, vr, vphi, vz, w, alive, tstate[0], tstate[1], tstate[2], tstate[3], tstate[4], tw,
-               charge, mass, n, is_bunch};
-  hipLaunchKernelGGL(k_tlm_particles, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g, f, tf, tj, s, pusher);
+  TlmSpecies s{state, tstate[0], tstate[1], tstate[2], tstate[3], tstate[4], tw, charge, mass, n};
+  const dim3 grid((unsigned)((n + 255) / 256));
+  using K = void (*)(GridDesc, AdjFields, TlmFields, TlmJ, TlmSpecies, int);
+  static const K kernels[4] = {k_tlm_particles<false, false>, k_tlm_particles<true, false>,
+                               k_tlm_particles<false, true>, k_tlm_particles<true, true>};
+  hipLaunchKernelGGL(kernels[(is_bunch != 0) + 2 * (state.cell != nullptr)], grid, dim3(256), 0, st, g, f, tf, tj, s,
+                     pusher);
 }
 
 void launch_tlm_objective(const GridDesc &g, const double *ez, double *const *const *tgrid, int k0, int k1,

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -378,6 +379,7 @@ int pdp3_ctx_destroy(pdp3_ctx *ctx) {
   dfree(c.rho_all);
   dfree(c.gauss);
   dfree(c.probe_ws);
+  dfree(c.adj_ws);
   dfree(c.rows);
   dfree(c.vol64);
   if (c.err_host) (void)hipHostFree(c.err_host);
@@ -1124,16 +1126,31 @@ struct DBuf {
   }
 };
 
-struct SpeciesCkpt {
-  std::vector<DBuf> bufs;  // native state arrays
+// arrays placed one after another in one block of device memory
+struct Layout {
+  std::vector<std::pair<void **, size_t>> items;
+  size_t total = 0;
+  size_t add(size_t bytes) {
+    const size_t at = total;
+    total += (bytes + 255) / 256 * 256;
+    return at;
+  }
+  template <class T>
+  void add(T **p, size_t n) {
+    items.emplace_back((void **)p, add(n * sizeof(T)));
+  }
+  void place(void *base) {
+    for (auto &it : items) *it.first = (char *)base + it.second;
+  }
 };
 
 // the state a loop iteration reads: fields E, H (and the rest of the grid for
-// the final restore) and every species' native particle arrays, plus the host
-// bookkeeping of time and bunches
+// the final restore) and every species' native particle arrays, one block of
+// device memory (own: allocated for it), plus the host bookkeeping of time and
+// bunches
 struct Checkpoint {
-  DBuf grid;  // components kER .. kRhoBunch
-  std::vector<SpeciesCkpt> sp;
+  void *mem = nullptr;
+  DBuf own;
   double time = 0;
   long long steps = 0;
   int next_bunch = 0;
@@ -1156,23 +1173,37 @@ std::vector<std::pair<void *, size_t>> native_arrays(Ctx &c, Species &sp) {
   return out;
 }
 
+// a checkpoint's arrays: offset in its block, the context's array, bytes
+struct CkptItem {
+  size_t at;
+  void *p;
+  size_t bytes;
+};
+size_t ckpt_items(Ctx &c, std::vector<CkptItem> *items) {
+  Layout l;
+  auto put = [&](void *p, size_t bytes) {
+    const size_t at = l.add(bytes);
+    if (items) items->push_back(CkptItem{at, p, bytes});
+  };
+  put(c.a[0], kCkComps * c.cells() * sizeof(double));
+  for (Species &sp : c.species)
+    for (auto &a : native_arrays(c, sp))
+      if (a.second) put(a.first, a.second);
+  return l.total;
+}
+
 int ckpt_save(pdp3_ctx *ctx, Checkpoint &ck) {
   Ctx &c = ctx->c;
-  const size_t gb = kCkComps * c.cells() * sizeof(double);
-  if (!ck.grid.p) HIP_TRY(ctx, hipMalloc(&ck.grid.p, gb));
-  HIP_TRY(ctx, hipMemcpyAsync(ck.grid.p, c.a[0], gb, hipMemcpyDeviceToDevice, c.stream));
-  if (ck.sp.empty()) ck.sp.resize(c.species.size());
-  for (size_t j = 0; j < c.species.size(); j++) {
-    auto arrs = native_arrays(c, c.species[j]);
-    auto &b = ck.sp[j].bufs;
-    if (b.empty()) {
-      b = std::vector<DBuf>(arrs.size());
-      for (size_t a = 0; a < arrs.size(); a++) HIP_TRY(ctx, hipMalloc(&b[a].p, std::max<size_t>(arrs[a].second, 1)));
-    }
-    for (size_t a = 0; a < arrs.size(); a++)
-      if (arrs[a].second)
-        HIP_TRY(ctx, hipMemcpyAsync(b[a].p, arrs[a].first, arrs[a].second, hipMemcpyDeviceToDevice, c.stream));
+  std::vector<CkptItem> items;
+  const size_t bytes = ckpt_items(c, &items);
+  if (!ck.mem) {
+    HIP_TRY(ctx, hipMalloc(&ck.own.p, bytes));
+    ck.mem = ck.own.p;
   }
+  std::vector<CopySeg> segs;
+  for (auto &it : items) segs.push_back(CopySeg{(char *)ck.mem + it.at, it.p, it.bytes});
+  launch_copies(segs, c.stream);
+  CHECK_LAUNCH(ctx);
   ck.time = c.current_time;
   ck.steps = c.steps_done;
   ck.next_bunch = c.next_bunch;
@@ -1184,31 +1215,44 @@ int ckpt_save(pdp3_ctx *ctx, Checkpoint &ck) {
 
 int ckpt_restore(pdp3_ctx *ctx, const Checkpoint &ck) {
   Ctx &c = ctx->c;
-  const size_t gb = kCkComps * c.cells() * sizeof(double);
-  HIP_TRY(ctx, hipMemcpyAsync(c.a[0], ck.grid.p, gb, hipMemcpyDeviceToDevice, c.stream));
-  for (size_t j = 0; j < c.species.size(); j++) {
-    auto arrs = native_arrays(c, c.species[j]);
-    for (size_t a = 0; a < arrs.size(); a++)
-      if (arrs[a].second)
-        HIP_TRY(ctx, hipMemcpyAsync(arrs[a].first, ck.sp[j].bufs[a].p, arrs[a].second, hipMemcpyDeviceToDevice,
-                                    c.stream));
-  }
+  std::vector<CkptItem> items;
+  ckpt_items(c, &items);
+  std::vector<CopySeg> segs;
+  for (auto &it : items) segs.push_back(CopySeg{it.p, (const char *)ck.mem + it.at, it.bytes});
+  launch_copies(segs, c.stream);
+  CHECK_LAUNCH(ctx);
   c.current_time = ck.time;
   c.steps_done = ck.steps;
   c.next_bunch = ck.next_bunch;
   c.order = ck.order;
   for (size_t j = 0; j < c.species.size(); j++) c.species[j].created = ck.created[j] != 0;
-  HIP_TRY(ctx, hipStreamSynchronize(c.stream));
   return PDP3_OK;
 }
 
-// FP64 particle state of one step, in the index space of the species (slots
-// of the FP64 form, logical order of the FP32 form's staging)
-struct SpeciesSnap {
-  DBuf r, z, vr, vphi, vz, alive;
-};
-
-long long adj_count(const Ctx &c, const Species &sp) { return is_f32(c) ? sp.n : sp.n_cap; }
+// the state of a species in native arrays (native_arrays' order); the weights,
+// which no step changes, are the species' own
+StateRef state_ref(const Ctx &c, const Species &sp, void *const *arr) {
+  StateRef s;
+  if (is_f32(c)) {
+    s.cell = (const uint32_t *)arr[0];
+    s.fa = (const float *)arr[1];
+    s.fb = (const float *)arr[2];
+    s.ur = (const float *)arr[3];
+    s.uphi = (const float *)arr[4];
+    s.uz = (const float *)arr[5];
+    s.fw = sp.f32.w;
+  } else {
+    s.r = (const double *)arr[0];
+    s.z = (const double *)arr[1];
+    s.vr = (const double *)arr[2];
+    s.vphi = (const double *)arr[3];
+    s.vz = (const double *)arr[4];
+    s.alive = (const uint8_t *)arr[5];
+    s.w = sp.f64.w;
+  }
+  return s;
+}
+constexpr int kNative = 6;  // arrays of native_arrays
 
 // the tangent-linear model carried along a forward sweep of the loop:
 // kTangentDirs directions of the particle weights; its grids are advanced by
@@ -1218,75 +1262,75 @@ long long adj_count(const Ctx &c, const Species &sp) { return is_f32(c) ? sp.n :
 struct TangentSweep {
   static constexpr int D = kTangentDirs;
   pdp3_ctx *ctx = nullptr;
-  DBuf tgrid_mem, phi_dev;
-  std::vector<Ctx> shadow;
+  DBuf mem;
+  Ctx shadow;  // the first direction's grids; the others follow, kNComp grids apart
+  double *tgrid = nullptr, *phi = nullptr;
   double *tg[D][kNComp] = {};
   double *const *tgp[D] = {};
-  std::vector<DBuf> tstate;  // per species: r, z, vr, vphi, vz tangents and the weight tangents (D x n each)
+  // per species: r, z, vr, vphi, vz tangents and the weight tangents (D x n_cap each)
+  std::vector<std::array<double *, 6>> ts;
 
+  size_t stride() const { return (size_t)kNComp * ctx->c.cells(); }
   int init(pdp3_ctx *c_, const double *const *dw) {
     ctx = c_;
     Ctx &c = ctx->c;
     const size_t cells = c.cells();
     const int nsp = (int)c.species.size();
-    HIP_TRY(ctx, hipMalloc(&tgrid_mem.p, (size_t)D * kNComp * cells * sizeof(double)));
-    HIP_TRY(ctx, hipMemsetAsync(tgrid_mem.p, 0, (size_t)D * kNComp * cells * sizeof(double), c.stream));
-    HIP_TRY(ctx, hipMalloc(&phi_dev.p, (1 + D) * sizeof(double)));
-    HIP_TRY(ctx, hipMemsetAsync(phi_dev.p, 0, (1 + D) * sizeof(double), c.stream));
-    shadow.assign(D, Ctx());
+    ts.resize((size_t)nsp);
+    Layout l;
+    l.add(&tgrid, D * stride());
+    l.add(&phi, 1 + D);
+    for (int j = 0; j < nsp; j++)
+      for (auto &p : ts[j]) l.add(&p, (size_t)c.species[j].n_cap * D);
+    const size_t zeroed = l.total;
+    double *tmp = nullptr;  // one direction of one species' weight tangents in logical order
+    long long most = 1;
+    for (int j = 0; j < nsp; j++)
+      if (c.species[j].chunked) most = std::max<long long>(most, c.species[j].n);
+    l.add(&tmp, (size_t)most);
+    HIP_TRY(ctx, hipMalloc(&mem.p, l.total));
+    l.place(mem.p);
+    HIP_TRY(ctx, hipMemsetAsync(mem.p, 0, zeroed, c.stream));
+    shadow.g = c.g;
+    shadow.stream = c.stream;
+    shadow.koef_e = c.koef_e;
+    shadow.koef_h = c.koef_h;
     for (int d = 0; d < D; d++) {
-      Ctx &sh = shadow[d];
-      sh.g = c.g;
-      sh.stream = c.stream;
-      sh.koef_e = c.koef_e;
-      sh.koef_h = c.koef_h;
-      for (int k = 0; k < kNComp; k++)
-        sh.a[k] = tg[d][k] = tgrid_mem.as<double>() + ((size_t)d * kNComp + k) * cells;
+      for (int k = 0; k < kNComp; k++) tg[d][k] = tgrid + ((size_t)d * kNComp + k) * cells;
       tgp[d] = tg[d];
     }
-    tstate = std::vector<DBuf>((size_t)nsp * 6);
+    for (int k = 0; k < kNComp; k++) shadow.a[k] = tg[0][k];
     for (int j = 0; j < nsp; j++) {
       Species &sp = c.species[j];
-      const long long n = adj_count(c, sp);
-      const size_t b = (size_t)std::max<long long>(n, 1) * D * sizeof(double);
-      for (int a = 0; a < 6; a++) {
-        HIP_TRY(ctx, hipMalloc(&tstate[j * 6 + a].p, b));
-        HIP_TRY(ctx, hipMemsetAsync(tstate[j * 6 + a].p, 0, b, c.stream));
+      if (!dw || !dw[j] || sp.n <= 0) continue;
+      if (!sp.chunked) {
+        HIP_TRY(ctx, hipMemcpyAsync(ts[j][5], dw[j], (size_t)D * sp.n * sizeof(double), hipMemcpyHostToDevice,
+                                    c.stream));
+        continue;
       }
-      if (dw && dw[j] && n > 0) {
-        // logical order -> the index space of the adjoint (FP64 form: slots)
-        std::vector<double> h((size_t)n * D, 0.0);
-        for (int d = 0; d < D; d++)
-          for (long long p = 0; p < n; p++) {
-            const long long l = (!is_f32(c) && sp.chunked) ? logical_of(p) : p;
-            if (l < sp.n) h[(size_t)d * n + p] = dw[j][(size_t)d * sp.n + l];
-          }
-        HIP_TRY(ctx, hipMemcpyAsync(tstate[j * 6 + 5].p, h.data(), h.size() * sizeof(double),
+      for (int d = 0; d < D; d++) {  // logical order -> slots
+        HIP_TRY(ctx, hipMemcpyAsync(tmp, dw[j] + (size_t)d * sp.n, (size_t)sp.n * sizeof(double),
                                     hipMemcpyHostToDevice, c.stream));
-        HIP_TRY(ctx, hipStreamSynchronize(c.stream));
+        launch_to_phys(c, tmp, ts[j][5] + (size_t)d * sp.n_cap, sp.n, sp.n_cap);
+        CHECK_LAUNCH(ctx);
       }
     }
+    HIP_TRY(ctx, hipStreamSynchronize(c.stream));  // dw is the caller's
     return PDP3_OK;
   }
   // after the H update of an iteration: E^n and Hh^n are final and the
   // particles are still at step n
   int after_h() {
     Ctx &c = ctx->c;
-    const size_t cells = c.cells();
-    for (int d = 0; d < D; d++) {
-      launch_h_update(shadow[d]);
-      launch_fill(tg[d][kJR], 3 * cells, 0.0, c.stream);  // J_r, J_phi, J_z are contiguous
-    }
+    launch_h_update(shadow, true, D, stride());
     const double *f6[6] = {c.a[kER], c.a[kEPhi], c.a[kEZ], c.a[kHHR], c.a[kHHPhi], c.a[kHHZ]};
     for (int j = 0; j < (int)c.species.size(); j++) {
       Species &sp = c.species[j];
-      const long long cnt = adj_count(c, sp);
-      if (cnt <= 0) continue;
-      if (is_f32(c)) launch_f64_from_f32(c, sp);  // logical-order FP64 staging
-      double *ts[5];
-      for (int a = 0; a < 5; a++) ts[a] = tstate[j * 6 + a].as<double>();
-      launch_tlm_particles(c.g, f6, tgp, sp.f64.r, sp.f64.z, sp.f64.vr, sp.f64.vphi, sp.f64.vz, sp.f64.w,
-                           sp.f64.alive, ts, tstate[j * 6 + 5].as<double>(), sp.charge, sp.mass, cnt,
+      if (sp.n_cap <= 0) continue;
+      void *arr[kNative];
+      auto native = native_arrays(c, sp);
+      for (int a = 0; a < kNative; a++) arr[a] = native[a].first;
+      launch_tlm_particles(c.g, f6, tgp, state_ref(c, sp, arr), ts[j].data(), ts[j][5], sp.charge, sp.mass, sp.n_cap,
                            sp.kind == PDP3_SPECIES_BUNCH, c.pusher, c.stream);
     }
     CHECK_LAUNCH(ctx);
@@ -1296,15 +1340,16 @@ struct TangentSweep {
   // objective's window, its tangent
   int after_step(bool in_window, int k0, int k1) {
     Ctx &c = ctx->c;
-    for (int d = 0; d < D; d++) launch_e_update(shadow[d]);
+    launch_e_update(shadow, D, stride());
     if (in_window && k1 >= k0)
-      launch_tlm_objective(c.g, c.a[kEZ], tgp, k0, k1, c.g.dt * c.g.dz, phi_dev.as<double>(), c.stream);
+      launch_tlm_objective(c.g, c.a[kEZ], tgp, k0, k1, c.g.dt * c.g.dz, phi, c.stream);
     CHECK_LAUNCH(ctx);
     return PDP3_OK;
   }
   int result(double *phi_out, double *dphi_out) {
     double out[1 + D];
-    HIP_TRY(ctx, hipMemcpy(out, phi_dev.p, sizeof(out), hipMemcpyDeviceToHost));
+    HIP_TRY(ctx, hipMemcpyAsync(out, phi, sizeof(out), hipMemcpyDeviceToHost, ctx->c.stream));
+    HIP_TRY(ctx, hipStreamSynchronize(ctx->c.stream));
     if (phi_out) *phi_out = out[0];
     if (dphi_out)
       for (int d = 0; d < D; d++) dphi_out[d] = out[1 + d];
@@ -1411,50 +1456,75 @@ int adjoint_impl(pdp3_ctx *ctx, int nsteps, int checkpoint_every, int window_ste
   objective_window(c, z_lo, z_hi, k0, k1);
   const double scale = c.g.dt * c.g.dz;
 
-  // forward with checkpoints (and the tangents, when requested)
-  const int nck = (nsteps + checkpoint_every - 1) / checkpoint_every;
+  const int K = checkpoint_every, nck = (nsteps + K - 1) / K;
   std::vector<Checkpoint> ck(nck);
   Checkpoint final_state;
+  // working memory: the adjoint grids (E twice: each pass writes the other set)
+  // and particle adjoints, cleared; a species' result in logical order; one
+  // segment's snapshots of E^n, Hh^n and the native particle states
+  double *lam_grid = nullptr, *phi_dev = nullptr, *out_dev = nullptr;
+  std::vector<std::array<double *, 6>> ls((size_t)nsp);  // r, z, vr, vphi, vz, w
+  const int steps_kept = std::min(K, nsteps);
+  std::vector<std::array<double *, 2>> fsnap(steps_kept);  // E, Hh: three components each
+  std::vector<std::array<void *, kNative>> psnap((size_t)steps_kept * nsp);
+  Layout work;
+  work.add(&lam_grid, 15 * cells);
+  work.add(&phi_dev, 1);
+  for (int j = 0; j < nsp; j++)
+    for (auto &p : ls[j]) work.add(&p, (size_t)c.species[j].n_cap);
+  const size_t zeroed = work.total;
+  size_t most = 1;
+  for (int j = 0; j < nsp; j++) most = std::max(most, (size_t)c.species[j].n);
+  work.add(&out_dev, most);
+  for (int t = 0; t < steps_kept; t++) {
+    for (auto &p : fsnap[t]) work.add(&p, 3 * cells);
+    for (int j = 0; j < nsp; j++) {
+      auto native = native_arrays(c, c.species[j]);
+      for (int a = 0; a < kNative; a++) work.add((char **)&psnap[(size_t)t * nsp + j][a], native[a].second);
+    }
+  }
+  // one block for everything, kept in the context, while that is small; else a
+  // block for the working memory and one for each checkpoint, given back at
+  // the end (an allocation costs more than a step of a small problem)
+  constexpr size_t kKeep = 1ull << 30;
+  const size_t ck_bytes = ckpt_items(c, nullptr), all = work.total + (size_t)(nck + 1) * ck_bytes;
+  DBuf work_own;
+  if (all <= kKeep) {
+    if (c.adj_ws_bytes < all) {
+      dfree(c.adj_ws);
+      c.adj_ws = nullptr;
+      c.adj_ws_bytes = 0;
+      HIP_TRY(ctx, hipMalloc(&c.adj_ws, all));
+      c.adj_ws_bytes = all;
+    }
+    work.place(c.adj_ws);
+    char *at = (char *)c.adj_ws + work.total;
+    for (auto &k : ck) {
+      k.mem = at;
+      at += ck_bytes;
+    }
+    final_state.mem = at;
+  } else {
+    HIP_TRY(ctx, hipMalloc(&work_own.p, work.total));
+    work.place(work_own.p);
+  }
+
+  // forward with checkpoints (and the tangents, when requested)
   TangentSweep tl;
   if (dw && (st = tl.init(ctx, dw))) return st;
   std::function<int()> tl_hook = [&]() { return tl.after_h(); };
   for (int n = 0; n < nsteps; n++) {
-    if (n % checkpoint_every == 0 && (st = ckpt_save(ctx, ck[n / checkpoint_every]))) return st;
+    if (n % K == 0 && (st = ckpt_save(ctx, ck[n / K]))) return st;
     if ((st = step_one(ctx, dw ? &tl_hook : nullptr))) return st;
     if (dw && (st = tl.after_step(n >= nsteps - window_steps, k0, k1))) return st;
   }
   if ((st = check_device_errors(ctx)) || (st = ckpt_save(ctx, final_state))) return st;
   if (dw && (st = tl.result(nullptr, dphi_tangent))) return st;
 
-  // adjoint state
-  DBuf lam_grid, phi_dev, ez_rows;
-  HIP_TRY(ctx, hipMalloc(&lam_grid.p, 12 * cells * sizeof(double)));
-  HIP_TRY(ctx, hipMemsetAsync(lam_grid.p, 0, 12 * cells * sizeof(double), c.stream));
-  double *lam[12];
-  for (int j = 0; j < 12; j++) lam[j] = lam_grid.as<double>() + (size_t)j * cells;
-  HIP_TRY(ctx, hipMalloc(&phi_dev.p, sizeof(double)));
-  HIP_TRY(ctx, hipMemsetAsync(phi_dev.p, 0, sizeof(double), c.stream));
-  const int K = checkpoint_every;
-  HIP_TRY(ctx, hipMalloc(&ez_rows.p, (size_t)K * c.g.nz * sizeof(double)));
-  std::vector<DBuf> lstate((size_t)nsp * 6);  // r, z, vr, vphi, vz, w per species
-  for (int j = 0; j < nsp; j++) {
-    const size_t n = (size_t)std::max<long long>(adj_count(c, c.species[j]), 1);
-    for (int a = 0; a < 6; a++) {
-      HIP_TRY(ctx, hipMalloc(&lstate[j * 6 + a].p, n * sizeof(double)));
-      HIP_TRY(ctx, hipMemsetAsync(lstate[j * 6 + a].p, 0, n * sizeof(double), c.stream));
-    }
-  }
-  // per-step snapshots of one segment: E^n, Hh^n and the FP64 particle states
-  DBuf fsnap;
-  HIP_TRY(ctx, hipMalloc(&fsnap.p, (size_t)K * 6 * cells * sizeof(double)));
-  std::vector<SpeciesSnap> psnap((size_t)K * nsp);
-  for (int t = 0; t < K; t++)
-    for (int j = 0; j < nsp; j++) {
-      const size_t n = (size_t)std::max<long long>(adj_count(c, c.species[j]), 1);
-      SpeciesSnap &s = psnap[(size_t)t * nsp + j];
-      for (DBuf *b : {&s.r, &s.z, &s.vr, &s.vphi, &s.vz}) HIP_TRY(ctx, hipMalloc(&b->p, n * sizeof(double)));
-      HIP_TRY(ctx, hipMalloc(&s.alive.p, n));
-    }
+  HIP_TRY(ctx, hipMemsetAsync(lam_grid, 0, zeroed, c.stream));
+  double *lam[12], *scaled[3];
+  for (int j = 0; j < 12; j++) lam[j] = lam_grid + (size_t)j * cells;
+  for (int j = 0; j < 3; j++) scaled[j] = lam_grid + (size_t)(12 + j) * cells;
 
   for (int seg = nck - 1; seg >= 0; seg--) {
     const int n0 = seg * K, n1 = std::min(nsteps, n0 + K);
@@ -1463,80 +1533,64 @@ int adjoint_impl(pdp3_ctx *ctx, int nsteps, int checkpoint_every, int window_ste
     for (int n = n0; n < n1; n++) {
       const int t = n - n0;
       std::function<int()> snap = [&]() -> int {
-        double *fs = fsnap.as<double>() + (size_t)t * 6 * cells;
-        const int comps[6] = {kER, kEPhi, kEZ, kHHR, kHHPhi, kHHZ};
-        for (int a = 0; a < 6; a++)
-          HIP_TRY(ctx, hipMemcpyAsync(fs + (size_t)a * cells, c.a[comps[a]], cells * sizeof(double),
-                                      hipMemcpyDeviceToDevice, c.stream));
+        std::vector<CopySeg> segs;
+        segs.push_back(CopySeg{fsnap[t][0], c.a[kER], 3 * cells * sizeof(double)});
+        segs.push_back(CopySeg{fsnap[t][1], c.a[kHHR], 3 * cells * sizeof(double)});
         for (int j = 0; j < nsp; j++) {
-          Species &sp = c.species[j];
-          SpeciesSnap &s = psnap[(size_t)t * nsp + j];
-          const long long n = adj_count(c, sp);
-          if (n <= 0) continue;
-          if (is_f32(c)) {
-            launch_f64_from_f32(c, sp);  // logical-order FP64 staging
-            CHECK_LAUNCH(ctx);
-          }
-          const double *src[5] = {sp.f64.r, sp.f64.z, sp.f64.vr, sp.f64.vphi, sp.f64.vz};
-          DBuf *dst[5] = {&s.r, &s.z, &s.vr, &s.vphi, &s.vz};
-          for (int a = 0; a < 5; a++)
-            HIP_TRY(ctx, hipMemcpyAsync(dst[a]->p, src[a], (size_t)n * sizeof(double), hipMemcpyDeviceToDevice,
-                                        c.stream));
-          HIP_TRY(ctx, hipMemcpyAsync(s.alive.p, sp.f64.alive, (size_t)n, hipMemcpyDeviceToDevice, c.stream));
+          auto native = native_arrays(c, c.species[j]);
+          for (int a = 0; a < kNative; a++)
+            if (native[a].second)
+              segs.push_back(CopySeg{psnap[(size_t)t * nsp + j][a], native[a].first, native[a].second});
         }
+        launch_copies(segs, c.stream);
+        CHECK_LAUNCH(ctx);
         return PDP3_OK;
       };
       if ((st = step_one(ctx, &snap))) return st;
-      HIP_TRY(ctx, hipMemcpyAsync(ez_rows.as<double>() + (size_t)t * c.g.nz, c.a[kEZ], c.g.nz * sizeof(double),
-                                  hipMemcpyDeviceToDevice, c.stream));
     }
-    if ((st = check_device_errors(ctx))) return st;
     // backward through the segment
     for (int n = n1 - 1; n >= n0; n--) {
       const int t = n - n0;
+      // E_z after step n: the next step's snapshot, or (at the segment's end) the context's
+      const double *ez = n + 1 < n1 ? fsnap[t + 1][0] + 2 * cells : c.a[kEZ];
       if (n >= nsteps - window_steps && k1 >= k0)
-        launch_adj_seed(c.g, ez_rows.as<double>() + (size_t)t * c.g.nz, lam[2], k0, k1, scale, phi_dev.as<double>(),
-                        c.stream);
-      launch_adj_fields_pre(c.g, lam, c.koef_e, c.koef_h, c.stream);
-      const double *fs = fsnap.as<double>() + (size_t)t * 6 * cells;
-      const double *f6[6] = {fs, fs + cells, fs + 2 * cells, fs + 3 * cells, fs + 4 * cells, fs + 5 * cells};
+        launch_adj_seed(c.g, ez, lam[2], k0, k1, scale, phi_dev, c.stream);
+      launch_adj_fields_pre(c.g, lam, scaled, c.koef_e, c.koef_h, c.stream);
+      const double *e = fsnap[t][0], *hh = fsnap[t][1];
+      const double *f6[6] = {e, e + cells, e + 2 * cells, hh, hh + cells, hh + 2 * cells};
       for (int j = 0; j < nsp; j++) {
         Species &sp = c.species[j];
-        SpeciesSnap &s = psnap[(size_t)t * nsp + j];
-        double *ls[5];
-        for (int a = 0; a < 5; a++) ls[a] = lstate[j * 6 + a].as<double>();
-        launch_adj_particles(c.g, f6, lam, s.r.as<double>(), s.z.as<double>(), s.vr.as<double>(),
-                             s.vphi.as<double>(), s.vz.as<double>(), sp.f64.w, s.alive.as<uint8_t>(), ls,
-                             lstate[j * 6 + 5].as<double>(), sp.charge, sp.mass, adj_count(c, sp),
-                             sp.kind == PDP3_SPECIES_BUNCH, c.pusher, c.stream);
+        launch_adj_particles(c.g, f6, lam, scaled, state_ref(c, sp, psnap[(size_t)t * nsp + j].data()), ls[j].data(),
+                             ls[j][5], sp.charge, sp.mass, sp.n_cap, sp.kind == PDP3_SPECIES_BUNCH, c.pusher,
+                             c.stream);
       }
-      launch_adj_fields_post(c.g, lam, c.koef_e, c.koef_h, c.stream);
+      launch_adj_fields_post(c.g, lam, scaled, c.koef_e, c.koef_h, c.stream);
       CHECK_LAUNCH(ctx);
+      for (int j = 0; j < 3; j++) std::swap(lam[j], scaled[j]);
     }
-    HIP_TRY(ctx, hipStreamSynchronize(c.stream));
   }
+  if ((st = check_device_errors(ctx))) return st;
   // results
   double phi = 0;
-  HIP_TRY(ctx, hipMemcpy(&phi, phi_dev.p, sizeof(double), hipMemcpyDeviceToHost));
+  HIP_TRY(ctx, hipMemcpyAsync(&phi, phi_dev, sizeof(double), hipMemcpyDeviceToHost, c.stream));
+  HIP_TRY(ctx, hipStreamSynchronize(c.stream));
   if (phi_out) *phi_out = phi;
   if (dphi_dw) {
     for (int j = 0; j < nsp; j++) {
-      if (!dphi_dw[j]) continue;
       Species &sp = c.species[j];
-      const long long n = adj_count(c, sp);
-      std::vector<double> h((size_t)std::max<long long>(n, 1));
-      HIP_TRY(ctx, hipMemcpy(h.data(), lstate[j * 6 + 5].p, (size_t)n * sizeof(double), hipMemcpyDeviceToHost));
-      if (!is_f32(c) && sp.chunked) {
-        for (long long p = 0; p < n; p++) {
-          const long long l = logical_of(p);
-          if (l < sp.n) dphi_dw[j][l] = h[(size_t)p];
-        }
-      } else {
-        std::memcpy(dphi_dw[j], h.data(), (size_t)sp.n * sizeof(double));
+      if (!dphi_dw[j] || sp.n <= 0) continue;
+      const double *src = ls[j][5];
+      if (sp.chunked) {
+        launch_to_logical(c, src, out_dev, sp.n);
+        CHECK_LAUNCH(ctx);
+        src = out_dev;
       }
+      HIP_TRY(ctx, hipMemcpyAsync(dphi_dw[j], src, (size_t)sp.n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
     }
   }
-  return ckpt_restore(ctx, final_state);
+  if ((st = ckpt_restore(ctx, final_state))) return st;
+  HIP_TRY(ctx, hipStreamSynchronize(c.stream));
+  return PDP3_OK;
 }
 
 }  // namespace

@@ -193,6 +193,9 @@ struct Ctx {
   // probe workspace: 5 per-cell sums of the temperature probe, then the
   // probe output (6 x cells doubles, allocated by the first probe)
   double *probe_ws = nullptr;
+  // the adjoint's working memory, kept between runs while it is small
+  void *adj_ws = nullptr;
+  size_t adj_ws_bytes = 0;
   // device address of the library's fixed no-allocation array on this
   // context's GPU (nullptr when it could not be resolved)
   double *noalloc = nullptr;
@@ -209,9 +212,11 @@ struct Ctx {
 constexpr int kMaxGroup = 4;
 
 // ---- launchers (each enqueues on ctx.stream) ----
-// reset_j: the same launch clears J and the bunch density
-void launch_h_update(Ctx &c, bool reset_j = false);
-void launch_e_update(Ctx &c);
+// reset_j: the same launch clears J and the bunch density; sets, stride: the
+// same update of `sets` grids, each component `stride` values from the last
+// set's (the coefficients are shared)
+void launch_h_update(Ctx &c, bool reset_j = false, int sets = 1, size_t stride = 0);
+void launch_e_update(Ctx &c, int sets = 1, size_t stride = 0);
 void launch_fill(double *p, size_t n, double v, hipStream_t s);
 void launch_gauss_residual(Ctx &c, const double *rho, double *out);
 
@@ -248,14 +253,31 @@ void ens_launch_inject(const EnsInjectItem *items, int n_items, int max_count, c
                        hipStream_t st);
 void ens_launch_count(long long *step, hipStream_t st);
 
+// one species' state in slots, in either form (cell: nullptr in the FP64 form)
+struct StateRef {
+  const double *r = nullptr, *z = nullptr, *vr = nullptr, *vphi = nullptr, *vz = nullptr, *w = nullptr;
+  const uint8_t *alive = nullptr;
+  const uint32_t *cell = nullptr;
+  const float *fa = nullptr, *fb = nullptr, *ur = nullptr, *uphi = nullptr, *uz = nullptr, *fw = nullptr;
+};
+// device-to-device copies, as few launches as possible
+struct CopySeg {
+  void *dst;
+  const void *src;
+  size_t bytes;
+};
+void launch_copies(const std::vector<CopySeg> &segs, hipStream_t st);
+
 // adjoint of one loop iteration (FP64); lam = adjoints of E_r, E_phi, E_z,
-// H_r, H_phi, H_z, Hh_r, Hh_phi, Hh_z, J_r, J_phi, J_z (12 grids)
-void launch_adj_fields_pre(const GridDesc &g, double *const *lam, const double *ke, const double *kh, hipStream_t st);
-void launch_adj_fields_post(const GridDesc &g, double *const *lam, const double *ke, const double *kh,
-                            hipStream_t st);
-void launch_adj_particles(const GridDesc &g, const double *const *fields6, double *const *lam, const double *r,
-                          const double *z, const double *vr, const double *vphi, const double *vz, const double *w,
-                          const uint8_t *alive, double *const *lstate, double *lw, double charge, double mass,
+// H_r, H_phi, H_z, Hh_r, Hh_phi, Hh_z, J_r, J_phi, J_z (12 grids); scaled:
+// three more E grids, which pre writes and which hold the adjoint of E^n after
+// post
+void launch_adj_fields_pre(const GridDesc &g, double *const *lam, double *const *scaled, const double *ke,
+                           const double *kh, hipStream_t st);
+void launch_adj_fields_post(const GridDesc &g, double *const *lam, double *const *scaled, const double *ke,
+                            const double *kh, hipStream_t st);
+void launch_adj_particles(const GridDesc &g, const double *const *fields6, double *const *lam, double *const *scaled,
+                          const StateRef &state, double *const *lstate, double *lw, double charge, double mass,
                           long long n, int is_bunch, int pusher, hipStream_t st);
 void launch_adj_seed(const GridDesc &g, const double *ez, double *lez, int k0, int k1, double scale, double *phi,
                      hipStream_t st);
@@ -263,12 +285,11 @@ void launch_adj_seed(const GridDesc &g, const double *ez, double *lez, int k0, i
 // directions at once): tgrid[d][comp] are direction d's tangent grids (E, Hh
 // read, J accumulated); tstate = 5 arrays (r, z, vr, vphi, vz) of
 // kTangentDirs x n tangents, updated in place; tw = kTangentDirs x n weight
-// tangents
+// tangents (n slots)
 constexpr int kTangentDirs = 4;
 void launch_tlm_particles(const GridDesc &g, const double *const *fields6, double *const *const *tgrid,
-                          const double *r, const double *z, const double *vr, const double *vphi, const double *vz,
-                          const double *w, const uint8_t *alive, double *const *tstate, const double *tw,
-                          double charge, double mass, long long n, int is_bunch, int pusher, hipStream_t st);
+                          const StateRef &state, double *const *tstate, const double *tw, double charge, double mass,
+                          long long n, int is_bunch, int pusher, hipStream_t st);
 // phi5[0] += scale sum E_z(0,k)^2, phi5[1 + d] += scale sum 2 E_z E_z-dot_d over k0..k1
 void launch_tlm_objective(const GridDesc &g, const double *ez, double *const *const *tgrid, int k0, int k1,
                           double scale, double *phi5, hipStream_t st);

@@ -96,15 +96,19 @@ __device__ __forceinline__ void h_tile(const GridDesc &g, const HPtrs &f, int i0
 // shape, cleared by the threads of their nodes (Current::reset_j and
 // ChargeDensity::reset_rho of the loop, which nothing between the two reads):
 // a launch of its own for that took 4.3 us of a small run's 39 us step
-__global__ void __launch_bounds__(HTile::kThreads) k_h_update(GridDesc g, HPtrs f, double *j) {
+__global__ void __launch_bounds__(HTile::kThreads) k_h_update(GridDesc g, HPtrs f, double *j,
+                                                              size_t stride) {
   __shared__ double s[3 * HTile::kLds];
+  // set blockIdx.z of the grids
+  const size_t z = blockIdx.z * stride;
+  f = HPtrs{f.er + z, f.ephi + z, f.ez + z, f.hr + z, f.hphi + z, f.hz + z, f.hhr + z, f.hhphi + z, f.hhz + z};
   if (j) {
     const int r = threadIdx.x / HTile::kCols, c = threadIdx.x - r * HTile::kCols;
     const int i = blockIdx.y * HTile::kRows + r, k = blockIdx.x * HTile::kCols + c;
     const size_t n = (size_t)g.nr * (size_t)g.nz;
     if (i < g.nr && k < g.nz)
 #pragma unroll
-      for (int a = 0; a < 4; a++) j[a * n + at(g, i, k)] = 0.0;
+      for (int a = 0; a < 4; a++) j[z + a * n + at(g, i, k)] = 0.0;
   }
   h_tile<HTile>(g, f, blockIdx.y * HTile::kRows, blockIdx.x * HTile::kCols, s);
 }
@@ -157,8 +161,10 @@ __device__ __forceinline__ void e_tile(const GridDesc &g, const EPtrs &f, int i0
   f.ez[p] = f.ez[p] * ke - (f.jz[p] - (hphi - hphi_d) / dr - (hphi + hphi_d) / (2.0 * dr * i)) * kh;
 }
 
-__global__ void __launch_bounds__(ETile::kThreads) k_e_update(GridDesc g, EPtrs f) {
+__global__ void __launch_bounds__(ETile::kThreads) k_e_update(GridDesc g, EPtrs f, size_t stride) {
   __shared__ double s[3 * ETile::kLds];
+  const size_t z = blockIdx.z * stride;
+  f = EPtrs{f.hr + z, f.hphi + z, f.hz + z, f.jr + z, f.jphi + z, f.jz + z, f.ke, f.kh, f.er + z, f.ephi + z, f.ez + z};
   e_tile<ETile>(g, f, blockIdx.y * ETile::kRows, blockIdx.x * ETile::kCols, s);
 }
 
@@ -294,16 +300,16 @@ EPtrs eptrs(Ctx &c) {
                c.a[kER], c.a[kEPhi], c.a[kEZ]};
 }
 
-void launch_h_update(Ctx &c, bool reset_j) {
+void launch_h_update(Ctx &c, bool reset_j, int sets, size_t stride) {
   // (all nz columns of tiles: the last column of J is cleared too)
-  dim3 grid((c.g.nz + HTile::kCols - 1) / HTile::kCols, (c.g.nr + HTile::kRows - 1) / HTile::kRows);
+  dim3 grid((c.g.nz + HTile::kCols - 1) / HTile::kCols, (c.g.nr + HTile::kRows - 1) / HTile::kRows, sets);
   hipLaunchKernelGGL(k_h_update, grid, dim3(HTile::kThreads), 0, c.stream, c.g, hptrs(c),
-                     reset_j ? c.a[kJR] : nullptr);
+                     reset_j ? c.a[kJR] : nullptr, stride);
 }
 
-void launch_e_update(Ctx &c) {
-  dim3 grid((c.g.nz - 1 + ETile::kCols - 1) / ETile::kCols, (c.g.nr - 1 + ETile::kRows - 1) / ETile::kRows);
-  hipLaunchKernelGGL(k_e_update, grid, dim3(ETile::kThreads), 0, c.stream, c.g, eptrs(c));
+void launch_e_update(Ctx &c, int sets, size_t stride) {
+  dim3 grid((c.g.nz - 1 + ETile::kCols - 1) / ETile::kCols, (c.g.nr - 1 + ETile::kRows - 1) / ETile::kRows, sets);
+  hipLaunchKernelGGL(k_e_update, grid, dim3(ETile::kThreads), 0, c.stream, c.g, eptrs(c), stride);
 }
 
 void launch_gauss_residual(Ctx &c, const double *rho, double *out) {
