@@ -103,6 +103,10 @@ struct TileMap {
   }
 };
 
+// the probes and the charge weighting walk a chunk per block, or 256 particles
+// where that would be fewer blocks than this
+constexpr long long kOneChunkBlocks = 800;
+
 // alive byte of the FP64 state: 0 dead, 1 alive, 2 padding slot
 constexpr uint8_t kPadSlot = 2;
 // FP32 cell word of a padding slot (a dead particle's word never equals it)

@@ -862,6 +862,44 @@ __global__ void __launch_bounds__(256) k_charge(GridDesc g, GlobalSink gs, Speci
   deposit_rho(g, sk, s.charge * s.w[i], r, z);
 }
 
+// plasma species: tiles of the chunked layout, as k_charge32_tiled
+template <int PPT>
+__global__ void __launch_bounds__(256) k_charge_tiled(GridDesc g, GlobalSink gs, SpeciesArgs s, long long n_cap) {
+  __shared__ double box[NodeSink::kSize];
+  using Map = TileMap<PPT, kWavesPerBlock>;
+  const long long base = Map::base(blockIdx.x);
+  int ai, ak;
+  {
+    bool live[3];
+    int ri[3], kk[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      live[j] = s.alive[base + j] == 1;
+      ri[j] = live[j] ? max(0, cell_r(g, s.r[base + j])) : 0;
+      kk[j] = live[j] ? max(0, cell_z(g, s.z[base + j])) : 0;
+    }
+    tile_anchor(live, ri, kk, ai, ak);
+  }
+  NodeSink sk;
+  sk.init(gs, gs.rho, box, ai, ak);
+  __syncthreads();
+  const long long first = base + Map::first(threadIdx.x);
+  for (int j = 0; j < PPT; j++) {
+    const long long i = first + (long long)j * 64;
+    if (s.alive[i] != 1) continue;
+    const double r = s.r[i], z = s.z[i];
+    if (!finite2(r, z)) {
+      atomicOr(gs.err, kErrNonfinite);
+      continue;
+    }
+    sk.begin_cell(max(0, cell_r(g, r)), max(0, cell_z(g, z)));
+    deposit_rho(g, sk, s.charge * s.w[i], r, z);
+  }
+  sk.flush();
+  __syncthreads();
+  sk.to_grid();
+}
+
 __global__ void k_gather(GridDesc g, Fields f, int which, const double *r, const double *z, int n, double *out,
                          int *err) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1017,7 +1055,14 @@ void launch_charge_weighting_f64(Ctx &c, Species &sp, double *rho) {
   if (sp.n_cap <= 0) return;
   GlobalSink gs = sink_of(c);
   if (rho) gs.rho = rho;
-  hipLaunchKernelGGL(k_charge, dim3(blocks_for(sp.n_cap)), dim3(256), 0, c.stream, c.g, gs, args_of(sp), sp.n_cap);
+  if (sp.chunked && sp.n_cap >= kOneChunkBlocks * kChunk)
+    hipLaunchKernelGGL(k_charge_tiled<4>, dim3((unsigned)(sp.n_cap / kChunk)), dim3(256), 0, c.stream, c.g, gs,
+                       args_of(sp), sp.n_cap);
+  else if (sp.chunked)
+    hipLaunchKernelGGL(k_charge_tiled<1>, dim3((unsigned)(sp.n_cap / 256)), dim3(256), 0, c.stream, c.g, gs, args_of(sp),
+                       sp.n_cap);
+  else
+    hipLaunchKernelGGL(k_charge, dim3(blocks_for(sp.n_cap)), dim3(256), 0, c.stream, c.g, gs, args_of(sp), sp.n_cap);
 }
 
 void launch_gather_f64(Ctx &c, int which, const double *r, const double *z, int n, double *out) {

@@ -7,7 +7,10 @@
 // z = (k + b) dz with v = u / sqrt(1 + u^2/c^2) in FP64, exactly as its
 // download.  Per-cell sums use FP64 atomics, so they match the reference's
 // serial sums to FP64 round-off of the summation order.
+#include <type_traits>
+
 #include "context.hpp"
+#include "sink.hpp"
 
 namespace pdp3 {
 
@@ -25,6 +28,12 @@ struct StateF64 {
   const double *r, *z, *vr, *vphi, *vz, *w;
   const uint8_t *alive;
   GridDesc g;
+  __device__ __forceinline__ bool cell_of(long long p, int &i, int &k) const {
+    if (alive[p] != 1) return false;
+    i = (int)ceil(r[p] / g.dr) - 1;
+    k = (int)ceil(z[p] / g.dz) - 1;
+    return true;
+  }
   __device__ __forceinline__ bool get(long long p, ProbeParticle &q) const {
     if (alive[p] != 1) return false;
     q.r = r[p];
@@ -43,6 +52,12 @@ struct StateF32 {
   const uint32_t *cell;
   const float *fa, *fb, *ur, *uphi, *uz, *w;
   GridDesc g;
+  __device__ __forceinline__ bool cell_of(long long p, int &i, int &k) const {
+    const uint32_t c = cell[p];
+    i = (int)((c >> 16) & 0x7FFF);
+    k = (int)(c & 0xFFFF);
+    return !(c & kDeadBit);
+  }
   __device__ __forceinline__ bool get(long long p, ProbeParticle &q) const {
     const uint32_t c = cell[p];
     if (c & kDeadBit) return false;  // dead particles and padding slots
@@ -60,25 +75,81 @@ struct StateF32 {
   }
 };
 
-// per cell: sum |v|, sum v_r, sum v_phi, sum v_z, count (src/temperatureClassic.cpp:83-102)
+// the anchor cell of a tile starting at slot `base` (slots base, +1, +2: its
+// logical particles 0, 16, 32)
 template <class S>
+__device__ __forceinline__ void probe_anchor(const S &st, long long base, long long n_cap, int &ai, int &ak) {
+  bool live[3];
+  int ri[3], kk[3];
+#pragma unroll
+  for (int j = 0; j < 3; j++) {
+    ri[j] = kk[j] = 0;
+    live[j] = base + j < n_cap && st.cell_of(base + j, ri[j], kk[j]);
+  }
+  tile_anchor(live, ri, kk, ai, ak);
+}
+
+// per cell: sum |v|, sum v_r, sum v_phi, sum v_z, count
+// (src/temperatureClassic.cpp:83-102).  PPT particles a lane: consecutive ones
+// of a plasma species (TileMap), whose sums for the lane's current cell stay in
+// registers and go to an LDS box of kR x kK cells, then to the grid; PPT 0: a
+// bunch, one particle a thread, through the same box.  (Five global atomics a
+// particle, 20 particles a cell, took 930 us for 1.05e7 particles.)
+template <class S, int PPT>
 __global__ void __launch_bounds__(256) k_temperature_sums(S st, long long n_cap, double *sums, int *err) {
+  constexpr int kR = 3, kK = 128, kV = 5, kPlane = kR * kK;
+  __shared__ double box[kV * kPlane];
+  using Map = TileMap<PPT ? PPT : 1, 4>;
   const GridDesc &g = st.g;
   const size_t cells = (size_t)g.nr * (size_t)g.nz;
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < n_cap;
-       p += (long long)gridDim.x * blockDim.x) {
+  const long long base = PPT ? Map::base(blockIdx.x) : (long long)blockIdx.x * 256;
+  int ai, ak;
+  probe_anchor(st, base, n_cap, ai, ak);
+  for (int t = threadIdx.x; t < kV * kPlane; t += blockDim.x) box[t] = 0.0;
+  __syncthreads();
+  const int bi = ai - 1, bk = ak - 2;
+  int ic = -1, kc = -1;
+  double acc[kV] = {};
+  auto flush = [&]() {
+    if (ic < 0) return;
+    const int li = ic - bi, lk = kc - bk;
+    if ((unsigned)li < (unsigned)kR && (unsigned)lk < (unsigned)kK) {
+#pragma unroll
+      for (int v = 0; v < kV; v++) atomicAdd(box + v * kPlane + li * kK + lk, acc[v]);
+    } else {
+#pragma unroll
+      for (int v = 0; v < kV; v++) unsafeAtomicAdd(sums + v * cells + (size_t)ic * (size_t)g.nz + kc, acc[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < kV; v++) acc[v] = 0.0;
+  };
+  const long long first = PPT ? base + Map::first(threadIdx.x) : base + threadIdx.x;
+#pragma unroll
+  for (int j = 0; j < (PPT ? PPT : 1); j++) {
+    const long long p = first + j * 64;
     ProbeParticle q;
-    if (!st.get(p, q)) continue;
+    if (p >= n_cap || !st.get(p, q)) continue;
     if ((unsigned)q.i >= (unsigned)g.nr || (unsigned)q.k >= (unsigned)g.nz) {
       atomicOr(err, kErrDomain);
       continue;
     }
-    const size_t c = (size_t)q.i * (size_t)g.nz + (size_t)q.k;
-    unsafeAtomicAdd(sums + c, sqrt(q.vr * q.vr + q.vphi * q.vphi + q.vz * q.vz));
-    unsafeAtomicAdd(sums + cells + c, q.vr);
-    unsafeAtomicAdd(sums + 2 * cells + c, q.vphi);
-    unsafeAtomicAdd(sums + 3 * cells + c, q.vz);
-    unsafeAtomicAdd(sums + 4 * cells + c, 1.0);
+    if (q.i != ic || q.k != kc) {
+      flush();
+      ic = q.i;
+      kc = q.k;
+    }
+    acc[0] += sqrt(q.vr * q.vr + q.vphi * q.vphi + q.vz * q.vz);
+    acc[1] += q.vr;
+    acc[2] += q.vphi;
+    acc[3] += q.vz;
+    acc[4] += 1.0;
+  }
+  flush();
+  __syncthreads();
+  for (int t = threadIdx.x; t < kV * kPlane; t += blockDim.x) {
+    const double x = box[t];
+    const int v = t / kPlane, rem = t - v * kPlane;
+    if (x != 0.0) unsafeAtomicAdd(sums + v * cells + (size_t)(bi + rem / kK) * (size_t)g.nz + (bk + rem % kK), x);
   }
 }
 
@@ -118,14 +189,23 @@ __global__ void __launch_bounds__(256) k_temperature_normalize(GridDesc g, const
 // ParticlesDensity::calc_density (src/particlesDensity.cpp:40-225), the
 // reference's expressions in its order (CYL_RNG_VOL, CELL_VOLUME, CYL_VOL of
 // include/geometry.h:33-39); mass_array = mass * w (src/particles.cpp:329)
-template <class S>
+template <class S, int PPT>
 __global__ void __launch_bounds__(256) k_density(S st, long long n_cap, double mass, double *out, int *err) {
+  __shared__ double box[NodeSink::kSize];
+  using Map = TileMap<PPT ? PPT : 1, 4>;
   const GridDesc &g = st.g;
   const double dr = g.dr, dz = g.dz;
-  for (long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x; p < n_cap;
-       p += (long long)gridDim.x * blockDim.x) {
+  const long long base = PPT ? Map::base(blockIdx.x) : (long long)blockIdx.x * 256;
+  int ai, ak;
+  probe_anchor(st, base, n_cap, ai, ak);
+  NodeSink sk;
+  sk.init(GlobalSink{g.nr, g.nz, nullptr, nullptr, err}, out, box, ai, ak);
+  __syncthreads();
+  const long long first = PPT ? base + Map::first(threadIdx.x) : base + threadIdx.x;
+  for (int j = 0; j < (PPT ? PPT : 1); j++) {
+    const long long p = first + j * 64;
     ProbeParticle q;
-    if (!st.get(p, q)) continue;
+    if (p >= n_cap || !st.get(p, q)) continue;
     int r_i = q.i;
     const int z_k = q.k;
     if (r_i < 0 || z_k < 0 || r_i > g.nr - 2 || z_k > g.nz - 2) {
@@ -172,17 +252,24 @@ __global__ void __launch_bounds__(256) k_density(S st, long long n_cap, double m
       w11 = kPi * dz2 * (r3 * r3 - r2 * r2) / v_2;
     }
     const double ro_p = m / kElMass / v_0;
-    const size_t c = (size_t)r_i * (size_t)g.nz + (size_t)z_k;
-    unsafeAtomicAdd(out + c, ro_p * w00);
-    unsafeAtomicAdd(out + c + g.nz, ro_p * w10);
-    unsafeAtomicAdd(out + c + 1, ro_p * w01);
-    unsafeAtomicAdd(out + c + g.nz + 1, ro_p * w11);
+    sk.begin_cell(r_i, z_k);
+    sk.add4<kCRho>(r_i, z_k, ro_p * w00, ro_p * w10, ro_p * w01, ro_p * w11);
   }
+  sk.flush();
+  __syncthreads();
+  sk.to_grid();
 }
 
-unsigned probe_blocks(long long n) {
-  long long b = (n + 255) / 256;
-  return (unsigned)(b < 1 ? 1 : (b > 16384 ? 16384 : b));
+// the launch of a probe kernel over a species: a chunk, 256 logical particles
+// (small species) or 256 slots (bunches) a block
+template <class Launch>
+void probe_launch(const Species &sp, Launch launch) {
+  if (!sp.chunked)
+    launch(std::integral_constant<int, 0>(), (unsigned)((sp.n_cap + 255) / 256));
+  else if (sp.n_cap >= kOneChunkBlocks * kChunk)
+    launch(std::integral_constant<int, 4>(), (unsigned)(sp.n_cap / kChunk));
+  else
+    launch(std::integral_constant<int, 1>(), (unsigned)(sp.n_cap / 256));
 }
 
 StateF64 state64(const Ctx &c, const Species &sp) {
@@ -201,11 +288,15 @@ bool launch_temperature(Ctx &c, Species &sp, double *sums, double *out) {
   if (sp.n_cap > 0) {
     if (c.precision == 1) {
       if (!sp.f32.cell) return false;
-      hipLaunchKernelGGL(k_temperature_sums<StateF32>, dim3(probe_blocks(sp.n_cap)), dim3(256), 0, c.stream,
-                         state32(c, sp), sp.n_cap, sums, c.err);
+      probe_launch(sp, [&](auto ppt, unsigned blocks) {
+        hipLaunchKernelGGL((k_temperature_sums<StateF32, ppt()>), dim3(blocks), dim3(256), 0, c.stream, state32(c, sp),
+                           sp.n_cap, sums, c.err);
+      });
     } else {
-      hipLaunchKernelGGL(k_temperature_sums<StateF64>, dim3(probe_blocks(sp.n_cap)), dim3(256), 0, c.stream,
-                         state64(c, sp), sp.n_cap, sums, c.err);
+      probe_launch(sp, [&](auto ppt, unsigned blocks) {
+        hipLaunchKernelGGL((k_temperature_sums<StateF64, ppt()>), dim3(blocks), dim3(256), 0, c.stream, state64(c, sp),
+                           sp.n_cap, sums, c.err);
+      });
     }
   }
   hipLaunchKernelGGL(k_temperature_normalize, dim3((unsigned)((cells + 255) / 256)), dim3(256), 0, c.stream, c.g,
@@ -218,11 +309,15 @@ bool launch_density(Ctx &c, Species &sp, double *out) {
   if (sp.n_cap <= 0) return true;
   if (c.precision == 1) {
     if (!sp.f32.cell) return false;
-    hipLaunchKernelGGL(k_density<StateF32>, dim3(probe_blocks(sp.n_cap)), dim3(256), 0, c.stream, state32(c, sp),
-                       sp.n_cap, sp.mass, out, c.err);
+    probe_launch(sp, [&](auto ppt, unsigned blocks) {
+      hipLaunchKernelGGL((k_density<StateF32, ppt()>), dim3(blocks), dim3(256), 0, c.stream, state32(c, sp), sp.n_cap,
+                         sp.mass, out, c.err);
+    });
   } else {
-    hipLaunchKernelGGL(k_density<StateF64>, dim3(probe_blocks(sp.n_cap)), dim3(256), 0, c.stream, state64(c, sp),
-                       sp.n_cap, sp.mass, out, c.err);
+    probe_launch(sp, [&](auto ppt, unsigned blocks) {
+      hipLaunchKernelGGL((k_density<StateF64, ppt()>), dim3(blocks), dim3(256), 0, c.stream, state64(c, sp), sp.n_cap,
+                         sp.mass, out, c.err);
+    });
   }
   return true;
 }

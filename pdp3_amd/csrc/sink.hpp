@@ -216,6 +216,84 @@ using TileSink = TileSinkT<false, 3>;       // plasma species
 using TileRhoSink = TileSinkT<false, 4>;    // an ensemble's tiles, bunch blocks among them
 using BunchSink = TileSinkT<true, 4, 16, 32>;
 
+// One grid's node deposits of a tile (charge weighting outside the loop, the
+// density probe): the four corners of the lane's current cell in registers, an
+// LDS box of kR x kK nodes, the grid.
+struct NodeSink {
+  static constexpr int kR = 4, kK = 128, kSize = kR * kK;
+  GlobalSink g;
+  double *out;  // the grid
+  double *box;  // LDS
+  int bi, bk, ic, kc;
+  double r00, r10, r01, r11;
+
+  __device__ __forceinline__ void init(const GlobalSink &gs, double *grid, double *lds, int ai, int ak) {
+    g = gs;
+    out = grid;
+    box = lds;
+    bi = ai - 1;
+    bk = ak - 2;
+    ic = kc = -1;
+    r00 = r10 = r01 = r11 = 0.0;
+    for (int t = threadIdx.x; t < kSize; t += blockDim.x) box[t] = 0.0;
+  }
+  __device__ __forceinline__ void grid_put(int i, int k, double v) {
+    if ((unsigned)i < (unsigned)g.nr && (unsigned)k < (unsigned)g.nz)
+      unsafeAtomicAdd(out + (size_t)i * (size_t)g.nz + (size_t)k, v);
+    else
+      atomicOr(g.err, kErrDomain);
+  }
+  __device__ __forceinline__ void put(int i, int k, double v) {
+    const int li = i - bi, lk = k - bk;
+    if ((unsigned)li < (unsigned)kR && (unsigned)lk < (unsigned)kK)
+      atomicAdd(box + li * kK + lk, v);
+    else
+      grid_put(i, k, v);
+  }
+  template <int C>
+  __device__ __forceinline__ void add(int i, int k, double v) {
+    const int di = i - ic, dk = k - kc;
+    if ((unsigned)di < 2u && (unsigned)dk < 2u) {
+      r00 += (di == 0 && dk == 0) ? v : 0.0;
+      r10 += (di == 1 && dk == 0) ? v : 0.0;
+      r01 += (di == 0 && dk == 1) ? v : 0.0;
+      r11 += (di == 1 && dk == 1) ? v : 0.0;
+      return;
+    }
+    put(i, k, v);
+  }
+  template <int C>
+  __device__ __forceinline__ void add4(int i, int k, double v00, double v10, double v01, double v11) {
+    if (i == ic && k == kc) {
+      r00 += v00; r10 += v10; r01 += v01; r11 += v11;
+      return;
+    }
+    put(i, k, v00);
+    put(i + 1, k, v10);
+    put(i, k + 1, v01);
+    put(i + 1, k + 1, v11);
+  }
+  __device__ __forceinline__ void flush() {
+    if (ic < 0) return;
+    put(ic, kc, r00);
+    put(ic + 1, kc, r10);
+    put(ic, kc + 1, r01);
+    put(ic + 1, kc + 1, r11);
+    r00 = r10 = r01 = r11 = 0.0;
+  }
+  __device__ __forceinline__ void begin_cell(int i, int k) {
+    if (i != ic || k != kc) {
+      flush();
+      ic = i;
+      kc = k;
+    }
+  }
+  __device__ __forceinline__ void to_grid() {  // after flush and __syncthreads
+    for (int t = threadIdx.x; t < kSize; t += blockDim.x)
+      if (box[t] != 0.0) grid_put(bi + t / kK, bk + t % kK, box[t]);
+  }
+};
+
 // The anchor cell of a tile of cell-sorted particles, from the cells (i, k)
 // of its logical particles 0, 16 and 32 (live: a living particle; uniform
 // values, so that the choice runs on the scalar unit): the median row of the

@@ -81,3 +81,68 @@ def test_probe_arguments(orc):
     d = gpu.density(0)
     assert d.shape == (9, 17) and np.count_nonzero(d) == 4
     gpu.close()
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("nr,nz,n,in_order", [
+    (9, 31, 700, True),         # less than a chunk
+    (40, 211, 5003, False),     # particles in no order: sums outside the tiles' boxes
+    (65, 1001, 822001, True),   # a chunk per block, several tiles a row
+    (65, 130, 830000, False),
+])
+def test_probes_by_size(nr, nz, n, in_order, precision):
+    """The probes and the charge of a plasma species and a bunch against numpy
+    on the downloaded state, at sizes on both sides of their launch rule.  The
+    sums run over at most some hundred terms a cell (FP64 round-off of their
+    order: 1e-12 holds with room); T is a difference of squares of those sums,
+    of order 1e-2 of them here (1e-9)."""
+    from pdp3_amd import capi
+
+    rng = np.random.default_rng(n)
+    d = 5e-4
+    sim = capi.Simulation(nr, nz, (nr - 1) * d, (nz - 1) * d, 0.5 * d / 3e8, precision=precision)
+    r = d / 2 + rng.random(n) * (nr - 2) * d
+    z = d / 2 + rng.random(n) * (nz - 2) * d
+    if in_order:
+        o = np.lexsort((z, np.ceil(r / d)))
+        r, z = r[o], z[o]
+    v = rng.normal(0, 4e5, (3, n))
+    sim.add_plasma(-1, 1.0, r, z, v[0], v[1], v[2], rng.uniform(1e4, 1e6, n))
+    nb = 901
+    sim.add_bunch_loaded(-1, 1.0, d * (0.1 + 3 * rng.random(nb)), d * (1 + 20 * rng.random(nb)), *rng.normal(0, 1e5, (3, nb)),
+                         rng.uniform(1e4, 1e6, nb))
+    rho_ref = 0.0
+    for j in range(2):
+        s = sim.download(j)
+        dr, dz = sim.dr, sim.dz
+        i, k = np.ceil(s["r"] / dr).astype(int) - 1, np.ceil(s["z"] / dz).astype(int) - 1
+        p = i * nz + k
+        add = lambda x: np.bincount(p, weights=x, minlength=nr * nz)  # noqa: E731
+        speed = np.sqrt(s["vr"] ** 2 + s["vphi"] ** 2 + s["vz"] ** 2)
+        cnt = add(np.ones_like(speed))
+        with np.errstate(divide="ignore", invalid="ignore"):
+            v2 = (add(speed) ** 2 - add(s["vr"]) ** 2 - add(s["vphi"]) ** 2 - add(s["vz"]) ** 2) / cnt ** 2
+        t = (9.1e-31 * v2 / 2 / 1.6e-19).reshape(nr, nz)
+        t[-1, :], t[:, -1] = 0.0, 0.0
+        got = sim.temperature(j)
+        assert np.array_equal(np.isnan(got), np.isnan(t))
+        assert normwise(np.nan_to_num(got), np.nan_to_num(t)) <= 1e-9
+        # ring volumes of the charge weighting, in cells (density and charge share them)
+        x, b = s["r"] / dr, s["z"] / dz - k
+        fi = i.astype(float)
+        lo = np.where(i == 0, 16 * (0.25 - (x - 0.5) ** 2) / (2 * x), ((fi + 0.5) ** 2 - (x - 0.5) ** 2) / (x * np.maximum(fi, 1)))
+        hi = ((x + 0.5) ** 2 - (fi + 0.5) ** 2) / (x * (fi + 1))
+        near = (i == 0) & (x <= 0.5)
+        lo = np.where(near, 16 * (0.5 - x + x * x) / (2 * x * x + 0.5), lo)
+        hi = np.where(near, 2 * x * (x + 1) / (2 * x * x + 0.5), hi)
+        m = s["w"] / (4 * np.pi * dr * dr * dz)
+        dens = np.zeros(nr * nz)
+        for q, wgt in ((p, lo * (1 - b)), (p + nz, hi * (1 - b)), (p + 1, lo * b), (p + nz + 1, hi * b)):
+            dens += np.bincount(q, weights=m * wgt, minlength=nr * nz)
+        dens = dens.reshape(nr, nz)
+        assert normwise(sim.density(j), dens) <= 1e-12
+        rho_ref = rho_ref - 1.6e-19 * dens
+    _, rho = sim.gauss_residual()
+    # the FP32 form weights the charge in FP32 (2^-24 a particle, 1e-6 of the maximum is far above it)
+    assert normwise(rho, rho_ref) <= (1e-12 if precision == 0 else 1e-6)
+    sim.close()
