@@ -4,6 +4,8 @@
 #include "../../include/pdp3_hip.h"
 
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <array>
@@ -14,6 +16,7 @@
 #include <new>
 #include <string>
 #include <functional>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -90,6 +93,90 @@ int upload_koef(pdp3_ctx *ctx) {
   HIP_TRY(ctx, hipMemcpyAsync(c.a[kEps], c.eps_host.data(), n * sizeof(double), hipMemcpyHostToDevice,
                               c.stream));
   HIP_TRY(ctx, hipStreamSynchronize(c.stream));
+  return PDP3_OK;
+}
+
+// whether most of a host range's pages are in memory (mincore)
+bool resident(const void *p, size_t bytes) {
+  const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
+  const uintptr_t a = (uintptr_t)p & ~(page - 1), b = ((uintptr_t)p + bytes + page - 1) & ~(page - 1);
+  std::vector<unsigned char> vec((b - a) / page);
+  if (mincore((void *)a, b - a, vec.data()) != 0) return true;
+  size_t in = 0;
+  for (unsigned char v : vec) in += v & 1;
+  return 8 * in >= 7 * vec.size();
+}
+
+// Device memory to pageable host memory, complete on return.  The runtime pins
+// the destination for a copy like this, which is fast for memory in use (228 us
+// for 4.2 MB) but takes each page fault of fresh memory on the way: 1083 us for
+// a newly allocated 4.2 MB array, 8.7 ms for 34 MB.  Such a destination is
+// filled from pinned buffers, by several threads that share its page faults
+// (522 us, 3.9 ms).  Threads pay from 1 MiB; below kStageFrom the runtime's own
+// staging is used, and throughout where nothing may be allocated (stage false).
+int to_host(pdp3_ctx *ctx, void *dst, const void *src, size_t bytes, bool stage = true) {
+  Ctx &c = ctx->c;
+  constexpr size_t kStageFrom = 192 << 10, kSlot = 512 << 10, kThreadsFrom = 1 << 20;
+  constexpr int kThreads = 4;
+  HostStage &hs = c.stage;
+  const bool staged = stage && bytes >= kStageFrom && !resident(dst, bytes);
+  if (staged && !hs.mem) {
+    if (hipHostMalloc(&hs.mem, HostStage::kSlots * kSlot, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      hs.mem = nullptr;
+    }
+    for (int j = 0; hs.mem && j < HostStage::kSlots; j++)
+      if (hipEventCreateWithFlags(&hs.ev[j], hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        hs.free_all();
+      }
+  }
+  if (!staged || !hs.mem) {
+    HIP_TRY(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
+    HIP_TRY(ctx, hipStreamSynchronize(c.stream));
+    return PDP3_OK;
+  }
+  static_assert(HostStage::kSlots == 2 * kThreads, "two slots a thread");
+  const size_t chunks = (bytes + kSlot - 1) / kSlot;
+  const int nt = bytes >= kThreadsFrom ? kThreads : 1;
+  std::array<hipError_t, kThreads> err{};
+  // thread t copies chunks t, t + nt, ..: one on its way into a slot while the
+  // one before is copied out of the other
+  auto work = [&](int t, bool helper) {
+    hipError_t e = helper ? hipSetDevice(c.device) : hipSuccess;
+    auto issue = [&](size_t j, int s) {
+      const size_t at = j * kSlot;
+      if (e == hipSuccess)
+        e = hipMemcpyAsync((char *)hs.mem + (2 * t + s) * kSlot, (const char *)src + at, std::min(kSlot, bytes - at),
+                           hipMemcpyDeviceToHost, c.stream);
+      if (e == hipSuccess) e = hipEventRecord(hs.ev[2 * t + s], c.stream);
+    };
+    if ((size_t)t < chunks) issue(t, 0);
+    int s = 0;
+    for (size_t j = t; j < chunks; j += nt, s ^= 1) {
+      if (j + nt < chunks) issue(j + nt, s ^ 1);
+      if (e == hipSuccess) e = hipEventSynchronize(hs.ev[2 * t + s]);
+      if (e != hipSuccess) break;
+      const size_t at = j * kSlot;
+      std::memcpy((char *)dst + at, (char *)hs.mem + (2 * t + s) * kSlot, std::min(kSlot, bytes - at));
+    }
+    err[t] = e;
+  };
+  std::array<std::thread, kThreads> helpers;
+  int started = 1;
+  try {
+    for (; started < nt; started++) helpers[started] = std::thread(work, started, true);
+  } catch (const std::system_error &) {
+    // fewer threads than wanted: this one takes their shares
+  }
+  work(0, false);
+  for (int t = 1; t < started; t++) helpers[t].join();
+  for (int t = started; t < nt; t++) work(t, false);
+  for (hipError_t e : err)
+    if (e != hipSuccess) {
+      (void)hipStreamSynchronize(c.stream);  // no copy into the slots is left in flight
+      HIP_TRY(ctx, e);
+    }
   return PDP3_OK;
 }
 
@@ -380,6 +467,7 @@ int pdp3_ctx_destroy(pdp3_ctx *ctx) {
   dfree(c.gauss);
   dfree(c.probe_ws);
   dfree(c.adj_ws);
+  c.stage.free_all();
   dfree(c.rows);
   dfree(c.vol64);
   if (c.err_host) (void)hipHostFree(c.err_host);
@@ -604,9 +692,7 @@ int pdp3_hfield_get_field(pdp3_ctx *ctx, const double *r, const double *z, int n
 int pdp3_grid_download(pdp3_ctx *ctx, int component, double *out) {
   if (!ctx || component < 0 || component >= kNComp || !out) return PDP3_ERR_BAD_ARG;
   Ctx &c = ctx->c;
-  HIP_TRY(ctx, hipMemcpyAsync(out, c.a[component], c.cells() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  HIP_TRY(ctx, hipStreamSynchronize(c.stream));
-  return PDP3_OK;
+  return to_host(ctx, out, c.a[component], c.cells() * sizeof(double));
 }
 
 int pdp3_grid_upload(pdp3_ctx *ctx, int component, const double *in) {
@@ -790,30 +876,27 @@ int pdp3_species_download(pdp3_ctx *ctx, int index, double *r, double *z, double
   if (!is_f32(c) && sp.chunked) {
     void *tmp = nullptr;
     HIP_TRY(ctx, hipMalloc(&tmp, b));
-    hipError_t e = hipSuccess;
-    for (int j = 0; j < 6 && e == hipSuccess; j++)
+    int st = PDP3_OK;
+    for (int j = 0; j < 6 && !st; j++)
       if (dst[j]) {
         launch_to_logical(c, src[j], (double *)tmp, sp.n);
-        e = hipMemcpyAsync(dst[j], tmp, b, hipMemcpyDeviceToHost, c.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+        st = to_host(ctx, dst[j], tmp, b);
       }
-    if (alive && e == hipSuccess) {
+    if (alive && !st) {
       launch_alive_to_logical(c, sp.f64.alive, (uint8_t *)tmp, sp.n);
-      e = hipMemcpyAsync(alive, tmp, (size_t)sp.n, hipMemcpyDeviceToHost, c.stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+      st = to_host(ctx, alive, tmp, (size_t)sp.n);
     }
     (void)hipFree(tmp);
-    if (e != hipSuccess) return fail(ctx, PDP3_ERR_HIP, hipGetErrorString(e));
-    return PDP3_OK;
+    return st;
   }
   if (is_f32(c)) {
     launch_f64_from_f32(c, sp);
     CHECK_LAUNCH(ctx);
   }
+  int st;
   for (int j = 0; j < 6; j++)
-    if (dst[j]) HIP_TRY(ctx, hipMemcpyAsync(dst[j], src[j], b, hipMemcpyDeviceToHost, c.stream));
-  if (alive) HIP_TRY(ctx, hipMemcpyAsync(alive, sp.f64.alive, (size_t)sp.n, hipMemcpyDeviceToHost, c.stream));
-  HIP_TRY(ctx, hipStreamSynchronize(c.stream));
+    if (dst[j] && (st = to_host(ctx, dst[j], src[j], b))) return st;
+  if (alive && (st = to_host(ctx, alive, sp.f64.alive, (size_t)sp.n))) return st;
   return PDP3_OK;
 }
 
@@ -874,8 +957,8 @@ namespace {
 // the Gauss residual into device buffers rho and res (cells() values each):
 // rho cleared by a fill kernel, then the charge weighting of every species of
 // the loop (bunches once they are created), then the residual, which writes
-// every node
-int gauss_into(pdp3_ctx *ctx, double *rho, double *res, double *residual_out, double *rho_out) {
+// every node; stage: see to_host
+int gauss_into(pdp3_ctx *ctx, double *rho, double *res, double *residual_out, double *rho_out, bool stage) {
   Ctx &c = ctx->c;
   int st;
   launch_fill(rho, c.cells(), 0.0, c.stream);
@@ -889,9 +972,8 @@ int gauss_into(pdp3_ctx *ctx, double *rho, double *res, double *residual_out, do
   CHECK_LAUNCH(ctx);
   if ((st = check_device_errors(ctx))) return st;
   const size_t b = c.cells() * sizeof(double);
-  if (residual_out) HIP_TRY(ctx, hipMemcpyAsync(residual_out, res, b, hipMemcpyDeviceToHost, c.stream));
-  if (rho_out) HIP_TRY(ctx, hipMemcpyAsync(rho_out, rho, b, hipMemcpyDeviceToHost, c.stream));
-  HIP_TRY(ctx, hipStreamSynchronize(c.stream));
+  if (residual_out && (st = to_host(ctx, residual_out, res, b, stage))) return st;
+  if (rho_out && (st = to_host(ctx, rho_out, rho, b, stage))) return st;
   return PDP3_OK;
 }
 }  // namespace
@@ -904,7 +986,7 @@ int pdp3_gauss_residual(pdp3_ctx *ctx, double *residual_out, double *rho_out) {
   int st;
   if (!c.rho_all && (st = dalloc(ctx, &c.rho_all, c.cells()))) return st;
   if (!c.gauss && (st = dalloc(ctx, &c.gauss, c.cells()))) return st;
-  return gauss_into(ctx, c.rho_all, c.gauss, residual_out, rho_out);
+  return gauss_into(ctx, c.rho_all, c.gauss, residual_out, rho_out, true);
 }
 
 int pdp3_gauss_residual_noalloc(pdp3_ctx *ctx, double *residual_out, double *rho_out) {
@@ -916,7 +998,7 @@ int pdp3_gauss_residual_noalloc(pdp3_ctx *ctx, double *residual_out, double *rho
                     std::to_string((long long)PDP3_NOALLOC_MAX_NODES) + " (PDP3_NOALLOC_MAX_NODES)");
   if (!c.noalloc)
     return fail(ctx, PDP3_ERR_HIP, "the device address of the no-allocation array could not be resolved");
-  return gauss_into(ctx, c.noalloc, c.noalloc + (size_t)PDP3_NOALLOC_MAX_NODES, residual_out, rho_out);
+  return gauss_into(ctx, c.noalloc, c.noalloc + (size_t)PDP3_NOALLOC_MAX_NODES, residual_out, rho_out, false);
 }
 
 int pdp3_temperature(pdp3_ctx *ctx, int index, double *out) {
@@ -929,9 +1011,7 @@ int pdp3_temperature(pdp3_ctx *ctx, int index, double *out) {
     return fail(ctx, PDP3_ERR_STATE, "the species has no particle state yet");
   CHECK_LAUNCH(ctx);
   if ((st = check_device_errors(ctx))) return st;
-  HIP_TRY(ctx, hipMemcpyAsync(out, res, c.cells() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  HIP_TRY(ctx, hipStreamSynchronize(c.stream));
-  return PDP3_OK;
+  return to_host(ctx, out, res, c.cells() * sizeof(double));
 }
 
 int pdp3_density(pdp3_ctx *ctx, int index, double *out) {
@@ -944,9 +1024,7 @@ int pdp3_density(pdp3_ctx *ctx, int index, double *out) {
     return fail(ctx, PDP3_ERR_STATE, "the species has no particle state yet");
   CHECK_LAUNCH(ctx);
   if ((st = check_device_errors(ctx))) return st;
-  HIP_TRY(ctx, hipMemcpyAsync(out, res, c.cells() * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  HIP_TRY(ctx, hipStreamSynchronize(c.stream));
-  return PDP3_OK;
+  return to_host(ctx, out, res, c.cells() * sizeof(double));
 }
 
 int pdp3_bunch_inject(pdp3_ctx *ctx, int index) {
@@ -1585,7 +1663,7 @@ int adjoint_impl(pdp3_ctx *ctx, int nsteps, int checkpoint_every, int window_ste
         CHECK_LAUNCH(ctx);
         src = out_dev;
       }
-      HIP_TRY(ctx, hipMemcpyAsync(dphi_dw[j], src, (size_t)sp.n * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+      if ((st = to_host(ctx, dphi_dw[j], src, (size_t)sp.n * sizeof(double)))) return st;
     }
   }
   if ((st = ckpt_restore(ctx, final_state))) return st;

@@ -160,8 +160,24 @@ struct KernelTimer {
   long long launches = 0;
 };
 
+// pinned buffers for copies to the host, allocated by the first that needs them
+struct HostStage {
+  static constexpr int kSlots = 8;
+  void *mem = nullptr;
+  hipEvent_t ev[kSlots] = {};
+  void free_all() {
+    for (auto &e : ev) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+    if (mem) (void)hipHostFree(mem);
+    mem = nullptr;
+  }
+};
+
 struct Ctx {
   GridDesc g{};
+  HostStage stage;
   double current_time = 0, start_time = 0, relaxation_time = 0, end_time = 0;
   int pusher = 0;
   int precision = 0;
