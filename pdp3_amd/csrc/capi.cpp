@@ -1707,10 +1707,13 @@ struct pdp3_ensemble {
   hipStream_t stream = nullptr;
   EnsFields *fields = nullptr;
   EnsParticles *parts = nullptr;
+  // the tile shape; until it is set or autotuned, tiles by each species' size
   int tile = 0;
+  bool tile_auto = true;
+  bool banded = false;  // the ensemble has sorted
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  int graph_tile = -1;
+  int graph_list = -1;  // the work list that the graph launches
   int sort_interval = 0;
   long long steps_done = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1745,27 +1748,27 @@ void ens_drop_graph(pdp3_ensemble *e) {
   if (e->graph) (void)hipGraphDestroy(e->graph);
   e->exec = nullptr;
   e->graph = nullptr;
-  e->graph_tile = -1;
+  e->graph_list = -1;
 }
 
 // one loop iteration of every instance (src/loadInitParam.cpp:471-587; the
 // bunch injections of init_beam from the device tables), captured once per
 // tile shape and replayed
 int ens_graph(pdp3_ensemble *e) {
-  if (e->exec && e->graph_tile == e->tile) return PDP3_OK;
+  const int list = e->tile_auto ? ens_auto_list(e->banded) : e->tile;
+  if (e->exec && e->graph_list == list) return PDP3_OK;
   ens_drop_graph(e);
   ENS_HIP(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
   ens_launch_inject(e->inj, e->n_inj, e->inj_max, e->step_dev, e->stream);
   ens_launch_h(e->fields, e->stream);
-  ens_launch_zero(e->fields, e->stream);
-  ens_launch_particles(e->parts, e->tile, e->stream);
+  ens_launch_particles(e->parts, list, e->stream);
   ens_launch_e(e->fields, e->stream);
   ens_launch_count(e->step_dev, e->stream);
   hipGraph_t g = nullptr;
   ENS_HIP(e, hipStreamEndCapture(e->stream, &g));
   e->graph = g;
   ENS_HIP(e, hipGraphInstantiate(&e->exec, e->graph, nullptr, nullptr, 0));
-  e->graph_tile = e->tile;
+  e->graph_list = list;
   return PDP3_OK;
 }
 
@@ -1948,6 +1951,7 @@ int pdp3_ensemble_step(pdp3_ensemble *e, int nsteps) {
       st = sort_multi(e->ms, e->cs, e->stream);
       if (st) return efail(e, st == -3 ? PDP3_ERR_OOM : PDP3_ERR_HIP, "ensemble sort failed");
       if (ens_particles_update(e->parts, e->cs) != 0) return efail(e, PDP3_ERR_HIP, "ensemble tables");
+      e->banded = true;
     }
     if ((st = ens_graph(e))) return st;
     // init_beam's bookkeeping (the bunches join the species list on the
@@ -1993,6 +1997,7 @@ int pdp3_ensemble_set_tile(pdp3_ensemble *e, int ppt, int waves) {
   for (int t = 0; t < kNumTiles; t++)
     if (kTileShapes[t][0] == ppt && kTileShapes[t][1] == waves) {
       e->tile = t;
+      e->tile_auto = false;
       return PDP3_OK;
     }
   return efail(e, PDP3_ERR_BAD_ARG, "unsupported tile shape");
@@ -2011,6 +2016,7 @@ int pdp3_ensemble_autotune(pdp3_ensemble *e, int steps_per_candidate, int *ppt, 
   long long saved_steps = e->timed_steps;
   int best = 0, st = PDP3_OK;
   double best_ms = 1e300;
+  e->tile_auto = false;
   for (int t = 0; t < kNumTiles; t++) {
     e->tile = t;
     e->timed_ms = 0;

@@ -91,15 +91,35 @@ struct TileMap {
   // slot of the tile's last logical particle, from its first slot
   static constexpr int kLast = kWhole ? kParticles - 1 : (kPPT - 1) * 64 + kGroup - 1;
   static_assert(kPPT % PPT == 0 && (kWhole ? kParticles % kChunk == 0 : kChunk % kParticles == 0), "tile shape");
-  __device__ __forceinline__ static long long base(long long tile) {
+  __host__ __device__ __forceinline__ static long long base(long long tile) {
     if (kWhole) return tile * kParticles;
     constexpr int kPer = kWhole ? 1 : kChunk / kParticles;
     return tile / kPer * kChunk + tile % kPer * kGroup;
   }
+  __device__ __forceinline__ static constexpr int ppt() { return PPT; }
+  __device__ __forceinline__ static constexpr int span() { return kSpan; }
+  __device__ __forceinline__ static constexpr int last() { return kLast; }
   // the thread's first slot, from the tile's
   __device__ __forceinline__ static unsigned first(unsigned t) {
     constexpr unsigned kTeam = kGroup * (kPPT / PPT);  // threads that share a chunk's lanes
     return t / kTeam * kChunk + t % kTeam / kGroup * (PPT * 64) + t % kGroup;
+  }
+};
+
+// the same map with the particles per lane known at run time only (2^lg): one
+// kernel then serves tiles of every size in one launch
+template <int WAVES>
+struct TileMapRt {
+  int lg;
+  __device__ __forceinline__ int ppt() const { return 1 << lg; }
+  __device__ __forceinline__ int particles() const { return (WAVES * 64) << lg; }
+  __device__ __forceinline__ bool whole() const { return particles() >= kChunk; }
+  __device__ __forceinline__ int group() const { return whole() ? 64 : particles() / kPPT; }
+  __device__ __forceinline__ int span() const { return whole() ? particles() : kChunk; }
+  __device__ __forceinline__ int last() const { return whole() ? particles() - 1 : (kPPT - 1) * 64 + group() - 1; }
+  __device__ __forceinline__ unsigned first(unsigned t) const {
+    const unsigned g = group(), team = g * (unsigned)(kPPT >> lg);
+    return t / team * kChunk + t % team / g * (64u << lg) + t % g;
   }
 };
 
@@ -245,16 +265,18 @@ void launch_gauss_residual(Ctx &c, const double *rho, double *out);
 struct EnsFields;
 EnsFields *ens_fields_build(const std::vector<Ctx *> &ctxs);  // nullptr: out of memory
 void ens_fields_free(EnsFields *e);
-void ens_launch_h(EnsFields *e, hipStream_t st);
+void ens_launch_h(EnsFields *e, hipStream_t st);  // and the reset of J and the bunch densities
 void ens_launch_e(EnsFields *e, hipStream_t st);
-void ens_launch_zero(EnsFields *e, hipStream_t st);
 // the plasma tiles and bunch blocks of every instance, one launch;
 // rebuild after a sort (particle arrays move)
 struct EnsParticles;
 EnsParticles *ens_particles_build(const std::vector<Ctx *> &ctxs);
 int ens_particles_update(EnsParticles *e, const std::vector<Ctx *> &ctxs);  // 0 on success
 void ens_particles_free(EnsParticles *e);
-void ens_launch_particles(EnsParticles *e, int tile, hipStream_t st);
+// the work list of a settable tile shape (index into kTileShapes), or of tiles
+// by the size of each species (ens_auto_list; banded: the ensemble has sorted)
+int ens_auto_list(bool banded);
+void ens_launch_particles(EnsParticles *e, int list, hipStream_t st);
 // bunch injection of an ensemble (Bunch::bunch_inject, src/bunch.cpp:87-124)
 // driven by a device step counter: per (instance, bunch) pair a table of the
 // first particle injected at each ensemble step (-1: none), computed on the

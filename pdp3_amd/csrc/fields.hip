@@ -262,6 +262,17 @@ __global__ void __launch_bounds__(HTile::kThreads) k_ens_h(const EnsGrid *__rest
   for (int it = blockIdx.x; it < n_tiles; it += gridDim.x) {
     const EnsRow r = tiles[it];
     const EnsGridG &G = reinterpret_cast<const EnsGridG *>(grids)[r.inst];
+    {  // Current::reset_j and the bunch density's reset on the tile's nodes
+       // (4.3e6 nodes: 99 us together, 75 + 21 us and a launch apart)
+      const int i = r.i0 + threadIdx.x / HTile::kCols, k = r.k0 + threadIdx.x % HTile::kCols;
+      if (i < G.g.nr && k < G.g.nz) {
+        const size_t p = at(G.g, i, k);
+        G.jr[p] = 0.0;
+        G.jphi[p] = 0.0;
+        G.jz[p] = 0.0;
+        G.rho[p] = 0.0;
+      }
+    }
     h_tile<HTile>(G.g, from_global(G.h), r.i0, r.k0, s);
     __syncthreads();  // the next tile rewrites the staged rows
   }
@@ -275,18 +286,6 @@ __global__ void __launch_bounds__(ETile::kThreads) k_ens_e(const EnsGrid *__rest
     const EnsGridG &G = reinterpret_cast<const EnsGridG *>(grids)[r.inst];
     e_tile<ETile>(G.g, from_global(G.e), r.i0, r.k0, s);
     __syncthreads();  // the next tile rewrites the staged rows
-  }
-}
-
-// Current::reset_j and the bunch density reset of every instance
-__global__ void __launch_bounds__(256) k_ens_zero(const EnsGrid *__restrict__ grids) {
-  const EnsGridG &G = reinterpret_cast<const EnsGridG *>(grids)[blockIdx.y];
-  const size_t n = (size_t)G.g.nr * (size_t)G.g.nz;
-  for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (size_t)gridDim.x * blockDim.x) {
-    G.jr[p] = 0.0;
-    G.jphi[p] = 0.0;
-    G.jz[p] = 0.0;
-    G.rho[p] = 0.0;
   }
 }
 
@@ -337,7 +336,7 @@ EnsFields *ens_fields_build(const std::vector<Ctx *> &ctxs) {
     Ctx &c = *ctxs[j];
     g.push_back(EnsGrid{c.g, hptrs(c), eptrs(c), c.a[kJR], c.a[kJPhi], c.a[kJZ], c.a[kRhoBunch]});
     for (int i0 = 0; i0 < c.g.nr; i0 += HTile::kRows)
-      for (int k0 = 0; k0 < c.g.nz - 1; k0 += HTile::kCols) hr.push_back(EnsRow{(int)j, i0, k0});
+      for (int k0 = 0; k0 < c.g.nz; k0 += HTile::kCols) hr.push_back(EnsRow{(int)j, i0, k0});
     for (int i0 = 0; i0 < c.g.nr - 1; i0 += ETile::kRows)
       for (int k0 = 0; k0 < c.g.nz - 1; k0 += ETile::kCols) er.push_back(EnsRow{(int)j, i0, k0});
   }
@@ -373,10 +372,6 @@ void ens_launch_h(EnsFields *e, hipStream_t st) {
 void ens_launch_e(EnsFields *e, hipStream_t st) {
   const int blocks = std::min(e->n_e, 256 * 16);
   hipLaunchKernelGGL(k_ens_e, dim3(blocks), dim3(ETile::kThreads), 0, st, e->grids, e->erows, e->n_e);
-}
-
-void ens_launch_zero(EnsFields *e, hipStream_t st) {
-  hipLaunchKernelGGL(k_ens_zero, dim3(64, e->n_inst), dim3(256), 0, st, e->grids);
 }
 
 }  // namespace pdp3

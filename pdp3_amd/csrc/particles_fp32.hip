@@ -719,19 +719,18 @@ __device__ __forceinline__ F32Args from_slot(const F32Args &p, long long base) {
 // one tile of a cell-sorted (chunked) species from slot `base` (TileMap): its
 // lanes read contiguous slots (coalesced) and each walks PPT consecutive
 // logical particles, mostly of one cell.
-template <int PPT, int WAVES, class Sink>
-__device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink &gs, long long base, long long n_cap,
-                                             double *box, float *fbox) {
+template <int WAVES, class Map>
+__device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink &gs, const Map &map, long long base,
+                                             long long n_cap, double *box, float *fbox) {
+  using Sink = TileSink;
   static_assert(kFK == Sink::kK, "the two boxes share their width");
-  using Map = TileMap<PPT, WAVES>;
   const F32Args q = from_slot(p, base);
-  const unsigned lim = (unsigned)min(n_cap - base, (long long)Map::kSpan);
-  const unsigned off0 = Map::first(threadIdx.x);
+  const unsigned lim = (unsigned)min(n_cap - base, (long long)map.span());
+  const unsigned off0 = map.first(threadIdx.x);
   // the lane's first particle is on its way while the boxes are set up
   PState nx{kDead, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (off0 < lim) nx = load_state_next(q, off0 * 4u);
-  // anchor samples: slot base + j is the logical particle 16 j of a plasma
-  // tile (the chunk-transposed layout), particle j of an ensemble's bunch block
+  // anchor samples: slot base + j is the logical particle 16 j of the tile
   int ai, ak;
   {
     bool live[3];
@@ -748,7 +747,7 @@ __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink 
   // the boxes' width: half of it when the tile's last particle (the last
   // slot its threads reach) lies within the first half of the anchor's row,
   // with one column to spare
-  const uint32_t cl = base + Map::kLast < n_cap ? p.cell[base + Map::kLast] : kDead;
+  const uint32_t cl = base + map.last() < n_cap ? p.cell[base + map.last()] : kDead;
   const bool narrow = !(cl & kDead) && cell_i(cl) == ai && cell_k(cl) - ak <= kFK / 2 - 5;
   const int width = narrow ? kFK / 2 : kFK;
   Sink sk;
@@ -759,11 +758,11 @@ __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink 
   // software pipeline: the state of the lane's next particle is loaded before
   // the current one is pushed; all its loads are waited for before the
   // current particle's stores, so the wait never includes stores in flight
-  for (int j = 0; j < PPT; j++) {
+  for (int j = 0; j < map.ppt(); j++) {
     const PState cur = nx;
     unsigned n = off0 + (unsigned)j * 64u, n1 = n + 64u;
     asm("" : "+v"(n), "+v"(n1));  // keeps the slots 32-bit offsets from the scalar bases (no 64-bit pointer per array)
-    if (j + 1 < PPT && n1 < lim) nx = load_state_next(q, n1 * 4u);
+    if (j + 1 < map.ppt() && n1 < lim) nx = load_state_next(q, n1 * 4u);
     POut o;
     const bool st = n < lim && step_state32(q, sk, fs, cur, o);
     wait_loads();
@@ -789,7 +788,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
   g.nr = q.nr;
   g.nz = q.nz;
   g.err = q.err;
-  fused32_tile<PPT, WAVES, TileSink>(q, g, TileMap<PPT, WAVES>::base(blockIdx.x), n_cap, box, fbox);
+  using Map = TileMap<PPT, WAVES>;
+  fused32_tile<WAVES>(q, g, Map(), Map::base(blockIdx.x), n_cap, box, fbox);
 }
 
 // bunches (plain layout): the same walk, the box anchored at the smallest
@@ -939,43 +939,52 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
     fused32_bunch_tile<kWavesPerBlock, 1>(p, gs, block * (kWavesPerBlock * 64), g.n_cap[s], lds);
   } else {
     p.want_rho = 0;
-    fused32_tile<PPT, kWavesPerBlock, TileSink>(p, gs, TileMap<PPT, kWavesPerBlock>::base(block), g.n_cap[s], lds,
-                                                reinterpret_cast<float *>(lds + TileSink::kSize));
+    using Map = TileMap<PPT, kWavesPerBlock>;
+    fused32_tile<kWavesPerBlock>(p, gs, Map(), Map::base(block), g.n_cap[s], lds,
+                                 reinterpret_cast<float *>(lds + TileSink::kSize));
   }
 }
 
 // ensembles: the plasma tiles and bunch blocks of every instance in one
 // launch, one block per item of the work list (a persistent grid striding
 // over the list kept the loop's state in scalar registers, which spilled).
-// Bunch blocks take the plasma tile path too (their particles are not cell
-// sorted, so most of their gathers and deposits take the boxes' HBM
-// fallbacks), which keeps the kernel at the plasma path's register count.
+// The tiles of a list may differ in size; its bunch blocks, the longest for
+// their particles (gathers from HBM), come first and hold one particle per
+// lane.  16 instances, 1.27e8 particles at 12 to 40 per cell, MI355X: 1646 us;
+// with the bunches on the tiles' walk (4096 particles each, mostly past the
+// boxes) and the sparse species in a launch of their own 1739 + 91 us.
 struct EnsItem {
   int arg;   // index into the per-(instance, species) argument tables
-  int kind;  // 0 plasma tile, 1 bunch block
+  int lg;    // plasma tile of 2^lg particles per lane; -1: bunch block, one per lane
   long long base, n_cap;
 };
 
-template <int PPT, int WAVES>
-// 5 waves per SIMD (96 VGPRs, 6 scalar registers spilled into vector lanes)
-// once the table pointers are global; with flat pointers it needed 121 VGPRs
-// and ran at 4
+// 5 waves per SIMD (96 VGPRs) once the table pointers are global; with flat
+// pointers it needed 121 VGPRs and ran at 4
+template <int WAVES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5)))
 k_ens_fused32(const F32Args *__restrict__ args, const GlobalSink *__restrict__ sinks,
               const EnsItem *__restrict__ items, int n_items) {
-  __shared__ double box[TileRhoSink::kSize];
-  __shared__ __align__(16) float fbox[kFBoxFloats];
+  constexpr int kBunch = BunchSink::kSize, kTile = TileSink::kSize + (kFBoxFloats + 1) / 2;
+  __shared__ __align__(16) double lds[kBunch > kTile ? kBunch : kTile];
   const int it = blockIdx.x;
   if (it >= n_items) return;
   const EnsItem item = items[it];
   const F32ArgsG *ag = reinterpret_cast<const F32ArgsG *>(args) + item.arg;
   const GlobalSinkG *sg = reinterpret_cast<const GlobalSinkG *>(sinks) + item.arg;
-  const F32Args a = from_global(*ag);
+  F32Args a = from_global(*ag);
   GlobalSink g = from_global(*sg);
   g.nr = a.nr;  // one copy of the grid size and error word (scalar registers)
   g.nz = a.nz;
   g.err = a.err;
-  fused32_tile<PPT, WAVES, TileRhoSink>(a, g, item.base, item.n_cap, box, fbox);
+  if (item.lg < 0) {
+    a.is_bunch = a.want_rho = 1;
+    fused32_bunch_tile<WAVES, 1>(a, g, item.base, item.n_cap, lds);
+  } else {
+    a.is_bunch = a.want_rho = 0;
+    fused32_tile<WAVES>(a, g, TileMapRt<WAVES>{item.lg}, item.base, item.n_cap, lds,
+                        reinterpret_cast<float *>(lds + TileSink::kSize));
+  }
 }
 
 // plain layout (bunches): one particle per thread, deposits straight to HBM
@@ -1344,45 +1353,67 @@ void launch_f64_from_f32(Ctx &c, Species &sp) {
                      sp.f32.w);
 }
 
+// the work lists: one per tile shape that can be set (index into kTileShapes),
+// and two whose tiles follow each species' size, for particles in cell order
+// and in the ensemble sort's bands (kNumTiles, kNumTiles + 1)
+constexpr int kEnsLists = kNumTiles + 2;
 struct EnsParticles {
   int n_args = 0;
   F32Args *args = nullptr;
   GlobalSink *sinks = nullptr;
-  // work list per tile shape (plasma tiles and bunch blocks), and at index
-  // kNumTiles the one-chunk tiles of the sparse plasma species (below
-  // kSparsePpc particles per cell), which the lists of the larger shapes leave
-  // out: a tile spans tile / ppc cells, and one chunk is the smallest tile
-  EnsItem *items[kNumTiles + 1] = {};
-  int n_items[kNumTiles + 1] = {};
+  EnsItem *items[kEnsLists] = {};
+  int n_items[kEnsLists] = {};
 };
 
 namespace {
+// a set shape's tiles are cut to one chunk for species below kSparsePpc
+// particles per cell (a tile spans tile / ppc cells)
 constexpr int kSparsePpc = 16;
-// the argument table and the work lists of the ensemble's species
-void ens_lists(const std::vector<Ctx *> &ctxs, std::vector<F32Args> *args,
-               std::vector<EnsItem> items[kNumTiles + 1]) {
+// particles per lane (2^lg) of a species' tiles of 4 waves: the largest tile
+// whose cells its boxes hold (the setting up of the boxes costs each tile the
+// same, a particle past them gathers from HBM); unlike a single run's, an
+// ensemble's tiles fill the GPU whatever their size.  In
+// bands of two rows (species below 32 particles per cell, once the ensemble has
+// sorted) a tile spans half as many columns.
+int ens_auto_lg(const Ctx &c, const Species &sp, bool banded) {
+  const double cells = (double)(c.g.nr - 1) * (double)(c.g.nz - 1);
+  const double rows = banded && sp.n < 32 * cells ? 2 : 1;
+  int lg = 4;
+  while (lg > 0 && (256 << lg) * cells > rows * (kFK - 4) * (double)sp.n) lg--;
+  return lg;
+}
+std::vector<EnsItem> ens_list(const std::vector<Ctx *> &ctxs, int list) {
+  std::vector<EnsItem> items, tiles;
+  const bool set = list < kNumTiles;
+  const int waves = set ? kTileShapes[list][1] : kWavesPerBlock;
   int a = 0;
   for (Ctx *cp : ctxs) {
     Ctx &c = *cp;
     // every species by index, a bunch whether or not it has been created
     // (until its injection its particles are dead and do nothing)
-    for (int j = 0; j < (int)c.species.size(); j++) {
-      Species &sp = c.species[j];
+    for (Species &sp : c.species) {
       if (sp.n_cap <= 0 || !sp.f32.cell) continue;
-      args->push_back(args32(c, sp));
-      const bool sparse = sp.chunked && sp.n < (long long)kSparsePpc * (c.g.nr - 1) * (c.g.nz - 1);
-      for (int t = 0; t <= kNumTiles; t++) {
-        // the one-chunk shape's own list holds every species; the others
-        // leave the sparse ones to the extra list
-        if (t < kNumTiles && t != kChunkTile && sparse) continue;
-        if (t == kNumTiles && !sparse) continue;
-        const int ts = t == kNumTiles ? kChunkTile : t;
-        const long long tile = (long long)kTileShapes[ts][1] * kTileShapes[ts][0] / kPPT * kChunk;
-        for (long long b = 0; b < sp.n_cap; b += tile) items[t].push_back(EnsItem{a, sp.chunked ? 0 : 1, b, sp.n_cap});
+      if (!sp.chunked) {
+        for (long long b = 0; b < sp.n_cap; b += waves * 64) items.push_back(EnsItem{a, -1, b, sp.n_cap});
+      } else {
+        int lg = 0;
+        while (set && (1 << lg) < kTileShapes[list][0]) lg++;
+        if (!set) lg = ens_auto_lg(c, sp, list == kNumTiles + 1);
+        if (set && sp.n < (long long)kSparsePpc * (c.g.nr - 1) * (c.g.nz - 1))
+          while ((waves * 64 << lg) > kChunk) lg--;
+        const long long tile = (long long)waves * 64 << lg;
+        for (long long t = 0; t * tile < sp.n_cap; t++) {
+          // TileMap::base
+          const long long per = tile < kChunk ? kChunk / tile : 1;
+          const long long base = tile < kChunk ? t / per * kChunk + t % per * (tile / kPPT) : t * tile;
+          tiles.push_back(EnsItem{a, lg, base, sp.n_cap});
+        }
       }
       a++;
     }
   }
+  items.insert(items.end(), tiles.begin(), tiles.end());
+  return items;
 }
 }  // namespace
 
@@ -1407,17 +1438,16 @@ int ens_particles_update(EnsParticles *e, const std::vector<Ctx *> &ctxs) {
 
 EnsParticles *ens_particles_build(const std::vector<Ctx *> &ctxs) {
   auto *e = new EnsParticles;
-  std::vector<F32Args> args;
-  std::vector<EnsItem> items[kNumTiles + 1];
-  ens_lists(ctxs, &args, items);
-  e->n_args = (int)args.size();
+  for (Ctx *cp : ctxs)
+    for (Species &sp : cp->species) e->n_args += sp.n_cap > 0 && sp.f32.cell ? 1 : 0;
   bool ok = hipMalloc((void **)&e->args, std::max(1, e->n_args) * sizeof(F32Args)) == hipSuccess &&
             hipMalloc((void **)&e->sinks, std::max(1, e->n_args) * sizeof(GlobalSink)) == hipSuccess;
-  for (int t = 0; ok && t <= kNumTiles; t++) {
-    e->n_items[t] = (int)items[t].size();
-    ok = hipMalloc((void **)&e->items[t], std::max<size_t>(1, items[t].size()) * sizeof(EnsItem)) == hipSuccess &&
-         (items[t].empty() || hipMemcpy(e->items[t], items[t].data(), items[t].size() * sizeof(EnsItem),
-                                        hipMemcpyHostToDevice) == hipSuccess);
+  for (int t = 0; t < kEnsLists && ok; t++) {
+    const std::vector<EnsItem> items = ens_list(ctxs, t);
+    const size_t bytes = items.size() * sizeof(EnsItem);
+    e->n_items[t] = (int)items.size();
+    ok = hipMalloc((void **)&e->items[t], std::max(bytes, sizeof(EnsItem))) == hipSuccess &&
+         (items.empty() || hipMemcpy(e->items[t], items.data(), bytes, hipMemcpyHostToDevice) == hipSuccess);
   }
   if (!ok || ens_particles_update(e, ctxs) != 0) {
     ens_particles_free(e);
@@ -1426,6 +1456,8 @@ EnsParticles *ens_particles_build(const std::vector<Ctx *> &ctxs) {
   return e;
 }
 
+int ens_auto_list(bool banded) { return kNumTiles + (banded ? 1 : 0); }
+
 void ens_particles_free(EnsParticles *e) {
   if (!e) return;
   if (e->args) (void)hipFree(e->args);
@@ -1433,14 +1465,6 @@ void ens_particles_free(EnsParticles *e) {
   for (auto *p : e->items)
     if (p) (void)hipFree(p);
   delete e;
-}
-
-template <int PPT, int WAVES>
-void ens_launch_t(EnsParticles *e, int t, hipStream_t st) {
-  const int blocks = e->n_items[t];
-  if (blocks <= 0) return;
-  hipLaunchKernelGGL((k_ens_fused32<PPT, WAVES>), dim3(blocks), dim3(WAVES * 64), 0, st, e->args, e->sinks,
-                     e->items[t], e->n_items[t]);
 }
 
 void ens_launch_inject(const EnsInjectItem *items, int n_items, int max_count, const long long *step,
@@ -1454,18 +1478,11 @@ void ens_launch_count(long long *step, hipStream_t st) {
   hipLaunchKernelGGL(k_ens_count, dim3(1), dim3(64), 0, st, step);
 }
 
-void ens_launch_particles(EnsParticles *e, int tile, hipStream_t st) {
-  switch (tile) {
-    case 0: ens_launch_t<16, 4>(e, 0, st); break;
-    case 1: ens_launch_t<16, 2>(e, 1, st); break;
-    case 2: ens_launch_t<16, 1>(e, 2, st); break;
-    case 3: ens_launch_t<8, 4>(e, 3, st); break;
-    case 4: ens_launch_t<8, 2>(e, 4, st); break;
-    default: ens_launch_t<4, 4>(e, 5, st); break;
-  }
-  // the sparse species on one-chunk tiles (their list is empty when the
-  // shape is the one-chunk shape itself, whose list holds them)
-  if (tile != kChunkTile) ens_launch_t<4, 4>(e, kNumTiles, st);
+void ens_launch_particles(EnsParticles *e, int list, hipStream_t st) {
+  const int n = e->n_items[list], waves = list < kNumTiles ? kTileShapes[list][1] : kWavesPerBlock;
+  if (n <= 0) return;
+  auto kernel = waves == 4 ? k_ens_fused32<4> : waves == 2 ? k_ens_fused32<2> : k_ens_fused32<1>;
+  hipLaunchKernelGGL(kernel, dim3(n), dim3(waves * 64), 0, st, e->args, e->sinks, e->items[list], n);
 }
 
 }  // namespace pdp3

@@ -67,12 +67,9 @@ struct GlobalSink {
 // 128 columns (a sorted block covers a run of cells along one row), the bunch
 // box 16 rows by 32 columns (a bunch block is a thin disc of particles
 // injected in the same step)
-// COMPS: 3, or 4 where rho is deposited too (RHO: also summed in registers)
-template <bool RHO, int COMPS, int BR = 4, int BK = 128>
+template <bool RHO, int BR = 4, int BK = 128>
 struct TileSinkT {
-  static constexpr int kComps = COMPS;
-  static_assert(COMPS == 3 || COMPS == 4, "J_r, J_phi, J_z and rho");
-  static_assert(COMPS == 4 || !RHO, "rho sums need the box's fourth component");
+  static constexpr int kComps = RHO ? 4 : 3;  // rho only where it is deposited
   static constexpr int kR = BR, kK = BK, kSize = kComps * BR * BK;
   GlobalSink g;
   double *box;  // LDS, kComps x kR x kK
@@ -87,7 +84,7 @@ struct TileSinkT {
 
   __device__ __forceinline__ void box_put(int comp, int i, int k, double v) {
     int li = i - bi, lk = k - bk;
-    if (comp < COMPS && (unsigned)li < (unsigned)BR && (unsigned)lk < (unsigned)bw)
+    if ((unsigned)li < (unsigned)BR && (unsigned)lk < (unsigned)bw)
       atomicAdd(box + (comp * BR + li) * BK + lk, v);
     else
       g.put(comp, i, k, v);
@@ -212,9 +209,8 @@ struct TileSinkT {
     }
   }
 };
-using TileSink = TileSinkT<false, 3>;       // plasma species
-using TileRhoSink = TileSinkT<false, 4>;    // an ensemble's tiles, bunch blocks among them
-using BunchSink = TileSinkT<true, 4, 16, 32>;
+using TileSink = TileSinkT<false>;  // plasma species: no rho
+using BunchSink = TileSinkT<true, 16, 32>;
 
 // One grid's node deposits of a tile (charge weighting outside the loop, the
 // density probe): the four corners of the lane's current cell in registers, an

@@ -84,6 +84,30 @@ def test_ensemble_tiles_and_autotune():
     ens.close()
 
 
+@pytest.mark.parametrize("ppc", [1, 3, 8, 15, 16, 31, 33])
+def test_ensemble_tiles_by_size(ppc):
+    """Tiles that follow each species' size (the shape is not set), in one
+    launch: from 256 particles to four chunks, partly filled last chunks, in
+    cell order and then in bands after the second sort; the tolerance is that
+    of the same instances at set shapes (FP64 sums in another order)."""
+    from pdp3_amd import capi
+    from pdp3_amd import workloads as wl
+
+    insts = [wl.Instance(cells_r=17, cells_z=61, ppc=ppc, density=1e17, bunch_ratio=0.2, seed=5, bunch_macro=257),
+             wl.Instance(cells_r=9, cells_z=130, ppc=3 * ppc, density=1e16, bunch_ratio=0.3, seed=6, bunch_macro=63)]
+    alone = [wl.build_instance(i) for i in insts]
+    members = [wl.build_instance(i) for i in insts]
+    for s in alone:
+        s.step(7)
+    ens = capi.Ensemble(members)
+    ens.step(3)
+    ens.set_sort_interval(2)
+    ens.step(4)
+    for a, m in zip(alone, members):
+        _compare(m, a, 1e-10)
+    ens.close()
+
+
 def test_ensemble_sort_orders_by_cell_or_band():
     """The ensemble's batched sort orders each instance's plasma stably by its
     key: row-major cells for instances with at least 32 particles per cell,
