@@ -11,14 +11,17 @@
 //   runs:    each wavefront's 64 consecutive keys split into runs of equal
 //            keys (a run never spans two wavefronts); one record (key,
 //            length) per run, in logical order
-//   records: stable LSD radix sort of the records by key, 8-bit digits:
-//              hist:    per block of 16384 records, a 256-bin digit histogram
+//   records: stable LSD radix sort of the records by key, digits of up to 10
+//            bits (the width that divides the key into the fewest equal parts):
+//              hist:    per block of 4096 records, a digit histogram
 //              scan:    exclusive scan of the bin-major histogram matrix
 //              scatter: per block, stable ranks from wavefront ballots (lanes
-//                       holding the same digit are matched with 8 ballots),
-//                       running per-wave digit counters in LDS
+//                       holding the same digit are matched with one ballot
+//                       per bit), running per-wave digit counters in LDS
 //   ranks:   exclusive scan of the run lengths in sorted order: each run's
 //            first rank; a particle's rank = its run's + its place in the run
+// The grids are sized for the record capacity (the number of records is known
+// on the device only); what lies past the records' number returns at once.
 // then every particle array is gathered through the resulting permutation in
 // one pass (for a particle that stayed in place the gather reads its own
 // slot, so a nearly sorted species is moved with coalesced reads).
@@ -28,11 +31,17 @@ namespace pdp3 {
 
 namespace {
 
+// A radix block: each lane holds 16 records of its wave in registers, their
+// loads all in flight at once: a scatter launch takes 15 us where there are few
+// (1e6 particles of 13 per cell) and 106 us for an ensemble of 1.3e8.  (4096
+// per wave, read one at a time in two passes, took 64 us and 290 us: a chain
+// of 128 loads.)
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-constexpr int kPerWave = 4096;
-constexpr int kPerBlock = kWaves * kPerWave;  // 16384
-constexpr int kBins = 256;
+constexpr int kPer = 16;  // records per lane
+constexpr int kPerBlock = kThreads * kPer;
+constexpr int kMaxDigit = 10;
+constexpr int kMaxBins = 1 << kMaxDigit;
 
 // the number of records present: the count on the device, or none when it
 // exceeds the capacity (that sort is then skipped)
@@ -41,40 +50,8 @@ __device__ __forceinline__ long long present(const uint32_t *count, long long ca
   return m <= cap ? m : 0;
 }
 
-__global__ void __launch_bounds__(kThreads) k_hist(const uint32_t *__restrict__ keys, const uint32_t *count,
-                                                   long long cap, int shift, uint32_t *__restrict__ hist,
-                                                   int nblocks) {
-  __shared__ uint32_t cnt[kBins];
-  const long long n = present(count, cap);
-  cnt[threadIdx.x] = 0;
-  __syncthreads();
-  long long base = (long long)blockIdx.x * kPerBlock;
-  long long end = min(base + (long long)kPerBlock, n);
-  for (long long j = base + threadIdx.x; j < end; j += kThreads) atomicAdd(&cnt[(keys[j] >> shift) & 0xFF], 1u);
-  __syncthreads();
-  hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = cnt[threadIdx.x];
-}
-
-// exclusive scan, three phases: per-block sums, scan of the sums, add back
-constexpr int kScanBlock = 1024;
-__global__ void __launch_bounds__(kScanBlock) k_scan_local(uint32_t *data, long long n, uint32_t *sums) {
-  __shared__ uint32_t s[kScanBlock];
-  long long j = (long long)blockIdx.x * kScanBlock + threadIdx.x;
-  uint32_t v = j < n ? data[j] : 0u;
-  s[threadIdx.x] = v;
-  __syncthreads();
-  for (int off = 1; off < kScanBlock; off <<= 1) {
-    uint32_t t = threadIdx.x >= (unsigned)off ? s[threadIdx.x - off] : 0u;
-    __syncthreads();
-    s[threadIdx.x] += t;
-    __syncthreads();
-  }
-  if (j < n) data[j] = s[threadIdx.x] - v;
-  if (threadIdx.x == kScanBlock - 1) sums[blockIdx.x] = s[threadIdx.x];
-}
-__global__ void k_scan_add(uint32_t *data, long long n, const uint32_t *sums) {
-  long long j = (long long)blockIdx.x * kScanBlock + threadIdx.x;
-  if (j < n) data[j] += sums[blockIdx.x];
+__host__ __device__ __forceinline__ uint32_t radix_blocks(long long n) {
+  return (uint32_t)((n + kPerBlock - 1) / kPerBlock);
 }
 
 __device__ __forceinline__ uint64_t lanemask_lt() {
@@ -82,76 +59,208 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
-// lanes (among `active`) whose digit equals this lane's digit
-__device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t active) {
+// lanes (among `active`) whose digit of `width` bits equals this lane's
+__device__ __forceinline__ uint64_t match_digit(uint32_t d, uint64_t active, int width) {
   uint64_t m = active;
-  for (int b = 0; b < 8; b++) {
+  for (int b = 0; b < width; b++) {
     uint64_t bal = __ballot((d >> b) & 1u);
     m &= ((d >> b) & 1u) ? bal : ~bal;
   }
   return m;
 }
 
-__global__ void __launch_bounds__(kThreads) k_scatter(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin,
-                                                      uint32_t *__restrict__ kout, uint32_t *__restrict__ vout,
-                                                      const uint32_t *count, long long cap, int shift,
-                                                      const uint32_t *__restrict__ offs, int nblocks) {
-  __shared__ uint32_t run[kWaves][kBins];
+// hist[digit * blocks + block], blocks = those that hold records
+__global__ void __launch_bounds__(kThreads) k_hist(const uint32_t *__restrict__ keys, const uint32_t *count,
+                                                   long long cap, int shift, int width, uint32_t *__restrict__ hist) {
+  __shared__ uint32_t cnt[kMaxBins];
   const long long n = present(count, cap);
-  const int wave = threadIdx.x / 64;
-  for (int t = threadIdx.x; t < kWaves * kBins; t += kThreads) run[t / kBins][t % kBins] = 0;
+  const uint32_t blocks = radix_blocks(n), bins = 1u << width;
+  if (blockIdx.x >= blocks) return;
+  const long long base = (long long)blockIdx.x * kPerBlock + threadIdx.x;
+  uint32_t key[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; u++) key[u] = base + u * kThreads < n ? keys[base + u * kThreads] : 0u;
+  for (uint32_t d = threadIdx.x; d < bins; d += kThreads) cnt[d] = 0;
   __syncthreads();
-  const long long base = (long long)blockIdx.x * kPerBlock + (long long)wave * kPerWave;
-  const unsigned lane = __lane_id();
-  // phase 1: per-wave digit totals
-  for (int it = 0; it < kPerWave / 64; it++) {
-    long long j = base + it * 64 + lane;
-    bool valid = j < n;
-    uint64_t active = __ballot(valid);
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const bool valid = base + u * kThreads < n;
+    const uint32_t d = (key[u] >> shift) & (bins - 1);
+    // records that are nearly in order mostly share their high digits
+    const uint64_t active = __ballot(valid);
     if (active == 0) break;
-    uint32_t d = valid ? (kin[j] >> shift) & 0xFF : 0u;
-    uint64_t m = match_digit(d, active);
-    if (valid && (m & lanemask_lt()) == 0) run[wave][d] += (uint32_t)__popcll(m);
+    const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);  // the valid lanes are a prefix
+    if (__ballot(valid && d == d0) == active) {
+      if (__lane_id() == 0) atomicAdd(&cnt[d0], (uint32_t)__popcll(active));
+    } else if (valid) {
+      atomicAdd(&cnt[d], 1u);
+    }
   }
   __syncthreads();
-  // bases: global offset of this block for the digit plus earlier waves
-  {
-    int d = threadIdx.x;
-    uint32_t acc = offs[(size_t)d * nblocks + blockIdx.x];
+  for (uint32_t d = threadIdx.x; d < bins; d += kThreads) hist[(size_t)d * blocks + blockIdx.x] = cnt[d];
+}
+
+__global__ void __launch_bounds__(kThreads) k_scatter(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                                      uint32_t *__restrict__ kout, uint32_t *__restrict__ vout,
+                                                      const uint32_t *count, long long cap, int shift, int width,
+                                                      const uint32_t *__restrict__ offs) {
+  __shared__ uint32_t run[kWaves][kMaxBins];
+  const long long n = present(count, cap);
+  const uint32_t blocks = radix_blocks(n), bins = 1u << width;
+  if (blockIdx.x >= blocks) return;
+  const int wave = threadIdx.x / 64;
+  const unsigned lane = __lane_id();
+  const long long base = (long long)blockIdx.x * kPerBlock + (long long)wave * (64 * kPer) + lane;
+  uint32_t key[kPer], val[kPer], place[kPer], off[kMaxBins / kThreads];
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const bool valid = base + u * 64 < n;
+    key[u] = valid ? kin[base + u * 64] : 0u;
+    val[u] = valid ? vin[base + u * 64] : 0u;
+  }
+#pragma unroll
+  for (int u = 0; u < kMaxBins / kThreads; u++) {
+    const uint32_t d = u * kThreads + threadIdx.x;
+    off[u] = d < bins ? offs[(size_t)d * blocks + blockIdx.x] : 0u;
+    for (int w = 0; w < kWaves; w++) run[w][d] = 0;
+  }
+  __syncthreads();
+  // each record's place among its wave's records of the same digit
+#pragma unroll
+  for (int u = 0; u < kPer; u++) {
+    const bool valid = base + u * 64 < n;
+    const uint64_t active = __ballot(valid);
+    if (active == 0) break;
+    const uint32_t d = (key[u] >> shift) & (bins - 1);
+    const uint64_t m = match_digit(d, active, width);
+    const uint32_t before = run[wave][d];
+    place[u] = before + (uint32_t)__popcll(m & lanemask_lt());
+    // every lane's read of run[] before the leaders' update
+    __builtin_amdgcn_wave_barrier();
+    if (valid && (m & lanemask_lt()) == 0) run[wave][d] = before + (uint32_t)__popcll(m);
+    __builtin_amdgcn_wave_barrier();
+  }
+  __syncthreads();
+  // the global offset of the block's records of each digit, then of each wave's
+#pragma unroll
+  for (int u = 0; u < kMaxBins / kThreads; u++) {
+    const uint32_t d = u * kThreads + threadIdx.x;
+    uint32_t acc = off[u];
     for (int w = 0; w < kWaves; w++) {
-      uint32_t c = run[w][d];
+      const uint32_t c = run[w][d];
       run[w][d] = acc;
       acc += c;
     }
   }
   __syncthreads();
-  // phase 2: stable positions and scatter
-  for (int it = 0; it < kPerWave / 64; it++) {
-    long long j = base + it * 64 + lane;
-    bool valid = j < n;
-    uint64_t active = __ballot(valid);
-    if (active == 0) break;
-    uint32_t key = valid ? kin[j] : 0u;
-    uint32_t d = (key >> shift) & 0xFF;
-    uint64_t m = match_digit(d, active);
-    uint32_t pos = run[wave][d] + (uint32_t)__popcll(m & lanemask_lt());
-    if (valid) {
-      kout[pos] = key;
-      vout[pos] = vin[j];
+#pragma unroll
+  for (int u = 0; u < kPer; u++)
+    if (base + u * 64 < n) {
+      const uint32_t pos = run[wave][(key[u] >> shift) & (bins - 1)] + place[u];
+      kout[pos] = key[u];
+      vout[pos] = val[u];
     }
-    // make every lane's read of run[] happen before the leaders update it
-    __builtin_amdgcn_wave_barrier();
-    if (valid && (m & lanemask_lt()) == 0) run[wave][d] += (uint32_t)__popcll(m);
-    __builtin_amdgcn_wave_barrier();
+}
+
+// ---- exclusive scan: the blocks' sums, then each block's scan from the sum
+// of those before it (the block adds them up itself).  S: size(), load(j),
+// store(j, scanned); one thread loads and stores an element, so that both may
+// be the same array. ----
+constexpr int kScanThreads = 1024, kScanPer = 4, kScanBlock = kScanThreads * kScanPer;
+// a block adding up more sums than this would cost more than scanning them first
+constexpr long long kScanSums = 8192;
+
+struct ScanArray {
+  uint32_t *p;
+  long long n;
+  __device__ __forceinline__ long long size() const { return n; }
+  __device__ __forceinline__ uint32_t load(long long j) const { return p[j]; }
+  __device__ __forceinline__ void store(long long j, uint32_t v) const { p[j] = v; }
+};
+// the histogram matrix of the records present
+struct ScanHist {
+  uint32_t *p;
+  const uint32_t *count;
+  long long cap;
+  int width;
+  __device__ __forceinline__ long long size() const { return (long long)radix_blocks(present(count, cap)) << width; }
+  __device__ __forceinline__ uint32_t load(long long j) const { return p[j]; }
+  __device__ __forceinline__ void store(long long j, uint32_t v) const { p[j] = v; }
+};
+// the run lengths in sorted order; each is replaced by its run's first rank
+struct ScanRuns {
+  const uint32_t *order;
+  uint32_t *len;
+  const uint32_t *count;
+  long long cap;
+  __device__ __forceinline__ long long size() const { return present(count, cap); }
+  __device__ __forceinline__ uint32_t load(long long j) const { return len[order[j]]; }
+  __device__ __forceinline__ void store(long long j, uint32_t v) const { len[order[j]] = v; }
+};
+
+// the exclusive prefix of v over the block and, in total, its sum; w: kScanThreads / 64 words of LDS
+__device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t *w, uint32_t &total) {
+  const unsigned lane = __lane_id(), wave = threadIdx.x >> 6;
+  uint32_t x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o);
+    if (lane >= (unsigned)o) x += y;
   }
+  __syncthreads();  // the last use of w
+  if (lane == 63) w[wave] = x;
+  __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (unsigned k = 0; k < kScanThreads / 64; k++) {
+    before += k < wave ? w[k] : 0u;
+    total += w[k];
+  }
+  return before + x - v;
+}
+
+template <class S>
+__global__ void __launch_bounds__(kScanThreads) k_scan_sums(S s, uint32_t *__restrict__ sums) {
+  __shared__ uint32_t w[kScanThreads / 64];
+  const long long n = s.size(), j0 = (long long)blockIdx.x * kScanBlock + threadIdx.x;
+  uint32_t v = 0, total;
+  if (j0 - threadIdx.x < n) {
+#pragma unroll
+    for (int u = 0; u < kScanPer; u++) v += j0 + u * kScanThreads < n ? s.load(j0 + u * kScanThreads) : 0u;
+  }
+  block_prefix(v, w, total);
+  if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+// scanned: sums holds the exclusive prefixes already
+template <class S>
+__global__ void __launch_bounds__(kScanThreads) k_scan_write(S s, const uint32_t *__restrict__ sums, int scanned) {
+  __shared__ uint32_t w[kScanThreads / 64];
+  const long long n = s.size(), j0 = (long long)blockIdx.x * kScanBlock + (long long)threadIdx.x * kScanPer;
+  if ((long long)blockIdx.x * kScanBlock >= n) return;
+  uint32_t v[kScanPer], base = 0, t = 0, total;
+#pragma unroll
+  for (int u = 0; u < kScanPer; u++) {
+    v[u] = j0 + u < n ? s.load(j0 + u) : 0u;
+    t += v[u];
+  }
+  if (scanned) {
+    base = sums[blockIdx.x];
+  } else if (blockIdx.x > 0) {
+    uint32_t b = 0;
+    for (unsigned k = threadIdx.x; k < blockIdx.x; k += kScanThreads) b += sums[k];
+    block_prefix(b, w, base);
+  }
+  uint32_t acc = base + block_prefix(t, w, total);
+#pragma unroll
+  for (int u = 0; u < kScanPer; u++)
+    if (j0 + u < n) {
+      s.store(j0 + u, acc);
+      acc += v[u];
+    }
 }
 
 // ---- runs of equal keys ----
-
-__global__ void k_fill_u32(uint32_t *p, long long n, uint32_t v) {
-  long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j < n) p[j] = v;
-}
 
 // the runs of this wavefront's keys (lanes >= the valid prefix are not
 // keys): heads = mask of first lanes; head, len = this lane's run
@@ -243,7 +352,8 @@ __device__ __forceinline__ uint32_t run_index(const ChunkRuns &cr, int m, uint32
   return r + (uint32_t)__popcll(below);
 }
 
-// runs per group of 256 logical keys
+// runs per group of 256 logical keys, and a zero behind the last group's (where
+// the scan leaves the number of runs)
 template <class K>
 __global__ void __launch_bounds__(256) k_run_count(K keys, long long nch, uint32_t *__restrict__ block_runs) {
   __shared__ uint32_t t[kCPB * kChunkLds];
@@ -256,6 +366,7 @@ __global__ void __launch_bounds__(256) k_run_count(K keys, long long nch, uint32
     const uint32_t *g = wc + threadIdx.x * 4;
     block_runs[(long long)blockIdx.x * kBlockGroups + threadIdx.x] = g[0] + g[1] + g[2] + g[3];
   }
+  if (blockIdx.x == 0 && threadIdx.x == 0) block_runs[nch * kGroups] = 0;
 }
 
 // one record (key, index, length) per run
@@ -280,21 +391,6 @@ __global__ void __launch_bounds__(256) k_run_emit(K keys, long long nch, const u
       rlen[r] = (uint32_t)cr.len[m];
     }
   }
-}
-
-// lens[t] = length of the t-th run in key order; after the scan of lens,
-// rfirst[run] = its first rank
-__global__ void k_run_lens(const uint32_t *__restrict__ order, const uint32_t *__restrict__ rlen,
-                           const uint32_t *count, long long cap, uint32_t *__restrict__ lens) {
-  const long long m = present(count, cap);
-  long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < cap) lens[t] = t < m ? rlen[order[t]] : 0u;
-}
-__global__ void k_run_first(const uint32_t *__restrict__ order, const uint32_t *__restrict__ lens,
-                            const uint32_t *count, long long cap, uint32_t *__restrict__ rfirst) {
-  const long long m = present(count, cap);
-  long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < m) rfirst[order[t]] = lens[t];
 }
 
 // src[rank] = the slot of the particle of that rank, indexed by logical
@@ -456,13 +552,15 @@ struct KeysMulti {
   __device__ __forceinline__ uint32_t operator()(long long j) const { return at_chunk(j - j % kChunk)(j); }
 };
 
-void exclusive_scan(uint32_t *data, long long n, uint32_t *tmp, hipStream_t s) {
-  long long nb = (n + kScanBlock - 1) / kScanBlock;
-  hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nb), dim3(kScanBlock), 0, s, data, n, tmp);
-  if (nb > 1) {
-    exclusive_scan(tmp, nb, tmp + nb, s);
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nb), dim3(kScanBlock), 0, s, data, n, tmp);
-  }
+// scans at most n elements (S::size() on the device may be fewer); sums:
+// scan_scratch(n) words
+template <class S>
+void exclusive_scan(const S &s, long long n, uint32_t *sums, hipStream_t st) {
+  const long long nb = (n + kScanBlock - 1) / kScanBlock;
+  const bool two = nb > kScanSums;
+  if (nb > 1) hipLaunchKernelGGL(k_scan_sums<S>, dim3((unsigned)nb), dim3(kScanThreads), 0, st, s, sums);
+  if (two) exclusive_scan(ScanArray{sums, nb}, nb, sums + nb, st);
+  hipLaunchKernelGGL(k_scan_write<S>, dim3((unsigned)nb), dim3(kScanThreads), 0, st, s, sums, two ? 1 : 0);
 }
 // scratch words exclusive_scan needs for n elements
 long long scan_scratch(long long n) {
@@ -474,19 +572,26 @@ long long scan_scratch(long long n) {
   return t + 1;
 }
 
-// stable LSD radix sort of m (key, val) pairs by the low `bits` bits of the
-// key; returns the buffers holding the result (a or b)
+int digit_width(int bits) {
+  const int passes = (bits + kMaxDigit - 1) / kMaxDigit;
+  return (bits + passes - 1) / passes;
+}
+// words of the histogram matrix and its scan
+long long hist_words(long long cap, int bits) { return (long long)radix_blocks(cap) << digit_width(bits); }
+
+// stable LSD radix sort of the (key, val) pairs by the low `bits` bits of the
+// key; returns the buffers holding the result (a or b).  hist: hist_words and
+// their scan's scratch
 void radix_pairs(uint32_t *&ka, uint32_t *&va, uint32_t *&kb, uint32_t *&vb, const uint32_t *count, long long cap,
-                 int bits, uint32_t *hist, uint32_t *tmp, hipStream_t st) {
-  const int passes = (bits + 7) / 8;
-  const int nblocks = (int)((cap + kPerBlock - 1) / kPerBlock);
-  const long long hist_n = (long long)kBins * nblocks;
-  for (int p = 0; p < passes; p++) {
-    const int shift = 8 * p;
-    hipLaunchKernelGGL(k_hist, dim3(nblocks), dim3(kThreads), 0, st, ka, count, cap, shift, hist, nblocks);
-    exclusive_scan(hist, hist_n, tmp, st);
-    hipLaunchKernelGGL(k_scatter, dim3(nblocks), dim3(kThreads), 0, st, ka, va, kb, vb, count, cap, shift, hist,
-                       nblocks);
+                 int bits, uint32_t *hist, hipStream_t st) {
+  const int width = digit_width(bits);
+  const uint32_t blocks = radix_blocks(cap);
+  const long long words = hist_words(cap, bits);
+  for (int shift = 0; shift < bits; shift += width) {
+    hipLaunchKernelGGL(k_hist, dim3(blocks), dim3(kThreads), 0, st, ka, count, cap, shift, width, hist);
+    exclusive_scan(ScanHist{hist, count, cap, width}, words, hist + words, st);
+    hipLaunchKernelGGL(k_scatter, dim3(blocks), dim3(kThreads), 0, st, ka, va, kb, vb, count, cap, shift, width,
+                       hist);
     std::swap(ka, kb);
     std::swap(va, vb);
   }
@@ -501,22 +606,34 @@ bool ensure_alt(void *&alt, size_t bytes) {
   return true;
 }
 
-// workspace bytes for n slots and cap run records (u32 words): src (n); group
-// counts (nb + 1); scratch for the scans of the group counts and run lengths
-// and for the records' digit histograms with their scan; the records (5 per
+// workspace bytes for n slots and cap run records of `bits` bits (u32 words):
+// src (n), before it is written the digit histograms with their scan, where
+// they fit; group counts (nb + 1); scratch for the scans of the group counts
+// and run lengths, and for the histograms that do not fit; the records (5 per
 // slot)
 struct SortWs {
-  long long nb, rec_hist, scratch;
+  long long nb, scratch;
+  bool hist_in_src;
   size_t bytes;
 };
-SortWs sort_ws(long long n, long long cap) {
+SortWs sort_ws(long long n, long long cap, int bits) {
   SortWs w;
   w.nb = (n + 255) / 256;
-  w.rec_hist = (long long)kBins * ((cap + kPerBlock - 1) / kPerBlock);
-  w.scratch = std::max(std::max(scan_scratch(w.nb + 1), scan_scratch(cap)), w.rec_hist + scan_scratch(w.rec_hist)) +
-              1024;
+  const long long words = hist_words(cap, bits), hist = words + scan_scratch(words);
+  w.hist_in_src = hist <= n;
+  w.scratch = std::max(std::max(scan_scratch(w.nb + 1), scan_scratch(cap)), w.hist_in_src ? 0 : hist);
   w.bytes = (size_t)(n + (w.nb + 1) + w.scratch + 5 * cap) * sizeof(uint32_t);
   return w;
+}
+// bits of the keys 0 .. nkeys - 1 (at least one)
+int key_bits(unsigned long long nkeys) {
+  int bits = 1;
+  while ((1ull << bits) < nkeys) bits++;
+  return bits;
+}
+// the keys of a species: cells, the dead particles' and the padding's
+unsigned long long cell_keys(const Ctx &c) {
+  return (unsigned long long)(c.g.nr - 1) * (unsigned long long)(c.g.nz - 1) + 2;
 }
 bool ensure_ws(Ctx &c, size_t need) {
   if (c.sort_ws_bytes >= need) return true;
@@ -570,7 +687,7 @@ size_t sort_periodic_bytes(const Ctx &c) {
   for (const Species &sp : c.species) {
     if (sp.kind != 0 || !sortable(c, sp)) continue;
     const long long cap = sp.rec_cap > 0 ? sp.rec_cap : std::min(sp.n_cap, sp.n_cap / 4 + 65536);
-    need = std::max(need, sort_ws(sp.n_cap, cap).bytes);
+    need = std::max(need, sort_ws(sp.n_cap, cap, key_bits(cell_keys(c))).bytes);
   }
   return need;
 }
@@ -588,7 +705,7 @@ int sort_prepare(Ctx &c, Species &sp) {
   if (sp.sort_prepared || !sortable(c, sp)) return 0;
   const long long n = sp.n_cap;
   if (sp.rec_cap <= 0) sp.rec_cap = std::min(n, n / 4 + 65536);
-  if (!ensure_runs(sp) || !ensure_ws(c, sort_ws(n, sp.rec_cap).bytes) || !ensure_alts(c, sp)) return -3;
+  if (!ensure_runs(sp) || !ensure_ws(c, sort_ws(n, sp.rec_cap, key_bits(cell_keys(c))).bytes) || !ensure_alts(c, sp)) return -3;
   sp.sort_prepared = true;
   return 0;
 }
@@ -599,8 +716,7 @@ int sort_species(Ctx &c, Species &sp, bool exact) {
   if (n % kChunk != 0) return -1;  // a chunked species fills whole chunks
   const uint32_t ncell = (uint32_t)(c.g.nr - 1) * (uint32_t)(c.g.nz - 1);
   const uint32_t dead_key = ncell;
-  int bits = 1;
-  while ((1ull << bits) <= (unsigned long long)dead_key + 1) bits++;
+  const int bits = key_bits(cell_keys(c));
   // record capacity: grown from the previous sort's run count (read back
   // asynchronously), so that no sort waits for the device
   const bool first = !sp.runs_host;
@@ -611,8 +727,8 @@ int sort_species(Ctx &c, Species &sp, bool exact) {
   if (4 * last > 3 * cap) cap = std::min(n, 2 * last + 65536);
   sp.rec_cap = cap;
   if (exact) cap = n;  // room for one run per particle: this sort cannot be skipped
-  const SortWs ws = sort_ws(n, cap);
-  const long long nb = ws.nb, rec_hist = ws.rec_hist, scratch = ws.scratch;
+  const SortWs ws = sort_ws(n, cap, bits);
+  const long long nb = ws.nb, scratch = ws.scratch;
   if (!ensure_ws(c, ws.bytes) || !ensure_alts(c, sp)) return -3;
   uint32_t *src = (uint32_t *)c.sort_ws, *block = src + n, *tmp = block + nb + 1;
   uint32_t *rk = tmp + scratch, *ri = rk + cap, *rk2 = ri + cap, *ri2 = rk2 + cap, *rlen = ri2 + cap;
@@ -622,14 +738,13 @@ int sort_species(Ctx &c, Species &sp, bool exact) {
   const bool f32 = c.precision == 1;
   // runs per group of 256 logical keys and their scan (block[nb] = the
   // number of runs); n is a whole number of chunks, one per block
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(1), 0, c.stream, block + nb, 1LL, 0u);
   const long long nch = n / kChunk;
   const unsigned chunks = (unsigned)nch, rblocks = (unsigned)((nch + kCPB - 1) / kCPB);
   if (f32)
     hipLaunchKernelGGL(k_run_count<KeysF32>, dim3(rblocks), dim3(256), 0, c.stream, k32, nch, block);
   else
     hipLaunchKernelGGL(k_run_count<KeysF64>, dim3(rblocks), dim3(256), 0, c.stream, k64, nch, block);
-  exclusive_scan(block, nb + 1, tmp, c.stream);
+  exclusive_scan(ScanArray{block, nb + 1}, nb + 1, tmp, c.stream);
   if (f32)
     hipLaunchKernelGGL(k_run_emit<KeysF32>, dim3(rblocks), dim3(256), 0, c.stream, k32, nch, block, count, cap, rk,
                        ri, rlen);
@@ -637,12 +752,8 @@ int sort_species(Ctx &c, Species &sp, bool exact) {
     hipLaunchKernelGGL(k_run_emit<KeysF64>, dim3(rblocks), dim3(256), 0, c.stream, k64, nch, block, count, cap, rk,
                        ri, rlen);
   // records by key (stable), then each run's first rank
-  radix_pairs(rk, ri, rk2, ri2, count, cap, bits, tmp, tmp + rec_hist, c.stream);
-  const unsigned mb = (unsigned)((cap + 255) / 256);
-  uint32_t *lens = rk2;  // free after the sort
-  hipLaunchKernelGGL(k_run_lens, dim3(mb), dim3(256), 0, c.stream, ri, rlen, count, cap, lens);
-  exclusive_scan(lens, cap, tmp, c.stream);
-  hipLaunchKernelGGL(k_run_first, dim3(mb), dim3(256), 0, c.stream, ri, lens, count, cap, rlen);
+  radix_pairs(rk, ri, rk2, ri2, count, cap, bits, ws.hist_in_src ? src : tmp, c.stream);
+  exclusive_scan(ScanRuns{ri, rlen, count, cap}, cap, tmp, c.stream);
   if (f32)
     hipLaunchKernelGGL(k_run_place<KeysF32>, dim3(rblocks), dim3(256), 0, c.stream, k32, nch, block, count, cap, rlen,
                        src);
@@ -760,8 +871,7 @@ int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream) 
   if (hipMemcpyAsync(ms.seg, ms.seg_host.data(), segs.size() * sizeof(MultiSeg), hipMemcpyHostToDevice, stream) !=
       hipSuccess)
     return -3;
-  int bits = 1;
-  while ((1ull << bits) <= (unsigned long long)keys) bits++;
+  const int bits = key_bits((unsigned long long)keys);
   // record capacity from the previous sort's run count (read back
   // asynchronously), as sort_species does
   if (!ms.runs_host) {
@@ -773,7 +883,7 @@ int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream) 
   long long cap = ms.rec_cap > 0 ? ms.rec_cap : std::min(n, n / 4 + 65536);
   if (4 * last > 3 * cap) cap = std::min(n, 2 * last + 65536);
   ms.rec_cap = cap;
-  const SortWs ws = sort_ws(n, cap);
+  const SortWs ws = sort_ws(n, cap, bits);
   if (ms.ws_bytes < ws.bytes) {
     if (ms.ws) (void)hipFree(ms.ws);
     ms.ws = nullptr;
@@ -781,23 +891,18 @@ int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream) 
     if (hipMalloc(&ms.ws, ws.bytes) != hipSuccess) return -3;
     ms.ws_bytes = ws.bytes;
   }
-  const long long nb = ws.nb, rec_hist = ws.rec_hist, scratch = ws.scratch;
+  const long long nb = ws.nb, scratch = ws.scratch;
   uint32_t *src = (uint32_t *)ms.ws, *block = src + n, *tmp = block + nb + 1;
   uint32_t *rk = tmp + scratch, *ri = rk + cap, *rk2 = ri + cap, *ri2 = rk2 + cap, *rlen = ri2 + cap;
   const uint32_t *count = block + nb;
   const KeysMulti km{ms.seg, ms.seg_of_chunk};
-  hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(1), 0, stream, block + nb, 1LL, 0u);
   const unsigned chunks = (unsigned)nch, rblocks = (unsigned)((nch + kCPB - 1) / kCPB);
   hipLaunchKernelGGL(k_run_count<KeysMulti>, dim3(rblocks), dim3(256), 0, stream, km, nch, block);
-  exclusive_scan(block, nb + 1, tmp, stream);
+  exclusive_scan(ScanArray{block, nb + 1}, nb + 1, tmp, stream);
   hipLaunchKernelGGL(k_run_emit<KeysMulti>, dim3(rblocks), dim3(256), 0, stream, km, nch, block, count, cap, rk, ri,
                      rlen);
-  radix_pairs(rk, ri, rk2, ri2, count, cap, bits, tmp, tmp + rec_hist, stream);
-  const unsigned mb = (unsigned)((cap + 255) / 256);
-  uint32_t *lens = rk2;
-  hipLaunchKernelGGL(k_run_lens, dim3(mb), dim3(256), 0, stream, ri, rlen, count, cap, lens);
-  exclusive_scan(lens, cap, tmp, stream);
-  hipLaunchKernelGGL(k_run_first, dim3(mb), dim3(256), 0, stream, ri, lens, count, cap, rlen);
+  radix_pairs(rk, ri, rk2, ri2, count, cap, bits, ws.hist_in_src ? src : tmp, stream);
+  exclusive_scan(ScanRuns{ri, rlen, count, cap}, cap, tmp, stream);
   hipLaunchKernelGGL(k_run_place<KeysMulti>, dim3(rblocks), dim3(256), 0, stream, km, nch, block, count, cap, rlen,
                      src);
   if (hipMemcpyAsync(ms.runs_host, count, sizeof(uint32_t), hipMemcpyDeviceToHost, stream) != hipSuccess ||

@@ -105,3 +105,57 @@ def test_periodic_sort_of_unsorted_state(precision):
     st = sims[1].download(0)
     key = _cell_keys(st, sims[1].dr, sims[1].dz, nr, nz)
     assert np.all(np.diff(key) >= 0)
+
+
+@pytest.mark.parametrize("cells_r,cells_z,n", [
+    (3, 3, 1), (3, 3, 4097),              # one digit
+    (7, 146, 5000), (3, 341, 5000),       # 1024 keys in one digit of 10 bits, 1025 in two of 6
+    (64, 128, 70000),                     # the histogram in the space of the permutation
+    (510, 514, 4096), (510, 514, 600000),  # 18 bits: two digits of 9
+    (1024, 1024, 700000),                 # 21 bits: three digits
+])
+def test_sort_by_size(cells_r, cells_z, n):
+    """Random particles, mostly a record each: digits of every width, partly
+    filled radix and scan blocks, one scan block and several."""
+    from pdp3_amd import capi
+
+    rng = np.random.default_rng(n + cells_z)
+    nr, nz, dr = cells_r + 1, cells_z + 1, 5e-4
+    sim = capi.Simulation(nr, nz, cells_r * dr, cells_z * dr, 0.5 * dr / 3e8, precision=0)
+    r = rng.uniform(dr / 2, (cells_r - 0.5) * dr, n)
+    z = rng.uniform(dr / 2, (cells_z - 0.5) * dr, n)
+    v = rng.standard_normal((3, n)) * 1e5
+    alive = (rng.random(n) > 0.05).astype(np.uint8)
+    idx = sim.add_plasma(-1, 1.0, r, z, v[0], v[1], v[2], np.ones(n), alive)
+    before = sim.download(idx)
+    key = _cell_keys(before, sim.dr, sim.dz, nr, nz)
+    order = np.argsort(np.where(before["alive"] == 1, key, cells_r * cells_z), kind="stable")
+    sim.sort()
+    after = sim.download(idx)
+    for k in ("r", "z", "vr", "vphi", "vz", "w", "alive"):
+        assert np.array_equal(after[k], before[k][order]), k
+    sim.close()
+
+
+def test_sort_of_many_scan_blocks():
+    """More run records' room than one pass over the scan blocks' sums takes
+    (3.4e7): the sums are scanned first."""
+    from pdp3_amd import capi
+
+    cells, ppc, dr = 1000, 35, 5e-4
+    sim = capi.Simulation(cells + 1, cells + 1, cells * dr, cells * dr, 0.5 * dr / 3e8, precision=1)
+    sim.boundary_conditions()
+    idx = sim.add_species(-1, 1.0, ppc * cells * cells)
+    sim.init_uniform(idx, 3, ppc, 1e14, 0, 1e3)
+    sim.step(10)
+    before = sim.download(idx)
+    sim.sort()
+    after = sim.download(idx)
+    key = _cell_keys(after, sim.dr, sim.dz, cells + 1, cells + 1)
+    key[after["alive"] != 1] = cells * cells
+    # FP32 states hold cell and place in it: a particle on a face may belong to
+    # either side of it
+    assert np.count_nonzero(np.diff(key) < 0) < 1e-4 * len(key)
+    for k in ("r", "z", "vz"):
+        assert np.array_equal(np.sort(after[k]), np.sort(before[k])), k
+    sim.close()
