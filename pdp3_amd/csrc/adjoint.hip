@@ -7,24 +7,21 @@
 //                       E^{n+1} = Ke E^n - Kh (J^n - C H^{n+1})
 // Backward, given the adjoints of E^{n+1}, H^{n+1} and the particle states:
 //   1. lambda_J = -Kh lambda_E;  lambda_H += C^T (Kh lambda_E);  lambda_E <- Ke lambda_E
-//   2. per particle, the vector-Jacobian product of P: the particle's step is
-//      re-executed in dual numbers (value + N directional derivatives) over
-//      its 12 inputs (r, z, v, the gathered E and H, w) in 12/N passes; every
-//      output (new r, z, v and each grid deposit) contributes its adjoint
-//      times its derivative; the adjoints of the gathered fields are scattered
-//      back to the nodes with the gather weights, the weight adjoint is
-//      accumulated per particle
+//   2. per particle, the vector-Jacobian product of P, written out in reverse:
+//      every output (new r, z, v and each grid deposit) passes its adjoint back
+//      to the 12 inputs (r, z, v, the gathered E and H, w); the adjoints of the
+//      gathered fields are scattered to the nodes with the gather weights, the
+//      weight adjoint is accumulated per particle
 //   3. lambda_alpha = lambda_H + lambda_Hh / 2;  lambda_E += A^T lambda_alpha;
 //      lambda_H <- lambda_H + lambda_Hh
 // The operators A (HField::calc_field, src/hField.cpp:93-157), C, Ke, Kh
 // (EField::calc_field, src/eField.cpp:85-170, PML in Ke / Kh) are transposed
-// node by node in pull form (no atomics).  The particle step follows
-// particles_fp64.hip expression for expression.
+// node by node in pull form (no atomics).
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "context.hpp"
-#include "crmath.hpp"
 #include "sink.hpp"
 
 namespace pdp3 {
@@ -108,28 +105,6 @@ __device__ __forceinline__ D operator/(D a, double b) {
   return r;
 }
 __device__ __forceinline__ D operator/(double a, D b) { return cst(a) / b; }
-__device__ __forceinline__ D dsqrt(D a) {
-  D r;
-  r.v = sqrt(a.v);
-  const double h = 0.5 / r.v;
-  for (int j = 0; j < kDN; j++) r.d[j] = a.d[j] * h;
-  return r;
-}
-__device__ __forceinline__ D dlog(D a) {
-  D r;
-  r.v = log(a.v);
-  for (int j = 0; j < kDN; j++) r.d[j] = a.d[j] / a.v;
-  return r;
-}
-// pow(y, -0.5) of lib::get_gamma_inv with the correctly rounded value
-__device__ __forceinline__ D drsqrt(D a) {
-  D r;
-  r.v = rsqrt_cr(a.v);
-  const double h = -0.5 * r.v * r.v * r.v;
-  for (int j = 0; j < kDN; j++) r.d[j] = a.d[j] * h;
-  return r;
-}
-
 constexpr double kC2 = kLightSpeed * kLightSpeed;
 
 // ------------------------------------------------------------ the particle
@@ -190,259 +165,7 @@ __device__ __forceinline__ int cell_number(double x, double dx) { return (int)ce
 __device__ __forceinline__ double cell_volume(int i, double dr, double dz) { return kPi * dz * dr * dr * 2.0 * i; }
 __device__ __forceinline__ double cyl_vol(double z, double r) { return kPi * z * r * r / 4.; }
 
-// the node weights of the four-node gather (src/eField.cpp:204-316) for one
-// component family; weights[] multiply F at (i_r, k), (i_r+1, k), (i_r, k+1),
-// (i_r+1, k+1).  Dual in (r, z).
-struct GatherW {
-  int ir, kz;
-  D w[4];
-};
-__device__ GatherW gather_w(const GridDesc &g, D radius, D longitude, bool lo, bool zhalf) {
-  const double dr = g.dr, dz = g.dz;
-  D r1 = radius - 0.5 * dr;
-  D r3 = radius + 0.5 * dr;
-  int i_r = lo ? cell_number(radius.v - 0.5 * dr, dr) : cell_number(radius.v, dr);
-  int k_z = zhalf ? cell_number(longitude.v - 0.5 * dz, dz) : cell_number(longitude.v, dz);
-  if (i_r < 0) i_r = 0;
-  if (k_z < 0) k_z = 0;
-  i_r = min(i_r, g.nr - 2);
-  k_z = min(k_z, g.nz - 2);
-  double vol_1, vol_2, r2;
-  if (lo) {
-    vol_1 = cell_volume(i_r + 1, dr, dz);
-    vol_2 = cell_volume(i_r + 3, dr, dz);
-    r2 = (i_r + 1) * dr;
-  } else {
-    vol_1 = (radius.v > dr) ? cell_volume(i_r, dr, dz) : cyl_vol(dz, dr);
-    r2 = (i_r + 0.5) * dr;
-    vol_2 = cell_volume(i_r + 2, dr, dz);
-  }
-  D dz1, dz2;
-  if (zhalf) {
-    dz1 = (k_z + 1.5) * dz - longitude;
-    dz2 = longitude - (k_z + 0.5) * dz;
-  } else {
-    dz1 = (k_z + 1) * dz - longitude;
-    dz2 = longitude - k_z * dz;
-  }
-  GatherW out;
-  out.ir = i_r;
-  out.kz = k_z;
-  // ring_term(F, dzx, ra, rb, vol) = F * pi * dzx * (rb^2 - ra^2) / vol
-  D a_in = r2 * r2 - r1 * r1, a_out = r3 * r3 - r2 * r2;
-  out.w[0] = kPi * dz1 * a_in / vol_1;
-  out.w[1] = kPi * dz1 * a_out / vol_2;
-  out.w[2] = kPi * dz2 * a_in / vol_1;
-  out.w[3] = kPi * dz2 * a_out / vol_2;
-  return out;
-}
-
-__device__ __forceinline__ D gather_d(const GridDesc &g, const double *F, D r, D z, bool lo, bool zhalf) {
-  GatherW gw = gather_w(g, r, z, lo, zhalf);
-  const double *row0 = F + (size_t)gw.ir * (size_t)g.nz + gw.kz;
-  const double *row1 = row0 + g.nz;
-  return gw.w[0] * row0[0] + gw.w[1] * row1[0] + gw.w[2] * row0[1] + gw.w[3] * row1[1];
-}
-
 constexpr int kAR = 0, kAPhi = 1, kAZ = 2;
-
-__device__ __forceinline__ D dot3(const D *a, const D *b) {
-  D res = cst(0.0);
-  res = res + a[0] * b[0];
-  res = res + a[1] * b[1];
-  res = res + a[2] * b[2];
-  return res;
-}
-
-// relativistic Boris (src/particles.cpp:1025-1150)
-__device__ void boris_d(D q, D m, double dt, D e[3], D b[3], D v[3]) {
-  D const1 = q * dt / (2 * m);
-  for (int j = 0; j < 3; j++) e[j] = e[j] * const1;
-  D bs = kMagnConst * const1;
-  for (int j = 0; j < 3; j++) b[j] = b[j] * bs;
-  D u[3], t[3];
-  for (int j = 0; j < 3; j++) u[j] = (fabs(v[j].v) < kMnzl) ? cst(0.0) : v[j];
-  D beta = dot3(u, u) / kC2;
-  D gamma = 1 / dsqrt(1.0 - beta);
-  for (int j = 0; j < 3; j++) u[j] = u[j] * gamma;
-  for (int j = 0; j < 3; j++) u[j] = u[j] + e[j];
-  gamma = drsqrt(1.0 + dot3(u, u) / kC2);
-  for (int j = 0; j < 3; j++) b[j] = b[j] * gamma;
-  D const2 = 2. / (1. + dot3(b, b));
-  for (int j = 0; j < 3; j++) t[j] = u[j];
-  u[0] = t[0] + const2 * ((t[1] - t[0] * b[2] + t[2] * b[0]) * b[2] - (t[2] + t[0] * b[1] - t[1] * b[0]) * b[1]);
-  u[1] = t[1] + const2 * (-(t[0] + t[1] * b[2] - t[2] * b[1]) * b[2] + (t[2] + t[0] * b[1] - t[1] * b[0]) * b[0]);
-  u[2] = t[2] + const2 * ((t[0] + t[1] * b[2] - t[2] * b[1]) * b[1] - (t[1] - t[0] * b[2] + t[2] * b[0]) * b[0]);
-  for (int j = 0; j < 3; j++) u[j] = u[j] + e[j];
-  gamma = drsqrt(1.0 + dot3(u, u) / kC2);
-  for (int j = 0; j < 3; j++) v[j] = u[j] * gamma;
-}
-
-// Vay with the reference's scaling (src/particles.cpp:1152-1254)
-__device__ void vay_d(D q, D m, double dt, D e[3], D b[3], D v[3]) {
-  D const1 = q * dt / (2 * m);
-  D s2 = 2 * const1;
-  for (int j = 0; j < 3; j++) e[j] = e[j] * s2;
-  D bs = kMagnConst * const1;
-  for (int j = 0; j < 3; j++) b[j] = b[j] * bs;
-  D u[3], t[3];
-  for (int j = 0; j < 3; j++) u[j] = (fabs(v[j].v) < kMnzl) ? cst(0.0) : v[j];
-  D beta = dot3(u, u) / kC2;
-  D gamma = 1 / dsqrt(1.0 - beta);
-  for (int j = 0; j < 3; j++) u[j] = u[j] * gamma;
-  for (int j = 0; j < 3; j++) t[j] = u[j];
-  for (int j = 0; j < 3; j++) b[j] = b[j] * s2;
-  for (int j = 0; j < 3; j++) u[j] = u[j] + e[j];
-  for (int j = 0; j < 3; j++) b[j] = b[j] * const1;
-  gamma = drsqrt(1.0 + dot3(t, t) / kC2);
-  u[0] = u[0] + gamma * (t[1] * b[2] - t[2] * b[1]);
-  u[1] = u[1] + gamma * (t[2] * b[0] - t[0] * b[2]);
-  u[2] = u[2] + gamma * (t[0] * b[1] - t[1] * b[0]);
-  gamma = drsqrt(1.0 + dot3(u, u) / kC2);
-  D alpha = 1. / gamma / gamma;
-  D B2 = dot3(b, b);
-  D sg = alpha - B2;
-  D ub = dot3(u, b);
-  D us2 = ub * ub;
-  alpha = 1. / dsqrt(0.5 * (sg + dsqrt(sg * sg + 4. * (B2 + us2))));
-  for (int j = 0; j < 3; j++) b[j] = b[j] * alpha;
-  sg = 1. / (1. + dot3(b, b));
-  alpha = dot3(u, b);
-  t[0] = sg * (u[0] + alpha * b[0] + b[2] * u[1] - b[1] * u[2]);
-  t[1] = sg * (u[1] + alpha * b[1] + b[0] * u[2] - b[2] * u[0]);
-  t[2] = sg * (u[2] + alpha * b[2] + b[1] * u[0] - b[0] * u[1]);
-  gamma = drsqrt(1.0 + dot3(t, t) / kC2);
-  for (int j = 0; j < 3; j++) v[j] = t[j] * gamma;
-}
-
-__device__ __forceinline__ D ring(D F, D dzx, D ra, D rb, double vol) { return F * kPi * dzx * (rb * rb - ra * ra) / vol; }
-
-// azimuthal_current_distribution, src/particles.cpp:688-784
-template <class S>
-__device__ void jphi_d(const GridDesc &g, S &sk, D q, D r, D z, D vphi) {
-  const double dr = g.dr, dz = g.dz;
-  int r_i = cell_number(r.v, dr), z_k = cell_number(z.v, dz);
-  if (r_i < 0) r_i = 0;
-  if (z_k < 0) z_k = 0;
-  D r1 = r - 0.5 * dr;
-  D r2 = cst((r_i + 0.5) * dr);
-  D r3 = r + 0.5 * dr;
-  D ro_v = q / (2. * kPi * dz * dr * r);
-  double v_1 = (r.v > dr) ? cell_volume(r_i, dr, dz) : cyl_vol(dz, dr);
-  double v_2 = cell_volume(r_i + 1, dr, dz);
-  D dz1 = (z_k + 0.5) * dz - (z - 0.5 * dz);
-  D dz2 = (z + 0.5 * dz) - (z_k + 0.5) * dz;
-  sk.add(kAPhi, r_i, z_k, ring(ro_v, dz1, r1, r2, v_1) * vphi);
-  sk.add(kAPhi, r_i + 1, z_k, ring(ro_v, dz1, r2, r3, v_2) * vphi);
-  sk.add(kAPhi, r_i, z_k + 1, ring(ro_v, dz2, r1, r2, v_1) * vphi);
-  sk.add(kAPhi, r_i + 1, z_k + 1, ring(ro_v, dz2, r2, r3, v_2) * vphi);
-}
-
-// (log(1+x) - x) / x without cancellation (series below |x| = 0.1)
-__device__ __forceinline__ D m_of_d(D x) {
-  if (fabs(x.v) < 0.1) {
-    D s = cst(-1.0 / 12.0);
-    const double c[] = {1.0 / 11.0, -0.1, 1.0 / 9.0, -0.125, 1.0 / 7.0, -1.0 / 6.0, 0.2, -0.25, 1.0 / 3.0, -0.5};
-    for (double ck : c) s = ck + x * s;
-    return x * s;
-  }
-  D l;
-  l.v = log1p(x.v);
-  for (int j = 0; j < kDN; j++) l.d[j] = x.d[j] / (1.0 + x.v);
-  return (l - x) / x;
-}
-
-// simple_current_distribution, src/particles.cpp:333-474.  Values: the
-// reference's expressions.  Derivatives: those of the same integrals written
-// without cancellation in cell units (r = (i + a) dr, rho = i + a,
-// x = drho / rho, M = (ln(1+x) - x) / x, N = -x / (1+x) - M):
-//   J_z[i]   = q dzeta / (4 pi dr^2 dt) [ (1-a)(2i+a)/rho - drho/2 + i(i+1)/rho M ] / i
-//   J_z[i+1] = q dzeta / (4 pi dr^2 dt) [ a(2i+1+a)/rho + drho/2 - i(i+1)/rho M ] / (i+1)
-//   J_r[k]   = q / (2 pi dr dz dt) [ drho((1-b)/2 - dzeta/4) + i(i+1)/(2 rho) (drho (1-b)/rho_e + dzeta N) ] / (i+1/2)
-//   J_r[k+1] = q / (2 pi dr dz dt) [ drho(b/2 + dzeta/4) + i(i+1)/(2 rho) (drho b/rho_e - dzeta N) ] / (i+1/2)
-// (and the polynomial forms on the axis cell).  The reference's forms are
-// differences of O(i) terms: their derivative loses ~1/x digits for nearly
-// axial paths, which a relativistic beam's particles are.
-template <class S>
-__device__ void segment_d(const GridDesc &g, S &acc, D q, D radius_new, D longitude_new, D radius_old,
-                          D longitude_old, int i_n, int k_n) {
-  const double dr = g.dr, dz = g.dz, delta_t = g.dt;
-  const double delta_r = radius_new.v - radius_old.v;
-  const double delta_z = longitude_new.v - longitude_old.v;
-  if ((fabs(delta_r) < kMnzl) || (fabs(delta_z) < kMnzl)) return;
-  // values, as the reference computes them
-  double vz0, vz1, vr0, vr1;
-  {
-    const double qv = q.v;
-    double k = delta_r / delta_z;
-    double b = radius_old.v;
-    double lg = log((k * delta_z + b) / b);
-    if (i_n >= 1) {
-      double ssd = qv / (2 * kPi * (i_n * dr) * dr * dz * delta_t * 2 * dr);
-      vz0 = ssd * (dr * delta_z - k * delta_z * delta_z / 2. - delta_z * b +
-                   dr * dr / k * ((i_n + 0.5) * (i_n + 0.5) - 0.25) * lg);
-      ssd = qv / (2 * kPi * ((i_n + 1) * dr) * dr * dz * delta_t * 2 * dr);
-      vz1 = ssd * (k * delta_z * delta_z / 2. + delta_z * b + delta_z * dr +
-                   dr * dr / k * (0.25 - (i_n + 0.5) * (i_n + 0.5)) * lg);
-    } else {
-      double ssd = qv / (2. * kPi * dr / 4. * dr * dz * delta_t * dr);
-      vz0 = ssd * (dr * delta_z - k * delta_z * delta_z / 2. - delta_z * b);
-      ssd = qv / (2 * kPi * dr * dr * dz * delta_t * 2 * dr);
-      vz1 = ssd * (k * delta_z * delta_z / 2. + delta_z * dr + delta_z * b);
-    }
-    k = -delta_z / delta_r;
-    const double r0 = (i_n + 0.5) * dr;
-    const double r1 = radius_old.v;
-    b = (k_n + 1.) * dz - longitude_old.v;
-    const double ssd = qv / (2 * kPi * r0 * dr * dz * delta_t * dz);
-    const double lr = log((radius_old.v + delta_r) / radius_old.v);
-    vr0 = ssd * (r0 * k * delta_r + k / 2. * delta_r * (radius_old.v + delta_r / 2.) +
-                 0.5 * delta_r * (b - k * (2 * r0 + r1)) +
-                 delta_r * (b - k * r1) * (4 * r0 * r0 - dr * dr) / (8 * radius_old.v * (radius_old.v + delta_r)) +
-                 (k * (r0 * r0 / 2. - dr * dr / 8.)) * lr);
-    b = longitude_old.v - k_n * dz;
-    vr1 = ssd * (-r0 * k * delta_r - k / 2. * delta_r * (radius_old.v + delta_r / 2.) +
-                 0.5 * delta_r * (b + k * (2 * r0 + r1)) +
-                 delta_r * (b + k * r1) * (4 * r0 * r0 - dr * dr) / (8 * radius_old.v * (radius_old.v + delta_r)) -
-                 (k * (r0 * r0 / 2. - dr * dr / 8.)) * lr);
-  }
-  // derivatives, from the cancellation-free forms
-  const double fi = (double)i_n;
-  D a = radius_old / dr - fi;
-  D bo = longitude_old / dz - (double)k_n;
-  D drho = (radius_new - radius_old) / dr;
-  D dzeta = (longitude_new - longitude_old) / dz;
-  D jz0, jz1, jr0, jr1;
-  if (i_n == 0) {
-    jz0 = 8.0 * (1.0 - 0.5 * drho - a);
-    jz1 = 0.5 * drho + 1.0 + a;
-    jr0 = drho * (0.5 * (1.0 - bo) - 0.25 * dzeta) * 2.0;
-    jr1 = drho * (0.5 * bo + 0.25 * dzeta) * 2.0;
-  } else {
-    D rs = fi + a;
-    D re = rs + drho;
-    D x = drho / rs;
-    D M = m_of_d(x);
-    D N = -(x / (1.0 + x)) - M;
-    const double ii = fi * (fi + 1.0);
-    jz0 = ((1.0 - a) * (2.0 * fi + a) / rs - 0.5 * drho + ii / rs * M) / fi;
-    jz1 = (a * (2.0 * fi + 1.0 + a) / rs + 0.5 * drho - ii / rs * M) / (fi + 1.0);
-    D cc = 0.5 * ii / rs;
-    jr0 = (drho * (0.5 * (1.0 - bo) - 0.25 * dzeta) + cc * (drho * (1.0 - bo) / re + dzeta * N)) / (fi + 0.5);
-    jr1 = (drho * (0.5 * bo + 0.25 * dzeta) + cc * (drho * bo / re - dzeta * N)) / (fi + 0.5);
-  }
-  D sz = q * dzeta / (4.0 * kPi * dr * dr * delta_t);
-  D sr = q / (2.0 * kPi * dr * dz * delta_t);
-  D out[4] = {sz * jz0, sz * jz1, sr * jr0, sr * jr1};
-  out[0].v = vz0;
-  out[1].v = vz1;
-  out[2].v = vr0;
-  out[3].v = vr1;
-  acc.add(kAZ, i_n, k_n, out[0]);
-  acc.add(kAZ, i_n + 1, k_n, out[1]);
-  acc.add(kAR, i_n, k_n, out[2]);
-  acc.add(kAR, i_n, k_n + 1, out[3]);
-}
 
 // strict_motion_weighting, src/particles.cpp:786-988
 template <class S>
@@ -525,175 +248,6 @@ __device__ void strict_d(const GridDesc &g, S &acc, D q, D radius_new, D longitu
       acc.add(kAR, i_n, k_n, wj * left_delta_z);
       acc.add(kAR, i_n, k_n + 1, wj * right_delta_z);
     }
-  }
-}
-
-struct SegD {
-  D rn, zn, ro, zo;
-  int i, k;
-};
-
-// current_distribution, src/particles.cpp:480-685
-template <class S>
-__device__ void deposit_j_d(const GridDesc &g, S &acc, D q, D pr, D pz, D por, D poz) {
-  const double dr = g.dr, dz = g.dz;
-  int i_n = cell_number(pr.v, dr), k_n = cell_number(pz.v, dz);
-  int i_o = cell_number(por.v, dr), k_o = cell_number(poz.v, dz);
-  if (i_n < 0) i_n = 0;
-  if (k_n < 0) k_n = 0;
-  if (i_o < 0) i_o = 0;
-  if (k_o < 0) k_o = 0;
-  if (por.v == (i_o + 1) * dr) i_o = i_n;
-  if (poz.v == (k_o + 1) * dz) k_o = k_n;
-  if (pr.v == (i_n + 1) * dr) i_n = i_o;
-  if (pz.v == (k_n + 1) * dz) k_n = k_o;
-  int res_cell = abs(i_n - i_o) + abs(k_n - k_o);
-  if ((fabs(pr.v - por.v) < kMnzl) || (fabs(pz.v - poz.v) < kMnzl)) {
-    strict_d(g, acc, q, pr, pz, por, poz);
-    return;
-  }
-  if (res_cell == 0) {  // the common case, without the segment list (which lives in scratch memory)
-    segment_d(g, acc, q, pr, pz, por, poz, i_n, k_n);
-    return;
-  }
-  SegD s[3];
-  int ns = 0;
-  if (res_cell == 1) {
-    if ((i_n != i_o) && (k_n == k_o)) {
-      if (por.v > (i_n + 1) * dr) {
-        D a = (por - pr) / (poz - pz);
-        D r_b = cst((i_n + 1) * dr);
-        D z_b = pz + (r_b - pr) / a;
-        s[0] = SegD{r_b, z_b, por, poz, i_n + 1, k_n};
-        s[1] = SegD{pr, pz, r_b, z_b, i_n, k_n};
-      } else {
-        D a = (pr - por) / (pz - poz);
-        D r_b = cst(i_n * dr);
-        D z_b = poz + (r_b - por) / a;
-        s[0] = SegD{r_b, z_b, por, poz, i_n - 1, k_n};
-        s[1] = SegD{pr, pz, r_b, z_b, i_n, k_n};
-      }
-      ns = 2;
-    } else if ((i_n == i_o) && (k_n != k_o)) {
-      if (poz.v < k_n * dz) {
-        D z_b = cst(k_n * dz);
-        D a = (pr - por) / (pz - poz);
-        D r_b = por + a * (z_b - poz);
-        s[0] = SegD{r_b, z_b, por, poz, i_n, k_n - 1};
-        s[1] = SegD{pr, pz, r_b, z_b, i_n, k_n};
-      } else {
-        D z_b = cst((k_n + 1) * dz);
-        D a = (por - pr) / (poz - pz);
-        D r_b = pr + a * (z_b - pz);
-        s[0] = SegD{r_b, z_b, por, poz, i_n, k_n + 1};
-        s[1] = SegD{pr, pz, r_b, z_b, i_n, k_n};
-      }
-      ns = 2;
-    }
-  } else if (res_cell == 2) {
-    if (i_o < i_n) {
-      if (k_o < k_n) {
-        D a = (pr - por) / (pz - poz);
-        D r1 = cst(i_n * dr);
-        D z1 = poz + (r1 - por) / a;
-        D z2 = cst(k_n * dz);
-        D r2 = por + (z2 - poz) * a;
-        if (z1.v < k_n * dz) {
-          s[0] = SegD{r1, z1, por, poz, i_n - 1, k_n - 1};
-          s[1] = SegD{r2, z2, r1, z1, i_n, k_n - 1};
-          s[2] = SegD{pr, pz, r2, z2, i_n, k_n};
-          ns = 3;
-        } else if (z1.v > k_n * dz) {
-          s[0] = SegD{r2, z2, por, poz, i_n - 1, k_n - 1};
-          s[1] = SegD{r1, z1, r2, z2, i_n - 1, k_n};
-          s[2] = SegD{pr, pz, r1, z1, i_n, k_n};
-          ns = 3;
-        }
-      } else {
-        D a = (pr - por) / (pz - poz);
-        D r1 = cst(i_n * dr);
-        D z1 = poz + (r1 - por) / a;
-        D z2 = cst((k_n + 1) * dz);
-        D r2 = por + -(poz - z2) * a;
-        if (z1.v > (k_n + 1) * dz) {
-          s[0] = SegD{r1, z1, por, poz, i_n - 1, k_n + 1};
-          s[1] = SegD{r2, z2, r1, z1, i_n, k_n + 1};
-          s[2] = SegD{pr, pz, r2, z2, i_n, k_n};
-          ns = 3;
-        } else if (z1.v < (k_n + 1) * dz) {
-          s[0] = SegD{r2, z2, por, poz, i_n - 1, k_n + 1};
-          s[1] = SegD{r1, z1, r2, z2, i_n - 1, k_n};
-          s[2] = SegD{pr, pz, r1, z1, i_n, k_n};
-          ns = 3;
-        }
-      }
-    } else if (i_o > i_n) {
-      if (k_o < k_n) {
-        D a = (pr - por) / (pz - poz);
-        D r1 = cst((i_n + 1) * dr);
-        D z1 = poz + -(por - r1) / a;
-        D z2 = cst(k_n * dz);
-        D r2 = por - -(z2 - poz) * a;
-        if (z1.v < (k_n)*dz) {
-          s[0] = SegD{r1, z1, por, poz, i_n + 1, k_n - 1};
-          s[1] = SegD{r2, z2, r1, z1, i_n, k_n - 1};
-          s[2] = SegD{pr, pz, r2, z2, i_n, k_n};
-          ns = 3;
-        } else if (z1.v > (k_n)*dz) {
-          s[0] = SegD{r2, z2, por, poz, i_n + 1, k_n - 1};
-          s[1] = SegD{r1, z1, r2, z2, i_n + 1, k_n};
-          s[2] = SegD{pr, pz, r1, z1, i_n, k_n};
-          ns = 3;
-        }
-      } else if (k_o > k_n) {
-        D a = (por - pr) / (poz - pz);
-        D r1 = cst((i_n + 1) * dr);
-        D z1 = pz + (r1 - pr) / a;
-        D z2 = cst((k_n + 1) * dz);
-        D r2 = pr + (z2 - pz) * a;
-        if (z1.v > (k_n + 1) * dz) {
-          s[0] = SegD{r1, z1, por, poz, i_n + 1, k_n + 1};
-          s[1] = SegD{r2, z2, r1, z1, i_n, k_n + 1};
-          s[2] = SegD{pr, pz, r2, z2, i_n, k_n};
-          ns = 3;
-        } else if (z1.v < (k_n + 1) * dz) {
-          s[0] = SegD{r2, z2, por, poz, i_n + 1, k_n + 1};
-          s[1] = SegD{r1, z1, r2, z2, i_n + 1, k_n};
-          s[2] = SegD{pr, pz, r1, z1, i_n, k_n};
-          ns = 3;
-        }
-      }
-    }
-  }
-#pragma nounroll
-  for (int t = 0; t < ns; t++) segment_d(g, acc, q, s[t].rn, s[t].zn, s[t].ro, s[t].zo, s[t].i, s[t].k);
-}
-
-// reflection_single / Bunch::reflection_single on the half-step point
-__device__ __forceinline__ void walls_d(const GridDesc &g, bool is_bunch, D &x, D &z, D &v0, D &v2, bool &alive) {
-  const double dr = g.dr, dz = g.dz;
-  const double radius_wall = g.r_size - dr / 2., longitude_wall = g.z_size - dz / 2.;
-  const double half_dr = dr / 2., half_dz = dz / 2.;
-  if (is_bunch) {
-    if (x.v > radius_wall) alive = false;
-    if (z.v > longitude_wall) alive = false;
-  } else {
-    if (x.v > radius_wall) {
-      x = radius_wall * 2. - x;
-      v0 = -v0;
-    }
-    if (z.v > longitude_wall) {
-      z = longitude_wall * 2. - z;
-      v2 = -v2;
-    }
-  }
-  if (x.v < half_dr) {
-    x = dr - x;
-    v0 = -v0;
-  }
-  if (z.v < half_dz) {
-    z = dz - z;
-    v2 = -v2;
   }
 }
 
@@ -962,9 +516,20 @@ __device__ __forceinline__ void m_and_slope(double x, double &M, double &dM) {
   }
 }
 
-// reverse of one straight piece inside cell (i, k), from the closed forms
-// above segment_d: S = sum lambda_J J and its derivatives with respect to the
-// piece's ends
+// The deposits of one straight piece inside cell (i, k)
+// (simple_current_distribution, src/particles.cpp:333-474), as integrals written
+// without cancellation in cell units (r = (i + a) dr, z = (k + b) dz, rho = i + a,
+// rho_e = rho + drho, x = drho / rho, M = (ln(1+x) - x) / x, N = -x / (1+x) - M):
+//   J_z[i]   = q dzeta / (4 pi dr^2 dt) [ (1-a)(2i+a)/rho - drho/2 + i(i+1)/rho M ] / i
+//   J_z[i+1] = q dzeta / (4 pi dr^2 dt) [ a(2i+1+a)/rho + drho/2 - i(i+1)/rho M ] / (i+1)
+//   J_r[k]   = q / (2 pi dr dz dt) [ drho((1-b)/2 - dzeta/4) + i(i+1)/(2 rho) (drho (1-b)/rho_e + dzeta N) ] / (i+1/2)
+//   J_r[k+1] = q / (2 pi dr dz dt) [ drho(b/2 + dzeta/4) + i(i+1)/(2 rho) (drho b/rho_e - dzeta N) ] / (i+1/2)
+// (and the polynomial forms on the axis cell).  The reference's forms are
+// differences of O(i) terms: their derivative loses ~1/x digits for nearly
+// axial paths, which a relativistic beam's particles are.
+//
+// Reverse of one piece: S = sum lambda_J J and its derivatives with respect to
+// the piece's ends.
 struct PieceAdj {
   double s, rn, zn, ro, zo;
 };
@@ -1043,14 +608,19 @@ struct StrictSink {
   }
 };
 
-// reverse of the J_r / J_z deposit of the straight path (ro, zo) -> (rn, zn)
-// (current_distribution, src/particles.cpp:480-685): the path is split at the
-// radial face r = rb (met at z1) and the axial face z = zb (met at r2) that it
-// crosses; with s the path parameter of the crossing, the adjoint of z1 goes
-// to the ends as (1-s, s) along z and times -dz/dr along r, that of r2 likewise
-__device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjGrid &lg, double q, double rn, double zn,
-                                                   double ro, double zo) {
+// the straight path (ro, zo) -> (rn, zn) (current_distribution,
+// src/particles.cpp:480-685): its ns pieces, split at the radial face r = rb
+// (met at z1) and the axial face z = zb (met at r2) that it crosses, rfirst: in
+// that order; the last piece lies in cell (i_n, k_n), those before it in
+// (i0, k0) and (i1, k1)
+struct Path {
+  int i_n, k_n, i0, k0, i1, k1, ns;
+  bool strict, rad, axi, rfirst;  // strict: along one axis, not split
+  double rb, zb, z1, r2, slope;
+};
+__device__ __forceinline__ Path split_path(const GridDesc &g, double rn, double zn, double ro, double zo) {
   const double dr = g.dr, dz = g.dz;
+  Path p;
   int i_n = max(cell_number(rn, dr), 0), k_n = max(cell_number(zn, dz), 0);
   int i_o = max(cell_number(ro, dr), 0), k_o = max(cell_number(zo, dz), 0);
   if (ro == (i_o + 1) * dr) i_o = i_n;
@@ -1058,54 +628,70 @@ __device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjG
   if (rn == (i_n + 1) * dr) i_n = i_o;
   if (zn == (k_n + 1) * dz) k_n = k_o;
   const int di = i_n - i_o, dk = k_n - k_o, res = abs(di) + abs(dk);
-  if ((fabs(rn - ro) < kMnzl) || (fabs(zn - zo) < kMnzl)) {
-    StrictSink sk{&g, &lg, {0.0, 0.0, 0.0, 0.0, 0.0}};
-    strict_d(g, sk, cst(q), seed(rn, 0), seed(zn, 1), seed(ro, 2), seed(zo, 3));
-    return sk.o;
-  }
-  // pieces: ns, the crossings in order (first / second), the cells before the last
-  int ns = 1, i0 = i_n, k0 = k_n, i1 = i_n, k1 = k_n;
-  bool rad = false, axi = false, rfirst = false;
-  double rb = 0.0, zb = 0.0, z1 = 0.0, r2 = 0.0;
-  const double slope = (rn - ro) / (zn - zo);
+  p.strict = (fabs(rn - ro) < kMnzl) || (fabs(zn - zo) < kMnzl);
+  p.ns = 1;
+  p.i_n = p.i0 = p.i1 = i_n;
+  p.k_n = p.k0 = p.k1 = k_n;
+  p.rad = p.axi = p.rfirst = false;
+  p.rb = p.zb = p.z1 = p.r2 = 0.0;
+  p.slope = (rn - ro) / (zn - zo);
   if (res == 1) {
-    ns = 2;
+    p.ns = 2;
     if (di != 0) {
-      rad = rfirst = true;
+      p.rad = p.rfirst = true;
       const bool up = !(ro > (i_n + 1) * dr);
-      rb = (up ? i_n : i_n + 1) * dr;
-      z1 = up ? zo + (rb - ro) / slope : zn + (rb - rn) / slope;
-      i0 = up ? i_n - 1 : i_n + 1;
+      p.rb = (up ? i_n : i_n + 1) * dr;
+      p.z1 = up ? zo + (p.rb - ro) / p.slope : zn + (p.rb - rn) / p.slope;
+      p.i0 = up ? i_n - 1 : i_n + 1;
     } else {
-      axi = true;
+      p.axi = true;
       const bool up = zo < k_n * dz;
-      zb = (up ? k_n : k_n + 1) * dz;
-      r2 = up ? ro + slope * (zb - zo) : rn + slope * (zb - zn);
-      k0 = up ? k_n - 1 : k_n + 1;
+      p.zb = (up ? k_n : k_n + 1) * dz;
+      p.r2 = up ? ro + p.slope * (p.zb - zo) : rn + p.slope * (p.zb - zn);
+      p.k0 = up ? k_n - 1 : k_n + 1;
     }
   } else if (res == 2) {
     // a path across a radial and an axial face; the other two-cell jumps are
     // too long for a step and are treated as the forward pass treats them
     const bool up = di > 0, right = dk > 0;
     if (di == 0 || (!up && dk == 0)) {
-      ns = 0;
+      p.ns = 0;
     } else {
-      rad = axi = true;
-      rb = (up ? i_n : i_n + 1) * dr;
-      zb = (right ? k_n : k_n + 1) * dz;
+      p.rad = p.axi = true;
+      p.rb = (up ? i_n : i_n + 1) * dr;
+      p.zb = (right ? k_n : k_n + 1) * dz;
       const bool from_new = !up && !right;
-      z1 = from_new ? zn + (rb - rn) / slope : zo + (rb - ro) / slope;
-      r2 = from_new ? rn + (zb - zn) * slope : ro + (zb - zo) * slope;
-      ns = z1 == zb ? 0 : 3;
-      rfirst = right ? z1 < zb : z1 > zb;
-      i0 = up ? i_n - 1 : i_n + 1;
-      k0 = right ? k_n - 1 : k_n + 1;
-      i1 = rfirst ? i_n : i0;
-      k1 = rfirst ? k0 : k_n;
+      p.z1 = from_new ? zn + (p.rb - rn) / p.slope : zo + (p.rb - ro) / p.slope;
+      p.r2 = from_new ? rn + (p.zb - zn) * p.slope : ro + (p.zb - zo) * p.slope;
+      p.ns = p.z1 == p.zb ? 0 : 3;
+      p.rfirst = right ? p.z1 < p.zb : p.z1 > p.zb;
+      p.i0 = up ? i_n - 1 : i_n + 1;
+      p.k0 = right ? k_n - 1 : k_n + 1;
+      p.i1 = p.rfirst ? i_n : p.i0;
+      p.k1 = p.rfirst ? p.k0 : k_n;
     }
   } else if (res > 2) {
-    ns = 0;
+    p.ns = 0;
   }
+  return p;
+}
+
+// reverse of the J_r / J_z deposit of the straight path (ro, zo) -> (rn, zn)
+// (current_distribution, src/particles.cpp:480-685): the path is split at the
+// radial face r = rb (met at z1) and the axial face z = zb (met at r2) that it
+// crosses; with s the path parameter of the crossing, the adjoint of z1 goes
+// to the ends as (1-s, s) along z and times -dz/dr along r, that of r2 likewise
+__device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjGrid &lg, double q, double rn, double zn,
+                                                   double ro, double zo) {
+  const Path c = split_path(g, rn, zn, ro, zo);
+  if (c.strict) {
+    StrictSink sk{&g, &lg, {0.0, 0.0, 0.0, 0.0, 0.0}};
+    strict_d(g, sk, cst(q), seed(rn, 0), seed(zn, 1), seed(ro, 2), seed(zo, 3));
+    return sk.o;
+  }
+  const int ns = c.ns;
+  const bool rfirst = c.rfirst;
+  const double rb = c.rb, zb = c.zb, z1 = c.z1, r2 = c.r2, slope = c.slope;
   // the crossings in path order
   const double cr0 = rfirst ? rb : r2, cz0 = rfirst ? z1 : zb;
   const double cr1 = rfirst ? r2 : rb, cz1 = rfirst ? zb : z1;
@@ -1116,7 +702,7 @@ __device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjG
     const bool first = t == 0, last = t == ns - 1;
     const PieceAdj p = segment_back(g, lg, q, last ? rn : first ? cr0 : cr1, last ? zn : first ? cz0 : cz1,
                                     first ? ro : t == 1 ? cr0 : cr1, first ? zo : t == 1 ? cz0 : cz1,
-                                    last ? i_n : first ? i0 : i1, last ? k_n : first ? k0 : k1);
+                                    last ? c.i_n : first ? c.i0 : c.i1, last ? c.k_n : first ? c.k0 : c.k1);
     o.s += p.s;
     if (first) {
       o.ro += p.ro;
@@ -1139,14 +725,14 @@ __device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjG
       c1z += p.zn;
     }
   }
-  if (rad) {
+  if (c.rad) {
     const double l = rfirst ? c0z : c1z, s = (rb - ro) / (rn - ro), is = 1.0 / slope;
     o.zo += (1.0 - s) * l;
     o.zn += s * l;
     o.ro -= is * (1.0 - s) * l;
     o.rn -= is * s * l;
   }
-  if (axi) {
+  if (c.axi) {
     const double l = rfirst ? c1r : c0r, s = (zb - zo) / (zn - zo);
     o.ro += (1.0 - s) * l;
     o.rn += s * l;
@@ -1291,22 +877,25 @@ __global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, 
     if (v == 0.0) continue;
     const int comp = t / (Box::kR * kABK), rem = t - comp * Box::kR * kABK;
     const int gi = b.bi + rem / kABK, gk = b.bk + rem % kABK;
-    // nodes off the grid never receive a stencil (gather_w clamps its cell)
+    // nodes off the grid never receive a stencil (the gathers clamp their cell)
     if ((unsigned)gi < (unsigned)g.nr && (unsigned)gk < (unsigned)g.nz)
       unsafeAtomicAdd(lf[comp] + (size_t)gi * (size_t)g.nz + gk, v);
   }
 }
 
 // ------------------------------------------------ tangent-linear (forward mode)
-// The same particle step in dual numbers, seeded with kDN tangent directions
-// of the state, of the gathered fields and of the weight instead of unit
-// vectors: the derivative parts of the outputs are the tangents of the new
-// state and of every deposit (J-dot, scattered with atomics).  Together with
-// the forward field updates applied to tangent grids this is the
+// The derivative of the same step along kDN tangent directions of the state,
+// of the fields and of the weight: what does not depend on the direction (the
+// push's intermediates, the gathers' and deposits' shares) is evaluated once,
+// and each direction takes the linear maps between them, one direction after
+// the other.  The tangents of the deposits (J-dot) are scattered with atomics.
+// Together with the forward field updates applied to tangent grids this is the
 // tangent-linear model of the loop, the exact transpose of what the adjoint
 // above computes; <dphi/dw, dw> from the adjoint must equal the tangent of phi
-// along dw to round-off (the dot-product test).
-
+// along dw to round-off (the dot-product test).  Re-executing the step in dual
+// numbers of four directions took 256 + 66 registers, 736 bytes of scratch and a
+// division per direction at every quotient: 184 us for 2.6e5 plasma particles
+// and 55 us for 8e3 of a bunch; this form takes 76 and 37 us.
 struct TlmFields {  // tangents of E^n and Hh^n, one set per direction
   const double *er[kDN], *ephi[kDN], *ez[kDN], *hhr[kDN], *hhphi[kDN], *hhz[kDN];
 };
@@ -1333,21 +922,18 @@ struct TlmSink {
   TlmJ j;
   double *box;  // LDS
   int bi, bk;   // node of box[.][0][0]
-  __device__ __forceinline__ void add(int comp, int i, int k, D v) {
-    if ((unsigned)i >= (unsigned)g->nr || (unsigned)k >= (unsigned)g->nz) return;
+  // node (i, k): its place in a plane of the box, -1 outside the box, -2 off the grid
+  __device__ __forceinline__ int node(int i, int k) const {
+    if ((unsigned)i >= (unsigned)g->nr || (unsigned)k >= (unsigned)g->nz) return -2;
     const int li = i - bi, lk = k - bk;
-    if ((unsigned)li < (unsigned)kR && (unsigned)lk < (unsigned)kK) {
-      double *q = box + (comp * kDN * kR + li) * kK + lk;
-#pragma unroll
-      for (int d = 0; d < kDN; d++)
-        if (v.d[d] != 0.0) atomicAdd(q + d * kR * kK, v.d[d]);
-      return;
-    }
-    const size_t p = (size_t)i * (size_t)g->nz + (size_t)k;
-#pragma unroll
-    for (int d = 0; d < kDN; d++) {
+    return (unsigned)li < (unsigned)kR && (unsigned)lk < (unsigned)kK ? li * kK + lk : -1;
+  }
+  __device__ __forceinline__ void put(int comp, int d, int node, int i, int k, double v) {
+    if (node >= 0) {
+      atomicAdd(box + (comp * kDN + d) * kR * kK + node, v);
+    } else if (node == -1) {
       double *J = comp == kAR ? j.jr[d] : comp == kAPhi ? j.jphi[d] : j.jz[d];
-      if (v.d[d] != 0.0) unsafeAtomicAdd(J + p, v.d[d]);
+      unsafeAtomicAdd(J + (size_t)i * (size_t)g->nz + (size_t)k, v);
     }
   }
   __device__ __forceinline__ void flush() const {
@@ -1362,99 +948,299 @@ struct TlmSink {
   }
 };
 
-// the gather of the tangent fields at the particle's (value) position: the
-// gather is linear in the field, so its tangent along the field is the same
-// weights applied to the tangent grid
-__device__ __forceinline__ double gather_value(const GridDesc &g, const double *F, double r, double z, bool lo,
-                                               bool zhalf) {
-  GatherW gw = gather_w(g, cst(r), cst(z), lo, zhalf);
-  const double *row0 = F + (size_t)gw.ir * (size_t)g.nz + gw.kz;
-  const double *row1 = row0 + g.nz;
-  return gw.w[0].v * row0[0] + gw.w[1].v * row1[0] + gw.w[2].v * row0[1] + gw.w[3].v * row1[1];
+#pragma clang fp contract(fast)
+// tangents of the push: the forward evaluation of boris_fwd / vay_fwd kept, and
+// the map of one direction
+struct BoostT {
+  Boost b;
+  bool x, y, z;  // components that are kept
+};
+__device__ __forceinline__ BoostT boost_t(V3 v) {
+  return BoostT{boost_of(v), !(fabs(v.x) < kMnzl), !(fabs(v.y) < kMnzl), !(fabs(v.z) < kMnzl)};
+}
+__device__ __forceinline__ V3 along(const BoostT &t, V3 dv) {
+  const V3 du = V3{t.x ? dv.x : 0.0, t.y ? dv.y : 0.0, t.z ? dv.z : 0.0};
+  return fma3(t.b.g0 * t.b.g0 * t.b.g0 / kC2 * dot(t.b.u, du), t.b.u, t.b.g0 * du);
+}
+// tangent of inv_gamma(u) u, g = inv_gamma(u)
+__device__ __forceinline__ V3 slow_t(double g, V3 u, V3 du) {
+  return fma3(-(g * g * g) / kC2 * dot(u, du), u, g * du);
+}
+struct BorisT {
+  BoostT b0;
+  V3 t, h, b, tp, w, u;
+  double g1, c2, g2;
+  __device__ __forceinline__ BorisT(V3 v, V3 e, V3 hs) : b0(boost_t(v)), h(hs) {
+    t = fma3(b0.b.g0, b0.b.u, e);
+    g1 = inv_gamma(t);
+    b = g1 * h;
+    tp = t + cross(t, b);
+    c2 = 2.0 / (1.0 + dot(b, b));
+    w = cross(tp, b);
+    u = fma3(c2, w, t) + e;
+    g2 = inv_gamma(u);
+  }
+  __device__ __forceinline__ V3 v() const { return g2 * u; }
+  __device__ __forceinline__ V3 along_dir(V3 dv, V3 de, V3 dh) const {
+    const V3 dt = along(b0, dv) + de;
+    const V3 db = fma3(-(g1 * g1 * g1) / kC2 * dot(t, dt), h, g1 * dh);
+    const V3 dtp = dt + cross(dt, b) + cross(t, db);
+    const V3 dw = cross(dtp, b) + cross(tp, db);
+    const V3 du = fma3(-c2 * c2 * dot(b, db), w, fma3(c2, dw, dt + de));
+    return slow_t(g2, u, du);
+  }
+};
+struct VayT {
+  BoostT b0;
+  V3 t, h, th, up, b, q, u;
+  double g1, ub, sg, root, al, s, al2, g3;
+  __device__ __forceinline__ VayT(V3 v, V3 e, V3 hs) : b0(boost_t(v)), h(hs) {
+    t = b0.b.g0 * b0.b.u;
+    g1 = inv_gamma(t);
+    th = cross(t, h);
+    up = fma3(g1, th, t + e);
+    const double B2 = dot(h, h);
+    ub = dot(up, h);
+    sg = 1.0 + dot(up, up) / kC2 - B2;
+    root = sqrt(sg * sg + 4. * (B2 + ub * ub));
+    al = 1.0 / sqrt(0.5 * (sg + root));
+    b = al * h;
+    s = 1.0 / (1.0 + dot(b, b));
+    al2 = dot(up, b);
+    q = fma3(al2, b, up) + cross(up, b);
+    u = s * q;
+    g3 = inv_gamma(u);
+  }
+  __device__ __forceinline__ V3 v() const { return g3 * u; }
+  __device__ __forceinline__ V3 along_dir(V3 dv, V3 de, V3 dh) const {
+    const V3 dt = along(b0, dv);
+    const V3 dth = cross(dt, h) + cross(t, dh);
+    const V3 dup = fma3(-(g1 * g1 * g1) / kC2 * dot(t, dt), th, fma3(g1, dth, dt + de));
+    const double dB2 = 2.0 * dot(h, dh), dub = dot(dup, h) + dot(up, dh);
+    const double dsg = 2.0 / kC2 * dot(up, dup) - dB2;
+    const double droot = (sg * dsg + 2.0 * dB2 + 4.0 * ub * dub) / root;
+    const V3 db = fma3(-0.25 * al * al * al * (dsg + droot), h, al * dh);
+    const double dal2 = dot(dup, b) + dot(up, db);
+    const V3 dq = fma3(dal2, b, fma3(al2, db, dup)) + (cross(dup, b) + cross(up, db));
+    return slow_t(g3, u, fma3(-2.0 * s * s * dot(b, db), q, s * dq));
+  }
+};
+
+// tangents of the J_phi deposit (azimuthal_current_distribution,
+// src/particles.cpp:688-784) of w charges q
+template <class Sink>
+__device__ __forceinline__ void jphi_tangent(const GridDesc &g, Sink &sk, double q, double w, double r, double z,
+                                             double vphi, const double (&tw)[kDN], const double (&tr)[kDN],
+                                             const double (&tz)[kDN], const double (&tv)[kDN]) {
+  const double dr = g.dr, dz = g.dz;
+  const int i = max(cell_number(r, dr), 0), k = max(cell_number(z, dz), 0);
+  const double r1 = r - 0.5 * dr, r2 = (i + 0.5) * dr, r3 = r + 0.5 * dr;
+  const double i1 = 1.0 / ((r > dr) ? cell_volume(i, dr, dz) : cyl_vol(dz, dr)), i2 = 1.0 / cell_volume(i + 1, dr, dz);
+  const double d1 = (k + 0.5) * dz - (z - 0.5 * dz), d2 = (z + 0.5 * dz) - (k + 0.5) * dz;
+  const double in = (r2 * r2 - r1 * r1) * i1, out = (r3 * r3 - r2 * r2) * i2;
+  const double ir = 1.0 / r, K = q * ir / (2. * dz * dr), P = w * K * vphi;
+  const double din = P * (-2.0 * r1 * i1), dout = P * (2.0 * r3 * i2);
+  const int n00 = sk.node(i, k), n10 = sk.node(i + 1, k), n01 = sk.node(i, k + 1), n11 = sk.node(i + 1, k + 1);
+#pragma unroll
+  for (int d = 0; d < kDN; d++) {
+    const double c = K * (w * tv[d] + vphi * tw[d]) - P * ir * tr[d];
+    const double ti = c * in + din * tr[d], to = c * out + dout * tr[d];
+    const double zi = P * in * tz[d], zo = P * out * tz[d];
+    sk.put(kAPhi, d, n00, i, k, ti * d1 - zi);
+    sk.put(kAPhi, d, n10, i + 1, k, to * d1 - zo);
+    sk.put(kAPhi, d, n01, i, k + 1, ti * d2 + zi);
+    sk.put(kAPhi, d, n11, i + 1, k + 1, to * d2 + zo);
+  }
 }
 
-template <bool BUNCH, class Sink>
-__device__ __forceinline__ void tlm_particle(const GridDesc &g, const AdjFields &f, const TlmFields &tf, Sink &sk,
-                                             const TlmSpecies &s, int pusher, long long i, bool live,
-                                             const AdjParticle &pt) {
-  const long long n = s.n;
-  if (!live) {
-    // dead (or padding) slots keep zero tangents; a particle injected later
-    // starts with zero tangents, as its injected state does not depend on w
+// the tangents of a path's ends
+struct PathT {
+  double rn[kDN], zn[kDN], ro[kDN], zo[kDN], w[kDN];
+};
+// strict_d's sink in the tangent step (see StrictSink): w times the deposits of
+// a unit weight, along each direction
+template <class Sink>
+struct StrictTangent {
+  Sink *sk;
+  const PathT *t;
+  double w;
+  __device__ __forceinline__ void add(int comp, int i, int k, D v) {
+    const int n = sk->node(i, k);
 #pragma unroll
-    for (int d = 0; d < kDN; d++) s.tr[d * n + i] = s.tz[d * n + i] = s.tvr[d * n + i] = s.tvphi[d * n + i] =
-        s.tvz[d * n + i] = 0.0;
+    for (int d = 0; d < kDN; d++)
+      sk->put(comp, d, n, i, k,
+              w * (v.d[0] * t->rn[d] + v.d[1] * t->zn[d] + v.d[2] * t->ro[d] + v.d[3] * t->zo[d]) + v.v * t->w[d]);
+  }
+};
+
+// tangents of the J_r / J_z deposit of w charges q on the path (ro, zo) -> (rn,
+// zn), piece by piece (the closed forms above segment_back)
+template <class Sink>
+__device__ __forceinline__ void deposit_j_tangent(const GridDesc &g, Sink &sk, double q, double w, double rn, double zn,
+                                                  double ro, double zo, const PathT &t) {
+  const double dr = g.dr, dz = g.dz, idr = 1.0 / dr, idz = 1.0 / dz;
+  const Path c = split_path(g, rn, zn, ro, zo);
+  if (c.strict) {
+    const PathT own = t;  // t itself stays in registers
+    StrictTangent<Sink> st{&sk, &own, w};
+    strict_d(g, st, cst(q), seed(rn, 0), seed(zn, 1), seed(ro, 2), seed(zo, 3));
     return;
   }
-  auto dual = [&](double v, const double *t) {
-    D x;
-    x.v = v;
+  const double kz = q / (4.0 * kPi * dr * dr * g.dt), kr = q / (2.0 * kPi * dr * dz * g.dt);
+  // path parameters of the crossings
+  const double sr = c.rad ? (c.rb - ro) / (rn - ro) : 0.0, sz = c.axi ? (c.zb - zo) / (zn - zo) : 0.0;
+  const double isl = c.rad ? 1.0 / c.slope : 0.0;
+#pragma nounroll
+  for (int n = 0; n < c.ns; n++) {
+    const bool first = n == 0, last = n == c.ns - 1;
+    // the piece ends at crossing n and begins at crossing n - 1; crossing n is
+    // the radial face's if
+    const bool nrad = first == c.rfirst, orad = (n == 1) == c.rfirst;
+    const double prn = last ? rn : nrad ? c.rb : c.r2, pzn = last ? zn : nrad ? c.z1 : c.zb;
+    const double pro = first ? ro : orad ? c.rb : c.r2, pzo = first ? zo : orad ? c.z1 : c.zb;
+    const int i = last ? c.i_n : first ? c.i0 : c.i1, k = last ? c.k_n : first ? c.k0 : c.k1;
+    if ((fabs(prn - pro) < kMnzl) || (fabs(pzn - pzo) < kMnzl)) continue;
+    const double fi = (double)i;
+    const double a = pro / dr - fi, b = pzo / dz - (double)k, drho = (prn - pro) / dr, dzeta = (pzn - pzo) / dz;
+    const double hdr = 0.5 * drho, ub = 1.0 - b, qdz = 0.25 * dzeta, p0 = 0.5 * ub - qdz, p1 = 0.5 * b + qdz;
+    // J_z = kz w dzeta (z0, z1), J_r = kr w (j0, j1); along a direction, with
+    // the tangents (ta, tb, tdr, tdz) of (a, b, drho, dzeta):
+    //   z0' = z0a ta + z0d tdr, j0' = j0a ta + j0b tb + j0d tdr + j0z tdz, and so on
+    double z0, z1, j0, j1, z0a, z1a, z0d, z1d, j0a, j1a, jb, j0d, j1d, jz;
+    if (i == 0) {
+      z0 = 8.0 * (1.0 - hdr - a);
+      z1 = hdr + 1.0 + a;
+      z0a = -8.0;
+      z1a = 1.0;
+      z0d = -4.0;
+      z1d = 0.5;
+      j0 = 2.0 * drho * p0;
+      j1 = 2.0 * drho * p1;
+      j0a = j1a = 0.0;
+      jb = drho;
+      j0d = 2.0 * p0;
+      j1d = 2.0 * p1;
+      jz = hdr;
+    } else {
+      const double i0 = 1.0 / fi, i1 = 1.0 / (fi + 1.0), ih = 1.0 / (fi + 0.5);
+      const double rs = fi + a, re = rs + drho, irs = 1.0 / rs, ire = 1.0 / re;
+      const double ii = fi * (fi + 1.0), x = drho * irs, u = drho * ire;
+      double M, dM;
+      m_and_slope(x, M, dM);
+      const double N = -u - M, iiM = ii * M, cc = 0.5 * ii * irs;
+      const double A0 = (1.0 - a) * (2.0 * fi + a) + iiM, A1 = a * (2.0 * fi + 1.0 + a) - iiM;
+      const double R0 = u * ub + dzeta * N, R1 = u * b - dzeta * N;
+      // derivatives of x, u and N along a and drho
+      const double xa = -x * irs, ua = -u * ire, ud = rs * ire * ire, Ma = dM * xa, Md = dM * irs;
+      const double Na = -ua - Ma, Nd = -ud - Md;
+      z0 = (A0 * irs - hdr) * i0;
+      z1 = (A1 * irs + hdr) * i1;
+      z0a = (((1.0 - 2.0 * fi - 2.0 * a) + ii * Ma) - A0 * irs) * irs * i0;
+      z1a = (((2.0 * fi + 1.0 + 2.0 * a) - ii * Ma) - A1 * irs) * irs * i1;
+      z0d = (ii * Md * irs - 0.5) * i0;
+      z1d = (0.5 - ii * Md * irs) * i1;
+      j0 = (drho * p0 + cc * R0) * ih;
+      j1 = (drho * p1 + cc * R1) * ih;
+      j0a = cc * (ua * ub + dzeta * Na - R0 * irs) * ih;
+      j1a = cc * (ua * b - dzeta * Na - R1 * irs) * ih;
+      jb = (hdr + cc * u) * ih;
+      j0d = (p0 + cc * (ud * ub + dzeta * Nd)) * ih;
+      j1d = (p1 + cc * (ud * b - dzeta * Nd)) * ih;
+      jz = (0.25 * drho - cc * N) * ih;
+    }
+    const int n00 = sk.node(i, k), n10 = sk.node(i + 1, k), n01 = sk.node(i, k + 1);
+    const double wz = w * kz, wr = w * kr;
 #pragma unroll
-    for (int d = 0; d < kDN; d++) x.d[d] = t[d * n + i];
-    return x;
-  };
-  D r = dual(pt.r, s.tr), z = dual(pt.z, s.tz);
-  D v[3] = {dual(pt.vr, s.tvr), dual(pt.vphi, s.tvphi), dual(pt.vz, s.tvz)};
-  D w = dual(pt.w, s.tw);
-  D q = s.charge * w, m = s.mass * w;
-  const D r_old = r, z_old = z;
-  const double r0v = r.v, z0v = z.v;
-  D e[3], h[3];
-  e[0] = gather_d(g, f.er, r, z, true, false);
-  e[1] = gather_d(g, f.ephi, r, z, false, false);
-  e[2] = gather_d(g, f.ez, r, z, false, true);
-  h[0] = gather_d(g, f.hhr, r, z, false, true);
-  h[1] = gather_d(g, f.hhphi, r, z, true, true);
-  h[2] = gather_d(g, f.hhz, r, z, true, false);
-#pragma unroll
-  for (int d = 0; d < kDN; d++) {
-    e[0].d[d] += gather_value(g, tf.er[d], r0v, z0v, true, false);
-    e[1].d[d] += gather_value(g, tf.ephi[d], r0v, z0v, false, false);
-    e[2].d[d] += gather_value(g, tf.ez[d], r0v, z0v, false, true);
-    h[0].d[d] += gather_value(g, tf.hhr[d], r0v, z0v, false, true);
-    h[1].d[d] += gather_value(g, tf.hhphi[d], r0v, z0v, true, true);
-    h[2].d[d] += gather_value(g, tf.hhz[d], r0v, z0v, true, false);
-  }
-  if (pusher == 1)
-    vay_d(q, m, g.dt, e, h, v);
-  else
-    boris_d(q, m, g.dt, e, h, v);
-  const double half_dt = g.dt / 2.;
-  D x = r + v[0] * half_dt;
-  D y = 0.0 + v[1] * half_dt;
-  z = z + v[2] * half_dt;
-  r = dsqrt(x * x + y * y);
-  jphi_d(g, sk, q, r, z, v[1]);
-  x = r + v[0] * half_dt;
-  y = 0.0 + v[1] * half_dt;
-  z = z + v[2] * half_dt;
-  bool alive = true;
-  walls_d(g, BUNCH, x, z, v[0], v[2], alive);
-  D rr = dsqrt(x * x + y * y);
-  D st = y / rr;
-  r = rr;
-  if (alive) {
-    deposit_j_d(g, sk, q, r, z, r_old, z_old);
-    D ct = dsqrt(1 - st * st);
-    D u2 = ct * v[0] - st * v[1];
-    D w2 = st * v[0] + ct * v[1];
-    v[0] = u2;
-    v[1] = w2;
-  }
-#pragma unroll
-  for (int d = 0; d < kDN; d++) {
-    const bool keep = alive;
-    s.tr[d * n + i] = keep ? r.d[d] : 0.0;
-    s.tz[d * n + i] = keep ? z.d[d] : 0.0;
-    s.tvr[d * n + i] = keep ? v[0].d[d] : 0.0;
-    s.tvphi[d * n + i] = keep ? v[1].d[d] : 0.0;
-    s.tvz[d * n + i] = keep ? v[2].d[d] : 0.0;
+    for (int d = 0; d < kDN; d++) {
+      double ern = t.rn[d], ezn = t.zn[d], ero = t.ro[d], ezo = t.zo[d];
+      if (c.ns > 1) {
+        // with s the path parameter of a crossing, the one with the radial
+        // face moves along z, that with the axial face along r
+        const double tz1 = (1.0 - sr) * ezo + sr * ezn - isl * ((1.0 - sr) * ero + sr * ern);
+        const double tr2 = (1.0 - sz) * ero + sz * ern - c.slope * ((1.0 - sz) * ezo + sz * ezn);
+        if (!last) {
+          ern = nrad ? 0.0 : tr2;
+          ezn = nrad ? tz1 : 0.0;
+        }
+        if (!first) {
+          ero = orad ? 0.0 : tr2;
+          ezo = orad ? tz1 : 0.0;
+        }
+      }
+      const double ta = ero * idr, tb = ezo * idz, tdr = (ern - ero) * idr, tdz = (ezn - ezo) * idz;
+      const double f = wz * tdz + kz * t.w[d] * dzeta, e = wz * dzeta, h = kr * t.w[d];
+      const double m = jb * tb + jz * tdz;
+      sk.put(kAZ, d, n00, i, k, f * z0 + e * (z0a * ta + z0d * tdr));
+      sk.put(kAZ, d, n10, i + 1, k, f * z1 + e * (z1a * ta + z1d * tdr));
+      sk.put(kAR, d, n00, i, k, h * j0 + wr * (j0a * ta + j0d * tdr - m));
+      sk.put(kAR, d, n01, i, k + 1, h * j1 + wr * (j1a * ta + j1d * tdr + m));
+    }
   }
 }
 
-template <bool BUNCH, bool F32>
-__global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, TlmFields tf, TlmJ tj, TlmSpecies s,
-                                                       int pusher) {
+template <class Push, bool BUNCH, class Sink>
+__device__ __forceinline__ void tlm_particle(const GridDesc &g, const AdjFields &f, const TlmFields &tf, Sink &sk,
+                                             const TlmSpecies &s, long long i, const AdjParticle &pt) {
+  constexpr bool kVay = std::is_same<Push, VayT>::value;
+  const long long n = s.n;
+  const double r0 = pt.r, z0 = pt.z, w = pt.w, half_dt = g.dt / 2.;
+  // the scales of the push's fields: q / m does not depend on w
+  const double c1 = s.charge * g.dt / (2 * s.mass);
+  const double es = kVay ? 2 * c1 : c1, bs = kVay ? kMagnConst * c1 * (2 * c1) * c1 : kMagnConst * c1;
+  const RingW wl = ring_lo(g, r0), wo = ring_own(g, r0);
+  const ColW co = col_w(g, z0, false), ch = col_w(g, z0, true);
+  const Gathered e0 = gather_grad(g, f.er, wl, co), e1 = gather_grad(g, f.ephi, wo, co);
+  const Gathered e2 = gather_grad(g, f.ez, wo, ch), h0 = gather_grad(g, f.hhr, wo, ch);
+  const Gathered h1 = gather_grad(g, f.hhphi, wl, ch), h2 = gather_grad(g, f.hhz, wl, co);
+  const Push push(V3{pt.vr, pt.vphi, pt.vz}, es * V3{e0.v, e1.v, e2.v}, bs * V3{h0.v, h1.v, h2.v});
+  const V3 v = push.v();
+  // first half step and rotation (step_v), then full_current_distribution
+  const double x1 = r0 + v.x * half_dt, y = v.y * half_dt, z1 = z0 + v.z * half_dt;
+  const double r1 = sqrt(x1 * x1 + y * y), ir1 = 1.0 / r1;
+  double x2 = r1 + v.x * half_dt, z2 = z1 + v.z * half_dt, sx, sz;
+  bool alive = true;
+  walls_sign(g, BUNCH, x2, z2, sx, sz, alive);
+  const double r2 = sqrt(x2 * x2 + y * y), ir2 = 1.0 / r2, st = y * ir2, ct = sqrt(1 - st * st);
+  const double vx = sx * v.x;  // after the walls
+  PathT t;
+  double tr1[kDN], tz1[kDN], tvp[kDN];  // at the J_phi deposit
+#pragma unroll
+  for (int d = 0; d < kDN; d++) {
+    const size_t p = (size_t)d * n + i;
+    const double tr = s.tr[p], tz = s.tz[p];
+    t.ro[d] = tr;
+    t.zo[d] = tz;
+    t.w[d] = s.tw[p];
+    const V3 de = es * V3{tr * e0.dr + tz * e0.dz + gather_grad(g, tf.er[d], wl, co).v,
+                          tr * e1.dr + tz * e1.dz + gather_grad(g, tf.ephi[d], wo, co).v,
+                          tr * e2.dr + tz * e2.dz + gather_grad(g, tf.ez[d], wo, ch).v};
+    const V3 dh = bs * V3{tr * h0.dr + tz * h0.dz + gather_grad(g, tf.hhr[d], wo, ch).v,
+                          tr * h1.dr + tz * h1.dz + gather_grad(g, tf.hhphi[d], wl, ch).v,
+                          tr * h2.dr + tz * h2.dz + gather_grad(g, tf.hhz[d], wl, co).v};
+    const V3 dv = push.along_dir(V3{s.tvr[p], s.tvphi[p], s.tvz[p]}, de, dh);
+    const double ty = dv.y * half_dt;
+    tr1[d] = (x1 * (tr + dv.x * half_dt) + y * ty) * ir1;
+    tz1[d] = tz + dv.z * half_dt;
+    tvp[d] = dv.y;
+    const double tx2 = sx * (tr1[d] + dv.x * half_dt);
+    t.rn[d] = (x2 * tx2 + y * ty) * ir2;
+    t.zn[d] = sz * (tz1[d] + dv.z * half_dt);
+    // rotation of the velocity by the second half step's angle
+    const double ts = (ty - st * t.rn[d]) * ir2, tc = -st / ct * ts, tvx = sx * dv.x;
+    s.tr[p] = alive ? t.rn[d] : 0.0;
+    s.tz[p] = alive ? t.zn[d] : 0.0;
+    s.tvr[p] = alive ? tc * vx + ct * tvx - ts * v.y - st * dv.y : 0.0;
+    s.tvphi[p] = alive ? ts * vx + st * tvx + tc * v.y + ct * dv.y : 0.0;
+    s.tvz[p] = alive ? sz * dv.z : 0.0;
+    __builtin_amdgcn_sched_barrier(0);  // one direction's registers at a time
+  }
+  jphi_tangent(g, sk, s.charge, w, r1, z1, v.y, t.w, tr1, tz1, tvp);
+  if (alive) deposit_j_tangent(g, sk, s.charge, w, r2, z2, r0, z0, t);
+}
+#pragma clang fp contract(off)
+
+template <bool VAY, bool BUNCH, bool F32>
+__global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, TlmFields tf, TlmJ tj, TlmSpecies s) {
   using Sink = TlmSink<BUNCH>;
   __shared__ double box[Sink::kSize];
   const long long i = adj_slot<BUNCH>();
@@ -1470,7 +1256,17 @@ __global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, 
   for (int t = threadIdx.x; t < Sink::kSize; t += blockDim.x) box[t] = 0.0;
   __syncthreads();
   Sink sk{&g, tj, box, ci - 1, ck - 2};
-  if (i < s.n) tlm_particle<BUNCH>(g, f, tf, sk, s, pusher, i, live, pt);
+  if (live) {
+    tlm_particle<typename std::conditional<VAY, VayT, BorisT>::type, BUNCH>(g, f, tf, sk, s, i, pt);
+  } else if (i < s.n) {
+    // dead (or padding) slots keep zero tangents; a particle injected later
+    // starts with zero tangents, as its injected state does not depend on w
+#pragma unroll
+    for (int d = 0; d < kDN; d++) {
+      const size_t p = (size_t)d * s.n + i;
+      s.tr[p] = s.tz[p] = s.tvr[p] = s.tvphi[p] = s.tvz[p] = 0.0;
+    }
+  }
   __syncthreads();
   sk.flush();
 }
@@ -1722,11 +1518,13 @@ void launch_tlm_particles(const GridDesc &g, const double *const *fields6, doubl
   }
   TlmSpecies s{state, tstate[0], tstate[1], tstate[2], tstate[3], tstate[4], tw, charge, mass, n};
   const dim3 grid((unsigned)((n + 255) / 256));
-  using K = void (*)(GridDesc, AdjFields, TlmFields, TlmJ, TlmSpecies, int);
-  static const K kernels[4] = {k_tlm_particles<false, false>, k_tlm_particles<true, false>,
-                               k_tlm_particles<false, true>, k_tlm_particles<true, true>};
-  hipLaunchKernelGGL(kernels[(is_bunch != 0) + 2 * (state.cell != nullptr)], grid, dim3(256), 0, st, g, f, tf, tj, s,
-                     pusher);
+  using K = void (*)(GridDesc, AdjFields, TlmFields, TlmJ, TlmSpecies);
+  static const K kernels[8] = {k_tlm_particles<false, false, false>, k_tlm_particles<true, false, false>,
+                               k_tlm_particles<false, true, false>,  k_tlm_particles<true, true, false>,
+                               k_tlm_particles<false, false, true>,  k_tlm_particles<true, false, true>,
+                               k_tlm_particles<false, true, true>,   k_tlm_particles<true, true, true>};
+  const int k = (pusher == 1) + 2 * (is_bunch != 0) + 4 * (state.cell != nullptr);
+  hipLaunchKernelGGL(kernels[k], grid, dim3(256), 0, st, g, f, tf, tj, s);
 }
 
 void launch_tlm_objective(const GridDesc &g, const double *ez, double *const *const *tgrid, int k0, int k1,
