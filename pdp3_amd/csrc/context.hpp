@@ -38,7 +38,8 @@ struct GridDesc {
   // the FP64 form's shared divisors, correctly rounded on the host: 1/dr,
   // 1/dz, CYL_VOL(dz, dr) and its reciprocal, and per radial index
   // i = 0 .. nr+1 the pair {CELL_VOLUME(i, dr, dz), 1/CELL_VOLUME(i, dr, dz)}
-  // (include/geometry.h:33-39), built at context creation
+  // (include/geometry.h:33-39), then those of the divisors of density_r and
+  // density_z (include/particles.h:169-178), built at context creation
   double inv_dr, inv_dz;
   double cyl, inv_cyl;
   const double2 *vol;

@@ -27,19 +27,16 @@ __device__ __forceinline__ double rsqrt_residual(double x, double c) {
   return (t - qe) - x * pe;
 }
 
-// 1/sqrt(x), correctly rounded except in exact-tie cases, for x > 0 finite
+// 1/sqrt(x), correctly rounded except in exact-tie cases, for x > 0 finite: two
+// Newton steps from the hardware's estimate leave y within an ulp, and of its
+// neighbours only the one that its residual points to can be nearer
 __device__ __forceinline__ double rsqrt_cr(double x) {
-  double y = 1.0 / sqrt(x);
-  double r0 = fabs(rsqrt_residual(x, y));
-  double yl = nextafter(y, 0.0), yh = nextafter(y, 1e308);
-  double rl = fabs(rsqrt_residual(x, yl)), rh = fabs(rsqrt_residual(x, yh));
-  double best = y, rb = r0;
-  if (rl < rb) {
-    best = yl;
-    rb = rl;
-  }
-  if (rh < rb) best = yh;
-  return best;
+  double y = __builtin_amdgcn_rsq(x);
+  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  const double r = rsqrt_residual(x, y);
+  const double c = __longlong_as_double(__double_as_longlong(y) + (r < 0.0 ? -1 : 1));
+  return fabs(rsqrt_residual(x, c)) < fabs(r) ? c : y;
 }
 
 // x / y, correctly rounded, from yr = 1/y correctly rounded: q = x yr lies

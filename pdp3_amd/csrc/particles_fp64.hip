@@ -51,63 +51,86 @@ constexpr double kC2 = kLightSpeed * kLightSpeed;
 constexpr double kInvC2 = 1.0 / kC2;
 
 // four-node ring-volume gather shared by EField::get_field
-// (src/eField.cpp:204-316) and HField::get_field (src/hField.cpp:159-267).
-// lo: radial index from r - dr/2 (E_r, H_z, H_phi); zhalf: axial index from
-// z - dz/2 (E_z, H_r, H_phi).  Indices are clamped at 0 as the reference does
-// and, beyond the reference, kept inside the array (flagged as a domain error).
-__device__ double gather4(const GridDesc &g, const double *__restrict__ F, double radius, double longitude,
-                          bool lo, bool zhalf, int *err) {
-  const double dr = g.dr, dz = g.dz;
-  double r1 = radius - 0.5 * dr;
-  double r3 = radius + 0.5 * dr;
-  int i_r = lo ? cell_r(g, radius - 0.5 * dr) : cell_r(g, radius);
-  int k_z = zhalf ? cell_z(g, longitude - 0.5 * dz) : cell_z(g, longitude);
-  if (i_r < 0) i_r = 0;
-  if (k_z < 0) k_z = 0;
-  if (i_r > g.nr - 2 || k_z > g.nz - 2) {
-    atomicOr(err, kErrDomain);
-    i_r = min(i_r, g.nr - 2);
-    k_z = min(k_z, g.nz - 2);
-  }
-  Vol vol_1, vol_2;
-  double r2, dz1, dz2;
+// (src/eField.cpp:204-316) and HField::get_field (src/hField.cpp:159-267): two
+// radial families (lo: the index from r - dr/2, for E_r, H_z, H_phi) and two
+// axial ones (half: from z - dz/2, for E_z, H_r, H_phi), each evaluated once.
+// Indices are clamped at 0 as the reference does and, beyond the reference, kept
+// inside the array (flagged as a domain error).
+struct Rings {
+  int i;
+  double in, out;  // rb^2 - ra^2 of the shares of rows i and i + 1
+  Vol v1, v2;
+};
+struct Cols {
+  int k;
+  double d1, d2;
+};
+__device__ __forceinline__ double ring_share(double F, double dzx, double ring, Vol vol) {
+  return div_cr(F * kPi * dzx * ring, vol.v, vol.inv);
+}
+__device__ __forceinline__ Rings rings_of(const GridDesc &g, double radius, bool lo, bool &out) {
+  const double dr = g.dr;
+  const double r1 = radius - 0.5 * dr, r3 = radius + 0.5 * dr;
+  Rings w;
+  w.i = max(lo ? cell_r(g, radius - 0.5 * dr) : cell_r(g, radius), 0);
+  out = out || w.i > g.nr - 2;
+  w.i = min(w.i, g.nr - 2);
+  double r2;
   if (lo) {
-    vol_1 = vol_cell(g, i_r + 1);
-    vol_2 = vol_cell(g, i_r + 3);
-    r2 = (i_r + 1) * dr;
+    w.v1 = vol_cell(g, w.i + 1);
+    w.v2 = vol_cell(g, w.i + 3);
+    r2 = (w.i + 1) * dr;
   } else {
-    vol_1 = (radius > dr) ? vol_cell(g, i_r) : vol_cyl(g);
-    r2 = (i_r + 0.5) * dr;
-    vol_2 = vol_cell(g, i_r + 2);
+    w.v1 = (radius > dr) ? vol_cell(g, w.i) : vol_cyl(g);
+    r2 = (w.i + 0.5) * dr;
+    w.v2 = vol_cell(g, w.i + 2);
   }
-  if (zhalf) {
-    dz1 = (k_z + 1.5) * dz - longitude;
-    dz2 = longitude - (k_z + 0.5) * dz;
-  } else {
-    dz1 = (k_z + 1) * dz - longitude;
-    dz2 = longitude - k_z * dz;
-  }
-  const double *row0 = F + (size_t)i_r * (size_t)g.nz;
+  w.in = r2 * r2 - r1 * r1;
+  w.out = r3 * r3 - r2 * r2;
+  return w;
+}
+__device__ __forceinline__ Cols cols_of(const GridDesc &g, double longitude, bool half, bool &out) {
+  const double dz = g.dz;
+  Cols c;
+  c.k = max(half ? cell_z(g, longitude - 0.5 * dz) : cell_z(g, longitude), 0);
+  out = out || c.k > g.nz - 2;
+  c.k = min(c.k, g.nz - 2);
+  c.d1 = (half ? (c.k + 1.5) * dz : (c.k + 1) * dz) - longitude;
+  c.d2 = longitude - (half ? (c.k + 0.5) * dz : c.k * dz);
+  return c;
+}
+__device__ __forceinline__ double gather4(const GridDesc &g, const double *__restrict__ F, const Rings &w,
+                                          const Cols &c) {
+  const double *row0 = F + (size_t)w.i * (size_t)g.nz;
   const double *row1 = row0 + g.nz;
   double acc = 0;
-  acc = acc + ring_term(row0[k_z], dz1, r1, r2, vol_1);
-  acc = acc + ring_term(row1[k_z], dz1, r2, r3, vol_2);
-  acc = acc + ring_term(row0[k_z + 1], dz2, r1, r2, vol_1);
-  acc = acc + ring_term(row1[k_z + 1], dz2, r2, r3, vol_2);
+  acc = acc + ring_share(row0[c.k], c.d1, w.in, w.v1);
+  acc = acc + ring_share(row1[c.k], c.d1, w.out, w.v2);
+  acc = acc + ring_share(row0[c.k + 1], c.d2, w.in, w.v1);
+  acc = acc + ring_share(row1[c.k + 1], c.d2, w.out, w.v2);
   return acc;
 }
 
-__device__ __forceinline__ void gather_e(const GridDesc &g, const Fields &f, double r, double z, double e[3],
-                                         int *err) {
-  e[0] = gather4(g, f.er, r, z, true, false, err);
-  e[1] = gather4(g, f.ephi, r, z, false, false, err);
-  e[2] = gather4(g, f.ez, r, z, false, true, err);
+struct GatherW {
+  Rings lo, own;
+  Cols co, ch;
+};
+__device__ __forceinline__ GatherW gather_weights(const GridDesc &g, double r, double z, int *err) {
+  bool out = false;
+  const GatherW w{rings_of(g, r, true, out), rings_of(g, r, false, out), cols_of(g, z, false, out),
+                  cols_of(g, z, true, out)};
+  if (out) atomicOr(err, kErrDomain);
+  return w;
 }
-__device__ __forceinline__ void gather_h(const GridDesc &g, const Fields &f, double r, double z, double h[3],
-                                         int *err) {
-  h[0] = gather4(g, f.hhr, r, z, false, true, err);
-  h[1] = gather4(g, f.hhphi, r, z, true, true, err);
-  h[2] = gather4(g, f.hhz, r, z, true, false, err);
+__device__ __forceinline__ void gather_e(const GridDesc &g, const Fields &f, const GatherW &w, double e[3]) {
+  e[0] = gather4(g, f.er, w.lo, w.co);
+  e[1] = gather4(g, f.ephi, w.own, w.co);
+  e[2] = gather4(g, f.ez, w.own, w.ch);
+}
+__device__ __forceinline__ void gather_h(const GridDesc &g, const Fields &f, const GatherW &w, double h[3]) {
+  h[0] = gather4(g, f.hhr, w.own, w.ch);
+  h[1] = gather4(g, f.hhphi, w.lo, w.ch);
+  h[2] = gather4(g, f.hhz, w.lo, w.co);
 }
 
 __device__ __forceinline__ double dot3(const double *a, const double *b) {
@@ -211,10 +234,8 @@ __device__ void deposit_jphi(const GridDesc &g, S &sk, double q, double r, doubl
   Vol v_2 = vol_cell(g, r_i + 1);
   double dz1 = (z_k + 0.5) * dz - (z - 0.5 * dz);
   double dz2 = (z + 0.5 * dz) - (z_k + 0.5) * dz;
-  sk.template add<kCPhi>(r_i, z_k, ring_term(ro_v, dz1, r1, r2, v_1) * vphi);
-  sk.template add<kCPhi>(r_i + 1, z_k, ring_term(ro_v, dz1, r2, r3, v_2) * vphi);
-  sk.template add<kCPhi>(r_i, z_k + 1, ring_term(ro_v, dz2, r1, r2, v_1) * vphi);
-  sk.template add<kCPhi>(r_i + 1, z_k + 1, ring_term(ro_v, dz2, r2, r3, v_2) * vphi);
+  sk.template add4<kCPhi>(r_i, z_k, ring_term(ro_v, dz1, r1, r2, v_1) * vphi, ring_term(ro_v, dz1, r2, r3, v_2) * vphi,
+                          ring_term(ro_v, dz2, r1, r2, v_1) * vphi, ring_term(ro_v, dz2, r2, r3, v_2) * vphi);
 }
 
 // Particles::charge_weighting for one particle, src/particles.cpp:101-226
@@ -227,43 +248,41 @@ __device__ void deposit_rho(const GridDesc &g, S &sk, double q, double r, double
   if (z_k < 0) z_k = 0;
   double dz1 = (z_k + 0.5) * dz - (z - 0.5 * dz);
   double dz2 = (z + 0.5 * dz) - (z_k + 0.5) * dz;
-  if (r > dr) {
-    double r1 = r - 0.5 * dr, r2 = (r_i + 0.5) * dr, r3 = r + 0.5 * dr;
-    double ro_v = q / (2. * kPi * dz * dr * r);
-    Vol v_1 = vol_cell(g, r_i), v_2 = vol_cell(g, r_i + 1);
-    sk.template add<kCRho>(r_i, z_k, ring_term(ro_v, dz1, r1, r2, v_1));
-    sk.template add<kCRho>(r_i + 1, z_k, ring_term(ro_v, dz1, r2, r3, v_2));
-    sk.template add<kCRho>(r_i, z_k + 1, ring_term(ro_v, dz2, r1, r2, v_1));
-    sk.template add<kCRho>(r_i + 1, z_k + 1, ring_term(ro_v, dz2, r2, r3, v_2));
-  } else if (r <= dr / 2.) {
+  double w00, w10, w01, w11;
+  if (!(r > dr) && r <= dr / 2.) {
     r_i = 0;
     double r2 = (r_i + 0.5) * dr, r3 = r + 0.5 * dr;
     double ro_v = q / (kPi * dz * (2. * r * r + dr * dr / 2.));
     Vol v_1 = vol_cyl(g), v_2 = vol_cell(g, r_i + 1);
-    sk.template add<kCRho>(r_i, z_k, div_cr(ro_v * kPi * dz1 * (dr * dr / 2. - r * dr + r * r), v_1.v, v_1.inv));
-    sk.template add<kCRho>(r_i + 1, z_k, ring_term(ro_v, dz1, r2, r3, v_2));
-    sk.template add<kCRho>(r_i, z_k + 1, div_cr(ro_v * kPi * dz2 * (dr * dr / 2. - r * dr + r * r), v_1.v, v_1.inv));
-    sk.template add<kCRho>(r_i + 1, z_k + 1, ring_term(ro_v, dz2, r2, r3, v_2));
+    w00 = div_cr(ro_v * kPi * dz1 * (dr * dr / 2. - r * dr + r * r), v_1.v, v_1.inv);
+    w10 = ring_term(ro_v, dz1, r2, r3, v_2);
+    w01 = div_cr(ro_v * kPi * dz2 * (dr * dr / 2. - r * dr + r * r), v_1.v, v_1.inv);
+    w11 = ring_term(ro_v, dz2, r2, r3, v_2);
   } else {
     double r1 = r - 0.5 * dr, r2 = (r_i + 0.5) * dr, r3 = r + 0.5 * dr;
     double ro_v = q / (2. * kPi * dz * dr * r);
-    Vol v_1 = vol_cyl(g), v_2 = vol_cell(g, r_i + 1);
-    sk.template add<kCRho>(r_i, z_k, ring_term(ro_v, dz1, r1, r2, v_1));
-    sk.template add<kCRho>(r_i + 1, z_k, ring_term(ro_v, dz1, r2, r3, v_2));
-    sk.template add<kCRho>(r_i, z_k + 1, ring_term(ro_v, dz2, r1, r2, v_1));
-    sk.template add<kCRho>(r_i + 1, z_k + 1, ring_term(ro_v, dz2, r2, r3, v_2));
+    Vol v_1 = (r > dr) ? vol_cell(g, r_i) : vol_cyl(g), v_2 = vol_cell(g, r_i + 1);
+    w00 = ring_term(ro_v, dz1, r1, r2, v_1);
+    w10 = ring_term(ro_v, dz1, r2, r3, v_2);
+    w01 = ring_term(ro_v, dz2, r1, r2, v_1);
+    w11 = ring_term(ro_v, dz2, r2, r3, v_2);
   }
+  sk.template add4<kCRho>(r_i, z_k, w00, w10, w01, w11);
 }
 
 // density prefactors, include/particles.h:169-178
 __device__ __forceinline__ double density_strict(double q, double r, double dr, double dz, double dt) {
   return q / (kPi * 4. * r * dz * dz * dr * dt);
 }
-__device__ __forceinline__ double density_r(double q, double r, double dr, double dz, double dt) {
-  return q / (2 * kPi * r * dr * dz * dt * 2 * dr);
+// density_r(i dr) (i = 0: of the axis cell's own term) and density_z((i + 1/2) dr)
+// by the context's table of their divisors
+__device__ __forceinline__ double density_r(const GridDesc &g, double q, int i) {
+  const double2 t = g.vol[(g.nr + 2) + i];
+  return div_cr(q, t.x, t.y);
 }
-__device__ __forceinline__ double density_z(double q, double r, double dr, double dz, double dt) {
-  return q / (2 * kPi * r * dr * dz * dt * dz);
+__device__ __forceinline__ double density_z(const GridDesc &g, double q, int i) {
+  const double2 t = g.vol[2 * (g.nr + 2) + i];
+  return div_cr(q, t.x, t.y);
 }
 
 // simple_current_distribution: one straight segment inside cell (i_n, k_n),
@@ -271,7 +290,7 @@ __device__ __forceinline__ double density_z(double q, double r, double dr, doubl
 template <class S>
 __device__ void segment(const GridDesc &g, S &acc, double q, double radius_new, double longitude_new,
                         double radius_old, double longitude_old, int i_n, int k_n) {
-  const double dr = g.dr, dz = g.dz, delta_t = g.dt;
+  const double dr = g.dr, dz = g.dz;
   double delta_r = radius_new - radius_old;
   double delta_z = longitude_new - longitude_old;
   if ((fabs(delta_r) < kMnzl) || (fabs(delta_z) < kMnzl)) return;
@@ -280,41 +299,43 @@ __device__ void segment(const GridDesc &g, S &acc, double q, double radius_new, 
   double lg = log((k * delta_z + b) / b);
   double wj0, wj1;
   if (i_n >= 1) {
-    double ssd = density_r(q, i_n * dr, dr, dz, delta_t);
+    double ssd = density_r(g, q, i_n);
     wj0 = ssd * (dr * delta_z - k * delta_z * delta_z / 2. - delta_z * b +
                  dr * dr / k * ((i_n + 0.5) * (i_n + 0.5) - 0.25) * lg);
-    ssd = density_r(q, (i_n + 1) * dr, dr, dz, delta_t);
+    ssd = density_r(g, q, i_n + 1);
     wj1 = ssd * (k * delta_z * delta_z / 2. + delta_z * b + delta_z * dr +
                  dr * dr / k * (0.25 - (i_n + 0.5) * (i_n + 0.5)) * lg);
   } else {
-    double ssd = q / (2. * kPi * dr / 4. * dr * dz * delta_t * dr);
+    double ssd = density_r(g, q, 0);
     wj0 = ssd * (dr * delta_z - k * delta_z * delta_z / 2. - delta_z * b);
-    ssd = density_r(q, dr, dr, dz, delta_t);
+    ssd = density_r(g, q, 1);
     wj1 = ssd * (k * delta_z * delta_z / 2. + delta_z * dr + delta_z * b);
   }
-  acc.template add<kCZ>(i_n, k_n, wj0);
-  acc.template add<kCZ>(i_n + 1, k_n, wj1);
+  acc.template add2<kCZ>(i_n, k_n, wj0, wj1);
   // J_r (identical in both radial branches)
   k = -delta_z / delta_r;
   double r0 = (i_n + 0.5) * dr;
   double r1 = radius_old;
   b = (k_n + 1.) * dz - longitude_old;
-  double ssd = density_z(q, r0, dr, dz, delta_t);
+  double ssd = density_z(g, q, i_n);
   double lr = log((radius_old + delta_r) / radius_old);
-  double wj = ssd * (r0 * k * delta_r + k / 2. * delta_r * (radius_old + delta_r / 2.) +
+  const double wr0 = ssd * (r0 * k * delta_r + k / 2. * delta_r * (radius_old + delta_r / 2.) +
                      0.5 * delta_r * (b - k * (2 * r0 + r1)) +
                      delta_r * (b - k * r1) * (4 * r0 * r0 - dr * dr) / (8 * radius_old * (radius_old + delta_r)) +
                      (k * (r0 * r0 / 2. - dr * dr / 8.)) * lr);
-  acc.template add<kCR>(i_n, k_n, wj);
   b = longitude_old - k_n * dz;
-  wj = ssd * (-r0 * k * delta_r - k / 2. * delta_r * (radius_old + delta_r / 2.) +
+  const double wr1 = ssd * (-r0 * k * delta_r - k / 2. * delta_r * (radius_old + delta_r / 2.) +
               0.5 * delta_r * (b + k * (2 * r0 + r1)) +
               delta_r * (b + k * r1) * (4 * r0 * r0 - dr * dr) / (8 * radius_old * (radius_old + delta_r)) -
               (k * (r0 * r0 / 2. - dr * dr / 8.)) * lr);
-  acc.template add<kCR>(i_n, k_n + 1, wj);
+  acc.template add2<kCR>(i_n, k_n, wr0, wr1);
 }
 
 // strict_motion_weighting, src/particles.cpp:786-988
+struct Pair {
+  double a, b;
+  int i, k;
+};
 template <class S>
 __device__ void strict_motion(const GridDesc &g, S &acc, double q, double radius_new,
                               double longitude_new, double radius_old, double longitude_old) {
@@ -330,6 +351,10 @@ __device__ void strict_motion(const GridDesc &g, S &acc, double q, double radius
   bool still_r = fabs(radius_new - radius_old) < kMnzl;
   bool still_z = fabs(longitude_new - longitude_old) < kMnzl;
   if (still_r && still_z) return;
+  // the node pairs of the path's pieces: (i, k), (i + 1, k) of J_z or (i, k),
+  // (i, k + 1) of J_r, deposited by one loop so that one copy of it is generated
+  Pair p0{0.0, 0.0, 0, 0}, p1 = p0;
+  int np = 0;
   if (still_r) {
     // strictly axial motion (:810-887); the reference's two `+ 0.` adds to
     // J_r are no-ops and are omitted
@@ -344,22 +369,20 @@ __device__ void strict_motion(const GridDesc &g, S &acc, double q, double radius
     int res_k = k_n - k_o;
     if (res_k == 0) {
       double delta_z = longitude_new - longitude_old;
-      acc.template add<kCZ>(i_n, k_n, wl * delta_z);
-      acc.template add<kCZ>(i_n + 1, k_n, wu * delta_z);
+      p0 = Pair{wl * delta_z, wu * delta_z, i_n, k_n};
+      np = 1;
     } else if (res_k == 1) {
       double delta_z = k_n * dz - longitude_old;
-      acc.template add<kCZ>(i_n, k_n - 1, wl * delta_z);
-      acc.template add<kCZ>(i_n + 1, k_n - 1, wu * delta_z);
+      p0 = Pair{wl * delta_z, wu * delta_z, i_n, k_n - 1};
       delta_z = longitude_new - k_n * dz;
-      acc.template add<kCZ>(i_n, k_n, wl * delta_z);
-      acc.template add<kCZ>(i_n + 1, k_n, wu * delta_z);
+      p1 = Pair{wl * delta_z, wu * delta_z, i_n, k_n};
+      np = 2;
     } else if (res_k == -1) {
       double delta_z = (k_n + 1) * dz - longitude_old;
-      acc.template add<kCZ>(i_n, k_n + 1, wl * delta_z);
-      acc.template add<kCZ>(i_n + 1, k_n + 1, wu * delta_z);
+      p0 = Pair{wl * delta_z, wu * delta_z, i_n, k_n + 1};
       delta_z = longitude_new - (k_n + 1) * dz;
-      acc.template add<kCZ>(i_n, k_n, wl * delta_z);
-      acc.template add<kCZ>(i_n + 1, k_n, wu * delta_z);
+      p1 = Pair{wl * delta_z, wu * delta_z, i_n, k_n};
+      np = 2;
     }
   } else if (still_z) {
     // strictly radial motion (:890-986)
@@ -372,16 +395,15 @@ __device__ void strict_motion(const GridDesc &g, S &acc, double q, double radius
       double ssd = density_strict(q, r0, dr, dz, delta_t);
       double wj = ssd * (delta_r - r0 * r0 / (radius_old + delta_r) + r0 * r0 / radius_old +
                          dr * dr / (4. * (radius_old + delta_r)) - dr * dr / (4. * radius_old));
-      acc.template add<kCR>(i_n, k_n, wj * left_delta_z);
-      acc.template add<kCR>(i_n, k_n + 1, wj * right_delta_z);
+      p0 = Pair{wj * left_delta_z, wj * right_delta_z, i_n, k_n};
+      np = 1;
     } else if (res_i == 1) {
       double delta_r = (i_n)*dr - radius_old;
       double r0 = (i_n - 0.5) * dr;
       double ssd = density_strict(q, r0, dr, dz, delta_t);
       double wj = ssd * (delta_r - r0 * r0 / (radius_old + delta_r) + r0 * r0 / radius_old +
                          dr * dr / (4. * (radius_old + delta_r)) - dr * dr / (4. * radius_old));
-      acc.template add<kCR>(i_n - 1, k_n, wj * left_delta_z);
-      acc.template add<kCR>(i_n - 1, k_n + 1, wj * right_delta_z);
+      p0 = Pair{wj * left_delta_z, wj * right_delta_z, i_n - 1, k_n};
       delta_r = radius_new - i_n * dr;
       r0 = (i_n + 0.5) * dr;
       ssd = density_strict(q, r0, dr, dz, delta_t);
@@ -389,16 +411,15 @@ __device__ void strict_motion(const GridDesc &g, S &acc, double q, double radius
       const double slip = g.strict_fix ? r0 * r0 / (i_n * dr) : r0 * r0 / i_n * dr;
       wj = ssd * (delta_r - r0 * r0 / (i_n * dr + delta_r) + slip +
                   dr * dr / (4. * (i_n * dr + delta_r)) - dr * dr / (4. * i_n * dr));
-      acc.template add<kCR>(i_n, k_n, wj * left_delta_z);
-      acc.template add<kCR>(i_n, k_n + 1, wj * right_delta_z);
+      p1 = Pair{wj * left_delta_z, wj * right_delta_z, i_n, k_n};
+      np = 2;
     } else if (res_i == -1) {
       double delta_r = (i_n + 1) * dr - radius_old;
       double r0 = (i_n + 1.5) * dr;
       double ssd = density_strict(q, r0, dr, dz, delta_t);
       double wj = ssd * (delta_r - r0 * r0 / (radius_old + delta_r) + r0 * r0 / radius_old +
                          dr * dr / (4. * (radius_old + delta_r)) - dr * dr / (4. * radius_old));
-      acc.template add<kCR>(i_n + 1, k_n, wj * left_delta_z);
-      acc.template add<kCR>(i_n + 1, k_n + 1, wj * right_delta_z);
+      p0 = Pair{wj * left_delta_z, wj * right_delta_z, i_n + 1, k_n};
       delta_r = radius_new - (i_n + 1) * dr;
       r0 = (i_n + 0.5) * dr;
       ssd = density_strict(q, r0, dr, dz, delta_t);
@@ -406,9 +427,17 @@ __device__ void strict_motion(const GridDesc &g, S &acc, double q, double radius
       const double slip1 = g.strict_fix ? r0 * r0 / ((i_n + 1) * dr) : r0 * r0 / (i_n + 1) * dr;
       wj = ssd * (delta_r - r0 * r0 / ((i_n + 1) * dr + delta_r) + slip1 +
                   dr * dr / (4. * ((i_n + 1) * dr + delta_r)) - dr * dr / (4. * (i_n + 1) * dr));
-      acc.template add<kCR>(i_n, k_n, wj * left_delta_z);
-      acc.template add<kCR>(i_n, k_n + 1, wj * right_delta_z);
+      p1 = Pair{wj * left_delta_z, wj * right_delta_z, i_n, k_n};
+      np = 2;
     }
+  }
+#pragma nounroll
+  for (int t = 0; t < np; t++) {
+    const Pair p = t == 0 ? p0 : p1;
+    if (still_r)
+      acc.template add2<kCZ>(p.i, p.k, p.a, p.b);
+    else
+      acc.template add2<kCR>(p.i, p.k, p.a, p.b);
   }
 }
 
@@ -605,8 +634,9 @@ __device__ bool push_half(const GridDesc &g, const Fields &f, int pusher, int *e
     return false;
   }
   double e[3], h[3];
-  gather_e(g, f, r, z, e, err);
-  gather_h(g, f, r, z, h, err);
+  const GatherW gw = gather_weights(g, r, z, err);
+  gather_e(g, f, gw, e);
+  gather_h(g, f, gw, h);
   bool ok = (pusher == 1) ? vay(q, m, g.dt, e, h, v) : boris(q, m, g.dt, e, h, v);
   if (!ok) {
     atomicOr(err, kErrSuperluminal);
@@ -676,16 +706,17 @@ __device__ __forceinline__ void step_particle(const GridDesc &g, const Fields &f
   if (!alive) s.alive[i] = 0;
 }
 
-// chunked plasma species: 4 wavefronts per block on one tile (TileMap), PPT
-// particles per lane, deposits through the tile sink; with the divisions taken from shared reciprocals (div_cr) the compiler's own
-// choice, 227 VGPRs (PPT > 1) at 2 waves per SIMD without spills, is the fastest: 25.9 ms
-// at cfg3 against 26.7 ms for the IEEE divisions at 3 waves (168 VGPRs, 12
-// spilled); forcing 3 waves with div_cr spills 146 VGPRs (43 ms)
-template <int PPT>
+// chunked plasma species: one particle per lane, a block on 256 consecutive
+// logical particles (TileMap), deposits through the tile's box.  The kernel is
+// bound by FP64 instructions (about 1500 a particle, of which 17 divisions, 7
+// square roots and 2 logarithms).  At 128 VGPRs four waves per SIMD run: 6318 us
+// for 1.0e8 particles at 50 per cell, 1302 us for 2.1e7 at 40.  Lanes that walk
+// 16 or 8 particles each and sum a cell's deposits in registers need 167 VGPRs
+// (three waves: 6968 and 1470 us).
 __device__ __forceinline__ void fused_tile(const GridDesc &g, const Fields &f, const GlobalSink &gs,
                                            const SpeciesArgs &s, long long n_cap, int pusher, long long tile,
                                            double *box) {
-  using Map = TileMap<PPT, kWavesPerBlock>;
+  using Map = TileMap<1, kWavesPerBlock>;
   const long long base = Map::base(tile);
   // anchor samples: slot base + j is the logical particle 16 j of the tile
   int ai, ak;
@@ -700,40 +731,33 @@ __device__ __forceinline__ void fused_tile(const GridDesc &g, const Fields &f, c
     }
     tile_anchor(live, ri, kk, ai, ak);
   }
-  TileSink sk;
-  box_init(box, ai, ak, TileSink::kK, sk, gs);
+  TileSinkOne sk;
+  box_init(box, ai, ak, TileSinkOne::kK, sk, gs);
   __syncthreads();
-  const long long first = base + Map::first(threadIdx.x);
-  for (int j = 0; j < PPT; j++) {
-    long long p = first + (long long)j * 64;
-    if (p < n_cap) step_particle(g, f, sk, gs.err, s, pusher, false, p);
-  }
-  sk.flush();
+  const long long p = base + Map::first(threadIdx.x);
+  if (p < n_cap) step_particle(g, f, sk, gs.err, s, pusher, false, p);
   __syncthreads();
   box_flush(box, sk);
 }
 
-template <int PPT>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_cap, int pusher) {
-  __shared__ double box[TileSink::kSize];
-  fused_tile<PPT>(g, f, gs, s, n_cap, pusher, blockIdx.x, box);
+  __shared__ double box[TileSinkOne::kSize];
+  fused_tile(g, f, gs, s, n_cap, pusher, blockIdx.x, box);
 }
 
-// bunches (plain layout): the tiled walk with the box anchored at the
-// smallest living cell of the block; PPT particles per lane (wave w of a
-// block takes the 64 * PPT slots from w * 64 * PPT), few for a small bunch so
-// that its blocks still spread over the GPU
+// bunches (plain layout): the same with the box anchored at the smallest
+// living cell of the block, PPT particles per lane (the lanes of a wave on
+// neighbouring slots): a bunch's block covers many cells, and the adding of its
+// box to the grid is shared by more particles where there are enough of them
 template <int PPT>
 __device__ __forceinline__ void fused_bunch(const GridDesc &g, const Fields &f, const GlobalSink &gs,
                                             const SpeciesArgs &s, long long n_cap, int pusher, long long block,
                                             double *box) {
-  const long long base = block * (kWavesPerBlock * 64 * PPT);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const long long cbase = base + (long long)wave * (64 * PPT) + lane;
+  const long long first = block * (kWavesPerBlock * 64 * PPT) + threadIdx.x;
   int ai = 0x7fffffff, ak = 0x7fffffff;
   for (int j = 0; j < PPT; j++) {
-    long long p = cbase + (long long)j * 64;
+    const long long p = first + j * (kWavesPerBlock * 64);
     if (p < n_cap && s.alive[p] == 1) {
       ai = min(ai, max(0, cell_r(g, s.r[p])));
       ak = min(ak, max(0, cell_z(g, s.z[p])));
@@ -741,22 +765,22 @@ __device__ __forceinline__ void fused_bunch(const GridDesc &g, const Fields &f, 
   }
   block_min2(ai, ak);
   if (ai == 0x7fffffff) return;
-  BunchSink sk;
-  box_init(box, ai, ak, BunchSink::kK, sk, gs);
+  BunchSinkOne sk;
+  box_init(box, ai, ak, BunchSinkOne::kK, sk, gs);
   __syncthreads();
+#pragma nounroll
   for (int j = 0; j < PPT; j++) {
-    long long p = cbase + (long long)j * 64;
+    const long long p = first + j * (kWavesPerBlock * 64);
     if (p < n_cap) step_particle(g, f, sk, gs.err, s, pusher, true, p);
   }
-  sk.flush();
   __syncthreads();
   box_flush(box, sk);
 }
 
 template <int PPT>
-__global__ void __launch_bounds__(256) k_fused_bunch(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s,
-                                                     long long n_cap, int pusher) {
-  __shared__ double box[BunchSink::kSize];
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+k_fused_bunch(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_cap, int pusher) {
+  __shared__ double box[BunchSinkOne::kSize];
   fused_bunch<PPT>(g, f, gs, s, n_cap, pusher, blockIdx.x, box);
 }
 
@@ -778,8 +802,8 @@ struct SpeciesArgsG {
 struct F64Group {
   SpeciesArgsG a[kMaxGroup];
 };
-__global__ void __launch_bounds__(256) k_fused_group(GridDesc g, Fields f, GlobalSink gs, F64Group grp, int pusher) {
-  __shared__ double box[BunchSink::kSize > TileSink::kSize ? BunchSink::kSize : TileSink::kSize];
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_fused_group(GridDesc g, Fields f, GlobalSink gs, F64Group grp, int pusher) {
+  __shared__ double box[BunchSinkOne::kSize > TileSinkOne::kSize ? BunchSinkOne::kSize : TileSinkOne::kSize];
   int t = 0;
 #pragma unroll
   for (int j = 1; j < kMaxGroup; j++) t += (int)blockIdx.x >= grp.a[j].first ? 1 : 0;
@@ -799,7 +823,7 @@ __global__ void __launch_bounds__(256) k_fused_group(GridDesc g, Fields f, Globa
   if (a.is_bunch)
     fused_bunch<1>(g, f, gs, s, a.n_cap, pusher, block, box);
   else
-    fused_tile<1>(g, f, gs, s, a.n_cap, pusher, block, box);
+    fused_tile(g, f, gs, s, a.n_cap, pusher, block, box);
 }
 
 // plain layout, one particle per thread, deposits straight to HBM
@@ -905,10 +929,11 @@ __global__ void k_gather(GridDesc g, Fields f, int which, const double *r, const
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   double v[3];
+  const GatherW gw = gather_weights(g, r[i], z[i], err);
   if (which == 0)
-    gather_e(g, f, r[i], z[i], v, err);
+    gather_e(g, f, gw, v);
   else
-    gather_h(g, f, r[i], z[i], v, err);
+    gather_h(g, f, gw, v);
   out[3 * i + 0] = v[0];
   out[3 * i + 1] = v[1];
   out[3 * i + 2] = v[2];
@@ -963,47 +988,20 @@ unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
 
 }  // namespace
 
-template <int PPT>
-void launch_tile64(Ctx &c, Species &sp) {
-  constexpr long long kTile = TileMap<PPT, kWavesPerBlock>::kParticles;
-  hipLaunchKernelGGL(k_fused_tiled<PPT>, dim3((unsigned)((sp.n_cap + kTile - 1) / kTile)), dim3(256), 0, c.stream, c.g,
-                     fields_of(c), sink_of(c), args_of(sp), sp.n_cap, c.pusher);
-}
-
-// Particles per lane by the size of the species.  Without a walk the kernel
-// needs 156 VGPRs (three waves per SIMD) and fills the GPU from the fewest
-// particles; a walk's hoisted constants and register sums bring it to 227 (two
-// waves), but it adds to LDS only when a lane changes cell, which wins once
-// every lane has many particles.  Kernel times in us, 16, 8, 4, 2, 1 per lane:
-//   1.6e5 particles, 10 per cell: 106   60   35   27   22
-//   2.6e6 particles, 20 per cell: 236  189  184  195  181
-//   1.0e7 particles, 20 per cell: 796  719  749  809  752
-//   1.0e8 particles, 100 per cell: 6448 6681 7118 7866 7288
-constexpr long long kOneEach = 8000000, kEightEach = 16000000;
-
 void launch_fused_f64(Ctx &c, Species &sp) {
   if (sp.n_cap <= 0) return;
-  if (sp.chunked) {
-    if (sp.n_cap < kOneEach)
-      launch_tile64<1>(c, sp);
-    else if (sp.n_cap < kEightEach)
-      launch_tile64<8>(c, sp);
-    else
-      launch_tile64<16>(c, sp);
-  } else {
-    // the most particles per lane that still give 1024 blocks
-    const long long n = sp.n_cap, per = (long long)kWavesPerBlock * 64;
-    if (n >= 1024 * per * kPPT)
-      hipLaunchKernelGGL(k_fused_bunch<kPPT>, dim3((unsigned)((n + per * kPPT - 1) / (per * kPPT))), dim3(256), 0,
-                         c.stream, c.g, fields_of(c), sink_of(c), args_of(sp), n, c.pusher);
-    else if (n >= 1024 * per * 4)
-      hipLaunchKernelGGL(k_fused_bunch<4>, dim3((unsigned)((n + per * 4 - 1) / (per * 4))), dim3(256), 0, c.stream,
-                         c.g, fields_of(c), sink_of(c), args_of(sp), n, c.pusher);
-    else
-      hipLaunchKernelGGL(k_fused_bunch<1>, dim3((unsigned)((n + per - 1) / per)), dim3(256), 0, c.stream, c.g,
-                         fields_of(c), sink_of(c), args_of(sp), n, c.pusher);
-  }
+  // a bunch: the most particles per lane that still give 1024 blocks
+  const long long n = sp.n_cap, per = (long long)kWavesPerBlock * 64;
+  const int ppt = sp.chunked || n < 1024 * per * 4 ? 1 : n < 1024 * per * 16 ? 4 : 16;
+  auto kernel = sp.chunked ? k_fused_tiled : ppt == 1 ? k_fused_bunch<1> : ppt == 4 ? k_fused_bunch<4> : k_fused_bunch<16>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)((n + per * ppt - 1) / (per * ppt))), dim3(256), 0, c.stream, c.g,
+                     fields_of(c), sink_of(c), args_of(sp), n, c.pusher);
 }
+
+// species that take longer than a launch's latency many times over have
+// launches of their own (the group's kernel holds both paths and spills a few
+// registers)
+constexpr long long kGroupBelow = 8000000, kGroupBunchBelow = 1048576;
 
 bool launch_group_f64(Ctx &c) {
   F64Group g;
@@ -1015,7 +1013,7 @@ bool launch_group_f64(Ctx &c) {
       Species &sp = c.species[j];
       if (sp.n_cap <= 0 || (sp.kind == 1) != (kind == 1)) continue;
       constexpr long long kPer = kWavesPerBlock * 64;
-      if (n == kMaxGroup || sp.n_cap >= (sp.chunked ? kOneEach : 1024 * kPer * 4)) return false;
+      if (n == kMaxGroup || sp.n_cap >= (sp.chunked ? kGroupBelow : kGroupBunchBelow)) return false;
       const SpeciesArgs s = args_of(sp);
       SpeciesArgsG &a = g.a[n++];
       a.r = (gptr<double>)s.r;

@@ -38,10 +38,6 @@ struct GlobalSink {
     else
       atomicOr(err, kErrDomain);
   }
-  template <int C>
-  __device__ __forceinline__ void add(int i, int k, double v) {
-    put(C, i, k, v);
-  }
   // a pair of nodes: (i, k), (i+1, k) for J_z; (i, k), (i, k+1) for J_r
   template <int C>
   __device__ __forceinline__ void add2(int i, int k, double v0, double v1) {
@@ -67,7 +63,10 @@ struct GlobalSink {
 // 128 columns (a sorted block covers a run of cells along one row), the bunch
 // box 16 rows by 32 columns (a bunch block is a thin disc of particles
 // injected in the same step)
-template <bool RHO, int BR = 4, int BK = 128>
+// ACC: the first level; without it (lanes that hold one particle) every
+// contribution goes to the box at once: 8 LDS atomics where the registers'
+// stencil takes 12, and no setting up of the registers
+template <bool RHO, int BR = 4, int BK = 128, bool ACC = true>
 struct TileSinkT {
   static constexpr int kComps = RHO ? 4 : 3;  // rho only where it is deposited
   static constexpr int kR = BR, kK = BK, kSize = kComps * BR * BK;
@@ -82,47 +81,39 @@ struct TileSinkT {
   double z0, z1;              // J_z at (ic, kc), (ic+1, kc)
   double x0, x1;              // J_r at (ic, kc), (ic, kc+1)
 
-  __device__ __forceinline__ void box_put(int comp, int i, int k, double v) {
-    int li = i - bi, lk = k - bk;
-    if ((unsigned)li < (unsigned)BR && (unsigned)lk < (unsigned)bw)
-      atomicAdd(box + (comp * BR + li) * BK + lk, v);
-    else
-      g.put(comp, i, k, v);
+  // whole stencils at once: one bounds check and atomics at fixed offsets; the
+  // nodes of one that leaves the box go to HBM, in a loop (one copy of put)
+  template <int C>
+  __device__ __forceinline__ void box_put2(int i, int k, double v0, double v1) {
+    const int li = i - bi, lk = k - bk;
+    if ((unsigned)li < (unsigned)(BR - (C == kCZ)) && (unsigned)lk < (unsigned)(bw - (C != kCZ))) {
+      double *q = box + (C * BR + li) * BK + lk;
+      atomicAdd(q, v0);
+      atomicAdd(q + (C == kCZ ? BK : 1), v1);
+      return;
+    }
+#pragma nounroll
+    for (int n = 0; n < 2; n++) g.put(C, i + (C == kCZ ? n : 0), k + (C == kCZ ? 0 : n), n ? v1 : v0);
   }
   template <int C>
-  __device__ __forceinline__ void add(int i, int k, double v) {
-    const int di = i - ic, dk = k - kc;
-    if (C == kCPhi || (C == kCRho && RHO)) {
-      if ((unsigned)di < 2u && (unsigned)dk < 2u) {
-        const double a00 = (di == 0 && dk == 0) ? v : 0.0, a10 = (di == 1 && dk == 0) ? v : 0.0;
-        const double a01 = (di == 0 && dk == 1) ? v : 0.0, a11 = (di == 1 && dk == 1) ? v : 0.0;
-        if (C == kCPhi) {
-          p00 += a00; p10 += a10; p01 += a01; p11 += a11;
-        } else {
-          r00 += a00; r10 += a10; r01 += a01; r11 += a11;
-        }
-        return;
-      }
-    } else if (C == kCZ) {
-      if (dk == 0 && (unsigned)di < 2u) {
-        z0 += di == 0 ? v : 0.0;
-        z1 += di == 1 ? v : 0.0;
-        return;
-      }
-    } else if (C == kCR) {
-      if (di == 0 && (unsigned)dk < 2u) {
-        x0 += dk == 0 ? v : 0.0;
-        x1 += dk == 1 ? v : 0.0;
-        return;
-      }
+  __device__ __forceinline__ void box_put4(int i, int k, double v00, double v10, double v01, double v11) {
+    const int li = i - bi, lk = k - bk;
+    if ((unsigned)li < (unsigned)(BR - 1) && (unsigned)lk < (unsigned)(bw - 1)) {
+      double *q = box + (C * BR + li) * BK + lk;
+      atomicAdd(q, v00);
+      atomicAdd(q + BK, v10);
+      atomicAdd(q + 1, v01);
+      atomicAdd(q + BK + 1, v11);
+      return;
     }
-    box_put(C, i, k, v);
+#pragma nounroll
+    for (int n = 0; n < 4; n++) g.put(C, i + (n & 1), k + (n >> 1), n < 2 ? (n ? v10 : v00) : (n == 2 ? v01 : v11));
   }
   // whole stencils: straight into the accumulators when they are centred on
   // the accumulator's cell (the common case: no select chains), else the box
   template <int C>
   __device__ __forceinline__ void add2(int i, int k, double v0, double v1) {
-    if (i == ic && k == kc) {
+    if (ACC && i == ic && k == kc) {
       if (C == kCZ) {
         z0 += v0;
         z1 += v1;
@@ -132,15 +123,11 @@ struct TileSinkT {
       }
       return;
     }
-    box_put(C, i, k, v0);
-    if (C == kCZ)
-      box_put(C, i + 1, k, v1);
-    else
-      box_put(C, i, k + 1, v1);
+    box_put2<C>(i, k, v0, v1);
   }
   template <int C>
   __device__ __forceinline__ void add4(int i, int k, double v00, double v10, double v01, double v11) {
-    if (i == ic && k == kc && (C == kCPhi || RHO)) {
+    if (ACC && i == ic && k == kc && (C == kCPhi || RHO)) {
       if (C == kCPhi) {
         p00 += v00; p10 += v10; p01 += v01; p11 += v11;
       } else {
@@ -148,10 +135,7 @@ struct TileSinkT {
       }
       return;
     }
-    box_put(C, i, k, v00);
-    box_put(C, i + 1, k, v10);
-    box_put(C, i, k + 1, v01);
-    box_put(C, i + 1, k + 1, v11);
+    box_put4<C>(i, k, v00, v10, v01, v11);
   }
   __device__ __forceinline__ void put_nz(int comp, int i, int k, double v) {
     if (v != 0.0) g.put(comp, i, k, v);
@@ -161,7 +145,7 @@ struct TileSinkT {
   // from one address (zeros included: cheaper than testing each value);
   // otherwise node by node to HBM
   __device__ __forceinline__ void flush() {
-    if (ic < 0) return;
+    if (!ACC || ic < 0) return;
     const int li = ic - bi, lk = kc - bk;
     if ((unsigned)li < (unsigned)(BR - 1) && (unsigned)lk < (unsigned)(bw - 1)) {
       double *q = box + li * BK + lk;
@@ -202,7 +186,7 @@ struct TileSinkT {
   }
   // the next particle's contributions are centred on cell (i, k)
   __device__ __forceinline__ void begin_cell(int i, int k) {
-    if (i != ic || k != kc) {
+    if (ACC && (i != ic || k != kc)) {
       flush();
       ic = i;
       kc = k;
@@ -211,6 +195,8 @@ struct TileSinkT {
 };
 using TileSink = TileSinkT<false>;  // plasma species: no rho
 using BunchSink = TileSinkT<true, 16, 32>;
+using TileSinkOne = TileSinkT<false, 4, 128, false>;  // one particle per lane
+using BunchSinkOne = TileSinkT<true, 16, 32, false>;
 
 // One grid's node deposits of a tile (charge weighting outside the loop, the
 // density probe): the four corners of the lane's current cell in registers, an
@@ -245,18 +231,6 @@ struct NodeSink {
       atomicAdd(box + li * kK + lk, v);
     else
       grid_put(i, k, v);
-  }
-  template <int C>
-  __device__ __forceinline__ void add(int i, int k, double v) {
-    const int di = i - ic, dk = k - kc;
-    if ((unsigned)di < 2u && (unsigned)dk < 2u) {
-      r00 += (di == 0 && dk == 0) ? v : 0.0;
-      r10 += (di == 1 && dk == 0) ? v : 0.0;
-      r01 += (di == 0 && dk == 1) ? v : 0.0;
-      r11 += (di == 1 && dk == 1) ? v : 0.0;
-      return;
-    }
-    put(i, k, v);
   }
   template <int C>
   __device__ __forceinline__ void add4(int i, int k, double v00, double v10, double v01, double v11) {
