@@ -435,17 +435,17 @@ int pdp3_ctx_create(int n_grid_r, int n_grid_z, double r_size, double z_size, do
     const double dr = c.g.dr, dz = c.g.dz;
     // and, behind them, the divisors of density_r(i dr) (i = 0: of the axis
     // cell's term, src/particles.cpp:389) and density_z((i + 1/2) dr)
-    // (include/particles.h:169-178)
+    // (include/particles.h:169-178), from i = -1
     const int rows = n_grid_r + 2;
-    std::vector<double2> vol((size_t)3 * rows);
-    for (int i = 0; i < rows; i++) {
-      const double v = kPi * dz * dr * dr * 2.0 * i;
+    std::vector<double2> vol((size_t)3 * rows + 1);
+    for (int i = -1; i < rows; i++) {
+      const double r0 = (i + 0.5) * dr, dens_z = 2 * kPi * r0 * dr * dz * delta_t * dz;
+      vol[2 * rows + 1 + i] = make_double2(dens_z, 1.0 / dens_z);
+      if (i < 0) continue;
+      const double v = kPi * dz * dr * dr * 2.0 * i, r = i * dr;
       vol[i] = make_double2(v, i ? 1.0 / v : 0.0);
-      const double r = i * dr, r0 = (i + 0.5) * dr;
       const double dens_r = i ? 2 * kPi * r * dr * dz * delta_t * 2 * dr : 2. * kPi * dr / 4. * dr * dz * delta_t * dr;
-      const double dens_z = 2 * kPi * r0 * dr * dz * delta_t * dz;
       vol[rows + i] = make_double2(dens_r, 1.0 / dens_r);
-      vol[2 * rows + i] = make_double2(dens_z, 1.0 / dens_z);
     }
     c.g.inv_dr = 1.0 / dr;
     c.g.inv_dz = 1.0 / dz;

@@ -37,8 +37,10 @@ __device__ __forceinline__ int cell_z(const GridDesc &g, double x) { return (int
 struct Vol {
   double v, inv;
 };
+// (the row of a particle outside the grid, whose deposits are refused node by
+// node, is kept inside the table)
 __device__ __forceinline__ Vol vol_cell(const GridDesc &g, int i) {
-  const double2 t = g.vol[i];
+  const double2 t = g.vol[min(i, g.nr + 1)];
   return Vol{t.x, t.y};
 }
 __device__ __forceinline__ Vol vol_cyl(const GridDesc &g) { return Vol{g.cyl, g.inv_cyl}; }
@@ -275,13 +277,13 @@ __device__ __forceinline__ double density_strict(double q, double r, double dr, 
   return q / (kPi * 4. * r * dz * dz * dr * dt);
 }
 // density_r(i dr) (i = 0: of the axis cell's own term) and density_z((i + 1/2) dr)
-// by the context's table of their divisors
+// (i = -1: below the axis) by the context's table of their divisors
 __device__ __forceinline__ double density_r(const GridDesc &g, double q, int i) {
-  const double2 t = g.vol[(g.nr + 2) + i];
+  const double2 t = g.vol[(g.nr + 2) + min(i, g.nr + 1)];
   return div_cr(q, t.x, t.y);
 }
 __device__ __forceinline__ double density_z(const GridDesc &g, double q, int i) {
-  const double2 t = g.vol[2 * (g.nr + 2) + i];
+  const double2 t = g.vol[2 * (g.nr + 2) + 1 + min(i, g.nr + 1)];
   return div_cr(q, t.x, t.y);
 }
 
