@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "context.hpp"
+#include "crmath.hpp"
 #include "sink.hpp"
 
 namespace pdp3 {
@@ -116,11 +117,23 @@ struct AdjGrid {
   const double *ljr, *ljphi, *ljz;             // adjoint of J^n
   double *ler, *lephi, *lez, *lhr, *lhphi, *lhz;  // adjoint of E^n, Hh^n (scatter, atomics)
 };
+// what a species' charge, mass and the grid's constants come to: the scales of
+// the push's E and H (q / m does not depend on the weight), and of the deposits
+// of one charge into J_z, J_r and J_phi
+struct StepScales {
+  double es, bs, kz, kr, kj;
+};
+StepScales scales_of(const GridDesc &g, double q, double m, bool vay) {
+  const double c1 = q * g.dt / (2 * m);
+  return StepScales{vay ? 2 * c1 : c1, vay ? kMagnConst * c1 * (2 * c1) * c1 : kMagnConst * c1,
+                    q / (4.0 * kPi * g.dr * g.dr * g.dt), q / (2.0 * kPi * g.dr * g.dz * g.dt), q / (2.0 * g.dz * g.dr)};
+}
 struct AdjSpecies {
   StateRef st;                          // state at step n
   double *lr, *lz, *lvr, *lvphi, *lvz;  // in: adjoint of the state after step n; out: before
   double *lw;                           // accumulated adjoint of the weight
-  double charge, mass;
+  double charge;
+  StepScales k;
   long long n;                          // slots
 };
 
@@ -166,7 +179,8 @@ __device__ __forceinline__ long long adj_slot() {
 // was in that order do not move it, as they would the smallest cell); (0, 0)
 // where none of the nine lives.  After 2400 steps without a sort 2.6e5 particles
 // at 8 per cell took the tangent step 231 us around the smallest cell in four
-// rows, 101 us around the median in six (76 and 69 us where they lie in order).
+// rows, 101 us around the median in six (76 and 69 us where they lie in order,
+// all with IEEE divisions).
 __device__ __forceinline__ void block_median(int &i, int &k, bool live) {
   constexpr int kN = 9, kEvery = 28;
   __shared__ unsigned long long cell[kN], med;
@@ -209,9 +223,21 @@ __device__ __forceinline__ void block_anchor(int &i, int &k, bool live) {
   }
 }
 
-__device__ __forceinline__ int cell_number(double x, double dx) { return (int)ceil(x / dx) - 1; }
-__device__ __forceinline__ double cell_volume(int i, double dr, double dz) { return kPi * dz * dr * dr * 2.0 * i; }
-__device__ __forceinline__ double cyl_vol(double z, double r) { return kPi * z * r * r / 4.; }
+// quotients by the context's constants and row volumes take their reciprocals
+// from the context (div_cr: correctly rounded, as the IEEE division): a quotient
+// is five FP64 operations instead of eleven and a quarter-rate reciprocal, and the
+// particle steps, bound by FP64 instructions at two waves per SIMD (211 VGPRs; three
+// spill 40 and take 290 us), had about fifty of them: reverse step of 2.6e6
+// particles 238 us with the IEEE quotients, 213 us
+__device__ __forceinline__ double per_dr(const GridDesc &g, double x) { return div_cr(x, g.dr, g.inv_dr); }
+__device__ __forceinline__ double per_dz(const GridDesc &g, double x) { return div_cr(x, g.dz, g.inv_dz); }
+__device__ __forceinline__ double per_c2(double x) { return div_cr(x, kC2, 1.0 / kC2); }
+__device__ __forceinline__ int cell_r(const GridDesc &g, double r) { return (int)ceil(per_dr(g, r)) - 1; }
+__device__ __forceinline__ int cell_z(const GridDesc &g, double z) { return (int)ceil(per_dz(g, z)) - 1; }
+// {volume, 1 / volume} of row i's cells (a row outside the grid is kept inside
+// the table; it receives and holds nothing), and of the axis cell
+__device__ __forceinline__ double2 vol_row(const GridDesc &g, int i) { return g.vol[min(i, g.nr + 1)]; }
+__device__ __forceinline__ double2 vol_axis(const GridDesc &g) { return make_double2(g.cyl, g.inv_cyl); }
 
 constexpr int kAR = 0, kAPhi = 1, kAZ = 2;
 
@@ -220,8 +246,8 @@ template <class S>
 __device__ void strict_d(const GridDesc &g, S &acc, D q, D radius_new, D longitude_new, D radius_old,
                          D longitude_old) {
   const double dr = g.dr, dz = g.dz, delta_t = g.dt;
-  int i_n = cell_number(radius_new.v, dr), k_n = cell_number(longitude_new.v, dz);
-  int i_o = cell_number(radius_old.v, dr), k_o = cell_number(longitude_old.v, dz);
+  int i_n = cell_r(g, radius_new.v), k_n = cell_z(g, longitude_new.v);
+  int i_o = cell_r(g, radius_old.v), k_o = cell_z(g, longitude_old.v);
   if (i_n < 0) i_n = 0;
   if (k_n < 0) k_n = 0;
   if (i_o < 0) i_o = 0;
@@ -326,19 +352,19 @@ struct Boost {
 __device__ __forceinline__ Boost boost_of(V3 v) {
   Boost b;
   b.u = V3{fabs(v.x) < kMnzl ? 0.0 : v.x, fabs(v.y) < kMnzl ? 0.0 : v.y, fabs(v.z) < kMnzl ? 0.0 : v.z};
-  b.g0 = 1.0 / sqrt(1.0 - dot(b.u, b.u) / kC2);
+  b.g0 = rsqrt_near(1.0 - per_c2(dot(b.u, b.u)));
   return b;
 }
 // adjoint of v from the adjoint of U = g0 u
 __device__ __forceinline__ V3 boost_back(const Boost &b, V3 v, V3 lU) {
-  const double s = b.g0 * b.g0 * b.g0 / kC2 * dot(lU, b.u);
+  const double s = per_c2(b.g0 * b.g0 * b.g0) * dot(lU, b.u);
   const V3 l = fma3(s, b.u, b.g0 * lU);
   return V3{fabs(v.x) < kMnzl ? 0.0 : l.x, fabs(v.y) < kMnzl ? 0.0 : l.y, fabs(v.z) < kMnzl ? 0.0 : l.z};
 }
-__device__ __forceinline__ double inv_gamma(V3 u) { return 1.0 / sqrt(1.0 + dot(u, u) / kC2); }
+__device__ __forceinline__ double inv_gamma(V3 u) { return rsqrt_near(1.0 + per_c2(dot(u, u))); }
 // adjoint of u added for an adjoint lg of g = inv_gamma(u)
 __device__ __forceinline__ V3 inv_gamma_back(double g, V3 u, double lg, V3 l) {
-  return fma3(-(g * g * g) / kC2 * lg, u, l);
+  return fma3(per_c2(-(g * g * g)) * lg, u, l);
 }
 
 // what the reverse sweep of a push keeps of its forward evaluation, recomputed
@@ -386,8 +412,8 @@ __device__ __forceinline__ V3 vay_fwd(V3 v, V3 e, V3 h) {
   const Boost b0 = boost_of(v);
   const V3 t = b0.g0 * b0.u;
   const V3 up = fma3(inv_gamma(t), cross(t, h), t + e);
-  const double B2 = dot(h, h), ub = dot(up, h), sg = 1.0 + dot(up, up) / kC2 - B2;
-  const double al = 1.0 / sqrt(0.5 * (sg + sqrt(sg * sg + 4. * (B2 + ub * ub))));
+  const double B2 = dot(h, h), ub = dot(up, h), sg = 1.0 + per_c2(dot(up, up)) - B2;
+  const double al = rsqrt_near(0.5 * (sg + sqrt(sg * sg + 4. * (B2 + ub * ub))));
   const V3 b = al * h;
   const V3 u = (1.0 / (1.0 + dot(b, b))) * (fma3(dot(up, b), b, up) + cross(up, b));
   return inv_gamma(u) * u;
@@ -398,9 +424,9 @@ __device__ __forceinline__ PushBack vay_back(V3 v, V3 e, V3 h, V3 lv) {
   const double g1 = inv_gamma(t);
   const V3 th = cross(t, h);
   const V3 up = fma3(g1, th, t + e);
-  const double B2 = dot(h, h), ub = dot(up, h), sg = 1.0 + dot(up, up) / kC2 - B2;
+  const double B2 = dot(h, h), ub = dot(up, h), sg = 1.0 + per_c2(dot(up, up)) - B2;
   const double root = sqrt(sg * sg + 4. * (B2 + ub * ub));
-  const double al = 1.0 / sqrt(0.5 * (sg + root));
+  const double al = rsqrt_near(0.5 * (sg + root));
   const V3 b = al * h;
   const double s = 1.0 / (1.0 + dot(b, b)), al2 = dot(up, b);
   const V3 q = fma3(al2, b, up) + cross(up, b);
@@ -437,9 +463,10 @@ struct RingW {
 };
 __device__ __forceinline__ RingW ring_lo(const GridDesc &g, double r) {
   RingW w;
-  w.ir = min(max(cell_number(r - 0.5 * g.dr, g.dr), 0), g.nr - 2);
+  w.ir = min(max(cell_r(g, r - 0.5 * g.dr), 0), g.nr - 2);
   const double r1 = r - 0.5 * g.dr, r3 = r + 0.5 * g.dr, r2 = (w.ir + 1) * g.dr;
-  const double p1 = kPi / cell_volume(w.ir + 1, g.dr, g.dz), p2 = kPi / cell_volume(w.ir + 3, g.dr, g.dz);
+  const double2 v1 = vol_row(g, w.ir + 1), v2 = vol_row(g, w.ir + 3);
+  const double p1 = div_cr(kPi, v1.x, v1.y), p2 = div_cr(kPi, v2.x, v2.y);
   w.in = p1 * (r2 * r2 - r1 * r1);
   w.out = p2 * (r3 * r3 - r2 * r2);
   w.din = -2.0 * p1 * r1;
@@ -448,10 +475,10 @@ __device__ __forceinline__ RingW ring_lo(const GridDesc &g, double r) {
 }
 __device__ __forceinline__ RingW ring_own(const GridDesc &g, double r) {
   RingW w;
-  w.ir = min(max(cell_number(r, g.dr), 0), g.nr - 2);
+  w.ir = min(max(cell_r(g, r), 0), g.nr - 2);
   const double r1 = r - 0.5 * g.dr, r3 = r + 0.5 * g.dr, r2 = (w.ir + 0.5) * g.dr;
-  const double p1 = kPi / ((r > g.dr) ? cell_volume(w.ir, g.dr, g.dz) : cyl_vol(g.dz, g.dr));
-  const double p2 = kPi / cell_volume(w.ir + 2, g.dr, g.dz);
+  const double2 v1 = (r > g.dr) ? vol_row(g, w.ir) : vol_axis(g), v2 = vol_row(g, w.ir + 2);
+  const double p1 = div_cr(kPi, v1.x, v1.y), p2 = div_cr(kPi, v2.x, v2.y);
   w.in = p1 * (r2 * r2 - r1 * r1);
   w.out = p2 * (r3 * r3 - r2 * r2);
   w.din = -2.0 * p1 * r1;
@@ -464,7 +491,7 @@ struct ColW {
 };
 __device__ __forceinline__ ColW col_w(const GridDesc &g, double z, bool half) {
   ColW c;
-  c.kz = min(max(cell_number(half ? z - 0.5 * g.dz : z, g.dz), 0), g.nz - 2);
+  c.kz = min(max(cell_z(g, half ? z - 0.5 * g.dz : z), 0), g.nz - 2);
   const double z0 = (half ? c.kz + 0.5 : c.kz) * g.dz;
   c.d1 = z0 + g.dz - z;
   c.d2 = z - z0;
@@ -528,19 +555,19 @@ __device__ __forceinline__ double lam_at(const GridDesc &g, const double *L, int
 // reverse of the J_phi deposit (azimuthal_current_distribution,
 // src/particles.cpp:688-784) of w charges q: adds to the adjoints of r, z,
 // v_phi; returns the weight's, sum lambda_J J / w
-__device__ __forceinline__ double jphi_back(const GridDesc &g, const double *L, double q, double w, double r, double z,
+__device__ __forceinline__ double jphi_back(const GridDesc &g, const double *L, double kj, double w, double r, double z,
                                             double vphi, double &lr, double &lz, double &lvphi) {
   const double dr = g.dr, dz = g.dz;
-  const int i = max(cell_number(r, dr), 0), k = max(cell_number(z, dz), 0);
+  const int i = max(cell_r(g, r), 0), k = max(cell_z(g, z), 0);
   const double r1 = r - 0.5 * dr, r2 = (i + 0.5) * dr, r3 = r + 0.5 * dr;
-  const double i1 = 1.0 / ((r > dr) ? cell_volume(i, dr, dz) : cyl_vol(dz, dr)), i2 = 1.0 / cell_volume(i + 1, dr, dz);
+  const double i1 = (r > dr) ? vol_row(g, i).y : g.inv_cyl, i2 = vol_row(g, i + 1).y;
   const double d1 = (k + 0.5) * dz - (z - 0.5 * dz), d2 = (z + 0.5 * dz) - (k + 0.5) * dz;
   const double l00 = lam_at(g, L, i, k) * i1, l10 = lam_at(g, L, i + 1, k) * i2;
   const double l01 = lam_at(g, L, i, k + 1) * i1, l11 = lam_at(g, L, i + 1, k + 1) * i2;
   const double in = r2 * r2 - r1 * r1, out = r3 * r3 - r2 * r2;
   const double lo = l00 * d1 + l01 * d2, hi = l10 * d1 + l11 * d2;
   const double G = in * lo + out * hi;
-  const double ir = 1.0 / r, K = q * ir / (2. * dz * dr);
+  const double ir = 1.0 / r, K = kj * ir;
   lvphi += w * K * G;
   lr += w * K * vphi * (2.0 * (r3 * hi - r1 * lo) - G * ir);
   lz += w * K * vphi * (in * (l01 - l00) + out * (l11 - l10));
@@ -581,17 +608,17 @@ __device__ __forceinline__ void m_and_slope(double x, double &M, double &dM) {
 struct PieceAdj {
   double s, rn, zn, ro, zo;
 };
-__device__ __forceinline__ PieceAdj segment_back(const GridDesc &g, const AdjGrid &lg, double q, double rn, double zn,
+__device__ __forceinline__ PieceAdj segment_back(const GridDesc &g, const AdjGrid &lg, const StepScales &s, double rn, double zn,
                                                  double ro, double zo, int i, int k) {
   const double dr = g.dr, dz = g.dz;
   PieceAdj o{0.0, 0.0, 0.0, 0.0, 0.0};
   if ((fabs(rn - ro) < kMnzl) || (fabs(zn - zo) < kMnzl)) return o;
-  const double fi = (double)i, idr = 1.0 / dr, idz = 1.0 / dz;
-  const double a = ro / dr - fi, b = zo / dz - (double)k, drho = (rn - ro) / dr, dzeta = (zn - zo) / dz;
-  const double kz = q / (4.0 * kPi * dr * dr * g.dt), kr = q / (2.0 * kPi * dr * dz * g.dt);
+  const double fi = (double)i;
+  const double a = per_dr(g, ro) - fi, b = per_dz(g, zo) - (double)k;
+  const double drho = per_dr(g, rn - ro), dzeta = per_dz(g, zn - zo);
   // lambda_J times the scales of the pairs (without the dzeta of J_z)
-  double gz0 = kz * lam_at(g, lg.ljz, i, k), gz1 = kz * lam_at(g, lg.ljz, i + 1, k);
-  double gr0 = kr * lam_at(g, lg.ljr, i, k), gr1 = kr * lam_at(g, lg.ljr, i, k + 1);
+  double gz0 = s.kz * lam_at(g, lg.ljz, i, k), gz1 = s.kz * lam_at(g, lg.ljz, i + 1, k);
+  double gr0 = s.kr * lam_at(g, lg.ljr, i, k), gr1 = s.kr * lam_at(g, lg.ljr, i, k + 1);
   const double hdr = 0.5 * drho, ub = 1.0 - b, qdz = 0.25 * dzeta;
   double sa, sb, sdr, sdz;
   if (i == 0) {
@@ -633,10 +660,10 @@ __device__ __forceinline__ PieceAdj segment_back(const GridDesc &g, const AdjGri
          sx * x * irs - st * t * ire;
     sdr = 0.5 * dzeta * (gz1 - gz0) + grp + sx * irs + st * rs * ire * ire;
   }
-  o.rn = sdr * idr;
-  o.ro = (sa - sdr) * idr;
-  o.zn = sdz * idz;
-  o.zo = (sb - sdz) * idz;
+  o.rn = sdr * g.inv_dr;
+  o.ro = (sa - sdr) * g.inv_dr;
+  o.zn = sdz * g.inv_dz;
+  o.zo = (sb - sdz) * g.inv_dz;
   return o;
 }
 
@@ -669,8 +696,8 @@ struct Path {
 __device__ __forceinline__ Path split_path(const GridDesc &g, double rn, double zn, double ro, double zo) {
   const double dr = g.dr, dz = g.dz;
   Path p;
-  int i_n = max(cell_number(rn, dr), 0), k_n = max(cell_number(zn, dz), 0);
-  int i_o = max(cell_number(ro, dr), 0), k_o = max(cell_number(zo, dz), 0);
+  int i_n = max(cell_r(g, rn), 0), k_n = max(cell_z(g, zn), 0);
+  int i_o = max(cell_r(g, ro), 0), k_o = max(cell_z(g, zo), 0);
   if (ro == (i_o + 1) * dr) i_o = i_n;
   if (zo == (k_o + 1) * dz) k_o = k_n;
   if (rn == (i_n + 1) * dr) i_n = i_o;
@@ -729,7 +756,7 @@ __device__ __forceinline__ Path split_path(const GridDesc &g, double rn, double 
 // radial face r = rb (met at z1) and the axial face z = zb (met at r2) that it
 // crosses; with s the path parameter of the crossing, the adjoint of z1 goes
 // to the ends as (1-s, s) along z and times -dz/dr along r, that of r2 likewise
-__device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjGrid &lg, double q, double rn, double zn,
+__device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjGrid &lg, const StepScales &k, double q, double rn, double zn,
                                                    double ro, double zo) {
   const Path c = split_path(g, rn, zn, ro, zo);
   if (c.strict) {
@@ -748,7 +775,7 @@ __device__ __forceinline__ PieceAdj deposit_j_back(const GridDesc &g, const AdjG
 #pragma nounroll
   for (int t = 0; t < ns; t++) {
     const bool first = t == 0, last = t == ns - 1;
-    const PieceAdj p = segment_back(g, lg, q, last ? rn : first ? cr0 : cr1, last ? zn : first ? cz0 : cz1,
+    const PieceAdj p = segment_back(g, lg, k, last ? rn : first ? cr0 : cr1, last ? zn : first ? cz0 : cz1,
                                     first ? ro : t == 1 ? cr0 : cr1, first ? zo : t == 1 ? cz0 : cz1,
                                     last ? c.i_n : first ? c.i0 : c.i1, last ? c.k_n : first ? c.k0 : c.k1);
     o.s += p.s;
@@ -826,9 +853,7 @@ __device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields 
   const double r0 = pt.r, z0 = pt.z, w = pt.w;
   const V3 v0 = {pt.vr, pt.vphi, pt.vz};
   const double half_dt = g.dt / 2.;
-  // the scales of the push's fields: q / m does not depend on w
-  const double c1 = s.charge * g.dt / (2 * s.mass);
-  const double es = VAY ? 2 * c1 : c1, bs = VAY ? kMagnConst * c1 * (2 * c1) * c1 : kMagnConst * c1;
+  const double es = s.k.es, bs = s.k.bs;
   V3 e, h;
   {
     const RingW wl = ring_lo(g, r0), wo = ring_own(g, r0);
@@ -852,7 +877,7 @@ __device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields 
     const double vx = sx * v.x;  // after the walls
     // rotation of the velocity by the second half step's angle
     const double lst = vx * o1 - v.y * o0 - st / ct * (vx * o0 + v.y * o1);
-    const PieceAdj p = deposit_j_back(g, lg, s.charge, r2, z2, r0, z0);
+    const PieceAdj p = deposit_j_back(g, lg, s.k, s.charge, r2, z2, r0, z0);
     lw += p.s;
     lr0 = w * p.ro;
     lz0 = w * p.zo;
@@ -864,7 +889,7 @@ __device__ __forceinline__ void adj_particle(const GridDesc &g, const AdjFields 
     lv.y = ct * o1 - st * o0 + half_dt * ly2;
     lv.z = sz * o2 + half_dt * lz1;
   }
-  lw += jphi_back(g, lg.ljphi, s.charge, w, r1, z1, v.y, lr1, lz1, lv.y);
+  lw += jphi_back(g, lg.ljphi, s.k.kj, w, r1, z1, v.y, lr1, lz1, lv.y);
   const double ir1 = 1.0 / r1, lx1 = lr1 * x1 * ir1;
   lr0 += lx1;
   lz0 += lz1;
@@ -907,8 +932,8 @@ __global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, 
   const bool live = i < s.n && adj_load<F32>(g, s.st, i, pt);
   int ci = INT_MAX, ck = INT_MAX;
   if (live) {
-    ci = max(cell_number(pt.r, g.dr), 0);
-    ck = max(cell_number(pt.z, g.dz), 0);
+    ci = max(cell_r(g, pt.r), 0);
+    ck = max(cell_z(g, pt.z), 0);
   }
   for (int t = threadIdx.x; t < kSize; t += blockDim.x) box[t] = 0.0;
   block_anchor<BUNCH, Box::kR, kABK>(ci, ck, live);
@@ -940,7 +965,7 @@ __global__ void __launch_bounds__(256) k_adj_particles(GridDesc g, AdjFields f, 
 // along dw to round-off (the dot-product test).  Re-executing the step in dual
 // numbers of four directions took 256 + 66 registers, 736 bytes of scratch and a
 // division per direction at every quotient: 184 us for 2.6e5 plasma particles
-// and 55 us for 8e3 of a bunch; this form takes 76 and 37 us.
+// and 55 us for 8e3 of a bunch; this form takes 63 and 33 us.
 struct TlmFields {  // tangents of E^n and Hh^n, one set per direction
   const double *er[kDN], *ephi[kDN], *ez[kDN], *hhr[kDN], *hhphi[kDN], *hhz[kDN];
 };
@@ -951,7 +976,8 @@ struct TlmSpecies {
   StateRef st;                          // state at step n (values)
   double *tr, *tz, *tvr, *tvphi, *tvz;  // kDN x n tangents: in at step n, out at n+1
   const double *tw;                     // kDN x n tangents of the weight
-  double charge, mass;
+  double charge;
+  StepScales k;
   long long n;                          // slots
 };
 
@@ -1005,11 +1031,11 @@ __device__ __forceinline__ BoostT boost_t(V3 v) {
 }
 __device__ __forceinline__ V3 along(const BoostT &t, V3 dv) {
   const V3 du = V3{t.x ? dv.x : 0.0, t.y ? dv.y : 0.0, t.z ? dv.z : 0.0};
-  return fma3(t.b.g0 * t.b.g0 * t.b.g0 / kC2 * dot(t.b.u, du), t.b.u, t.b.g0 * du);
+  return fma3(per_c2(t.b.g0 * t.b.g0 * t.b.g0) * dot(t.b.u, du), t.b.u, t.b.g0 * du);
 }
 // tangent of inv_gamma(u) u, g = inv_gamma(u)
 __device__ __forceinline__ V3 slow_t(double g, V3 u, V3 du) {
-  return fma3(-(g * g * g) / kC2 * dot(u, du), u, g * du);
+  return fma3(per_c2(-(g * g * g)) * dot(u, du), u, g * du);
 }
 struct BorisT {
   BoostT b0;
@@ -1028,7 +1054,7 @@ struct BorisT {
   __device__ __forceinline__ V3 v() const { return g2 * u; }
   __device__ __forceinline__ V3 along_dir(V3 dv, V3 de, V3 dh) const {
     const V3 dt = along(b0, dv) + de;
-    const V3 db = fma3(-(g1 * g1 * g1) / kC2 * dot(t, dt), h, g1 * dh);
+    const V3 db = fma3(per_c2(-(g1 * g1 * g1)) * dot(t, dt), h, g1 * dh);
     const V3 dtp = dt + cross(dt, b) + cross(t, db);
     const V3 dw = cross(dtp, b) + cross(tp, db);
     const V3 du = fma3(-c2 * c2 * dot(b, db), w, fma3(c2, dw, dt + de));
@@ -1046,9 +1072,9 @@ struct VayT {
     up = fma3(g1, th, t + e);
     const double B2 = dot(h, h);
     ub = dot(up, h);
-    sg = 1.0 + dot(up, up) / kC2 - B2;
+    sg = 1.0 + per_c2(dot(up, up)) - B2;
     root = sqrt(sg * sg + 4. * (B2 + ub * ub));
-    al = 1.0 / sqrt(0.5 * (sg + root));
+    al = rsqrt_near(0.5 * (sg + root));
     b = al * h;
     s = 1.0 / (1.0 + dot(b, b));
     al2 = dot(up, b);
@@ -1060,7 +1086,7 @@ struct VayT {
   __device__ __forceinline__ V3 along_dir(V3 dv, V3 de, V3 dh) const {
     const V3 dt = along(b0, dv);
     const V3 dth = cross(dt, h) + cross(t, dh);
-    const V3 dup = fma3(-(g1 * g1 * g1) / kC2 * dot(t, dt), th, fma3(g1, dth, dt + de));
+    const V3 dup = fma3(per_c2(-(g1 * g1 * g1)) * dot(t, dt), th, fma3(g1, dth, dt + de));
     const double dB2 = 2.0 * dot(h, dh), dub = dot(dup, h) + dot(up, dh);
     const double dsg = 2.0 / kC2 * dot(up, dup) - dB2;
     const double droot = (sg * dsg + 2.0 * dB2 + 4.0 * ub * dub) / root;
@@ -1074,16 +1100,16 @@ struct VayT {
 // tangents of the J_phi deposit (azimuthal_current_distribution,
 // src/particles.cpp:688-784) of w charges q
 template <class Sink>
-__device__ __forceinline__ void jphi_tangent(const GridDesc &g, Sink &sk, double q, double w, double r, double z,
+__device__ __forceinline__ void jphi_tangent(const GridDesc &g, Sink &sk, double kj, double w, double r, double z,
                                              double vphi, const double (&tw)[kDN], const double (&tr)[kDN],
                                              const double (&tz)[kDN], const double (&tv)[kDN]) {
   const double dr = g.dr, dz = g.dz;
-  const int i = max(cell_number(r, dr), 0), k = max(cell_number(z, dz), 0);
+  const int i = max(cell_r(g, r), 0), k = max(cell_z(g, z), 0);
   const double r1 = r - 0.5 * dr, r2 = (i + 0.5) * dr, r3 = r + 0.5 * dr;
-  const double i1 = 1.0 / ((r > dr) ? cell_volume(i, dr, dz) : cyl_vol(dz, dr)), i2 = 1.0 / cell_volume(i + 1, dr, dz);
+  const double i1 = (r > dr) ? vol_row(g, i).y : g.inv_cyl, i2 = vol_row(g, i + 1).y;
   const double d1 = (k + 0.5) * dz - (z - 0.5 * dz), d2 = (z + 0.5 * dz) - (k + 0.5) * dz;
   const double in = (r2 * r2 - r1 * r1) * i1, out = (r3 * r3 - r2 * r2) * i2;
-  const double ir = 1.0 / r, K = q * ir / (2. * dz * dr), P = w * K * vphi;
+  const double ir = 1.0 / r, K = kj * ir, P = w * K * vphi;
   const double din = P * (-2.0 * r1 * i1), dout = P * (2.0 * r3 * i2);
   const int n00 = sk.node(i, k), n10 = sk.node(i + 1, k), n01 = sk.node(i, k + 1), n11 = sk.node(i + 1, k + 1);
 #pragma unroll
@@ -1121,9 +1147,9 @@ struct StrictTangent {
 // tangents of the J_r / J_z deposit of w charges q on the path (ro, zo) -> (rn,
 // zn), piece by piece (the closed forms above segment_back)
 template <class Sink>
-__device__ __forceinline__ void deposit_j_tangent(const GridDesc &g, Sink &sk, double q, double w, double rn, double zn,
+__device__ __forceinline__ void deposit_j_tangent(const GridDesc &g, Sink &sk, const StepScales &sc, double q, double w, double rn, double zn,
                                                   double ro, double zo, const PathT &t) {
-  const double dr = g.dr, dz = g.dz, idr = 1.0 / dr, idz = 1.0 / dz;
+  const double idr = g.inv_dr, idz = g.inv_dz;
   const Path c = split_path(g, rn, zn, ro, zo);
   if (c.strict) {
     const PathT own = t;  // t itself stays in registers
@@ -1131,7 +1157,7 @@ __device__ __forceinline__ void deposit_j_tangent(const GridDesc &g, Sink &sk, d
     strict_d(g, st, cst(q), seed(rn, 0), seed(zn, 1), seed(ro, 2), seed(zo, 3));
     return;
   }
-  const double kz = q / (4.0 * kPi * dr * dr * g.dt), kr = q / (2.0 * kPi * dr * dz * g.dt);
+  const double kz = sc.kz, kr = sc.kr;
   // path parameters of the crossings
   const double sr = c.rad ? (c.rb - ro) / (rn - ro) : 0.0, sz = c.axi ? (c.zb - zo) / (zn - zo) : 0.0;
   const double isl = c.rad ? 1.0 / c.slope : 0.0;
@@ -1146,7 +1172,8 @@ __device__ __forceinline__ void deposit_j_tangent(const GridDesc &g, Sink &sk, d
     const int i = last ? c.i_n : first ? c.i0 : c.i1, k = last ? c.k_n : first ? c.k0 : c.k1;
     if ((fabs(prn - pro) < kMnzl) || (fabs(pzn - pzo) < kMnzl)) continue;
     const double fi = (double)i;
-    const double a = pro / dr - fi, b = pzo / dz - (double)k, drho = (prn - pro) / dr, dzeta = (pzn - pzo) / dz;
+    const double a = per_dr(g, pro) - fi, b = per_dz(g, pzo) - (double)k;
+    const double drho = per_dr(g, prn - pro), dzeta = per_dz(g, pzn - pzo);
     const double hdr = 0.5 * drho, ub = 1.0 - b, qdz = 0.25 * dzeta, p0 = 0.5 * ub - qdz, p1 = 0.5 * b + qdz;
     // J_z = kz w dzeta (z0, z1), J_r = kr w (j0, j1); along a direction, with
     // the tangents (ta, tb, tdr, tdz) of (a, b, drho, dzeta):
@@ -1226,12 +1253,9 @@ __device__ __forceinline__ void deposit_j_tangent(const GridDesc &g, Sink &sk, d
 template <class Push, bool BUNCH, class Sink>
 __device__ __forceinline__ void tlm_particle(const GridDesc &g, const AdjFields &f, const TlmFields &tf, Sink &sk,
                                              const TlmSpecies &s, long long i, const AdjParticle &pt) {
-  constexpr bool kVay = std::is_same<Push, VayT>::value;
   const long long n = s.n;
   const double r0 = pt.r, z0 = pt.z, w = pt.w, half_dt = g.dt / 2.;
-  // the scales of the push's fields: q / m does not depend on w
-  const double c1 = s.charge * g.dt / (2 * s.mass);
-  const double es = kVay ? 2 * c1 : c1, bs = kVay ? kMagnConst * c1 * (2 * c1) * c1 : kMagnConst * c1;
+  const double es = s.k.es, bs = s.k.bs;
   const RingW wl = ring_lo(g, r0), wo = ring_own(g, r0);
   const ColW co = col_w(g, z0, false), ch = col_w(g, z0, true);
   const Gathered e0 = gather_grad(g, f.er, wl, co), e1 = gather_grad(g, f.ephi, wo, co);
@@ -1279,8 +1303,8 @@ __device__ __forceinline__ void tlm_particle(const GridDesc &g, const AdjFields 
     s.tvz[p] = alive ? sz * dv.z : 0.0;
     __builtin_amdgcn_sched_barrier(0);  // one direction's registers at a time
   }
-  jphi_tangent(g, sk, s.charge, w, r1, z1, v.y, t.w, tr1, tz1, tvp);
-  if (alive) deposit_j_tangent(g, sk, s.charge, w, r2, z2, r0, z0, t);
+  jphi_tangent(g, sk, s.k.kj, w, r1, z1, v.y, t.w, tr1, tz1, tvp);
+  if (alive) deposit_j_tangent(g, sk, s.k, s.charge, w, r2, z2, r0, z0, t);
 }
 #pragma clang fp contract(off)
 
@@ -1293,8 +1317,8 @@ __global__ void __launch_bounds__(256) k_tlm_particles(GridDesc g, AdjFields f, 
   const bool live = i < s.n && adj_load<F32>(g, s.st, i, pt);
   int ci = INT_MAX, ck = INT_MAX;
   if (live) {
-    ci = max(cell_number(pt.r, g.dr), 0);
-    ck = max(cell_number(pt.z, g.dz), 0);
+    ci = max(cell_r(g, pt.r), 0);
+    ck = max(cell_z(g, pt.z), 0);
   }
   for (int t = threadIdx.x; t < Sink::kSize; t += blockDim.x) box[t] = 0.0;
   block_anchor<BUNCH, Sink::kR, Sink::kK>(ci, ck, live);
@@ -1524,7 +1548,7 @@ void launch_adj_particles(const GridDesc &g, const double *const *fields6, doubl
   if (n <= 0) return;
   AdjFields f{fields6[0], fields6[1], fields6[2], fields6[3], fields6[4], fields6[5]};
   AdjGrid lg{lam[9], lam[10], lam[11], scaled[0], scaled[1], scaled[2], lam[6], lam[7], lam[8]};
-  AdjSpecies s{state, lstate[0], lstate[1], lstate[2], lstate[3], lstate[4], lw, charge, mass, n};
+  AdjSpecies s{state, lstate[0], lstate[1], lstate[2], lstate[3], lstate[4], lw, charge, scales_of(g, charge, mass, pusher == 1), n};
   const dim3 grid((unsigned)((n + 255) / 256));
   using K = void (*)(GridDesc, AdjFields, AdjGrid, AdjSpecies);
   static const K kernels[8] = {k_adj_particles<false, false, false>, k_adj_particles<true, false, false>,
@@ -1559,7 +1583,7 @@ void launch_tlm_particles(const GridDesc &g, const double *const *fields6, doubl
     tj.jphi[d] = a[kJPhi];
     tj.jz[d] = a[kJZ];
   }
-  TlmSpecies s{state, tstate[0], tstate[1], tstate[2], tstate[3], tstate[4], tw, charge, mass, n};
+  TlmSpecies s{state, tstate[0], tstate[1], tstate[2], tstate[3], tstate[4], tw, charge, scales_of(g, charge, mass, pusher == 1), n};
   const dim3 grid((unsigned)((n + 255) / 256));
   using K = void (*)(GridDesc, AdjFields, TlmFields, TlmJ, TlmSpecies);
   static const K kernels[8] = {k_tlm_particles<false, false, false>, k_tlm_particles<true, false, false>,

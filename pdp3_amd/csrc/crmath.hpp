@@ -27,13 +27,17 @@ __device__ __forceinline__ double rsqrt_residual(double x, double c) {
   return (t - qe) - x * pe;
 }
 
-// 1/sqrt(x), correctly rounded except in exact-tie cases, for x > 0 finite: two
-// Newton steps from the hardware's estimate leave y within an ulp, and of its
-// neighbours only the one that its residual points to can be nearer
-__device__ __forceinline__ double rsqrt_cr(double x) {
+// 1/sqrt(x) within an ulp, for x > 0 finite: two Newton steps from the hardware's
+// estimate
+__device__ __forceinline__ double rsqrt_near(double x) {
   double y = __builtin_amdgcn_rsq(x);
   y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-  y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
+  return fma(0.5 * y, fma(-x * y, y, 1.0), y);
+}
+// correctly rounded except in exact-tie cases: of y's neighbours only the one
+// that its residual points to can be nearer
+__device__ __forceinline__ double rsqrt_cr(double x) {
+  const double y = rsqrt_near(x);
   const double r = rsqrt_residual(x, y);
   const double c = __longlong_as_double(__double_as_longlong(y) + (r < 0.0 ? -1 : 1));
   return fabs(rsqrt_residual(x, c)) < fabs(r) ? c : y;
