@@ -86,6 +86,7 @@ template <int PPT, int WAVES>
 struct TileMap {
   static constexpr int kParticles = WAVES * 64 * PPT;
   static constexpr bool kWhole = kParticles >= kChunk;
+  static constexpr bool kShort = PPT <= 2;  // a lane's walk is too short to share anything over it
   static constexpr int kGroup = kWhole ? 64 : kParticles / kPPT;
   // slots from the tile's first one that its threads may reach
   static constexpr int kSpan = kWhole ? kParticles : kChunk;
@@ -111,6 +112,7 @@ struct TileMap {
 // kernel then serves tiles of every size in one launch
 template <int WAVES>
 struct TileMapRt {
+  static constexpr bool kShort = false;
   int lg;
   __device__ __forceinline__ int ppt() const { return 1 << lg; }
   __device__ __forceinline__ int particles() const { return (WAVES * 64) << lg; }

@@ -19,6 +19,8 @@
 #include <cstring>
 #include <vector>
 
+#include <type_traits>
+
 #include "context.hpp"
 #include "sink.hpp"
 
@@ -169,7 +171,11 @@ __device__ __forceinline__ void row_entries(int i, float4 &t0, float4 &t1) {
   t1 = make_float4(i ? (float)(1.0 / fi) : 0.f, (float)(1.0 / (fi + 1)), (float)(1.0 / (fi + 0.5)), (float)(fi * (fi + 1)));
 }
 
-struct GlobalFields {
+// (HZ: H_z in the order of the box's)
+template <bool HZ>
+struct GlobalFieldsT {
+  __device__ __forceinline__ GlobalFieldsT() {}
+  __device__ __forceinline__ GlobalFieldsT(const float *, int, int, int) {}
   // the two table entries of row i (clamped only for memory safety: a corrupt
   // cell word is caught by the gathers' domain check)
   __device__ __forceinline__ void row(const F32Args &p, int i, float4 &t0, float4 &t1) const {
@@ -184,9 +190,11 @@ struct GlobalFields {
     e[2] = gather(p, field(p, kEZ), p.escale, ro, zh);
     h[0] = gather(p, field(p, kHHR), p.bscale, ro, zh);
     h[1] = gather(p, field(p, kHHPhi), p.bscale, rl, zh);
-    h[2] = gather(p, field(p, kHHZ), p.bscale, rl, zo);
+    h[2] = gather<HZ>(p, field(p, kHHZ), p.bscale, rl, zo);
   }
 };
+using GlobalFields = GlobalFieldsT<false>;
+using TileGlobalFields = GlobalFieldsT<true>;
 
 // rows bi..bi+kFR-1, columns bk..bk+width-1 of the six components, anchored
 // two rows and two columns below the tile's anchor cell (ai, ak): a particle
@@ -216,6 +224,7 @@ struct BoxFields {
   const float *box;  // LDS
   int ai, ak;        // anchor cell of the tile
   int width;         // columns filled
+  __device__ __forceinline__ BoxFields(const float *b, int i, int k, int w) : box(b), ai(i), ak(k), width(w) {}
   // the box's row entries (an LDS read for every particle), replaced by the
   // entries evaluated in place for a row outside the box.  A global load here
   // would make the read a flat load, whose wait also waits for the next
@@ -722,7 +731,11 @@ __device__ __forceinline__ F32Args from_slot(const F32Args &p, long long base) {
 template <int WAVES, class Map>
 __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink &gs, const Map &map, long long base,
                                              long long n_cap, double *box, float *fbox) {
-  using Sink = TileSink;
+  // one or two particles per lane: no register sums and no field box, whose
+  // filling (15 to 30 loads a lane and a barrier) takes longer than the
+  // particles' 24 loads each from L2
+  using Sink = typename std::conditional<Map::kShort, TileSinkOne, TileSink>::type;
+  using Fields = typename std::conditional<Map::kShort, TileGlobalFields, BoxFields>::type;
   static_assert(kFK == Sink::kK, "the two boxes share their width");
   const F32Args q = from_slot(p, base);
   const unsigned lim = (unsigned)min(n_cap - base, (long long)map.span());
@@ -752,9 +765,9 @@ __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink 
   const int width = narrow ? kFK / 2 : kFK;
   Sink sk;
   box_init(box, ai, ak, width, sk, gs);
-  field_box_fill<WAVES>(p, fbox, ai, ak, width);
+  if (!Map::kShort) field_box_fill<WAVES>(p, fbox, ai, ak, width);
   __syncthreads();
-  const BoxFields fs{fbox, ai, ak, width};
+  const Fields fs(fbox, ai, ak, width);
   // software pipeline: the state of the lane's next particle is loaded before
   // the current one is pushed; all its loads are waited for before the
   // current particle's stores, so the wait never includes stores in flight
@@ -797,7 +810,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
 // one block of a bunch (plain layout): WAVES chunks of kChunk slots from
 // `base`; the register / LDS sink is anchored at the smallest cell of the
 // block's living particles (a bunch block is a thin disc injected in one step)
-template <int WAVES, int PPT>
+template <int WAVES, int PPT, class Fields = GlobalFields>
 __device__ __forceinline__ void fused32_bunch_tile(const F32Args &p, const GlobalSink &gs, long long base,
                                                    long long n_cap, double *box) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -815,15 +828,18 @@ __device__ __forceinline__ void fused32_bunch_tile(const F32Args &p, const Globa
   }
   block_min2(ai, ak);
   if (ai == 0x7fffffff) return;  // no living particle in the block (uniform over the block)
-  BunchSink sk;
-  box_init(box, ai, ak, BunchSink::kK, sk, gs);
+  // (neighbouring slots of a bunch are not in one cell: register sums help
+  // only where a lane walks several)
+  using Sink = typename std::conditional<PPT == 1, BunchSinkOne, BunchSink>::type;
+  Sink sk;
+  box_init(box, ai, ak, Sink::kK, sk, gs);
   __syncthreads();
   const F32Args q = from_slot(p, base);
   const unsigned lim = (unsigned)min(n_cap - base, (long long)WAVES * 64 * PPT);
   const unsigned off0 = (unsigned)(wave * 64 * PPT + lane);
   for (int j = 0; j < PPT; j++) {
     const unsigned n = off0 + (unsigned)j * 64u;
-    if (n < lim) step_particle32(q, sk, GlobalFields(), n);
+    if (n < lim) step_particle32(q, sk, Fields(), n);
   }
   sk.flush();
   __syncthreads();
@@ -979,7 +995,7 @@ k_ens_fused32(const F32Args *__restrict__ args, const GlobalSink *__restrict__ s
   g.err = a.err;
   if (item.lg < 0) {
     a.is_bunch = a.want_rho = 1;
-    fused32_bunch_tile<WAVES, 1>(a, g, item.base, item.n_cap, lds);
+    fused32_bunch_tile<WAVES, 1, TileGlobalFields>(a, g, item.base, item.n_cap, lds);
   } else {
     a.is_bunch = a.want_rho = 0;
     fused32_tile<WAVES>(a, g, TileMapRt<WAVES>{item.lg}, item.base, item.n_cap, lds,
@@ -1228,26 +1244,33 @@ void launch_tile(int tile, hipStream_t st, const F32Args &p, const GlobalSink &g
 }
 
 // the shape for a species of a context whose shape was neither set nor
-// autotuned: the largest that covers at most kFK - 8 cells of a sorted species
-// (its boxes then serve all of its particles) and still fills the GPU; a
-// species without either runs on 256-particle tiles.  A shape of 4 or 8
-// particles per lane and more needs two full rounds or more of blocks (five
-// blocks on each of 256 CUs) to be worth its longer walk.  Kernel times in us,
-// shapes 16x4, 8x4, 4x4, 2x4, 1x4:
-//   1.6e5 particles, 10 per cell:  56.4   34.9   22.7   17.3   15.0
-//   9.8e5 particles, 30 per cell:  55.6   37.8   30.2   30.0   41.6
-//   1.3e6 particles, 10 per cell:  73.6   51.6   34.7   37.4   48.5
-//   2.6e6 particles, 20 per cell:  79.3   57.5   53.0   60.2   91.8
-//   2.1e7 particles, 40 per cell: 238    273    303    428    671
-//   2.1e8 particles, 100 per cell: 2126  2432   2866   4048   6755
+// autotuned: of the shapes with boxes the largest that covers at most kFK - 8
+// cells of a sorted species (its boxes then serve all of its particles) and has
+// enough blocks for its long walk (sixteen on each of 256 CUs, or six of 4x4);
+// smaller species run on the shapes without boxes, two particles per lane where
+// that leaves three blocks on each CU, else one.  Kernel times in us right after a
+// sort, shapes 16x4, 8x4, 4x4, 2x4, 1x4:
+//   1.6e5 particles, 10 per cell:   56     35     23     12.2   11.9
+//   1.0e6 twice, 13 per cell (Vay):  -      -     49     47      -
+//   2.6e6 particles, 20 per cell:   79     58     50     59      -
+//   2.1e7 particles, 40 per cell:  238    273    303      -      -
+//   2.1e8 particles, 100 per cell: 2126  2432   2866      -      -
+// and of the whole step 5 to 45 steps after it (500 eV: most lanes meet another
+// cell with every particle):
+//   1.6e5 particles, 10 per cell:  107      -     35     24     21
+//   6.6e5 particles, 40 per cell:  108      -     45     37     43
+//   9.8e5 particles, 15 per cell:  133      -     61     48     51
+//   2.6e6 particles, 20 per cell:  248    108    101     93     97
+//   7.9e6 particles, 30 per cell:  325    226    220    218      -
+//   2.1e7 particles, 40 per cell:  529    499    516    556    580
 int auto_tile(const Ctx &c, const Species &sp) {
   const double cells = (double)(c.g.nr - 1) * (c.g.nz - 1);
   const struct {
     int tile, particles, blocks;
-  } shapes[] = {{0, 4096, 4096}, {3, 2048, 4096}, {5, 1024, 800}, {6, 512, 400}};
+  } shapes[] = {{0, 4096, 4096}, {3, 2048, 4096}, {5, 1024, 1536}};
   for (const auto &s : shapes)
     if (sp.n >= (long long)s.particles * s.blocks && s.particles * cells <= (kFK - 8) * (double)sp.n) return s.tile;
-  return 7;
+  return sp.n >= 512 * 768 ? 6 : 7;
 }
 
 void launch_fused_f32(Ctx &c, Species &sp) {

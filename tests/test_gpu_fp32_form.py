@@ -254,8 +254,9 @@ def test_tile_shapes_agree_and_autotune():
 @pytest.mark.parametrize("cells_r,cells_z,ppc", [
     (21, 43, 3),      # 256-particle tiles, the last chunk mostly padding
     (9, 1000, 1),     # the same, tiles that overrun the field box
-    (64, 256, 16),    # 512-particle tiles
-    (128, 512, 15),   # one chunk per tile
+    (64, 256, 16),    # 256-particle tiles, whole chunks
+    (128, 512, 15),   # 512-particle tiles
+    (128, 1024, 13),  # one chunk per tile
     (256, 1024, 33),  # 2048-particle tiles, half the field box's width
     (512, 2048, 17),  # the same, its whole width
 ])
