@@ -290,7 +290,7 @@ int pdp3_adjoint_run(pdp3_ctx *ctx, int nsteps, int checkpoint_every, int window
  * PDP3_TANGENT_DIRS directions of the particle weights.  dw[j] holds species
  * j's PDP3_TANGENT_DIRS x n weight tangents, direction-major, in its logical
  * particle order (a NULL entry: zero).  The tangents are carried forward
- * through the FP64 plain form's particle step in dual numbers and through the
+ * through the derivative of the FP64 plain form's particle step and through the
  * field updates themselves, i.e. the linearisation that pdp3_adjoint_run
  * transposes (around the context's own trajectory, FP32 or FP64 form): for
  * every direction d, sum over particles of dphi_dw * dw[d] equals dphi_out[d]

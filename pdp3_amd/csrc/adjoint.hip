@@ -30,8 +30,9 @@ namespace pdp3 {
 namespace {
 
 constexpr int kDN = 4;  // directions
-static_assert(kDN == kTangentDirs, "the tangent-linear model runs one direction per dual slot");
+static_assert(kDN == kTangentDirs, "the tangent-linear model runs kDN directions");
 
+// dual numbers of kDN directions (strict_d, whose four inputs they are)
 struct D {
   double v;
   double d[kDN];

@@ -1345,7 +1345,7 @@ constexpr int kNative = 6;  // arrays of native_arrays
 // kTangentDirs directions of the particle weights; its grids are advanced by
 // the context's own (linear) field updates through shadow contexts that
 // share the geometry, PML coefficients and stream; the particle tangents by
-// the dual-number step (launch_tlm_particles) right after each H update
+// the tangent particle step (launch_tlm_particles) right after each H update
 struct TangentSweep {
   static constexpr int D = kTangentDirs;
   pdp3_ctx *ctx = nullptr;

@@ -166,7 +166,7 @@ def test_fd_converges_to_adjoint_smooth(orc):
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("pusher", [0, 1])
 def test_reverse_step_matches_tangent(pusher, precision):
-    """The reverse-mode particle step against the dual-number one, both pushers
+    """The reverse-mode particle step against the tangent one, both pushers
     and forms, on paths that reach every branch: a hot plasma that crosses
     radial and axial faces (both in one step too) and reflects at the axis and
     the walls, dead particles, an odd grid, a bunch on purely
