@@ -175,37 +175,6 @@ __device__ __forceinline__ long long adj_slot() {
   return TileMap<1, 4>::base(blockIdx.x) + TileMap<1, 4>::first(threadIdx.x);
 }
 
-// the cell that a plasma block's boxes are centred on: the median of nine of its
-// particles in the order of cells (a few that have drifted off since the species
-// was in that order do not move it, as they would the smallest cell); (0, 0)
-// where none of the nine lives.  After 2400 steps without a sort 2.6e5 particles
-// at 8 per cell took the tangent step 231 us around the smallest cell in four
-// rows, 101 us around the median in six (76 and 69 us where they lie in order,
-// all with IEEE divisions).
-__device__ __forceinline__ void block_median(int &i, int &k, bool live) {
-  constexpr int kN = 9, kEvery = 28;
-  __shared__ unsigned long long cell[kN], med;
-  if (threadIdx.x % kEvery == kEvery / 2 && threadIdx.x < kN * kEvery)
-    cell[threadIdx.x / kEvery] = live ? (unsigned long long)i << 32 | (unsigned)k : ~0ull;
-  if (threadIdx.x == 0) med = 0;
-  __syncthreads();
-  if (threadIdx.x < kN) {
-    const unsigned me = threadIdx.x;
-    const unsigned long long mine = cell[me];
-    int less = 0, all = 0;
-#pragma unroll
-    for (unsigned j = 0; j < kN; j++) {
-      const unsigned long long o = cell[j];
-      all += o != ~0ull;
-      less += o < mine || (o == mine && j < me);
-    }
-    if (mine != ~0ull && less == all / 2) med = mine;
-  }
-  __syncthreads();
-  i = (int)(med >> 32);
-  k = (int)med;
-}
-
 // node of box[.][0][0] of kR x kK nodes, from the thread's cell (INT_MAX: dead): a bunch
 // block's boxes begin one row and two columns below its smallest cell, a plasma
 // block's lie around its median cell.  (After a barrier, which the cleared box

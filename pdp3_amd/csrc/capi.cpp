@@ -1079,6 +1079,7 @@ int step_one(pdp3_ctx *ctx, const std::function<int()> *after_h) {
   }
   if (after_h && (st = (*after_h)())) return st;
   // (live timing keeps plasma and bunch launches apart)
+  for (Species &sp : c.species) sp.steps_unsorted++;
   if (!c.profiling && (is_f32(c) ? launch_group_f32(c) : launch_group_f64(c))) {
     CHECK_LAUNCH(ctx);
   } else {

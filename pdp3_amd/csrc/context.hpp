@@ -168,6 +168,7 @@ struct Species {
   long long rec_cap = 0;
   uint32_t *runs_host = nullptr;
   hipEvent_t runs_ev = nullptr;
+  long long steps_unsorted = 0;  // steps since it was created or sorted
   bool sort_prepared = false;  // the buffers of periodic sorts are allocated
   // bunch
   double *inject_u = nullptr;

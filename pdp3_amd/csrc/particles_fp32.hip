@@ -734,18 +734,21 @@ __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink 
   // one or two particles per lane: no register sums and no field box, whose
   // filling (15 to 30 loads a lane and a barrier) takes longer than the
   // particles' 24 loads each from L2
-  using Sink = typename std::conditional<Map::kShort, TileSinkOne, TileSink>::type;
+  using Sink = typename std::conditional<Map::kShort, TileSinkTall, TileSink>::type;
   using Fields = typename std::conditional<Map::kShort, TileGlobalFields, BoxFields>::type;
-  static_assert(kFK == Sink::kK, "the two boxes share their width");
   const F32Args q = from_slot(p, base);
   const unsigned lim = (unsigned)min(n_cap - base, (long long)map.span());
   const unsigned off0 = map.first(threadIdx.x);
   // the lane's first particle is on its way while the boxes are set up
   PState nx{kDead, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   if (off0 < lim) nx = load_state_next(q, off0 * 4u);
-  // anchor samples: slot base + j is the logical particle 16 j of the tile
-  int ai, ak;
-  {
+  Sink sk;
+  int ai = 0, ak = 0, width = 0;
+  if constexpr (Map::kShort) {
+    tall_init(box, cell_i(nx.c), cell_k(nx.c), !(nx.c & kDead), Map::kParticles, p.n, sk, gs);
+  } else {
+    static_assert(kFK == Sink::kK, "the two boxes share their width");
+    // anchor samples: slot base + j is the logical particle 16 j of the tile
     bool live[3];
     int ri[3], kk[3];
 #pragma unroll
@@ -756,17 +759,16 @@ __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink 
       kk[j] = cell_k(c);
     }
     tile_anchor(live, ri, kk, ai, ak);
+    // the boxes' width: half of it when the tile's last particle (the last
+    // slot its threads reach) lies within the first half of the anchor's row,
+    // with one column to spare
+    const uint32_t cl = base + map.last() < n_cap ? p.cell[base + map.last()] : kDead;
+    const bool narrow = !(cl & kDead) && cell_i(cl) == ai && cell_k(cl) - ak <= kFK / 2 - 5;
+    width = narrow ? kFK / 2 : kFK;
+    box_init(box, ai, ak, width, sk, gs);
+    field_box_fill<WAVES>(p, fbox, ai, ak, width);
+    __syncthreads();
   }
-  // the boxes' width: half of it when the tile's last particle (the last
-  // slot its threads reach) lies within the first half of the anchor's row,
-  // with one column to spare
-  const uint32_t cl = base + map.last() < n_cap ? p.cell[base + map.last()] : kDead;
-  const bool narrow = !(cl & kDead) && cell_i(cl) == ai && cell_k(cl) - ak <= kFK / 2 - 5;
-  const int width = narrow ? kFK / 2 : kFK;
-  Sink sk;
-  box_init(box, ai, ak, width, sk, gs);
-  if (!Map::kShort) field_box_fill<WAVES>(p, fbox, ai, ak, width);
-  __syncthreads();
   const Fields fs(fbox, ai, ak, width);
   // software pipeline: the state of the lane's next particle is loaded before
   // the current one is pushed; all its loads are waited for before the
@@ -788,7 +790,7 @@ __device__ __forceinline__ void fused32_tile(const F32Args &p, const GlobalSink 
 
 template <int PPT, int WAVES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_fused32_tiled(F32Args p, GlobalSink gs, long long n_cap) {
-  __shared__ double box[TileSink::kSize];
+  __shared__ double box[PPT <= 2 ? TileSinkTall::kSize : TileSink::kSize];
   __shared__ __align__(16) float fbox[kFBoxFloats];
   // launched for the chunked layout only, i.e. plasma species: no bunch walls
   // and no charge density (constants here drop their code and registers)
@@ -942,6 +944,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
   constexpr int kBunch = BunchSink::kSize, kTile = TileSink::kSize + (kFBoxFloats + 1) / 2;
   __shared__ __align__(16) double lds[kBunch > kTile ? kBunch : kTile];
   static_assert(TileSink::kSize % 2 == 0, "the field box behind the current box is 16-byte aligned");
+  static_assert(TileSinkTall::kSize <= kTile, "a small tile's box takes the place of both");
   int s = 0;
 #pragma unroll
   for (int t = 1; t < kMaxGroup; t++) s += (int)blockIdx.x >= g.first[t] ? 1 : 0;
@@ -1250,8 +1253,8 @@ void launch_tile(int tile, hipStream_t st, const F32Args &p, const GlobalSink &g
 // smaller species run on the shapes without boxes, two particles per lane where
 // that leaves three blocks on each CU, else one.  Kernel times in us right after a
 // sort, shapes 16x4, 8x4, 4x4, 2x4, 1x4:
-//   1.6e5 particles, 10 per cell:   56     35     23     12.2   11.9
-//   1.0e6 twice, 13 per cell (Vay):  -      -     49     47      -
+//   1.6e5 particles, 10 per cell:   56     35     23     12.2   10.9
+//   1.0e6 twice, 13 per cell (Vay):  -      -     49     42      -
 //   2.6e6 particles, 20 per cell:   79     58     50     59      -
 //   2.1e7 particles, 40 per cell:  238    273    303      -      -
 //   2.1e8 particles, 100 per cell: 2126  2432   2866      -      -
@@ -1263,13 +1266,20 @@ void launch_tile(int tile, hipStream_t st, const F32Args &p, const GlobalSink &g
 //   2.6e6 particles, 20 per cell:  248    108    101     93     97
 //   7.9e6 particles, 30 per cell:  325    226    220    218      -
 //   2.1e7 particles, 40 per cell:  529    499    516    556    580
+// A species that has not been sorted for kDrift steps runs on the shapes without
+// boxes whatever its size: its particles have drifted off the rows and columns
+// that the larger tiles' boxes hold (1 eV, 10-step passes: 4e6
+// particles at 20 per cell 2.0 ms in order on 4x4 and 2.2 on 2x4, 5.6 and 2.5
+// after 2000 steps; two species of 1.35e7 at 45 per cell 4.8 on 8x4 and 5.8, 14.2
+// and 6.5; the lines cross after about 400 and 800 steps).
+constexpr long long kDrift = 500;
 int auto_tile(const Ctx &c, const Species &sp) {
   const double cells = (double)(c.g.nr - 1) * (c.g.nz - 1);
   const struct {
     int tile, particles, blocks;
   } shapes[] = {{0, 4096, 4096}, {3, 2048, 4096}, {5, 1024, 1536}};
   for (const auto &s : shapes)
-    if (sp.n >= (long long)s.particles * s.blocks && s.particles * cells <= (kFK - 8) * (double)sp.n) return s.tile;
+    if (sp.steps_unsorted <= kDrift && sp.n >= (long long)s.particles * s.blocks && s.particles * cells <= (kFK - 8) * (double)sp.n) return s.tile;
   return sp.n >= 512 * 768 ? 6 : 7;
 }
 

@@ -709,7 +709,7 @@ __device__ __forceinline__ void step_particle(const GridDesc &g, const Fields &f
 }
 
 // chunked plasma species: one particle per lane, a block on 256 consecutive
-// logical particles (TileMap), deposits through the tile's box.  The kernel is
+// logical particles (TileMap), deposits through a box around their median cell.  The kernel is
 // bound by FP64 instructions (about 1500 a particle, of which 17 divisions, 7
 // square roots and 2 logarithms).  At 128 VGPRs four waves per SIMD run: 6318 us
 // for 1.0e8 particles at 50 per cell, 1302 us for 2.1e7 at 40.  Lanes that walk
@@ -720,23 +720,11 @@ __device__ __forceinline__ void fused_tile(const GridDesc &g, const Fields &f, c
                                            double *box) {
   using Map = TileMap<1, kWavesPerBlock>;
   const long long base = Map::base(tile);
-  // anchor samples: slot base + j is the logical particle 16 j of the tile
-  int ai, ak;
-  {
-    bool live[3];
-    int ri[3], kk[3];
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-      live[j] = base + j < n_cap && s.alive[base + j] == 1;
-      ri[j] = live[j] ? max(0, cell_r(g, s.r[base + j])) : 0;
-      kk[j] = live[j] ? max(0, cell_z(g, s.z[base + j])) : 0;
-    }
-    tile_anchor(live, ri, kk, ai, ak);
-  }
-  TileSinkOne sk;
-  box_init(box, ai, ak, TileSinkOne::kK, sk, gs);
-  __syncthreads();
   const long long p = base + Map::first(threadIdx.x);
+  const bool live = p < n_cap && s.alive[p] == 1;
+  TileSinkTall sk;
+  tall_init(box, live ? max(0, cell_r(g, s.r[p])) : 0, live ? max(0, cell_z(g, s.z[p])) : 0, live, Map::kParticles, n_cap,
+            sk, gs);
   if (p < n_cap) step_particle(g, f, sk, gs.err, s, pusher, false, p);
   __syncthreads();
   box_flush(box, sk);
@@ -744,7 +732,7 @@ __device__ __forceinline__ void fused_tile(const GridDesc &g, const Fields &f, c
 
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_cap, int pusher) {
-  __shared__ double box[TileSinkOne::kSize];
+  __shared__ double box[TileSinkTall::kSize];
   fused_tile(g, f, gs, s, n_cap, pusher, blockIdx.x, box);
 }
 
@@ -805,7 +793,7 @@ struct F64Group {
   SpeciesArgsG a[kMaxGroup];
 };
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_fused_group(GridDesc g, Fields f, GlobalSink gs, F64Group grp, int pusher) {
-  __shared__ double box[BunchSinkOne::kSize > TileSinkOne::kSize ? BunchSinkOne::kSize : TileSinkOne::kSize];
+  __shared__ double box[BunchSinkOne::kSize > TileSinkTall::kSize ? BunchSinkOne::kSize : TileSinkTall::kSize];
   int t = 0;
 #pragma unroll
   for (int j = 1; j < kMaxGroup; j++) t += (int)blockIdx.x >= grp.a[j].first ? 1 : 0;

@@ -730,6 +730,7 @@ int sort_species(Ctx &c, Species &sp, bool exact) {
   const SortWs ws = sort_ws(n, cap, bits);
   const long long nb = ws.nb, scratch = ws.scratch;
   if (!ensure_ws(c, ws.bytes) || !ensure_alts(c, sp)) return -3;
+  sp.steps_unsorted = 0;
   uint32_t *src = (uint32_t *)c.sort_ws, *block = src + n, *tmp = block + nb + 1;
   uint32_t *rk = tmp + scratch, *ri = rk + cap, *rk2 = ri + cap, *ri2 = rk2 + cap, *rlen = ri2 + cap;
   const uint32_t *count = block + nb;  // the number of runs, after the scan

@@ -285,3 +285,69 @@ def test_tile_chosen_by_size(cells_r, cells_z, ppc):
         sim.close()
     for n in out[0]:
         assert normwise(out[0][n], out[1][n]) <= 1e-11, (n, normwise(out[0][n], out[1][n]))
+
+
+@pytest.mark.parametrize("precision,cells_r,cells_z,n", [
+    (1, 33, 131, 20000),    # 256-particle tiles, 4 per cell: the box's whole width
+    (1, 16, 64, 30011),     # the same, half its width
+    (1, 64, 256, 393216),   # 512-particle tiles
+    (1, 200, 801, 400001),  # the same, the whole width
+    (0, 33, 131, 20000),
+    (0, 16, 64, 30011),
+])
+def test_small_tiles_of_particles_in_no_order(precision, cells_r, cells_z, n):
+    """Tiles whose particles lie anywhere on the grid (most deposits miss the
+    box), some of them dead: fields and states as with the particles in cell
+    order, up to the order of the FP64 sums (see above; states are compared
+    particle by particle after one step, whose inputs are the same)."""
+    from pdp3_amd import capi
+
+    d = 5e-4
+    rng = np.random.default_rng(n)
+    r, z = rng.uniform(d / 2, (cells_r - 0.5) * d, n), rng.uniform(d / 2, (cells_z - 0.5) * d, n)
+    v = 1e7 * rng.standard_normal((3, n))
+    w = rng.uniform(1, 2, n)
+    alive = (rng.random(n) > 0.03).astype(np.uint8)
+    out = []
+    for order in (np.arange(n), np.lexsort((np.ceil(z / d), np.ceil(r / d)))):
+        sim = capi.Simulation(cells_r + 1, cells_z + 1, cells_r * d, cells_z * d, 0.5 * d / 3e8, precision=precision)
+        sim.boundary_conditions()
+        for name in ("E_r", "E_phi", "E_z", "H_r", "H_phi", "H_z"):
+            g = np.random.default_rng(len(name)).standard_normal((cells_r + 1, cells_z + 1))
+            sim.set_field(name, (1e6 if name[0] == "E" else 2e3) * g)
+        idx = sim.add_plasma(-1, 1.0, r[order], z[order], v[0][order], v[1][order], v[2][order], w[order], alive[order])
+        sim.step(1)
+        st = sim.download(idx)
+        back = np.argsort(order)
+        out.append({k: st[k][back] for k in ("r", "z", "vr", "vphi", "vz", "alive")})
+        out[-1].update({k: sim.field(k) for k in ("J_r", "J_phi", "J_z", "E_z")})
+        sim.close()
+    for k in ("r", "z", "vr", "vphi", "vz", "alive"):
+        assert np.array_equal(out[0][k], out[1][k]), k
+    for k in ("J_r", "J_phi", "J_z", "E_z"):
+        assert normwise(out[0][k], out[1][k]) <= 1e-11, (k, normwise(out[0][k], out[1][k]))
+
+
+def test_tile_of_a_species_long_unsorted():
+    """After 500 steps without a sort a species of any size runs on the small
+    tiles.  The plasma is thin enough for its fields not to feed back: J is that
+    of the 16 x 4 shape up to the order of the FP64 sums."""
+    from pdp3_amd import capi
+
+    d, cells_r, cells_z, ppc = 5e-4, 128, 1024, 13
+    out = []
+    for shape in (None, (16, 4)):
+        sim = capi.Simulation(cells_r + 1, cells_z + 1, cells_r * d, cells_z * d, 0.5 * d / 3e8,
+                              precision=capi.PREC_FP32)
+        sim.boundary_conditions()
+        idx = sim.add_species(-1, 1.0, ppc * cells_r * cells_z)
+        sim.init_uniform(idx, 11, ppc, 1e2, 0, 1.0)
+        if shape:
+            sim.set_tile(*shape)
+        for steps in (499, 3):
+            sim.step(steps)
+            out.append({n: sim.field(n) for n in ("J_r", "J_phi", "J_z")})
+        sim.close()
+    for a, b in ((out[0], out[2]), (out[1], out[3])):
+        for n in a:
+            assert normwise(a[n], b[n]) <= 1e-11, (n, normwise(a[n], b[n]))
