@@ -1525,7 +1525,7 @@ void launch_adj_particles(const GridDesc &g, const double *const *fields6, doubl
                                k_adj_particles<false, true, false>,  k_adj_particles<true, true, false>,
                                k_adj_particles<false, false, true>,  k_adj_particles<true, false, true>,
                                k_adj_particles<false, true, true>,   k_adj_particles<true, true, true>};
-  hipLaunchKernelGGL(kernels[(pusher == 1) + 2 * (is_bunch != 0) + 4 * (state.cell != nullptr)], grid, dim3(256), 0, st,
+  hipLaunchKernelGGL(kernels[(pusher == 1) + 2 * (is_bunch != 0) + 4 * state.f32], grid, dim3(256), 0, st,
                      g, f, lg, s);
 }
 
@@ -1560,7 +1560,7 @@ void launch_tlm_particles(const GridDesc &g, const double *const *fields6, doubl
                                k_tlm_particles<false, true, false>,  k_tlm_particles<true, true, false>,
                                k_tlm_particles<false, false, true>,  k_tlm_particles<true, false, true>,
                                k_tlm_particles<false, true, true>,   k_tlm_particles<true, true, true>};
-  const int k = (pusher == 1) + 2 * (is_bunch != 0) + 4 * (state.cell != nullptr);
+  const int k = (pusher == 1) + 2 * (is_bunch != 0) + 4 * state.f32;
   hipLaunchKernelGGL(kernels[k], grid, dim3(256), 0, st, g, f, tf, tj, s);
 }
 

@@ -1248,9 +1248,15 @@ struct Checkpoint {
 
 constexpr int kCkComps = kRhoBunch + 1;
 
+// a species of the FP32 form has no native arrays until it is loaded; the loop
+// leaves it out, and so do checkpoints, snapshots and derivatives
+bool has_state(const Ctx &c, const Species &sp) { return sp.n_cap > 0 && (!is_f32(c) || sp.f32.cell); }
+
+// a species' kNative arrays and their bytes (0 without a state)
+constexpr int kNative = 6;
 std::vector<std::pair<void *, size_t>> native_arrays(Ctx &c, Species &sp) {
   std::vector<std::pair<void *, size_t>> out;
-  const size_t n = (size_t)sp.n_cap;
+  const size_t n = has_state(c, sp) ? (size_t)sp.n_cap : 0;
   if (is_f32(c)) {
     out.push_back({sp.f32.cell, n * sizeof(int32_t)});
     for (float *a : {sp.f32.fr, sp.f32.fz, sp.f32.vr, sp.f32.vphi, sp.f32.vz}) out.push_back({a, n * sizeof(float)});
@@ -1321,7 +1327,8 @@ int ckpt_restore(pdp3_ctx *ctx, const Checkpoint &ck) {
 // which no step changes, are the species' own
 StateRef state_ref(const Ctx &c, const Species &sp, void *const *arr) {
   StateRef s;
-  if (is_f32(c)) {
+  s.f32 = is_f32(c);
+  if (s.f32) {
     s.cell = (const uint32_t *)arr[0];
     s.fa = (const float *)arr[1];
     s.fb = (const float *)arr[2];
@@ -1340,7 +1347,6 @@ StateRef state_ref(const Ctx &c, const Species &sp, void *const *arr) {
   }
   return s;
 }
-constexpr int kNative = 6;  // arrays of native_arrays
 
 // the tangent-linear model carried along a forward sweep of the loop:
 // kTangentDirs directions of the particle weights; its grids are advanced by
@@ -1414,7 +1420,7 @@ struct TangentSweep {
     const double *f6[6] = {c.a[kER], c.a[kEPhi], c.a[kEZ], c.a[kHHR], c.a[kHHPhi], c.a[kHHZ]};
     for (int j = 0; j < (int)c.species.size(); j++) {
       Species &sp = c.species[j];
-      if (sp.n_cap <= 0) continue;
+      if (!has_state(c, sp)) continue;
       void *arr[kNative];
       auto native = native_arrays(c, sp);
       for (int a = 0; a < kNative; a++) arr[a] = native[a].first;
@@ -1648,6 +1654,7 @@ int adjoint_impl(pdp3_ctx *ctx, int nsteps, int checkpoint_every, int window_ste
       const double *f6[6] = {e, e + cells, e + 2 * cells, hh, hh + cells, hh + 2 * cells};
       for (int j = 0; j < nsp; j++) {
         Species &sp = c.species[j];
+        if (!has_state(c, sp)) continue;  // its adjoints stay 0
         launch_adj_particles(c.g, f6, lam, scaled, state_ref(c, sp, psnap[(size_t)t * nsp + j].data()), ls[j].data(),
                              ls[j][5], sp.charge, sp.mass, sp.n_cap, sp.kind == PDP3_SPECIES_BUNCH, c.pusher,
                              c.stream);

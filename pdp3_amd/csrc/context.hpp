@@ -299,8 +299,9 @@ void ens_launch_inject(const EnsInjectItem *items, int n_items, int max_count, c
                        hipStream_t st);
 void ens_launch_count(long long *step, hipStream_t st);
 
-// one species' state in slots, in either form (cell: nullptr in the FP64 form)
+// one species' state in slots, in the form of its context
 struct StateRef {
+  bool f32 = false;
   const double *r = nullptr, *z = nullptr, *vr = nullptr, *vphi = nullptr, *vz = nullptr, *w = nullptr;
   const uint8_t *alive = nullptr;
   const uint32_t *cell = nullptr;
