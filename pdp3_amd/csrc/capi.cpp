@@ -4,8 +4,6 @@
 #include "../../include/pdp3_hip.h"
 
 #include <hip/hip_runtime.h>
-#include <sys/mman.h>
-#include <unistd.h>
 
 #include <algorithm>
 #include <array>
@@ -16,7 +14,6 @@
 #include <new>
 #include <string>
 #include <functional>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -96,87 +93,10 @@ int upload_koef(pdp3_ctx *ctx) {
   return PDP3_OK;
 }
 
-// whether most of a host range's pages are in memory (mincore)
-bool resident(const void *p, size_t bytes) {
-  const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
-  const uintptr_t a = (uintptr_t)p & ~(page - 1), b = ((uintptr_t)p + bytes + page - 1) & ~(page - 1);
-  std::vector<unsigned char> vec((b - a) / page);
-  if (mincore((void *)a, b - a, vec.data()) != 0) return true;
-  size_t in = 0;
-  for (unsigned char v : vec) in += v & 1;
-  return 8 * in >= 7 * vec.size();
-}
-
-// Device memory to pageable host memory, complete on return.  The runtime pins
-// the destination for a copy like this, which is fast for memory in use (228 us
-// for 4.2 MB) but takes each page fault of fresh memory on the way: 1083 us for
-// a newly allocated 4.2 MB array, 8.7 ms for 34 MB.  Such a destination is
-// filled from pinned buffers, by several threads that share its page faults
-// (522 us, 3.9 ms).  Threads pay from 1 MiB; below kStageFrom the runtime's own
-// staging is used, and throughout where nothing may be allocated (stage false).
+// device memory to pageable host memory, complete on return; stage: see copy_to_host
 int to_host(pdp3_ctx *ctx, void *dst, const void *src, size_t bytes, bool stage = true) {
   Ctx &c = ctx->c;
-  constexpr size_t kStageFrom = 192 << 10, kSlot = 512 << 10, kThreadsFrom = 1 << 20;
-  constexpr int kThreads = 4;
-  HostStage &hs = c.stage;
-  const bool staged = stage && bytes >= kStageFrom && !resident(dst, bytes);
-  if (staged && !hs.mem) {
-    if (hipHostMalloc(&hs.mem, HostStage::kSlots * kSlot, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      hs.mem = nullptr;
-    }
-    for (int j = 0; hs.mem && j < HostStage::kSlots; j++)
-      if (hipEventCreateWithFlags(&hs.ev[j], hipEventDisableTiming) != hipSuccess) {
-        (void)hipGetLastError();
-        hs.free_all();
-      }
-  }
-  if (!staged || !hs.mem) {
-    HIP_TRY(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.stream));
-    HIP_TRY(ctx, hipStreamSynchronize(c.stream));
-    return PDP3_OK;
-  }
-  static_assert(HostStage::kSlots == 2 * kThreads, "two slots a thread");
-  const size_t chunks = (bytes + kSlot - 1) / kSlot;
-  const int nt = bytes >= kThreadsFrom ? kThreads : 1;
-  std::array<hipError_t, kThreads> err{};
-  // thread t copies chunks t, t + nt, ..: one on its way into a slot while the
-  // one before is copied out of the other
-  auto work = [&](int t, bool helper) {
-    hipError_t e = helper ? hipSetDevice(c.device) : hipSuccess;
-    auto issue = [&](size_t j, int s) {
-      const size_t at = j * kSlot;
-      if (e == hipSuccess)
-        e = hipMemcpyAsync((char *)hs.mem + (2 * t + s) * kSlot, (const char *)src + at, std::min(kSlot, bytes - at),
-                           hipMemcpyDeviceToHost, c.stream);
-      if (e == hipSuccess) e = hipEventRecord(hs.ev[2 * t + s], c.stream);
-    };
-    if ((size_t)t < chunks) issue(t, 0);
-    int s = 0;
-    for (size_t j = t; j < chunks; j += nt, s ^= 1) {
-      if (j + nt < chunks) issue(j + nt, s ^ 1);
-      if (e == hipSuccess) e = hipEventSynchronize(hs.ev[2 * t + s]);
-      if (e != hipSuccess) break;
-      const size_t at = j * kSlot;
-      std::memcpy((char *)dst + at, (char *)hs.mem + (2 * t + s) * kSlot, std::min(kSlot, bytes - at));
-    }
-    err[t] = e;
-  };
-  std::array<std::thread, kThreads> helpers;
-  int started = 1;
-  try {
-    for (; started < nt; started++) helpers[started] = std::thread(work, started, true);
-  } catch (const std::system_error &) {
-    // fewer threads than wanted: this one takes their shares
-  }
-  work(0, false);
-  for (int t = 1; t < started; t++) helpers[t].join();
-  for (int t = started; t < nt; t++) work(t, false);
-  for (hipError_t e : err)
-    if (e != hipSuccess) {
-      (void)hipStreamSynchronize(c.stream);  // no copy into the slots is left in flight
-      HIP_TRY(ctx, e);
-    }
+  HIP_TRY(ctx, copy_to_host(c.stage, c.device, c.stream, dst, src, bytes, stage));
   return PDP3_OK;
 }
 

@@ -8,6 +8,8 @@
 #include <string>
 #include <vector>
 
+#include "host_copy.hpp"
+
 namespace pdp3 {
 
 // constants, include/constant.h:10-27 (the reference's rounded SI values)
@@ -182,21 +184,6 @@ struct KernelTimer {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> pool;
   double total_ms = 0;
   long long launches = 0;
-};
-
-// pinned buffers for copies to the host, allocated by the first that needs them
-struct HostStage {
-  static constexpr int kSlots = 8;
-  void *mem = nullptr;
-  hipEvent_t ev[kSlots] = {};
-  void free_all() {
-    for (auto &e : ev) {
-      if (e) (void)hipEventDestroy(e);
-      e = nullptr;
-    }
-    if (mem) (void)hipHostFree(mem);
-    mem = nullptr;
-  }
 };
 
 struct Ctx {
