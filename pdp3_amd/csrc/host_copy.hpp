@@ -9,9 +9,7 @@
 #include <array>
 #include <cstdint>
 #include <cstring>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 namespace pdp3 {
 
@@ -47,15 +45,19 @@ struct HostStage {
   }
 };
 
-// whether most of a host range's pages are in memory (mincore)
+// whether most of a host range's pages are in memory (mincore, some pages at a time)
 inline bool resident(const void *p, size_t bytes) {
   const uintptr_t page = (uintptr_t)sysconf(_SC_PAGESIZE);
   const uintptr_t a = (uintptr_t)p & ~(page - 1), b = ((uintptr_t)p + bytes + page - 1) & ~(page - 1);
-  std::vector<unsigned char> vec((b - a) / page);
-  if (mincore((void *)a, b - a, vec.data()) != 0) return true;
+  const size_t pages = (b - a) / page;
+  std::array<unsigned char, 4096> vec;
   size_t in = 0;
-  for (unsigned char v : vec) in += v & 1;
-  return 8 * in >= 7 * vec.size();
+  for (size_t at = 0; at < pages; at += vec.size()) {
+    const size_t n = std::min(vec.size(), pages - at);
+    if (mincore((void *)(a + at * page), n * page, vec.data()) != 0) return true;
+    for (size_t j = 0; j < n; j++) in += vec[j] & 1;
+  }
+  return 8 * in >= 7 * pages;
 }
 
 // a device made current for a scope
@@ -105,8 +107,9 @@ inline hipError_t copy_staged(HostStage &hs, int device, hipStream_t stream, voi
   int started = 1;
   try {
     for (; started < nt; started++) helpers[started] = std::thread(work, started, true);
-  } catch (const std::system_error &) {
-    // fewer threads than wanted: this one takes their shares
+  } catch (...) {
+    // fewer threads than wanted (no thread or no memory for one): this one
+    // takes their shares
   }
   work(0, false);
   for (int t = 1; t < started; t++) helpers[t].join();

@@ -1,7 +1,7 @@
 """Host logic of the copies to the host (pdp3_amd/csrc/host_copy.hpp), on a fake
 HIP runtime of two devices (tests/native/fakehip): the copies through pinned
-slots work whatever the calling thread's current device is, and every failure
-of what they need ends in a plain copy."""
+slots work whatever the calling thread's current device is, every failure of
+what they need ends in a plain copy, and no exception leaves them."""
 import os
 import subprocess
 
@@ -21,7 +21,7 @@ def program(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["same_device", "other_device_current", "record_fails", "no_pinned_memory",
-                                  "no_threads"])
+                                  "no_threads", "no_host_memory"])
 def test_copy(program, case):
     r = subprocess.run([program, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (case, r.returncode, r.stderr)
