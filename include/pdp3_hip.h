@@ -255,15 +255,19 @@ int pdp3_density(pdp3_ctx *ctx, int index, double *out);
 /* tile shape of the FP32 particle kernel (no reference counterpart):
  * particles walked per lane (ppt, 4 / 8 / 16) and wavefronts per block
  * (waves); supported pairs: (16,4) (16,2) (16,1) (8,4) (8,2) (4,4).  The
- * FP64 form has one shape.  pdp3_autotune runs steps_per_candidate real steps
- * of the simulation with each shape, times the plasma kernel and keeps the
- * fastest (the steps advance the simulation; results differ between shapes
- * only by the order of FP64 sums).  Until one of the two is called, each
- * species runs on the shape that suits its size (down to 256 particles per
- * block, smaller than the shapes that can be set) and pdp3_get_tile returns
- * 16 x 4. */
+ * FP64 form has one shape.  Until pdp3_set_tile each species runs on the
+ * shape that suits its size (the automatic choice: down to 256 particles per
+ * block, smaller than the shapes that can be set).  pdp3_autotune runs
+ * 6 x steps_per_candidate real steps of the simulation, on the shapes that can
+ * be set and on the automatic choice (which takes the place of (16,2) unless it
+ * is one of the shapes), and keeps the fastest; ppt and waves are the fastest
+ * of the shapes, also where the automatic choice is kept.  Results differ
+ * between shapes only by the order of FP64 sums.  pdp3_get_tile returns the
+ * shape that was set or found ((16,4) at first), pdp3_species_tile the one that
+ * a plasma species' next step runs on. */
 int pdp3_set_tile(pdp3_ctx *ctx, int ppt, int waves);
 int pdp3_get_tile(const pdp3_ctx *ctx, int *ppt, int *waves);
+int pdp3_species_tile(const pdp3_ctx *ctx, int index, int *ppt, int *waves);
 int pdp3_autotune(pdp3_ctx *ctx, int steps_per_candidate, int *ppt, int *waves);
 
 /* ---- adjoint (no reference counterpart) ----
@@ -348,10 +352,12 @@ int pdp3_ensemble_step(pdp3_ensemble *e, int nsteps);
 int pdp3_ensemble_set_sort_interval(pdp3_ensemble *e, int sort_interval);
 /* device time of the stepped graphs since the last call (HIP events), and the step count */
 int pdp3_ensemble_timing(pdp3_ensemble *e, double *total_ms, long long *steps);
-/* tile shape of the ensemble's particle kernel, as pdp3_set_tile; the
- * autotuner times steps_per_candidate real steps per shape and keeps the fastest */
+/* tile shape of the ensemble's particle kernel, as pdp3_set_tile and
+ * pdp3_autotune (the automatic choice by each species' size is always a
+ * candidate of its own, in the place of (16,2)) */
 int pdp3_ensemble_set_tile(pdp3_ensemble *e, int ppt, int waves);
 int pdp3_ensemble_get_tile(const pdp3_ensemble *e, int *ppt, int *waves);
+int pdp3_ensemble_species_tile(const pdp3_ensemble *e, int member, int index, int *ppt, int *waves);
 int pdp3_ensemble_autotune(pdp3_ensemble *e, int steps_per_candidate, int *ppt, int *waves);
 
 /* live timing with HIP events on the context's stream (no reference

@@ -88,9 +88,11 @@ SIGNATURES = {
     "pdp3_ensemble_timing": (_I, [_P, _D, C.POINTER(C.c_longlong)]),
     "pdp3_ensemble_set_tile": (_I, [_P, _I, _I]),
     "pdp3_ensemble_get_tile": (_I, [_P, C.POINTER(_I), C.POINTER(_I)]),
+    "pdp3_ensemble_species_tile": (_I, [_P, _I, _I, C.POINTER(_I), C.POINTER(_I)]),
     "pdp3_ensemble_autotune": (_I, [_P, _I, C.POINTER(_I), C.POINTER(_I)]),
     "pdp3_set_tile": (_I, [_P, _I, _I]),
     "pdp3_get_tile": (_I, [_P, C.POINTER(_I), C.POINTER(_I)]),
+    "pdp3_species_tile": (_I, [_P, _I, C.POINTER(_I), C.POINTER(_I)]),
     "pdp3_autotune": (_I, [_P, _I, C.POINTER(_I), C.POINTER(_I)]),
     "pdp3_profile_enable": (_I, [_P, _I]),
     "pdp3_profile_get": (_I, [_P, _I, _D, C.POINTER(C.c_longlong)]),
@@ -366,8 +368,15 @@ class Simulation:
         self._chk(self.L.pdp3_get_tile(self.h, C.byref(a), C.byref(b)))
         return a.value, b.value
 
+    def species_tile(self, idx):
+        """(ppt, waves) that plasma species idx's next step runs on"""
+        a, b = _I(), _I()
+        self._chk(self.L.pdp3_species_tile(self.h, int(idx), C.byref(a), C.byref(b)))
+        return a.value, b.value
+
     def autotune(self, steps_per_candidate=2):
-        """Times real steps with every tile shape, keeps the fastest; returns (ppt, waves)."""
+        """Times real steps with the tile shapes and the automatic choice, keeps
+        the fastest; returns the fastest shape's (ppt, waves)."""
         a, b = _I(), _I()
         self._chk(self.L.pdp3_autotune(self.h, int(steps_per_candidate), C.byref(a), C.byref(b)))
         return a.value, b.value
@@ -457,6 +466,11 @@ class Ensemble:
     def tile(self):
         a, b = _I(), _I()
         self._chk(self.L.pdp3_ensemble_get_tile(self.h, C.byref(a), C.byref(b)))
+        return a.value, b.value
+
+    def species_tile(self, member, idx):
+        a, b = _I(), _I()
+        self._chk(self.L.pdp3_ensemble_species_tile(self.h, int(member), int(idx), C.byref(a), C.byref(b)))
         return a.value, b.value
 
     def autotune(self, steps_per_candidate=2):

@@ -131,6 +131,9 @@ void free_species(Species &sp) {
 }
 
 bool is_f32(const Ctx &c) { return c.precision == PDP3_PREC_FP32; }
+// a species of the FP32 form has no native arrays until it is loaded; the loop
+// leaves it out, and so do checkpoints, snapshots and derivatives
+bool has_state(const Ctx &c, const Species &sp) { return sp.n_cap > 0 && (!is_f32(c) || sp.f32.cell); }
 
 // FP64 arrays: the live state in the species' layout (n_cap slots) in the
 // FP64 form, a logical-order staging copy (n entries) in the FP32 form
@@ -168,7 +171,7 @@ struct TimedScope {
   int kernel;
   hipEvent_t a = nullptr, b = nullptr;
   TimedScope(Ctx &cc, int k) : c(cc), kernel(k) {
-    if (!c.profiling) return;
+    if (!(k == kTimerTune ? c.tuning : c.profiling)) return;
     KernelTimer &t = c.timers[kernel];
     if (!t.pool.empty()) {
       a = t.pool.back().first;
@@ -181,7 +184,7 @@ struct TimedScope {
     (void)hipEventRecord(a, c.stream);
   }
   ~TimedScope() {
-    if (!c.profiling || !a) return;
+    if (!a) return;
     (void)hipEventRecord(b, c.stream);
     c.timers[kernel].pending.emplace_back(a, b);
   }
@@ -193,6 +196,7 @@ void harvest_timers(Ctx &c) {
       float ms = 0;
       if (hipEventElapsedTime(&ms, ev.first, ev.second) == hipSuccess) {
         t.total_ms += ms;
+        t.min_ms = std::min(t.min_ms, (double)ms);
         t.launches++;
       }
       t.pool.push_back(ev);
@@ -1000,11 +1004,14 @@ int step_one(pdp3_ctx *ctx, const std::function<int()> *after_h) {
   if (after_h && (st = (*after_h)())) return st;
   // (live timing keeps plasma and bunch launches apart)
   for (Species &sp : c.species) sp.steps_unsorted++;
-  if (!c.profiling && (is_f32(c) ? launch_group_f32(c) : launch_group_f64(c))) {
-    CHECK_LAUNCH(ctx);
-  } else {
-    for (int j : c.order)
-      if ((st = particles_fused(ctx, c.species[j]))) return st;
+  {
+    TimedScope ts(c, kTimerTune);
+    if (!c.profiling && (is_f32(c) ? launch_group_f32(c) : launch_group_f64(c))) {
+      CHECK_LAUNCH(ctx);
+    } else {
+      for (int j : c.order)
+        if ((st = particles_fused(ctx, c.species[j]))) return st;
+    }
   }
   if ((st = pdp3_efield_calc(ctx))) return st;
   c.current_time = c.current_time + c.g.dt;  // src/loadInitParam.cpp:586
@@ -1084,34 +1091,68 @@ int pdp3_get_tile(const pdp3_ctx *ctx, int *ppt, int *waves) {
   return PDP3_OK;
 }
 
+int pdp3_species_tile(const pdp3_ctx *ctx, int index, int *ppt, int *waves) {
+  if (!ctx || index < 0 || index >= (int)ctx->c.species.size()) return PDP3_ERR_BAD_ARG;
+  const Ctx &c = ctx->c;
+  const Species &sp = c.species[index];
+  if (sp.kind != PDP3_SPECIES_PLASMA) return PDP3_ERR_BAD_ARG;
+  const int t = !is_f32(c) ? kNumTiles + 1 : c.tile_auto ? auto_tile(c, sp) : c.tile;
+  if (ppt) *ppt = kTileShapes[t][0];
+  if (waves) *waves = kTileShapes[t][1];
+  return PDP3_OK;
+}
+
+namespace {
+// the settable shape that all plasma species of the loop take by their sizes, else -1
+int common_auto_tile(const Ctx &c) {
+  int tile = -1;
+  for (const Species &sp : c.species) {
+    if (sp.kind != PDP3_SPECIES_PLASMA || !has_state(c, sp)) continue;
+    const int t = auto_tile(c, sp);
+    if (t >= kNumTiles || (tile >= 0 && t != tile)) return -1;
+    tile = t;
+  }
+  return tile;
+}
+constexpr int kAutoSlot = 1;  // 16 x 2: never the fastest (see auto_tile's table)
+}  // namespace
+
 int pdp3_autotune(pdp3_ctx *ctx, int steps_per_candidate, int *ppt, int *waves) {
   if (!ctx || steps_per_candidate < 1) return PDP3_ERR_BAD_ARG;
   Ctx &c = ctx->c;
   if (!is_f32(c)) return pdp3_get_tile(ctx, ppt, waves);  // one tile shape in the FP64 form
-  // each candidate times real steps of the simulation on the plasma kernel
-  const bool was_profiling = c.profiling;
-  KernelTimer saved = c.timers[PDP3_KERNEL_PARTICLES];
-  int st, best = 0;
-  double best_ms = 1e300;
-  c.tile_auto = false;
-  for (int t = 0; t < kNumTiles; t++) {
-    c.tile = t;
-    c.profiling = true;
-    if ((st = check_device_errors(ctx))) break;
-    c.timers[PDP3_KERNEL_PARTICLES].total_ms = 0;
-    c.timers[PDP3_KERNEL_PARTICLES].launches = 0;
-    if ((st = pdp3_step(ctx, steps_per_candidate))) break;
-    if ((st = check_device_errors(ctx))) break;
-    const double ms = c.timers[PDP3_KERNEL_PARTICLES].total_ms;
+  // each candidate times real steps of the simulation, launched as any step
+  // is; the automatic choice is one of the candidates, in the place of a
+  // settable shape unless it is itself one of them
+  const bool was_profiling = c.profiling, was_auto = c.tile_auto;
+  const int was_tile = c.tile, own = common_auto_tile(c);
+  int st = PDP3_OK, best = 0;
+  double best_ms = 1e300, auto_ms = 1e300;
+  c.profiling = false;
+  c.tuning = true;
+  KernelTimer &timer = c.timers[kTimerTune];
+  auto measure = [&](int tile, bool automatic, double *ms) {
+    c.tile = tile;
+    c.tile_auto = automatic;
+    if ((st = check_device_errors(ctx))) return;
+    timer.min_ms = 1e300;
+    if ((st = pdp3_step(ctx, steps_per_candidate))) return;
+    *ms = timer.min_ms;
+  };
+  if (own < 0) measure(c.tile, true, &auto_ms);
+  for (int t = 0; !st && t < kNumTiles; t++) {
+    if (own < 0 && t == kAutoSlot) continue;
+    double ms = 1e300;
+    measure(t, false, &ms);
     if (ms < best_ms) {
       best_ms = ms;
       best = t;
     }
   }
-  c.tile = best;
+  c.tuning = false;
   c.profiling = was_profiling;
-  c.timers[PDP3_KERNEL_PARTICLES].total_ms = saved.total_ms;
-  c.timers[PDP3_KERNEL_PARTICLES].launches = saved.launches;
+  c.tile = st ? was_tile : best;
+  c.tile_auto = st ? was_auto : auto_ms < best_ms || best == own;
   if (st) return st;
   return pdp3_get_tile(ctx, ppt, waves);
 }
@@ -1167,10 +1208,6 @@ struct Checkpoint {
 };
 
 constexpr int kCkComps = kRhoBunch + 1;
-
-// a species of the FP32 form has no native arrays until it is loaded; the loop
-// leaves it out, and so do checkpoints, snapshots and derivatives
-bool has_state(const Ctx &c, const Species &sp) { return sp.n_cap > 0 && (!is_f32(c) || sp.f32.cell); }
 
 // a species' kNative arrays and their bytes (0 without a state)
 constexpr int kNative = 6;
@@ -1688,11 +1725,13 @@ void ens_drop_graph(pdp3_ensemble *e) {
   e->graph_list = -1;
 }
 
+int ens_particle_list(const pdp3_ensemble *e) { return e->tile_auto ? ens_auto_list(e->banded) : e->tile; }
+
 // one loop iteration of every instance (src/loadInitParam.cpp:471-587; the
 // bunch injections of init_beam from the device tables), captured once per
 // tile shape and replayed
 int ens_graph(pdp3_ensemble *e) {
-  const int list = e->tile_auto ? ens_auto_list(e->banded) : e->tile;
+  const int list = ens_particle_list(e);
   if (e->exec && e->graph_list == list) return PDP3_OK;
   ens_drop_graph(e);
   ENS_HIP(e, hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
@@ -1947,24 +1986,42 @@ int pdp3_ensemble_get_tile(const pdp3_ensemble *e, int *ppt, int *waves) {
   return PDP3_OK;
 }
 
+int pdp3_ensemble_species_tile(const pdp3_ensemble *e, int member, int index, int *ppt, int *waves) {
+  if (!e || member < 0 || member >= (int)e->cs.size()) return PDP3_ERR_BAD_ARG;
+  const Ctx &c = *e->cs[member];
+  if (index < 0 || index >= (int)c.species.size() || c.species[index].kind != PDP3_SPECIES_PLASMA)
+    return PDP3_ERR_BAD_ARG;
+  const int list = ens_particle_list(e);
+  if (ppt) *ppt = 1 << ens_lg(c, c.species[index], list);
+  if (waves) *waves = list < kNumTiles ? kTileShapes[list][1] : kWavesPerBlock;
+  return PDP3_OK;
+}
+
 int pdp3_ensemble_autotune(pdp3_ensemble *e, int steps_per_candidate, int *ppt, int *waves) {
   if (!e || steps_per_candidate < 1) return PDP3_ERR_BAD_ARG;
-  double saved_ms = e->timed_ms;
-  long long saved_steps = e->timed_steps;
+  const double saved_ms = e->timed_ms;
+  const long long saved_steps = e->timed_steps;
+  const bool was_auto = e->tile_auto;
+  const int was_tile = e->tile;
   int best = 0, st = PDP3_OK;
-  double best_ms = 1e300;
-  e->tile_auto = false;
-  for (int t = 0; t < kNumTiles; t++) {
-    e->tile = t;
+  double best_ms = 1e300, auto_ms = 1e300;
+  // the tiles by size are the first candidate, in the place of 16 x 2
+  for (int t = -1; !st && t < kNumTiles; t++) {
+    if (t == kAutoSlot) continue;
+    e->tile_auto = t < 0;
+    e->tile = std::max(t, 0);
     e->timed_ms = 0;
     e->timed_steps = 0;
     if ((st = pdp3_ensemble_step(e, steps_per_candidate))) break;
-    if (e->timed_ms < best_ms) {
+    if (t < 0) {
+      auto_ms = e->timed_ms;
+    } else if (e->timed_ms < best_ms) {
       best_ms = e->timed_ms;
       best = t;
     }
   }
-  e->tile = best;
+  e->tile = st ? was_tile : best;
+  e->tile_auto = st ? was_auto : auto_ms < best_ms;
   e->timed_ms = saved_ms;
   e->timed_steps = saved_steps;
   if (st) return st;

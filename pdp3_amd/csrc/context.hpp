@@ -74,9 +74,10 @@ __host__ __device__ __forceinline__ long long logical_of(long long p) {
 }
 
 // tile shapes of the FP32 particle kernel: particles per lane (PPT) and waves
-// per block; the autotuner picks one per context
+// per block.  The first kNumTiles can be set; the last two are small tiles that
+// only the automatic choice takes
 constexpr int kNumTiles = 6;
-constexpr int kTileShapes[kNumTiles][2] = {{16, 4}, {16, 2}, {16, 1}, {8, 4}, {8, 2}, {4, 4}};
+constexpr int kTileShapes[kNumTiles + 2][2] = {{16, 4}, {16, 2}, {16, 1}, {8, 4}, {8, 2}, {4, 4}, {2, 4}, {1, 4}};
 
 // Which slots of a chunked species a block of WAVES wavefronts walks with PPT
 // particles per lane.  A tile is kParticles consecutive logical particles: a
@@ -182,9 +183,11 @@ struct Species {
 struct KernelTimer {
   std::vector<std::pair<hipEvent_t, hipEvent_t>> pending;
   std::vector<std::pair<hipEvent_t, hipEvent_t>> pool;
-  double total_ms = 0;
+  double total_ms = 0, min_ms = 1e300;
   long long launches = 0;
 };
+// a timer of the autotuner's own, behind those of the PDP3_KERNEL_* classes
+constexpr int kTimerTune = 5;
 
 struct Ctx {
   GridDesc g{};
@@ -205,7 +208,8 @@ struct Ctx {
   int *err_host = nullptr; // pinned mirror
   std::string last_error;
   bool profiling = false;
-  KernelTimer timers[5];
+  bool tuning = false;  // the particle launches of a step are timed together (kTimerTune)
+  KernelTimer timers[kTimerTune + 1];
   int sort_interval = 0;
   // tile shape of the FP32 particle kernel (index into kTileShapes); until it
   // is set or autotuned each species runs on the shape that suits its size
@@ -267,6 +271,8 @@ void ens_particles_free(EnsParticles *e);
 // the work list of a settable tile shape (index into kTileShapes), or of tiles
 // by the size of each species (ens_auto_list; banded: the ensemble has sorted)
 int ens_auto_list(bool banded);
+// particles per lane (2^lg) of a plasma species' tiles in a work list
+int ens_lg(const Ctx &c, const Species &sp, int list);
 void ens_launch_particles(EnsParticles *e, int list, hipStream_t st);
 // bunch injection of an ensemble (Bunch::bunch_inject, src/bunch.cpp:87-124)
 // driven by a device step counter: per (instance, bunch) pair a table of the
@@ -343,7 +349,7 @@ void launch_bunch_inject_f64(Ctx &c, Species &sp, unsigned start, unsigned count
 // FP32 form
 void launch_fused_f32(Ctx &c, Species &sp);
 bool launch_group_f32(Ctx &c);  // as launch_group_f64
-int auto_tile(const Ctx &c, const Species &sp);  // kTileShapes index, or 6 / 7: 2 / 1 particles per lane x 4
+int auto_tile(const Ctx &c, const Species &sp);  // kTileShapes index
 void launch_charge_weighting_f32(Ctx &c, Species &sp, double *rho = nullptr);
 void launch_bunch_inject_f32(Ctx &c, Species &sp, unsigned start, unsigned count, double dl);
 bool launch_f32_from_f64(Ctx &c, Species &sp);  // pack absolute FP64 state into cell form

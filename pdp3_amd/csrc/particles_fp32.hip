@@ -1415,10 +1415,21 @@ int ens_auto_lg(const Ctx &c, const Species &sp, bool banded) {
   while (lg > 0 && (256 << lg) * cells > rows * (kFK - 4) * (double)sp.n) lg--;
   return lg;
 }
+}  // namespace
+
+int ens_lg(const Ctx &c, const Species &sp, int list) {
+  if (list >= kNumTiles) return ens_auto_lg(c, sp, list == kNumTiles + 1);
+  int lg = 0;
+  while ((1 << lg) < kTileShapes[list][0]) lg++;
+  if (sp.n < (long long)kSparsePpc * (c.g.nr - 1) * (c.g.nz - 1))
+    while ((kTileShapes[list][1] * 64 << lg) > kChunk) lg--;
+  return lg;
+}
+
+namespace {
 std::vector<EnsItem> ens_list(const std::vector<Ctx *> &ctxs, int list) {
   std::vector<EnsItem> items, tiles;
-  const bool set = list < kNumTiles;
-  const int waves = set ? kTileShapes[list][1] : kWavesPerBlock;
+  const int waves = list < kNumTiles ? kTileShapes[list][1] : kWavesPerBlock;
   int a = 0;
   for (Ctx *cp : ctxs) {
     Ctx &c = *cp;
@@ -1429,11 +1440,7 @@ std::vector<EnsItem> ens_list(const std::vector<Ctx *> &ctxs, int list) {
       if (!sp.chunked) {
         for (long long b = 0; b < sp.n_cap; b += waves * 64) items.push_back(EnsItem{a, -1, b, sp.n_cap});
       } else {
-        int lg = 0;
-        while (set && (1 << lg) < kTileShapes[list][0]) lg++;
-        if (!set) lg = ens_auto_lg(c, sp, list == kNumTiles + 1);
-        if (set && sp.n < (long long)kSparsePpc * (c.g.nr - 1) * (c.g.nz - 1))
-          while ((waves * 64 << lg) > kChunk) lg--;
+        const int lg = ens_lg(c, sp, list);
         const long long tile = (long long)waves * 64 << lg;
         for (long long t = 0; t * tile < sp.n_cap; t++) {
           // TileMap::base

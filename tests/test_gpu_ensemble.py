@@ -202,3 +202,26 @@ def test_ensemble_injected_bunches(sort_interval):
             assert sa["alive"].sum() > 0
             for k in ("r", "z", "vr", "vphi", "vz"):
                 assert normwise(sm[k], sa[k]) <= 1e-10, (j, k)
+
+
+def test_ensemble_autotune_keeps_the_automatic_choice():
+    """Members of 1 and 40 particles per cell: tiles by each member's size are
+    faster than any one shape (the sparse member's tiles overrun every set
+    shape's boxes), and the autotuner keeps them; six times the steps, as ever."""
+    from pdp3_amd import capi
+    from pdp3_amd import workloads as wl
+
+    insts = [wl.Instance(cells_r=64, cells_z=4096, ppc=1, density=1e17, bunch_ratio=0.1, seed=5, bunch_macro=100),
+             wl.Instance(cells_r=64, cells_z=1024, ppc=40, density=1e17, bunch_ratio=0.1, seed=6, bunch_macro=100)]
+    members = [wl.build_instance(i) for i in insts]
+    ens = capi.Ensemble(members)
+    automatic = [ens.species_tile(m, 0) for m in range(2)]
+    assert automatic[0][0] < automatic[1][0]
+    t0 = members[0].time
+    best = ens.autotune(8)
+    assert abs(members[0].time - t0 - 48 * members[0].dt) <= 1e-6 * members[0].dt
+    assert best in [(16, 4), (16, 1), (8, 4), (8, 2), (4, 4)] and ens.tile() == best
+    assert [ens.species_tile(m, 0) for m in range(2)] == automatic
+    ens.set_tile(8, 2)
+    assert ens.species_tile(1, 0) == (8, 2)
+    ens.close()
