@@ -1205,6 +1205,7 @@ struct Checkpoint {
   int next_bunch = 0;
   std::vector<int> order;
   std::vector<char> created;
+  std::vector<long long> unsorted;
 };
 
 constexpr int kCkComps = kRhoBunch + 1;
@@ -1260,7 +1261,11 @@ int ckpt_save(pdp3_ctx *ctx, Checkpoint &ck) {
   ck.next_bunch = c.next_bunch;
   ck.order = c.order;
   ck.created.clear();
-  for (auto &sp : c.species) ck.created.push_back(sp.created ? 1 : 0);
+  ck.unsorted.clear();
+  for (auto &sp : c.species) {
+    ck.created.push_back(sp.created ? 1 : 0);
+    ck.unsorted.push_back(sp.steps_unsorted);
+  }
   return PDP3_OK;
 }
 
@@ -1276,7 +1281,10 @@ int ckpt_restore(pdp3_ctx *ctx, const Checkpoint &ck) {
   c.steps_done = ck.steps;
   c.next_bunch = ck.next_bunch;
   c.order = ck.order;
-  for (size_t j = 0; j < c.species.size(); j++) c.species[j].created = ck.created[j] != 0;
+  for (size_t j = 0; j < c.species.size(); j++) {
+    c.species[j].created = ck.created[j] != 0;
+    c.species[j].steps_unsorted = ck.unsorted[j];
+  }
   return PDP3_OK;
 }
 

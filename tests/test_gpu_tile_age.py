@@ -1,0 +1,34 @@
+"""The order that the automatic tile choice takes a plasma species to be in: in
+order when loaded so and after a sort, out of order after 500 steps without one.
+1.64e6 particles at 10 per cell run on 4 x 4 tiles in order, 2 x 4 out of it."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CR, CZ, PPC, D = 160, 1024, 10, 5e-4
+ORDERED, UNORDERED = (4, 4), (2, 4)
+
+
+def _sim(load=True):
+    from pdp3_amd import capi
+
+    sim = capi.Simulation(CR + 1, CZ + 1, CR * D, CZ * D, 0.5 * D / 3e8, precision=capi.PREC_FP32)
+    sim.boundary_conditions()
+    idx = sim.add_species(-1, 1.0, PPC * CR * CZ)
+    if load:
+        sim.init_uniform(idx, 3, PPC, 1e12, 0, 1.0)
+    return sim
+
+
+def test_adjoint_replays_do_not_age():
+    """The adjoint's replayed steps are no steps of the run: 300 steps and a
+    gradient over 150 leave the species 450 steps old."""
+    sim = _sim()
+    sim.step(300)
+    sim.adjoint_run(150, 50, 10, 0.2, 0.3)
+    assert sim.species_tile(0) == ORDERED
+    sim.step(51)
+    assert sim.species_tile(0) == UNORDERED
+    sim.sort()
+    assert sim.species_tile(0) == ORDERED
+    sim.close()
