@@ -1950,6 +1950,7 @@ int pdp3_ensemble_step(pdp3_ensemble *e, int nsteps) {
     for (Ctx *c : e->cs) {
       c->current_time = c->current_time + c->g.dt;  // src/loadInitParam.cpp:586
       c->steps_done++;
+      for (Species &sp : c->species) sp.steps_unsorted++;
     }
     e->steps_done++;
     // close the timed interval before a sort (which runs outside the graph)

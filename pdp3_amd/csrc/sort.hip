@@ -919,6 +919,7 @@ int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream) 
     void **bp[7] = {(void **)&b.cell, (void **)&b.fr, (void **)&b.fz, (void **)&b.vr, (void **)&b.vphi,
                     (void **)&b.vz, (void **)&b.w};
     for (int k = 0; k < 7; k++) std::swap(*ap[k], *bp[k]);
+    e.second->steps_unsorted = 0;
   }
   return 0;
 }

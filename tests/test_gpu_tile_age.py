@@ -32,3 +32,20 @@ def test_adjoint_replays_do_not_age():
     sim.sort()
     assert sim.species_tile(0) == ORDERED
     sim.close()
+
+
+def test_ensemble_steps_age_and_sorts_renew():
+    """Steps and sorts of an ensemble count as a single run's."""
+    from pdp3_amd import capi
+
+    for interval, want in ((0, UNORDERED), (300, ORDERED)):
+        sims = [_sim(), _sim()]
+        ens = capi.Ensemble(sims)
+        ens.set_sort_interval(interval)
+        ens.step(400)
+        assert [s.species_tile(0) for s in sims] == [ORDERED, ORDERED]
+        ens.step(101)
+        ens.close()
+        assert [s.species_tile(0) for s in sims] == [want, want]
+        for s in sims:
+            s.close()
