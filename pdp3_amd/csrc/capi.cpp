@@ -210,6 +210,7 @@ int check_device_errors(pdp3_ctx *ctx) {
   HIP_TRY(ctx, hipMemcpyAsync(c.err_host, c.err, sizeof(int), hipMemcpyDeviceToHost, c.stream));
   HIP_TRY(ctx, hipStreamSynchronize(c.stream));
   harvest_timers(c);
+  for (Species &sp : c.species) settle_sort(sp);
   int e = *c.err_host;
   if (e) {
     HIP_TRY(ctx, hipMemsetAsync(c.err, 0, sizeof(int), c.stream));
@@ -1758,6 +1759,7 @@ int ens_graph(pdp3_ensemble *e) {
 
 int ens_check(pdp3_ensemble *e) {
   ENS_HIP(e, hipStreamSynchronize(e->stream));
+  if (e->ms.counted) settle_sort_multi(e->ms, e->cs);
   for (pdp3_ctx *ctx : e->ctxs) {
     int st = check_device_errors(ctx);
     if (st) return efail(e, st, std::string("instance: ") + ctx->c.last_error);

@@ -172,6 +172,10 @@ struct Species {
   uint32_t *runs_host = nullptr;
   hipEvent_t runs_ev = nullptr;
   long long steps_unsorted = 0;  // steps since it was created or sorted
+  // the last sort, while it is not known whether it found room for its records
+  // (it is skipped where it did not): steps_unsorted before it, else -1
+  long long unsorted_before = -1;
+  long long sort_cap = 0;
   bool sort_prepared = false;  // the buffers of periodic sorts are allocated
   // bunch
   double *inject_u = nullptr;
@@ -406,6 +410,7 @@ struct MultiSort {
   uint32_t *runs_host = nullptr;       // pinned: the previous sort's run count
   hipEvent_t runs_ev = nullptr;
   bool counted = false;
+  long long sort_cap = 0;              // record space of the last sort
   std::vector<MultiSeg> seg_host;      // the table's source (kept for the asynchronous copy)
 };
 // sort the plasma species of the given contexts in one launch sequence on
@@ -413,6 +418,10 @@ struct MultiSort {
 // swaps each species' arrays with its second buffer.  0, -1 (a species not
 // in whole chunks), -3 (allocation or HIP error)
 int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream);
+// after a sort whose run count has arrived: a skipped sort leaves its species'
+// steps_unsorted as if it had not been
+void settle_sort(Species &sp);
+void settle_sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs);
 void sort_multi_free(MultiSort &ms);
 size_t sort_periodic_bytes(const Ctx &c);
 int sort_shrink_ws(Ctx &c, size_t need);

@@ -710,6 +710,19 @@ int sort_prepare(Ctx &c, Species &sp) {
   return 0;
 }
 
+void settle_sort(Species &sp) {
+  if (sp.unsorted_before >= 0 && sp.runs_host && (long long)*sp.runs_host > sp.sort_cap) sp.steps_unsorted += sp.unsorted_before;
+  sp.unsorted_before = -1;
+}
+
+void settle_sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs) {
+  for (Ctx *c : cs)
+    for (Species &sp : c->species) {
+      if (sp.unsorted_before >= 0 && (long long)*ms.runs_host > ms.sort_cap) sp.steps_unsorted += sp.unsorted_before;
+      sp.unsorted_before = -1;
+    }
+}
+
 int sort_species(Ctx &c, Species &sp, bool exact) {
   const long long n = sp.n_cap;
   if (!sortable(c, sp)) return 0;
@@ -722,6 +735,7 @@ int sort_species(Ctx &c, Species &sp, bool exact) {
   const bool first = !sp.runs_host;
   if (!ensure_runs(sp)) return -3;
   if (!first && hipEventSynchronize(sp.runs_ev) != hipSuccess) return -3;
+  settle_sort(sp);
   const long long last = *sp.runs_host;
   long long cap = sp.rec_cap > 0 ? sp.rec_cap : std::min(n, n / 4 + 65536);
   if (4 * last > 3 * cap) cap = std::min(n, 2 * last + 65536);
@@ -730,6 +744,8 @@ int sort_species(Ctx &c, Species &sp, bool exact) {
   const SortWs ws = sort_ws(n, cap, bits);
   const long long nb = ws.nb, scratch = ws.scratch;
   if (!ensure_ws(c, ws.bytes) || !ensure_alts(c, sp)) return -3;
+  sp.unsorted_before = exact ? -1 : sp.steps_unsorted;
+  sp.sort_cap = cap;
   sp.steps_unsorted = 0;
   uint32_t *src = (uint32_t *)c.sort_ws, *block = src + n, *tmp = block + nb + 1;
   uint32_t *rk = tmp + scratch, *ri = rk + cap, *rk2 = ri + cap, *ri2 = rk2 + cap, *rlen = ri2 + cap;
@@ -868,6 +884,7 @@ int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream) 
   // previous copy from seg_host has completed (the last sort's run-count
   // event, waited for below or above, comes after it on the stream)
   if (ms.counted && hipEventSynchronize(ms.runs_ev) != hipSuccess) return -3;
+  if (ms.counted) settle_sort_multi(ms, cs);
   ms.seg_host = segs;
   if (hipMemcpyAsync(ms.seg, ms.seg_host.data(), segs.size() * sizeof(MultiSeg), hipMemcpyHostToDevice, stream) !=
       hipSuccess)
@@ -883,7 +900,7 @@ int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream) 
   const long long last = ms.counted ? (long long)*ms.runs_host : 0;
   long long cap = ms.rec_cap > 0 ? ms.rec_cap : std::min(n, n / 4 + 65536);
   if (4 * last > 3 * cap) cap = std::min(n, 2 * last + 65536);
-  ms.rec_cap = cap;
+  ms.rec_cap = ms.sort_cap = cap;
   const SortWs ws = sort_ws(n, cap, bits);
   if (ms.ws_bytes < ws.bytes) {
     if (ms.ws) (void)hipFree(ms.ws);
@@ -919,6 +936,7 @@ int sort_multi(MultiSort &ms, const std::vector<Ctx *> &cs, hipStream_t stream) 
     void **bp[7] = {(void **)&b.cell, (void **)&b.fr, (void **)&b.fz, (void **)&b.vr, (void **)&b.vphi,
                     (void **)&b.vz, (void **)&b.w};
     for (int k = 0; k < 7; k++) std::swap(*ap[k], *bp[k]);
+    e.second->unsorted_before = e.second->steps_unsorted;
     e.second->steps_unsorted = 0;
   }
   return 0;
