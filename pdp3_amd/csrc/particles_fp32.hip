@@ -807,35 +807,33 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
   fused32_tile<WAVES>(q, g, Map(), Map::base(blockIdx.x), n_cap, box, fbox);
 }
 
-// bunches (plain layout): the same walk, the box anchored at the smallest
-// living cell of the block
-// one block of a bunch (plain layout): WAVES chunks of kChunk slots from
-// `base`; the register / LDS sink is anchored at the smallest cell of the
-// block's living particles (a bunch block is a thin disc injected in one step)
+// one block of a bunch (plain layout): WAVES x 64 x PPT slots from `base`; the
+// box takes the shape that suits the cells of the block's living particles
+// (bunch_init)
 template <int WAVES, int PPT, class Fields = GlobalFields>
 __device__ __forceinline__ void fused32_bunch_tile(const F32Args &p, const GlobalSink &gs, long long base,
                                                    long long n_cap, double *box) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long long cbase = base + (long long)wave * (64 * PPT) + lane;
-  int ai = 0x7fffffff, ak = 0x7fffffff;
+  int i0 = 0x7fffffff, k0 = 0x7fffffff, i1 = -1, k1 = -1;
   for (int j = 0; j < PPT; j++) {
     long long n = cbase + (long long)j * 64;
     if (n < n_cap) {
       uint32_t c = p.cell[n];
       if (!(c & kDead)) {
-        ai = min(ai, cell_i(c));
-        ak = min(ak, cell_k(c));
+        const int i = cell_i(c), k = cell_k(c);
+        i0 = min(i0, i);
+        k0 = min(k0, k);
+        i1 = max(i1, i);
+        k1 = max(k1, k);
       }
     }
   }
-  block_min2(ai, ak);
-  if (ai == 0x7fffffff) return;  // no living particle in the block (uniform over the block)
   // (neighbouring slots of a bunch are not in one cell: register sums help
   // only where a lane walks several)
   using Sink = typename std::conditional<PPT == 1, BunchSinkOne, BunchSink>::type;
   Sink sk;
-  box_init(box, ai, ak, Sink::kK, sk, gs);
-  __syncthreads();
+  if (!bunch_init<WAVES>(box, i0, k0, i1, k1, sk, gs)) return;
   const F32Args q = from_slot(p, base);
   const unsigned lim = (unsigned)min(n_cap - base, (long long)WAVES * 64 * PPT);
   const unsigned off0 = (unsigned)(wave * 64 * PPT + lane);

@@ -736,8 +736,8 @@ k_fused_tiled(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_ca
   fused_tile(g, f, gs, s, n_cap, pusher, blockIdx.x, box);
 }
 
-// bunches (plain layout): the same with the box anchored at the smallest
-// living cell of the block, PPT particles per lane (the lanes of a wave on
+// bunches (plain layout): the same with the box in the shape that suits the
+// block's cells (bunch_init), PPT particles per lane (the lanes of a wave on
 // neighbouring slots): a bunch's block covers many cells, and the adding of its
 // box to the grid is shared by more particles where there are enough of them
 template <int PPT>
@@ -745,19 +745,19 @@ __device__ __forceinline__ void fused_bunch(const GridDesc &g, const Fields &f, 
                                             const SpeciesArgs &s, long long n_cap, int pusher, long long block,
                                             double *box) {
   const long long first = block * (kWavesPerBlock * 64 * PPT) + threadIdx.x;
-  int ai = 0x7fffffff, ak = 0x7fffffff;
+  int i0 = 0x7fffffff, k0 = 0x7fffffff, i1 = -1, k1 = -1;
   for (int j = 0; j < PPT; j++) {
     const long long p = first + j * (kWavesPerBlock * 64);
     if (p < n_cap && s.alive[p] == 1) {
-      ai = min(ai, max(0, cell_r(g, s.r[p])));
-      ak = min(ak, max(0, cell_z(g, s.z[p])));
+      const int i = max(0, cell_r(g, s.r[p])), k = max(0, cell_z(g, s.z[p]));
+      i0 = min(i0, i);
+      k0 = min(k0, k);
+      i1 = max(i1, i);
+      k1 = max(k1, k);
     }
   }
-  block_min2(ai, ak);
-  if (ai == 0x7fffffff) return;
   BunchSinkOne sk;
-  box_init(box, ai, ak, BunchSinkOne::kK, sk, gs);
-  __syncthreads();
+  if (!bunch_init<kWavesPerBlock>(box, i0, k0, i1, k1, sk, gs)) return;
 #pragma nounroll
   for (int j = 0; j < PPT; j++) {
     const long long p = first + j * (kWavesPerBlock * 64);

@@ -61,20 +61,22 @@ struct GlobalSink {
 };
 
 // BR x BK nodes per component; the plasma box spans 4 rows (i0-1 .. i0+2) by
-// 128 columns (a sorted block covers a run of cells along one row), the bunch
-// box 16 rows by 32 columns (a bunch block is a thin disc of particles
-// injected in the same step)
+// 128 columns (a sorted block covers a run of cells along one row).  A bunch
+// block is a thin disc of particles injected in the same step: its box has
+// BR x BK nodes in 16, 32 or 64 rows (bunch_init)
 // ACC: the first level; without it (lanes that hold one particle) every
 // contribution goes to the box at once: 8 LDS atomics where the registers'
 // stencil takes 12, and no setting up of the registers
 template <bool RHO, int BR = 4, int BK = 128, bool ACC = true>
 struct TileSinkT {
+  static constexpr bool kBunch = RHO;
   static constexpr int kComps = RHO ? 4 : 3;  // rho only where it is deposited
   static constexpr int kR = BR, kK = BK, kSize = kComps * BR * BK;
   GlobalSink g;
   double *box;  // LDS, kComps x kR x kK
   int bi, bk;   // node coordinates of box[.][0][0]
   int bw;       // columns of the box in use (a multiple of the wavefront or kK)
+  int shift;    // bunches: log2 of the box's columns
   int ic, kc;   // cell of the register accumulator
   // scalar accumulators (no arrays: a runtime index would push them to scratch)
   double p00, p10, p01, p11;  // J_phi corners (ic+di, kc+dk)
@@ -82,33 +84,42 @@ struct TileSinkT {
   double z0, z1;              // J_z at (ic, kc), (ic+1, kc)
   double x0, x1;              // J_r at (ic, kc), (ic, kc+1)
 
+  // a node past the box.  (Zeros, such as the J_phi of a bunch without v_phi, a
+  // third of its atomics, are left out, as flush leaves them out.)
+  __device__ __forceinline__ void past_put(int comp, int i, int k, double v) {
+    if (ACC || v != 0.0) g.put(comp, i, k, v);
+  }
+  __device__ __forceinline__ int rows() const { return RHO ? (BR * BK) >> shift : BR; }
+  __device__ __forceinline__ int stride() const { return RHO ? 1 << shift : BK; }
+  __device__ __forceinline__ double *at(int li, int lk) const { return box + (RHO ? li << shift : li * BK) + lk; }
   // whole stencils at once: one bounds check and atomics at fixed offsets; the
   // nodes of one that leaves the box go to HBM, in a loop (one copy of put)
   template <int C>
   __device__ __forceinline__ void box_put2(int i, int k, double v0, double v1) {
     const int li = i - bi, lk = k - bk;
-    if ((unsigned)li < (unsigned)(BR - (C == kCZ)) && (unsigned)lk < (unsigned)(bw - (C != kCZ))) {
-      double *q = box + (C * BR + li) * BK + lk;
+    if ((unsigned)li < (unsigned)(rows() - (C == kCZ)) && (unsigned)lk < (unsigned)(bw - (C != kCZ))) {
+      double *q = at(li, lk) + C * BR * BK;
       atomicAdd(q, v0);
-      atomicAdd(q + (C == kCZ ? BK : 1), v1);
+      atomicAdd(q + (C == kCZ ? stride() : 1), v1);
       return;
     }
 #pragma nounroll
-    for (int n = 0; n < 2; n++) g.put(C, i + (C == kCZ ? n : 0), k + (C == kCZ ? 0 : n), n ? v1 : v0);
+    for (int n = 0; n < 2; n++) past_put(C, i + (C == kCZ ? n : 0), k + (C == kCZ ? 0 : n), n ? v1 : v0);
   }
   template <int C>
   __device__ __forceinline__ void box_put4(int i, int k, double v00, double v10, double v01, double v11) {
     const int li = i - bi, lk = k - bk;
-    if ((unsigned)li < (unsigned)(BR - 1) && (unsigned)lk < (unsigned)(bw - 1)) {
-      double *q = box + (C * BR + li) * BK + lk;
+    if ((unsigned)li < (unsigned)(rows() - 1) && (unsigned)lk < (unsigned)(bw - 1)) {
+      double *q = at(li, lk) + C * BR * BK;
       atomicAdd(q, v00);
-      atomicAdd(q + BK, v10);
+      atomicAdd(q + stride(), v10);
       atomicAdd(q + 1, v01);
-      atomicAdd(q + BK + 1, v11);
+      atomicAdd(q + stride() + 1, v11);
       return;
     }
 #pragma nounroll
-    for (int n = 0; n < 4; n++) g.put(C, i + (n & 1), k + (n >> 1), n < 2 ? (n ? v10 : v00) : (n == 2 ? v01 : v11));
+    for (int n = 0; n < 4; n++)
+      past_put(C, i + (n & 1), k + (n >> 1), n < 2 ? (n ? v10 : v00) : (n == 2 ? v01 : v11));
   }
   // whole stencils: straight into the accumulators when they are centred on
   // the accumulator's cell (the common case: no select chains), else the box
@@ -148,21 +159,22 @@ struct TileSinkT {
   __device__ __forceinline__ void flush() {
     if (!ACC || ic < 0) return;
     const int li = ic - bi, lk = kc - bk;
-    if ((unsigned)li < (unsigned)(BR - 1) && (unsigned)lk < (unsigned)(bw - 1)) {
-      double *q = box + li * BK + lk;
+    if ((unsigned)li < (unsigned)(rows() - 1) && (unsigned)lk < (unsigned)(bw - 1)) {
+      double *q = at(li, lk);
       constexpr int C = BR * BK;
+      const int BS = stride();
       atomicAdd(q + kCPhi * C, p00);
-      atomicAdd(q + kCPhi * C + BK, p10);
+      atomicAdd(q + kCPhi * C + BS, p10);
       atomicAdd(q + kCPhi * C + 1, p01);
-      atomicAdd(q + kCPhi * C + BK + 1, p11);
+      atomicAdd(q + kCPhi * C + BS + 1, p11);
       if (RHO) {
         atomicAdd(q + kCRho * C, r00);
-        atomicAdd(q + kCRho * C + BK, r10);
+        atomicAdd(q + kCRho * C + BS, r10);
         atomicAdd(q + kCRho * C + 1, r01);
-        atomicAdd(q + kCRho * C + BK + 1, r11);
+        atomicAdd(q + kCRho * C + BS + 1, r11);
       }
       atomicAdd(q + kCZ * C, z0);
-      atomicAdd(q + kCZ * C + BK, z1);
+      atomicAdd(q + kCZ * C + BS, z1);
       atomicAdd(q + kCR * C, x0);
       atomicAdd(q + kCR * C + 1, x1);
     } else {
@@ -297,13 +309,14 @@ __device__ __forceinline__ void tile_anchor(const bool (&live)[3], const int (&i
 
 // block prologue: anchor the box one row and two columns below the given
 // cell (the tile's anchor, or a bunch block's smallest cell) and clear its
-// first `width` columns
+// first `width` columns (bunch_init has cleared a bunch's)
 template <class T>
 __device__ __forceinline__ void box_init(double *box, int anchor_i, int anchor_k, int width, T &s,
                                          const GlobalSink &g) {
-  constexpr int kRow = T::kK < 64 ? T::kK : 64;  // columns cleared or added at a time
-  for (int t = threadIdx.x / kRow; t < T::kComps * T::kR; t += blockDim.x / kRow)
-    for (int c = threadIdx.x % kRow; c < width; c += kRow) box[t * T::kK + c] = 0.0;
+  if (!T::kBunch) {
+    for (int t = threadIdx.x / 64; t < T::kComps * T::kR; t += blockDim.x / 64)
+      for (int c = threadIdx.x % 64; c < width; c += 64) box[t * T::kK + c] = 0.0;
+  }
   s.g = g;
   s.box = box;
   s.bi = anchor_i - 1;
@@ -319,9 +332,18 @@ __device__ __forceinline__ void box_init(double *box, int anchor_i, int anchor_k
 // block epilogue: add the box to the grid (after __syncthreads)
 template <class T>
 __device__ __forceinline__ void box_flush(const double *box, const T &s) {
-  constexpr int kRow = T::kK < 64 ? T::kK : 64;
-  for (int t = threadIdx.x / kRow; t < T::kComps * T::kR; t += blockDim.x / kRow)
-    for (int c = threadIdx.x % kRow; c < s.bw; c += kRow) {
+  if (T::kBunch) {
+    constexpr int kPlane = T::kR * T::kK;
+    for (int t = threadIdx.x; t < T::kSize; t += blockDim.x) {
+      const double v = box[t];
+      if (v == 0.0) continue;
+      const int n = t % kPlane;
+      s.g.put(t / kPlane, s.bi + (n >> s.shift), s.bk + (n & (s.bw - 1)), v);
+    }
+    return;
+  }
+  for (int t = threadIdx.x / 64; t < T::kComps * T::kR; t += blockDim.x / 64)
+    for (int c = threadIdx.x % 64; c < s.bw; c += 64) {
       const double v = box[t * T::kK + c];
       if (v == 0.0) continue;
       const int comp = t / T::kR;
@@ -352,6 +374,54 @@ __device__ __forceinline__ void block_min2(int &i, int &k) {
     i = min(i, mi[w]);
     k = min(k, mk[w]);
   }
+}
+
+// block prologue of a bunch: the box lies one row and two columns below the
+// smallest cell of the block's living particles, in the shape (16 x 32, 32 x 16,
+// 64 x 8 nodes) that covers the most of the cells up to the largest, three rows
+// and four columns of it being margins.  (i, k), (i1, k1): the thread's smallest
+// and largest cell (INT_MAX, -1: none living); false: none lives in the block.
+// Particles past a 16 x 32 box alone made a bunch of 20 rows, in the order of
+// injection, a chain of grid atomics: 1e5 and 1e6 particles 185 and 1880 us
+// (FP64; 173 and 1957 in FP32), 20 and 94 us (16 and 75) in its own shape; of four
+// rows 19 and 94 us as before.  The choice is scalar arithmetic after one barrier.
+template <int WAVES, class T>
+__device__ __forceinline__ bool bunch_init(double *box, int i, int k, int i1, int k1, T &s, const GlobalSink &g) {
+  // the block's extent: minima of i, k, ~i1 and ~k1
+  __shared__ int part[4][WAVES];
+  int m[4] = {i, k, ~i1, ~k1};
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int j = 0; j < 4; j++) m[j] = min(m[j], __shfl_xor(m[j], off));
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int j = 0; j < 4; j++) part[j][threadIdx.x >> 6] = m[j];
+  for (int t = threadIdx.x; t < T::kSize; t += blockDim.x) box[t] = 0.0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+#pragma unroll
+    for (int w = 0; w < WAVES; w++) m[j] = min(m[j], part[j][w]);
+    m[j] = __builtin_amdgcn_readfirstlane(m[j]);
+  }
+  if (m[0] == 0x7fffffff) return false;
+  const int ni = ~m[2] - m[0] + 1, nk = ~m[3] - m[1] + 1;
+  constexpr int kNodes = T::kR * T::kK;
+  s.shift = 5;
+  if (ni > T::kR - 3) {
+    int best = 0;
+#pragma unroll
+    for (int t = 5; t >= 3; t--) {
+      const int cells = min(ni, (kNodes >> t) - 3) * min(nk, (1 << t) - 4);
+      if (cells > best) {
+        best = cells;
+        s.shift = t;
+      }
+    }
+  }
+  static_assert(T::kBunch && T::kK == 32, "the first shape");
+  box_init(box, m[0], m[1], 1 << s.shift, s, g);
+  return true;
 }
 
 // the cell that a plasma block's boxes are centred on: the median of nine of its
