@@ -972,7 +972,7 @@ struct TlmSink {
   __device__ __forceinline__ void put(int comp, int d, int node, int i, int k, double v) {
     if (node >= 0) {
       atomicAdd(box + (comp * kDN + d) * kR * kK + node, v);
-    } else if (node == -1) {
+    } else if (node == -1 && v != 0.0) {  // 0 along directions that do not reach the particle
       double *J = comp == kAR ? j.jr[d] : comp == kAPhi ? j.jphi[d] : j.jz[d];
       unsafeAtomicAdd(J + (size_t)i * (size_t)g->nz + (size_t)k, v);
     }
