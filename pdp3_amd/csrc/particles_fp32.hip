@@ -1004,14 +1004,6 @@ k_ens_fused32(const F32Args *__restrict__ args, const GlobalSink *__restrict__ s
   }
 }
 
-// plain layout (bunches): one particle per thread, deposits straight to HBM
-__global__ void __launch_bounds__(256) k_fused32_plain(F32Args p, GlobalSink gs, long long n_cap) {
-  const long long base = (long long)blockIdx.x * blockDim.x;
-  if (base + threadIdx.x >= n_cap) return;
-  GlobalSink sk = gs;
-  step_particle32(from_slot(p, base), sk, GlobalFields(), threadIdx.x);
-}
-
 __global__ void k_charge32(F32Args p, GlobalSink gs, long long n_cap) {
   const long long n = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (n >= n_cap) return;
@@ -1021,7 +1013,7 @@ __global__ void k_charge32(F32Args p, GlobalSink gs, long long n_cap) {
   deposit_rho(p, sk, p.w[n], cell_i(c), p.fa[n], cell_k(c), p.fb[n]);
 }
 
-// plasma species: tiles of the chunked layout (the plain kernel's four global
+// plasma species: tiles of the chunked layout (k_charge32's four global
 // atomics a particle, 20 of them on each node, took 401 us for 1.05e7
 // particles)
 template <int PPT>

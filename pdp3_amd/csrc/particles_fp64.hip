@@ -816,15 +816,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
     fused_tile(g, f, gs, s, a.n_cap, pusher, block, box);
 }
 
-// plain layout, one particle per thread, deposits straight to HBM
-__global__ void __launch_bounds__(256) k_fused_plain(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s,
-                                                     long long n_cap, int pusher, int want_rho) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_cap) return;
-  GlobalSink sk = gs;
-  step_particle(g, f, sk, gs.err, s, pusher, want_rho != 0, i);
-}
-
 __global__ void __launch_bounds__(256) k_step_v(GridDesc g, Fields f, int *err, SpeciesArgs s, long long n_cap,
                                                 int pusher) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
