@@ -84,10 +84,10 @@ struct TileSinkT {
   double z0, z1;              // J_z at (ic, kc), (ic+1, kc)
   double x0, x1;              // J_r at (ic, kc), (ic, kc+1)
 
-  // a node past the box.  (Zeros, such as the J_phi of a bunch without v_phi, a
-  // third of its atomics, are left out, as flush leaves them out.)
+  // a node past the box.  (A bunch's zeros, such as the J_phi of one without v_phi,
+  // a third of its atomics, are left out, as flush leaves them out.)
   __device__ __forceinline__ void past_put(int comp, int i, int k, double v) {
-    if (ACC || v != 0.0) g.put(comp, i, k, v);
+    if (ACC || !RHO || v != 0.0) g.put(comp, i, k, v);
   }
   __device__ __forceinline__ int rows() const { return RHO ? (BR * BK) >> shift : BR; }
   __device__ __forceinline__ int stride() const { return RHO ? 1 << shift : BK; }
