@@ -39,7 +39,7 @@ BYTES_PER_PARTICLE = {"fp32": 52.0, "fp64": 90.0}
 BYTES_PER_CELL = 72.0
 
 
-AUTOTUNE_STEPS = 12  # 6 tile shapes x 2 steps
+AUTOTUNE_STEPS = 12  # 6 candidates x 2 steps
 
 
 def run_form(wl, capi, w, precision, steps, warmup, sort_interval):
@@ -48,10 +48,11 @@ def run_form(wl, capi, w, precision, steps, warmup, sort_interval):
     sim.step(warmup)
     sim.sync()
     # the library's autotuner picks the tile shape of the FP32 particle kernel
-    # (AUTOTUNE_STEPS real steps: 2 per shape); the FP64 form has one shape and
+    # (AUTOTUNE_STEPS real steps: 2 per candidate); the FP64 form has one shape and
     # takes the same steps, so that both forms are compared at one time
     if precision == capi.PREC_FP32:
-        tile = list(sim.autotune(AUTOTUNE_STEPS // 6))
+        sim.autotune(AUTOTUNE_STEPS // 6)
+        tile = list(sim.species_tile(0))
     else:
         tile = None
         sim.step(AUTOTUNE_STEPS)
@@ -251,7 +252,7 @@ def traffic_from_profile(name):
 def bench_ensemble(a):
     """cfg4: 128 independent instances (per-instance grid, density, ppc, bunch
     ratio drawn from the seed), FP32 form, one graph replay per step with one
-    particle launch; the tile shape picked by the autotuner."""
+    particle launch; the tiles picked by the autotuner."""
     from pdp3_amd import capi
     from pdp3_amd import workloads as wl
 
@@ -262,13 +263,14 @@ def bench_ensemble(a):
     sims = [wl.build_instance(i, injected=not a.loaded_bunches) for i in insts]
     ens = capi.Ensemble(sims)
     ens.set_sort_interval(a.sort_interval)
-    tile = ens.autotune(1)
+    ens.autotune(1)
     ens.step(a.warmup)
     ens.timing()
     t0 = time.perf_counter()
     ens.step(a.steps)
     t1 = time.perf_counter()
     dev_ms, n = ens.timing()
+    tiles = sorted({ens.species_tile(m, 0) for m in range(len(sims))}, reverse=True)
     value = n_part * a.steps / (t1 - t0)
     out = {
         "metric": "particle-steps/s (ensemble, FP32 form)", "value": value, "unit": "particle-steps/s",
@@ -277,7 +279,8 @@ def bench_ensemble(a):
         "config": {"workload": f"cfg4: {len(insts)} r-z instances, r cells in 64/128/256 x z cells in "
                                f"512..4096, 5..40 ppc, densities 1e16..1e18, Gaussian bunches "
                                f"{'loaded at t = 0' if a.loaded_bunches else 'injected over 6 sigma_z / v'}",
-                   "particles": n_part, "cells": cells, "tile_ppt_waves": list(tile),
+                   "particles": n_part, "cells": cells,
+                   "tile_ppt_waves": [list(t) for t in tiles] if len(tiles) > 1 else list(tiles[0]),
                    "sort_interval": a.sort_interval},
         "device_ms_per_step": dev_ms / max(n, 1),
         "roofline": {"bound": "hbm", "achieved": (n_part * BYTES_PER_PARTICLE["fp32"] + cells * 304.0)

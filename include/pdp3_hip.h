@@ -284,7 +284,12 @@ int pdp3_autotune(pdp3_ctx *ctx, int steps_per_candidate, int *ppt, int *waves);
  * context's own forward trajectory: FP32 or FP64 form), with checkpoints of
  * the full state every checkpoint_every steps and recomputation between
  * them.  The context ends in the forward end state.  Requires
- * sort_interval 0 (a fixed particle order). */
+ * sort_interval 0 (a fixed particle order).  A species that was added and not
+ * loaded has no state: its derivatives are 0.
+ * Device memory: the checkpoints, one segment's states and the adjoint fields and
+ * particles.  Where that is at most 1 GiB the context keeps it for its next run,
+ * until it is destroyed (each member of a batch its own); more is given back at
+ * the end of the call. */
 int pdp3_adjoint_run(pdp3_ctx *ctx, int nsteps, int checkpoint_every, int window_steps, double z_lo,
                      double z_hi, double *phi_out, double *const *dphi_dw);
 
@@ -321,8 +326,8 @@ int pdp3_adjoint_tangent_run(pdp3_ctx *ctx, int nsteps, int checkpoint_every, in
  * the device.  Member m writes phi_out[m] and dphi_dw[m][j] (species j, as
  * pdp3_adjoint_run; dphi_dw or dphi_dw[m] may be NULL); status_out[m]
  * (may be NULL) receives its status, the return value is the first nonzero
- * one.  Every member holds its own checkpoints at once; a context may appear
- * only once. */
+ * one.  Every member holds its own checkpoints at once, and afterwards what
+ * pdp3_adjoint_run keeps; a context may appear only once. */
 int pdp3_adjoint_run_batch(pdp3_ctx *const *ctxs, int n, int nsteps, int checkpoint_every, int window_steps,
                            double z_lo, double z_hi, double *phi_out, double *const *const *dphi_dw,
                            int *status_out);
@@ -333,9 +338,9 @@ int pdp3_objective_run(pdp3_ctx *ctx, int nsteps, int window_steps, double z_lo,
 /* ---- ensembles (no reference counterpart) ----
  * Independent instances (contexts set up with the calls above: any grid,
  * PML, plasma, loaded bunches; FP32 form, one common delta_t) advanced
- * together: per step one graph replay with an H launch, a J / rho reset, ONE
- * particle launch over the plasma tiles and bunch blocks of every instance,
- * and an E launch.  The contexts stay owned by the caller and must not be
+ * together: per step one graph replay with an H launch, which also resets J and
+ * rho, ONE particle launch over the plasma tiles and bunch blocks of every
+ * instance, and an E launch.  The contexts stay owned by the caller and must not be
  * stepped on their own while the ensemble lives; their clocks advance with
  * the ensemble.  Bunches may be loaded (pdp3_bunch_add_loaded) or injected
  * (pdp3_bunch_add): the injections run inside the graph from a device step

@@ -196,9 +196,10 @@ __device__ __forceinline__ void block_anchor(int &i, int &k, bool live) {
 // quotients by the context's constants and row volumes take their reciprocals
 // from the context (div_cr: correctly rounded, as the IEEE division): a quotient
 // is five FP64 operations instead of eleven and a quarter-rate reciprocal, and the
-// particle steps, bound by FP64 instructions at two waves per SIMD (211 VGPRs; three
-// spill 40 and take 290 us), had about fifty of them: reverse step of 2.6e6
-// particles 238 us with the IEEE quotients, 213 us
+// particle steps, bound by their instructions at two waves per SIMD (211 VGPRs; three
+// spill 40 and take 290 us; the reverse step 1743 vector instructions a particle, 976
+// of them FP64), had about fifty of them: reverse step of 2.6e6 particles 238 us with
+// the IEEE quotients, 213 us
 __device__ __forceinline__ double per_dr(const GridDesc &g, double x) { return div_cr(x, g.dr, g.inv_dr); }
 __device__ __forceinline__ double per_dz(const GridDesc &g, double x) { return div_cr(x, g.dz, g.inv_dz); }
 __device__ __forceinline__ double per_c2(double x) { return div_cr(x, kC2, 1.0 / kC2); }
@@ -479,10 +480,9 @@ __device__ __forceinline__ Gathered gather_grad(const GridDesc &g, const double 
 }
 
 // the adjoints of the gathered fields of one block's particles are summed in
-// an LDS box of kR x kABK nodes per component (anchored one row and two
-// columns below the block's smallest cell) and added to the grid once per
-// block; stencils outside the box go to the grid directly.  A plasma block
-// lies along one row.  A bunch block spans the bunch's radius: in four rows
+// an LDS box of kR x kABK nodes per component (block_anchor) and added to the
+// grid once per block; stencils outside the box go to the grid directly.  A plasma
+// block lies along one row.  A bunch block spans the bunch's radius: in four rows
 // most of its 24 atomics a particle went to the same few grid nodes, and 6.4e4
 // bunch particles took as long as 2.6e6 plasma particles (330 us).
 constexpr int kABK = 64, kABComp = 6;
@@ -953,9 +953,8 @@ struct TlmSpecies {
 
 // deposit tangents: every contribution v at node (i, k) adds its derivative
 // part (one per direction) to the tangent J grids, through an LDS box of kR x
-// kK nodes per component and direction for the nodes around the block's
-// smallest cell (a particle's 48 global atomics, those of a bunch all on the
-// same few nodes, were most of the kernel)
+// kK nodes per component and direction (block_anchor; a particle's 48 global
+// atomics, those of a bunch all on the same few nodes, were most of the kernel)
 template <bool BUNCH>
 struct TlmSink {
   static constexpr int kR = BUNCH ? 16 : 6, kK = BUNCH ? 32 : 64, kSize = 3 * kDN * kR * kK;

@@ -112,7 +112,8 @@ struct TileMap {
 };
 
 // the same map with the particles per lane known at run time only (2^lg): one
-// kernel then serves tiles of every size in one launch
+// kernel then serves tiles of every size in one launch (the small ones fill boxes
+// too: it has one walk)
 template <int WAVES>
 struct TileMapRt {
   static constexpr bool kShort = false;

@@ -160,8 +160,11 @@ __device__ __forceinline__ float gather(const F32Args &p, const double *__restri
 // from HBM / L2 per particle; BoxFields serves the particles of a cell-sorted
 // block from an LDS copy (converted to FP32 once per node) of the nodes their
 // cells can touch, and falls back to HBM for the rest.  Both evaluate the same
-// FP32 expression on the same FP32-rounded node values, so the result does not
-// depend on the source.
+// FP32 expression on the same FP32-rounded node values; the result does not
+// depend on the source but for H_z, which the tiles (BoxFields, TileGlobalFields)
+// and an ensemble's bunches interpolate in another order than a single run's
+// bunches (GlobalFields).  So a bunch particle alone and in an ensemble may differ
+// by the rounding of its H_z; the orders are those that either has had all along.
 // the two table entries of row i (the host builds p.rows with the same FP64
 // expressions, so both give the same FP32 values)
 __device__ __forceinline__ void row_entries(int i, float4 &t0, float4 &t1) {
@@ -927,7 +930,7 @@ __device__ __forceinline__ GlobalSink from_global(const GlobalSinkG &g) {
 
 // The species of one simulation in one launch: where none of them fills the
 // GPU a launch is bound by the latency of its blocks (a 1e3-particle bunch
-// takes 9.6 us beside a 1.6e5-particle plasma's 15), and they overlap.
+// takes 11.0 us, a 1.6e5-particle plasma 11.3, both in one launch 12.1).
 // first[s]: the first block of species s; the bunches come first, their
 // blocks (one particle per lane, global gathers) take the longest.
 struct F32Group {
@@ -1258,10 +1261,13 @@ void launch_tile(int tile, hipStream_t st, const F32Args &p, const GlobalSink &g
 //   2.1e7 particles, 40 per cell:  529    499    516    556    580
 // A species that has not been sorted for kDrift steps runs on the shapes without
 // boxes whatever its size: its particles have drifted off the rows and columns
-// that the larger tiles' boxes hold (1 eV, 10-step passes: 4e6
-// particles at 20 per cell 2.0 ms in order on 4x4 and 2.2 on 2x4, 5.6 and 2.5
+// that the larger tiles' boxes hold (1 eV, steps of half a cell at c, 10-step passes:
+// 4e6 particles at 20 per cell 2.0 ms in order on 4x4 and 2.2 on 2x4, 5.6 and 2.5
 // after 2000 steps; two species of 1.35e7 at 45 per cell 4.8 on 8x4 and 5.8, 14.2
-// and 6.5; the lines cross after about 400 and 800 steps).
+// and 6.5; the lines cross after about 400 and 800 steps).  A hotter plasma drifts
+// off sooner: the count of steps is late for it, and no worse than one shape for
+// all.  Loaded in no order the shapes do not matter (2.1e7: 7514 and 7506 us): the
+// deposits wait for the grid.
 constexpr long long kDrift = 500;
 int auto_tile(const Ctx &c, const Species &sp) {
   const double cells = (double)(c.g.nr - 1) * (c.g.nz - 1);

@@ -709,10 +709,10 @@ __device__ __forceinline__ void step_particle(const GridDesc &g, const Fields &f
 }
 
 // chunked plasma species: one particle per lane, a block on 256 consecutive
-// logical particles (TileMap), deposits through a box around their median cell.  The kernel is
-// bound by FP64 instructions (about 1500 a particle, of which 17 divisions, 7
-// square roots and 2 logarithms).  At 128 VGPRs four waves per SIMD run: 6318 us
-// for 1.0e8 particles at 50 per cell, 1302 us for 2.1e7 at 40.  Lanes that walk
+// logical particles (TileMap), deposits through a box around their median cell.  The
+// kernel is bound by its instructions: 1570 vector instructions a particle, 912 of
+// them FP64 and 21 of these reciprocals and roots, one every 5.3 cycles of a SIMD.
+// At 128 VGPRs four waves per SIMD run: 6318 us for 1.0e8 particles at 50 per cell, 1302 us for 2.1e7 at 40.  Lanes that walk
 // 16 or 8 particles each and sum a cell's deposits in registers need 167 VGPRs
 // (three waves: 6968 and 1470 us).
 __device__ __forceinline__ void fused_tile(const GridDesc &g, const Fields &f, const GlobalSink &gs,
@@ -776,8 +776,8 @@ k_fused_bunch(GridDesc g, Fields f, GlobalSink gs, SpeciesArgs s, long long n_ca
 
 // The species of one simulation in one launch, one particle per lane: where
 // none of them fills the GPU a launch is bound by the latency of its blocks (a
-// 1e3-particle bunch takes 14 us beside a 1.6e5-particle plasma's 22), and they
-// overlap.  first[s]: the first block of species s.  The pointers are in the
+// 1e3-particle bunch takes 12.6 us, a 1.6e5-particle plasma 18.9, both in one
+// launch 18.9).  first[s]: the first block of species s.  The pointers are in the
 // global address space (SpeciesArgs read from an array would have generic ones).
 template <class T>
 using gptr = __attribute__((address_space(1))) T *;

@@ -2,19 +2,20 @@
 // and the bunch rho, all FP64).
 //
 // GlobalSink: bounds-checked hardware FP64 atomics straight to HBM (used by
-// the split entry points and by bunches, whose particles are not sorted).
+// the split entry points and for the charge of bunches).
 //
-// TileSink: three levels, for cell-sorted particles walked by one lane in
-// runs of the same cell:
+// TileSinkT: three levels, for particles walked by one lane in runs of the same
+// cell:
 //   1. registers: the contributions of the current cell (ic, kc) to its
 //      J_phi / rho corners (ic..ic+1, kc..kc+1), J_z nodes (ic..ic+1, kc) and
 //      J_r nodes (ic, kc..kc+1) are summed in FP64 registers and flushed only
 //      when the lane moves to a particle in another cell;
-//   2. an LDS box of kBoxR x kBoxK nodes per component anchored at the
-//      block's first particle, filled with LDS FP64 atomics;
+//   2. an LDS box of nodes around the block's cells (tile_anchor, tall_init,
+//      bunch_init), filled with LDS FP64 atomics;
 //   3. nodes outside the box go to GlobalSink.
 // After the block the box is added to HBM once (one atomic per touched node).
-// Small tiles, of one or two particles per lane, leave out the first level.
+// Small tiles, of one or two particles per lane, and the bunches whose lanes hold
+// one leave out the first level, the FP64 kernels altogether.
 #pragma once
 
 #include "context.hpp"
